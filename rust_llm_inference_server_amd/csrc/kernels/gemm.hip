@@ -2,7 +2,8 @@
 // reference's Linear holds them: crates/model/src/layers.rs:17-19, 65-69, 82).
 //
 //  * gemm_plain: any sizes, float32 accumulation with ordinary FMAs (no matrix-core
-//    shortcut), operands float32 or bfloat16.  This is the product of the true 32-bit path.
+//    shortcut), operands float32 or bfloat16.  Float32 throughout with K in steps of four goes to
+//    gemm_f32.hip instead.
 //  * gemm_bf16_mfma: bfloat16 operands on the matrix cores (v_mfma_f32_32x32x16_bf16),
 //    float32 accumulation, output bfloat16 or float32.  K must be a multiple of 8.
 //  * gemm_bf16_skinny: the decode shape, up to 64 rows of x.  Each weight row is read once

@@ -775,7 +775,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
            partials: bool = False) -> torch.Tensor:
     """``x @ w.T`` for ``x (T, K)`` and ``w (N, K)``, float32 accumulation.
 
-    A float32 weight (or float32 ``x``) takes the plain FMA kernel, the true 32-bit product.
+    Float32 throughout takes the 32-bit kernels on the matrix cores' 32-bit form (K and strides
+    multiples of 4; the same bits for a row whichever rows share the call); other sizes, and a
+    float32 weight or ``x`` beside bfloat16, the plain FMA kernel.
     bfloat16 operands take the streaming kernel up to 16 rows; more rows go to the library's
     GEMM (hipBLASLt, through its own entry points), or with ``BF16_GEMM = "own"`` to the skinny
     kernel up to 64 rows and the hand-written matrix-core GEMM beyond.
@@ -843,6 +845,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         name = "rlis_gemm_bf16_skinny" if T <= SKINNY_MAX_ROWS else "rlis_gemm_bf16_mfma"
         lib.call(name, x.data_ptr(), w.data_ptr(), y.data_ptr(), _DT[out_dtype], T, N, K, ldx,
                  ldw, N, stream)
+    elif (x.dtype == w.dtype == out_dtype == torch.float32 and K % 4 == 0 and ldx % 4 == 0
+          and ldw % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+        lib.call("rlis_gemm_f32", x.data_ptr(), w.data_ptr(), y.data_ptr(), T, N, K, ldx, ldw, N,
+                 stream)
     else:
         lib.call("rlis_gemm_plain", x.data_ptr(), _dt(x), w.data_ptr(), _dt(w), y.data_ptr(),
                  _DT[out_dtype], T, N, K, ldx, ldw, N, stream)

@@ -152,6 +152,33 @@ def test_linear_float32(ops, T, N, K):
     torch.testing.assert_close(ops.linear(x, w), want, atol=2e-5, rtol=1e-5)
 
 
+@pytest.mark.parametrize("N,K", [(3, 4), (331, 172), (64, 320), (65, 2048), (130, 2052), (33, 3104),
+                                 (2048, 3072), (20, 8200), (48, 14336), (17000, 64)])
+def test_linear_float32_same_bits_for_any_number_of_rows(ops, N, K):
+    """The 32-bit product's kernels (up to 16 and 32 rows, tiles of 64 x 32 and 64 x 64 with k whole,
+    in halves and in quarters; runs of k whole and cut): within the bound of a sum of float32
+    products, K / 64 + 19 roundings of 2^-24 on any way through (a run of K / 16 in steps of four,
+    the sums of four runs and four parts), and the same bits for a row whichever rows share the
+    call, x strided or not."""
+    rows = (1, 15, 16, 17, 32, 33, 64, 65, 129, 300)
+    base = rnd(max(rows), K + 8, seed=1)
+    x, w = base[:, :K], rnd(N, K, seed=2)
+    want = x.double() @ w.double().t()
+    bound = (K / 64 + 19) * 2.0 ** -24 * 4 * (x.double().abs() @ w.double().abs().t())
+    full = ops.linear(x, w)
+    assert bool(((full.double() - want).abs() <= bound).all())
+    for T in rows:
+        assert torch.equal(ops.linear(x[:T], w), full[:T]), T
+        assert torch.equal(ops.linear(x[:T].contiguous(), w), full[:T]), T
+    # infinities and NaN stay in their rows, also beside a k that is cut
+    bad = x[:40].clone()
+    bad[3, K - 1], bad[20, 0] = float("inf"), float("nan")
+    got = ops.linear(bad, w)
+    keep = [i for i in range(40) if i not in (3, 20)]
+    assert torch.equal(got[keep], full[:40][keep])
+    assert bool(torch.isnan(got[20]).all()) and not bool(torch.isfinite(got[3]).any())
+
+
 @pytest.mark.parametrize("out_dtype", DTYPES)
 @pytest.mark.parametrize("T,N,K", [(1, 2048, 2048), (1, 331, 104), (8, 3072, 2048), (16, 100, 64),
                                    (2, 2048, 8192), (7, 2049, 14336), (3, 128256, 2048), (4, 7, 520),
