@@ -55,6 +55,7 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
   // reads row 0 instead and is not stored: no load stands under a condition, so that the
   // compiler can count the loads in flight and wait for the oldest tile alone.
   constexpr int cols_per_tile = GATED ? TR / 2 : TR;
+// (non-temporal, as in the kernel for up to 16 rows)
 #define RLIS_WIDE_LOAD_TILE(a, tile_)                                                           \
   {                                                                                             \
     const int tl_ = (tile_);                                                                    \
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
       const int c = GATED ? (2 * p) % cols_per_tile : 2 * p;   /* column within the tile */     \
       const long long up = (GATED && 2 * p >= cols_per_tile) ? (long long)N * sh.ldw : 0;       \
       GlobalBf16 ptr = col0 + c < N ? w_tile + (long long)c * sh.ldw + up : w_lane;             \
-      const Bits4 v_ = *(GlobalU4)ptr;                                                          \
+      const Bits4 v_ = __builtin_nontemporal_load((GlobalU4)ptr);                               \
       a[p].x = v_.x;            /* member by member: a struct copy would go through scratch */  \
       a[p].y = v_.y;                                                                            \
       a[p].z = v_.z;                                                                            \
