@@ -656,7 +656,7 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     bfloat16 it is the split-k kernel's partial sums added in order (the library's products with
     a float32 result are slow at such row counts: 25 us against 6 + 3 for 64 x 2,048 x 2,048);
     otherwise ``linear(x, w, float32)``."""
-    if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 \
+    if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and not _rows_kernel(x, w) \
             and STREAM_MAX_ROWS < x.shape[0] <= SPLITK_MAX_ROWS and x.shape[0] > stream_rows(x.shape[1]):
         y = linear(x, w, torch.float32, partials=True)
         return weighted_sum(y, 1.0, None) if y.dim() == 3 else y
@@ -771,6 +771,42 @@ def _try_out(x, w, y, out_f32, T, N, K, ldx, ldw, slices, ws, stream, partial=Fa
         tune_log.append((T, N, K, slices, chosen.value, float(us[0]), float(us[1])))
 
 
+# The kernel for 17 to 64 rows (gemm_rows.hip; ``STREAM_WIDE_MAX_ROWS`` up to 16 switches it off
+# with the streaming kernel's form for 17 to 32 rows).  Beyond 32 rows a product of more than this
+# many weight rows goes to the library: x is read as often as W there, and tiles of 64 rows read
+# it more often than the library's (1B output head, 128,256 rows, 64 rows of x: 130 against 120 us;
+# 32 rows of x 108 against 113; gate/up of the 8B shape, 28,672: 53 against 56).
+ROWS_MAX_ROWS = 64
+ROWS_LIBRARY_N = 32768
+
+
+def _rows_kernel(x: torch.Tensor, w: torch.Tensor, gated: bool = False) -> bool:
+    """Whether the kernel for 17 to 64 rows takes ``x @ w.T`` (``gated``: gate and up rows)."""
+    T, K = x.shape
+    N = w.shape[0]
+    return (STREAM_MAX_ROWS < T <= ROWS_MAX_ROWS and STREAM_WIDE_MAX_ROWS > STREAM_MAX_ROWS
+            and BF16_GEMM == "library"
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and K % 128 == 0 and N % (16 if gated else 8) == 0 and (T <= 32 or N <= ROWS_LIBRARY_N)
+            and x.stride(1) == 1 and w.stride(1) == 1
+            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) >= K and w.stride(0) >= K
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and 2 * N * w.stride(0) < 1 << 32 and 2 * T * x.stride(0) < 1 << 32)
+
+
+def _rows_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, slices: int = 1,
+                 gated: bool = False, ss: Optional[torch.Tensor] = None, eps: float = 0.0
+                 ) -> torch.Tensor:
+    T, K = x.shape
+    N = w.shape[0] // 2 if gated else w.shape[0]
+    y = torch.empty((T, N) if slices == 1 else (slices, T, N), dtype=out_dtype, device=x.device)
+    lib.call("rlis_gemm_bf16_rows", x.data_ptr(), w.data_ptr(), y.data_ptr(),
+             2 if gated else int(out_dtype == torch.float32), T, N, K, slices, x.stride(0), w.stride(0),
+             N, T * N, None if ss is None else ss.data_ptr(), 0 if ss is None else ss.shape[1],
+             0 if ss is None else ss.stride(0), float(eps), lib.stream_ptr())
+    return y
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
            partials: bool = False) -> torch.Tensor:
     """``x @ w.T`` for ``x (T, K)`` and ``w (N, K)``, float32 accumulation.
@@ -778,13 +814,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     Float32 throughout takes the 32-bit kernels on the matrix cores' 32-bit form (K and strides
     multiples of 4; the same bits for a row whichever rows share the call); other sizes, and a
     float32 weight or ``x`` beside bfloat16, the plain FMA kernel.
-    bfloat16 operands take the streaming kernel up to 16 rows; more rows go to the library's
+    bfloat16 operands take the streaming kernel up to 16 rows (32 over short rows) and the kernel
+    for 17 to 64 rows beyond (``_rows_kernel``); more rows, and other sizes, go to the library's
     GEMM (hipBLASLt, through its own entry points), or with ``BF16_GEMM = "own"`` to the skinny
     kernel up to 64 rows and the hand-written matrix-core GEMM beyond.
 
     ``partials``: the caller hands the result to the residual stream and takes it as a stack
     ``(S, T, N)`` of float32 partial sums too (one per k slice of the streaming kernel, or of
-    the split-k kernel that 17 to 64 rows take, added in order by ``add_rmsnorm`` /
+    the kernels that 17 to 64 rows take, added in order by ``add_rmsnorm`` /
     ``add_residual``) where that saves a pass."""
     ldx = _rows_contig(x, "linear x")
     ldw = _rows_contig(w, "linear weight")
@@ -803,6 +840,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         lib.call("rlis_gemm_bf16_stream", x.data_ptr(), w.data_ptr(), y.data_ptr(),
                  _DT[y.dtype], T, N, K, ldx, ldw, N, T * N, 0, stream)
         return y
+    if bf16 and STREAM_MAX_ROWS < T <= ROWS_MAX_ROWS and out_dtype in _DT and _rows_kernel(x, w):
+        slices = lib.load().rlis_gemm_bf16_rows_slices(N, K) if partials else 1
+        return _rows_linear(x, w, torch.float32 if slices > 1 else out_dtype, slices)
     if bf16 and aligned and partials and STREAM_MAX_ROWS < T <= SPLITK_MAX_ROWS:
         slices = lib.load().rlis_gemm_bf16_splitk_slices(N, K)
         y = torch.empty((slices, T, N), dtype=torch.float32, device=x.device)
@@ -995,6 +1035,9 @@ def linear_scaled(xw: torch.Tensor, ss: torch.Tensor, eps: float, w: torch.Tenso
         if N % 2:
             raise KernelError("linear_scaled: a gated weight needs an even number of rows")
         N //= 2
+    if _rows_kernel(xw, w, gated) and out_dtype in ((torch.bfloat16,) if gated else _DT) \
+            and ss.stride(0) % 4 == 0 and ss.stride(1) == 1 and ss.data_ptr() % 16 == 0:
+        return _rows_linear(xw, w, out_dtype, gated=gated, ss=ss, eps=eps)
     y = torch.empty((T, N), dtype=out_dtype, device=xw.device)
     lib.call("rlis_gemm_bf16_stream_scaled", xw.data_ptr(), w.data_ptr(), y.data_ptr(),
              _DT[out_dtype], T, N, K, xw.stride(0), w.stride(0), N, int(bool(gated)),
@@ -1005,7 +1048,7 @@ def linear_scaled(xw: torch.Tensor, ss: torch.Tensor, eps: float, w: torch.Tenso
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]`` of shape ``(2 I, K)``.
 
-    Up to 16 rows of bfloat16 (64 with ``BF16_GEMM = "own"``) take one kernel that never stores
+    Up to 64 rows of bfloat16 take one kernel (of a K that it takes) that never stores
     the ``(T, 2 I)`` intermediate; everything else is the product followed by the SwiGLU
     kernel."""
     T, K = x.shape
@@ -1021,6 +1064,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     streamed = fusable and T <= stream_rows(K) and _one_item_per_wave(K)
     skinny = fusable and not streamed and T <= SKINNY_MAX_ROWS and \
         (BF16_GEMM == "own" or T <= STREAM_MAX_ROWS)
+    if fusable and not streamed and K == w_gate_up.shape[1] and _rows_kernel(x, w_gate_up, gated=True):
+        return _rows_linear(x, w_gate_up, torch.bfloat16, gated=True)
     if not (streamed or skinny):
         return swiglu(linear(x, w_gate_up, x.dtype))
     y = torch.empty((T, two_i // 2), dtype=torch.bfloat16, device=x.device)

@@ -67,6 +67,7 @@ _SIGNATURES = {
     "rlis_copy_pages": [P, I, I, L, L, P, P, I, P],
     "rlis_gemm_plain": [P, I, P, I, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, P],
+    "rlis_gemm_bf16_rows": [P, P, P, I, I, I, I, I, L, L, L, L, P, I, I, F, P],
     "rlis_gemm_bf16_mfma": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny_swiglu": [P, P, P, I, I, I, L, L, L, P],
@@ -118,6 +119,8 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     lib.rlis_gemm_bf16_stream_slices.restype = c_int
     lib.rlis_gemm_bf16_stream_slices.argtypes = [I]
+    lib.rlis_gemm_bf16_rows_slices.restype = c_int
+    lib.rlis_gemm_bf16_rows_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_splitk_slices.restype = c_int
     lib.rlis_gemm_bf16_splitk_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_stream_join_tiles.restype = c_int

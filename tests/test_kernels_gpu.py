@@ -144,6 +144,53 @@ def test_swiglu(ops, dtype, T, I):
 
 
 # ------------------------------------------------------------------- products
+@pytest.mark.parametrize("N,K", [(8, 128), (72, 256), (1000, 384), (3072, 2048), (2048, 8192), (264, 14336),
+                                 (5120, 640), (16384, 256), (4096, 1536)])
+def test_linear_rows_kernel(ops, N, K):
+    """The kernel for 17 to 64 rows (tiles of 16, 32 and 64 weight rows, several tiles to a
+    workgroup, stages that wrap round, one to four slices of k; plain, float32, partial sums,
+    gated, scaled) against float64 products of the same bf16-rounded operands, within K roundings
+    of 2^-24 of the sum of magnitudes and a rounding to bfloat16 (2^-8) where the result is stored
+    so; and the same bits for a row with 17 rows in the call as with 64."""
+    base = rnd(64, K + 16, dtype=torch.bfloat16, seed=1)
+    x, w = base[:, :K], rnd(2 * N, K, dtype=torch.bfloat16, seed=2, scale=0.05)
+    want = x.double() @ w.double().t()
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    wn = w[:N]
+    assert ops._rows_kernel(x, wn) and ops._rows_kernel(x, w, gated=True)
+    full = ops._rows_linear(x, wn, torch.float32)
+    assert bool(((full.double() - want[:, :N]).abs() <= bound[:, :N]).all())
+    half = ops._rows_linear(x, wn, torch.bfloat16)
+    assert torch.equal(half, full.to(torch.bfloat16))
+    from rust_llm_inference_server_amd.ops import lib
+    slices = lib.load().rlis_gemm_bf16_rows_slices(N, K)
+    assert slices in (1, 2, 4) and K % (128 * slices) == 0
+    parts = ops._rows_linear(x, wn, torch.float32, slices)
+    total = parts if slices == 1 else parts[0] + sum(parts[i] for i in range(1, slices))
+    assert bool(((total.double() - want[:, :N]).abs() <= bound[:, :N]).all())
+    gated = ops._rows_linear(x, w, torch.bfloat16, gated=True)
+    g, u = want[:, :N], want[:, N:]
+    unit = torch.nn.functional.silu(g) * u
+    # (the slope of silu is at most 1.1, |silu(g)| at most |g|; stored once)
+    off = 1.1 * bound[:, :N] * u.abs() + g.abs() * bound[:, N:] + 1.1 * bound[:, :N] * bound[:, N:]
+    assert bool(((gated.double() - unit).abs() <= 2.0 ** -8 * unit.abs() + 1.01 * off + 1e-30).all())
+    count = K // 16
+    ss = torch.zeros(64, -(-count // 4) * 4, device=DEV)[:, :count]
+    ss.copy_((x.float() ** 2).reshape(64, count, 16).sum(-1))
+    scale = torch.rsqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+    scaled = ops._rows_linear(x, wn, torch.float32, ss=ss, eps=1e-5)
+    torch.testing.assert_close(scaled.double(), full.double() * scale, rtol=1e-5, atol=1e-30)
+    for T in (17, 31, 32, 33, 49):
+        assert torch.equal(ops._rows_linear(x[:T], wn, torch.float32), full[:T]), T
+        few = ops._rows_linear(x[:T].contiguous(), wn, torch.float32, slices)
+        assert torch.equal(few, parts[..., :T, :]), T
+        assert torch.equal(ops._rows_linear(x[:T], w, torch.bfloat16, gated=True), gated[:T]), T
+        assert torch.equal(ops._rows_linear(x[:T], wn, torch.float32, ss=ss, eps=1e-5), scaled[:T]), T
+    # the public entry points take it where nothing else is pinned, and only then
+    assert torch.equal(ops.linear(x, wn), half) and torch.equal(ops.linear_swiglu(x, w), gated)
+    assert not ops._rows_kernel(x[:16], wn) and not ops._rows_kernel(x[:, 1:], wn[:, 1:])
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 331, 100), (5, 100, 172), (64, 130, 96), (65, 257, 100),
                                    (200, 3072, 2048), (3, 7, 5)])
 def test_linear_float32(ops, T, N, K):
