@@ -20,6 +20,7 @@
 // context are merged with weights e^(m_i - max m) over the non-empty ones (metal:276-304).
 //
 //  * attn_generic: one wave per (token, query head); any way of cutting the batch.
+//  * attn_tiles_f32: float32, sixteen queries of a head per wave on the matrix cores' 32-bit form.
 //  * attn_decode: one query token per sequence; a workgroup serves up to 8 query heads of one
 //    KV head, so K and V are read once per group; contexts are split into partitions.
 //  * attn_reduce: merges the partitions.
@@ -151,6 +152,192 @@ RLIS_API int rlis_attn_generic(const void* q, int dtype, long long q_stride, voi
 #undef BY_DPL
 #undef LAUNCH
   RLIS_LAUNCH_CHECK("attn_generic");
+  return 0;
+}
+
+// ============================================================== tiles of queries, float32
+// One wave per 16 neighbouring tokens and query head, on v_mfma_f32_16x16x4_f32 (float32 operands
+// and multiply-adds).  Keys are walked in blocks of 16 from absolute multiples of 16 on: S^T = K Q^T
+// leaves a lane the scores of its query (lane % 16) for the keys 4 g + i of its group g = lane / 16,
+// which is how P^T enters O^T = V^T P^T, so probabilities stay in their registers; K rows and rows of
+// V^T are loaded straight into operand layout, 16 bytes a lane, the next block's while this one is
+// multiplied.  A query's blocks and sums do not depend on the tokens beside it: a key that it does
+// not see adds an exact zero.  A tile that spans sequences walks them one after the other.
+//
+// attn_generic, a wave per query, is bound by its chain (every key's product summed by one lane, one
+// load each): three prompts of 96 tokens on average, 32 heads of 64, took 242 us; this takes 16.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int J /* d / 16 */>
+__global__ __launch_bounds__(256) void attn_tiles_f32_kernel(
+    const float* __restrict__ q, long long q_stride, float* __restrict__ out, long long out_stride,
+    const float* __restrict__ k_pages, const float* __restrict__ v_pages,
+    const int* __restrict__ block_tables, int max_pages, const int* __restrict__ seq_of_token,
+    const int* __restrict__ positions, int T, int nh, int nkv, int page_size, float scale, int window,
+    const float* __restrict__ slopes, const float* __restrict__ head_scales, float softcap,
+    const float* __restrict__ sinks, int chunk) {
+  constexpr int d = 16 * J;
+  const int lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  const int t0 = blockIdx.x * 16, h = blockIdx.y * 4 + (int)(threadIdx.x / 64);
+  if (h >= nh) return;
+  const int kvh = h / (nh / nkv);
+  const float slope = slopes ? slopes[h] : 0.f;
+  if (head_scales) scale *= head_scales[h];
+  const float inv_cap = softcap > 0.f ? 1.0f / softcap : 0.f;
+  const int t = min(t0 + r, T - 1);                   // this lane's query
+  const int pos = positions[t], seq = seq_of_token[t];
+  const int lo = first_visible(pos, window, chunk);
+  f32x4 qv[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) qv[j] = *(const f32x4*)(q + (long long)t * q_stride + h * d + 16 * j + 4 * g) * scale;
+
+  const int last = min(t0 + 16, T) - 1;
+  for (int first = t0; first <= last;) {
+    // queries [first, next) are of one sequence; they are wave-uniform
+    const int cur = __shfl(seq, first - t0, 64);
+    const unsigned long long same = __ballot(seq == cur) & 0xffffull;
+    int next = first;
+    while (next <= last && (same >> (next - t0) & 1)) ++next;
+    const bool mine = r >= first - t0 && r < next - t0;
+    const int* table = block_tables + (long long)cur * max_pages;
+    const int end = __shfl(pos, next - 1 - t0, 64) + 1;
+    int begin = end;
+    for (int i = first; i < next; ++i) begin = min(begin, __shfl(lo, i - t0, 64));
+    begin &= ~15;
+
+    float m = -INFINITY, l = 0.f;
+    f32x4 acc[J], kv[J], vv[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const auto load = [&](int k0) {
+      // (past the last key the last one's page is read again: it is masked)
+      const int kk = min(k0 + r, end - 1), vk = min(k0 + 4 * g, (end - 1) & ~3);
+      const long long kp = table[kk / page_size], vp = table[vk / page_size];
+      const float* kr = k_pages + ((kp * nkv + kvh) * page_size + kk % page_size) * d + 4 * g;
+      const float* vr = v_pages + ((vp * nkv + kvh) * d + r) * page_size + vk % page_size;
+#pragma unroll
+      for (int j = 0; j < J; ++j) kv[j] = *(const f32x4*)(kr + 16 * j);
+#pragma unroll
+      for (int j = 0; j < J; ++j) vv[j] = *(const f32x4*)(vr + (long long)16 * j * page_size);
+    };
+    load(begin);
+    for (int k0 = begin; k0 < end; k0 += 16) {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[j][i], qv[j][i], s, 0, 0, 0);
+      }
+      f32x4 vc[J];
+#pragma unroll
+      for (int j = 0; j < J; ++j) vc[j] = vv[j];
+      load(k0 + 16);
+      float top = -INFINITY;
+      bool sees[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = k0 + 4 * g + i;
+        sees[i] = mine && key >= lo && key <= pos;
+        float x = s[i];
+        if (softcap > 0.f) x = softcap * tanhf(x * inv_cap);
+        x += slope * (float)(key - pos);
+        s[i] = x;
+        if (sees[i]) top = fmaxf(top, x);
+      }
+      top = xor32_max(xor16_max(top));
+      const float m_new = fmaxf(m, top);
+      const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
+      m = m_new;
+      float p[4], add = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[i] = sees[i] ? expf(s[i] - m_new) : 0.f;
+        add += p[i];
+      }
+      l = l * corr + add;                            // this lane's keys; the groups meet at the end
+      bool odd = false;                              // a value that is no finite number
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        acc[j] *= corr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (k0 + 4 * g + i >= end) vc[j][i] = 0.f; // (whatever the page holds there)
+          odd |= !(fabsf(vc[j][i]) < INFINITY);
+        }
+      }
+      if (__ballot(odd) == 0) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vc[j][i], p[i], acc[j], 0, 0, 0);
+        }
+      } else {
+        // key by key, and only into the queries that see it: zero times infinity is NaN
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const bool seen = __shfl((int)sees[u % 4], u / 4 * 16 + r, 64);
+#pragma unroll
+          for (int j = 0; j < J; ++j) {
+            const f32x4 a = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                g == u / 4 ? vc[j][u % 4] : 0.f, g == u / 4 ? p[u % 4] : 0.f, acc[j], 0, 0, 0);
+            if (seen) acc[j] = a;
+          }
+        }
+      }
+    }
+    l = xor32_sum(xor16_sum(l));
+    if (sinks) {
+      // the sink counts once in the denominator: e^sink beside the keys' e^score
+      const float sink = sinks[h];
+      const float m_new = fmaxf(m, sink);
+      const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
+      l = l * corr + expf(sink - m_new);
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[j] *= corr;
+    }
+    const float inv_l = 1.0f / l;
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        *(f32x4*)(out + (long long)t * out_stride + h * d + 16 * j + 4 * g) = acc[j] * inv_l;
+    }
+    first = next;
+  }
+}
+
+// Rows [0, T) of q, any mix of sequences (each one's tokens side by side in ascending order); d 16,
+// 32, 64, 128 or 256; page_size a multiple of 4; q, out and their strides in steps of 16 bytes.
+RLIS_API int rlis_attn_tiles_f32(const void* q, long long q_stride, void* out, long long out_stride,
+                                 const void* k_pages, const void* v_pages, const int* block_tables,
+                                 int max_pages, const int* seq_of_token, const int* positions, int T,
+                                 int nh, int nkv, int d, int page_size, float scale, int window,
+                                 const float* slopes, const float* head_scales, float softcap,
+                                 const float* sinks, int chunk, hipStream_t stream) {
+  RLIS_REQUIRE(T >= 0 && nh > 0 && nkv > 0 && page_size > 0 && page_size % 4 == 0,
+               "attn_tiles_f32: bad sizes");
+  RLIS_REQUIRE(chunk >= 0 && (chunk == 0 || window == 0), "attn_tiles_f32: a window or chunks, not both");
+  RLIS_REQUIRE(nh % nkv == 0 && nh <= 4 * 65535, "attn_tiles_f32: bad head counts");
+  RLIS_REQUIRE(q_stride % 4 == 0 && out_stride % 4 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+                   (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0,
+               "attn_tiles_f32: rows must lie on 16-byte boundaries");
+  if (T == 0) return 0;
+  dim3 grid(ceil_div(T, 16), ceil_div(nh, 4));
+#define LAUNCH(J)                                                                                    \
+  attn_tiles_f32_kernel<J><<<grid, 256, 0, stream>>>(                                                \
+      (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, \
+      block_tables, max_pages, seq_of_token, positions, T, nh, nkv, page_size, scale, window, slopes,  \
+      head_scales, softcap, sinks, chunk)
+  switch (d) {
+    case 16: LAUNCH(1); break;
+    case 32: LAUNCH(2); break;
+    case 64: LAUNCH(4); break;
+    case 128: LAUNCH(8); break;
+    case 256: LAUNCH(16); break;
+    default: RLIS_REQUIRE(false, "attn_tiles_f32: head_dim %d is not 16, 32, 64, 128 or 256", d);
+  }
+#undef LAUNCH
+  RLIS_LAUNCH_CHECK("attn_tiles_f32");
   return 0;
 }
 

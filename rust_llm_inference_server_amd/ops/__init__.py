@@ -1463,11 +1463,25 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
         raise KernelError("attention: only the matrix-core kernels rotate, and only the decode "
                           "kernel stores")
     if kind == "generic":
-        lib.call("rlis_attn_generic", qkv.data_ptr(), _dt(qkv), q_stride, out.data_ptr(), nh * d,
-                 k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), max_pages,
-                 _i32(step.seq_of_token, "seq_of_token", T), _i32(step.positions, "positions", T),
-                 T, nh, nkv, d, page_size, float(scale), win, slopes_ptr, scales_ptr, softcap,
-                 sinks_ptr, kept, span, stream)
+        # float32: portions of prompts go in tiles of 16 queries; single tokens, which lead the
+        # step, each walk their own sequence and stay apart
+        rows = T
+        if (force is None and qkv.dtype == torch.float32 and d in (16, 32, 64, 128, 256) and not kept
+                and page_size % 4 == 0 and q_stride % 4 == 0 and qkv.data_ptr() % 16 == 0
+                and k_pages.data_ptr() % 16 == 0 and v_pages.data_ptr() % 16 == 0):
+            rows = step.num_single
+        seqs, poss = _i32(step.seq_of_token, "seq_of_token", T), _i32(step.positions, "positions", T)
+        if rows:
+            lib.call("rlis_attn_generic", qkv.data_ptr(), _dt(qkv), q_stride, out.data_ptr(), nh * d,
+                     k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), max_pages, seqs,
+                     poss, rows, nh, nkv, d, page_size, float(scale), win, slopes_ptr, scales_ptr,
+                     softcap, sinks_ptr, kept, span, stream)
+        if rows < T:
+            lib.call("rlis_attn_tiles_f32", qkv.data_ptr() + 4 * rows * q_stride, q_stride,
+                     out.data_ptr() + 4 * rows * nh * d, nh * d, k_pages.data_ptr(),
+                     v_pages.data_ptr(), block_tables.data_ptr(), max_pages, seqs + 4 * rows,
+                     poss + 4 * rows, T - rows, nh, nkv, d, page_size, float(scale), win, slopes_ptr,
+                     scales_ptr, softcap, sinks_ptr, span, stream)
         return out
     if kind not in ("decode", "prefill"):
         raise KernelError(f"attention: unknown kernel '{kind}'")

@@ -915,6 +915,41 @@ def test_attention_mixed_batch(ops, dtype, nh, nkv, d, ps, kind):
     torch.testing.assert_close(got.float().cpu(), want, **tol(dtype, 2e-5, 2e-2))
 
 
+@pytest.mark.parametrize("nh,nkv,d,ps", [(4, 1, 16, 16), (6, 2, 32, 8), (32, 8, 64, 16), (5, 1, 128, 4),
+                                         (3, 3, 256, 64)])
+@pytest.mark.parametrize("form", ["plain", "window", "chunk", "shaped"])
+def test_attention_float32_tiles(ops, nh, nkv, d, ps, form):
+    """float32 portions in tiles of 16 queries on the matrix cores, single tokens in front of them:
+    tiles that span sequences and end inside one, keys that start inside a block and a page, a
+    window, chunks, and a bias, head scales, a cap and sinks, against the kernel of one wave per
+    query (both sum in float32: some 300 roundings of values around 1).  Then a value that is
+    infinite and one that is NaN, late in a sequence: the queries in front of them keep their
+    bits."""
+    cached, new = [9, 0, 5, 40, 0, 130, 17], [1, 1, 33, 70, 2, 49, 3]
+    qkv, kp, vp, bt, step, ks, vs, cu = paged_case(cached, new, nh, nkv, d, ps, torch.float32, seed=nh)
+    assert step.num_single == 2
+    options = {"plain": {}, "window": {}, "chunk": {"chunk": 48},
+               "shaped": {"bias_slopes": rnd(nh, seed=7, scale=0.02), "softcap": 3.0, "sinks": rnd(nh, seed=8),
+                          "head_scales": 1.0 + rnd(nh, seed=9, scale=0.1)}}[form]
+    window = 37 if form == "window" else None
+
+    def run(values, force=None):
+        return ops.paged_attention(qkv, nh, nkv, d, kp, values, ps, bt, step, 1.0 / math.sqrt(d), window,
+                                   force=force, **options)
+
+    got, want = run(vp), run(vp, "generic")
+    torch.testing.assert_close(got, want, atol=2e-5, rtol=2e-5)
+    assert torch.equal(got[:2], want[:2])
+    page, off = int(bt[3, 100 // ps]), 100 % ps                # position 100 of the sequence with 40 cached
+    for bad in (float("inf"), float("nan")):
+        broken = vp.clone()
+        broken[page, :, :, off] = bad
+        rows = run(broken)
+        keep = [i for i in range(rows.shape[0]) if not cu[3] + 60 <= i < cu[4]]
+        assert torch.equal(rows[keep], got[keep])
+        assert not bool(torch.isfinite(rows[cu[3] + 60]).any())
+
+
 @pytest.mark.parametrize("nh,nkv,d,ps", [(32, 8, 64, 16), (24, 8, 128, 16), (6, 2, 32, 8), (5, 5, 48, 16),
                                          (34, 2, 16, 16)])
 @pytest.mark.parametrize("window", [None, 70])
