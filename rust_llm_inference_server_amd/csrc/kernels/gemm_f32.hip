@@ -8,15 +8,20 @@
 // (a multiple of 16, from K alone: f32_run).  Inside a run the sum grows in steps of 16 k, four
 // instructions a step, instruction i multiplying k = 16 j + 4 g + i of the four lane groups g.
 // The sums of four runs in a row are added in ascending order to a part, the parts likewise to
-// the result.  Both kernels below do exactly that, so a row's result does not depend on how many
+// the result.  All kernels below do exactly that, so a row's result does not depend on how many
 // rows share the call, nor on the kernel or tile that takes it.
 //
-//  * gemm_f32_stream: up to 32 rows, bound by reading W once.  A workgroup takes 16 weight rows
+//  * gemm_f32_ring: up to 16 rows over K in whole 1024s, bound by reading W once.  W and x come
+//    into LDS by direct loads that leave a wave 16 KB ahead of its products, with no registers held
+//    for them and whole lines (256 bytes of a row) per load.  At 4 rows, weights cold (MI355X, us,
+//    stream kernel -> this): 3072 x 2048 10.8 -> 8.6, 2048 x 2048 10.2 -> 7.9, 16384 x 2048 30.2 ->
+//    24.7 (5.4 TB/s), 2048 x 8192 30 -> 21, 128256 x 2048 182 -> 177 (5.9 TB/s), 4096 x 14336 39
+//    (6.1 TB/s); at 16 rows 2048 x 8192 37 -> 22.
+//  * gemm_f32_stream: other K, and 17 to 32 rows.  A workgroup takes 16 weight rows
 //    at a time, one wave per run of k, so a wave's loads of a tile are all in flight at once
 //    (8 KB) and the next tile's are asked for before this one's products; runs of up to 128 k
-//    keep x in registers over all tiles.  The waves' sums meet in LDS.  At 4 rows of the 1B
-//    shape, weights cold (MI355X, us, gemm_plain -> this): q/k/v 245 -> 10.9, output 240 -> 10.2,
-//    gate/up 250 -> 30 (4.5 TB/s), head 487 (hot) -> 181 (5.8 TB/s), down 940 -> 30: there, and
+//    keep x in registers over all tiles.  The waves' sums meet in LDS.  At 32 rows of the 1B
+//    shape, weights cold: q/k/v 16, output 16, gate/up 40, head 242, down 59 us: there, and
 //    wherever the long form runs, x is loaded as often as W, and a load of either takes its
 //    compute unit about 24 ns (56 clocks, sixteen row pieces of 64 bytes), which bounds it.
 //  * gemm_f32_tiles: more rows, bound by the matrix cores (154 TFLOP/s for a large library
@@ -60,8 +65,8 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int k, int e
 // The sum of a tile's runs, which lie in LDS as [run][group of rows][lane], for rows t * 16 .. + 15
 // of x: stored by one wave.
 template <int TG>
-__device__ __forceinline__ void store_tile(const float* red, int runs, int t, int tile, float* Y,
-                                           int T, int N, long long ldy, int vec_out) {
+__device__ __forceinline__ void store_tile(const float* red, int runs, int t, int tile, int rows,
+                                           float* Y, int T, int N, long long ldy, int vec_out) {
   const int lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   f32x4 s;
   for (int q0 = 0; q0 < runs; q0 += kPartRuns) {
@@ -70,8 +75,8 @@ __device__ __forceinline__ void store_tile(const float* red, int runs, int t, in
       p += *(const f32x4*)(red + (q * TG + t) * 256 + lane * 4);
     s = q0 == 0 ? p : s + p;
   }
-  const int token = t * 16 + r, n = tile * 16 + 4 * g;
-  if (token >= T) return;
+  const int token = t * 16 + r, n = tile * rows + 4 * g;
+  if (token >= T || 4 * g >= rows) return;
   float* y = Y + token * ldy + n;
   if (vec_out && n + 4 <= N) {
     *(f32x4*)y = s;
@@ -134,7 +139,7 @@ __global__ __launch_bounds__(kMaxRuns * 64) void gemm_f32_stream_kernel(
     __syncthreads();
     // (the next tile writes the other buffer; this one is written again behind the barrier that
     // its readers reach only when they are done)
-    for (int t = wave; t < TG; t += waves) store_tile<TG>(part, waves, t, tile, Y, T, N, ldy, vec_out);
+    for (int t = wave; t < TG; t += waves) store_tile<TG>(part, waves, t, tile, 16, Y, T, N, ldy, vec_out);
   }
 }
 
@@ -213,7 +218,7 @@ __global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(
         if (++m_run == 2) {                            // the end of a tile
           m_run = 0;
           __syncthreads();
-          if (wave < TG) store_tile<TG>(part, runs, wave, tile, Y, T, N, ldy, vec_out);
+          if (wave < TG) store_tile<TG>(part, runs, wave, tile, 16, Y, T, N, ldy, vec_out);
           buf ^= 1;
           tile += gridDim.x;
           if (tile >= tiles) break;
@@ -221,6 +226,100 @@ __global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(
       }
     }
   }
+}
+
+// Up to 16 rows over K in whole 1024s (whole runs of a multiple of 64 k): W and x go straight from
+// memory into LDS, every wave through a ring of its own, so that nothing waits for another wave but
+// the tile's end.  What bounds it is the bytes in flight (a compute unit holds 128 KB of them; reading
+// W once runs at 5.5 to 6 TB/s from 100 MB up).  Eight waves of two runs each; a chunk is 64 k (256 bytes) of RW * 4 weight rows
+// and XW * 4 rows of x, asked for as soon as its place has been read.  Row r's piece i lies at piece
+// i ^ (r % 16).  Tiles of 8 or 12 rows fill half or three quarters of a product (lanes beyond read
+// a row twice).
+template <int RW, int XW>
+__host__ __device__ constexpr int ring_chunks() {
+  return std::min(6, 16384 / ((RW + XW) * 1024));
+}
+template <int RW, int XW>
+__global__ __launch_bounds__(512) void gemm_f32_ring_kernel(
+    const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int T, int N,
+    int run, int tiles, uint32_t ldx, uint32_t ldw, long long ldy, int vec_out) {
+#ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
+  constexpr int PER = RW + XW, CHUNK = PER * 1024, NB = ring_chunks<RW, XW>();
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ring_smem[];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int r = lane % 16, g = lane / 16;
+  unsigned char* ring = ring_smem + wave * NB * CHUNK;
+  float* red = (float*)(ring_smem + 8 * NB * CHUNK);            // [2][16 runs][64 lanes][4]
+  const int chunks = run / 64 * 2;                              // of this wave's two runs
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + 2 * wave * run), 0, 0xffffffff, 0x00027000);
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(W + 2 * wave * run), 0, 0xffffffff, 0x00027000);
+  // instruction i brings rows 4 i .. + 3 of a chunk, 16 lanes a row
+  uint32_t src[PER];
+  const auto place = [&](int row) { return (uint32_t)((r ^ (row & 15)) * 16); };
+#pragma unroll
+  for (int i = 0; i < XW; ++i) src[RW + i] = (uint32_t)min(4 * i + g, T - 1) * ldx * 4 + place(4 * i + g);
+  const auto weight_rows = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < RW; ++i)
+      src[i] = (uint32_t)min(tile * 4 * RW + 4 * i + g, N - 1) * ldw * 4 + place(4 * i + g);
+  };
+  int a_tile = blockIdx.x, a_chunk = 0;
+  const auto ask = [&](int buf) {
+    unsigned char* base = ring + buf * CHUNK;
+    const int at = a_chunk * 256;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (i < RW)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr)(base + i * 1024), 16, src[i], at, 0, 2);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr)(base + i * 1024), 16, src[i], at, 0, 0);
+    }
+    if (++a_chunk == chunks) {             // (past the last tile its last row is read again)
+      a_chunk = 0;
+      a_tile += gridDim.x;
+      weight_rows(a_tile);
+    }
+  };
+  weight_rows(a_tile);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) ask(b);
+  const int w_row = r < 4 * RW ? r : r - 4 * RW, x_row = min(r, 4 * XW - 1);
+  int buf = 0, side = 0;
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, side ^= 1) {
+    float* part = red + side * 16 * 256;
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < chunks / 2; ++c) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * (NB - 1)) : "memory");
+        const unsigned char* base = ring + buf * CHUNK;
+        f32x4 w[4], x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          w[j] = *(const f32x4*)(base + w_row * 256 + ((4 * j + g) ^ w_row) * 16);
+          x[j] = *(const f32x4*)(base + RW * 1024 + x_row * 256 + ((4 * j + g) ^ x_row) * 16);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the chunk has been read
+        __builtin_amdgcn_sched_barrier(0);
+        ask(buf);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc = mfma_f32(w[j][i], x[j][i], acc);
+        }
+        buf = buf + 1 == NB ? 0 : buf + 1;
+      }
+      *(f32x4*)(part + (2 * wave + half) * 256 + lane * 4) = acc;
+    }
+    __syncthreads();
+    // (the next tile writes the other side; this one is written again behind the barrier that its
+    // reader reaches only when it is done)
+    if (wave == 0) store_tile<1>(part, 16, 0, tile, 4 * RW, Y, T, N, ldy, vec_out);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // (loads past the last tile)
+#endif
 }
 
 // ------------------------------------------------------------------ more rows
@@ -384,6 +483,20 @@ int compute_units() {
   return n;
 }
 
+template <int RW, int XW>
+int launch_ring(const float* X, const float* W, float* Y, int T, int N, int run, int cus, long long ldx,
+                long long ldw, long long ldy, int vec, hipStream_t stream) {
+  static LdsGrant grant;
+  constexpr int bytes = 8 * ring_chunks<RW, XW>() * (RW + XW) * 1024 + 2 * 16 * 1024;
+  const auto kernel = gemm_f32_ring_kernel<RW, XW>;
+  const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
+  RLIS_REQUIRE(e == hipSuccess, "gemm_f32: %s", hipGetErrorString(e));
+  const int tiles = ceil_div(N, 4 * RW);
+  kernel<<<std::min(tiles, cus), 512, bytes, stream>>>(X, W, Y, T, N, run, tiles, (uint32_t)ldx,
+                                                       (uint32_t)ldw, ldy, vec);
+  return 0;
+}
+
 template <int TG>
 void launch_stream(const float* X, const float* W, float* Y, int T, int N, int K, int run, int cus,
                    long long ldx, long long ldw, long long ldy, int vec, hipStream_t stream) {
@@ -443,7 +556,36 @@ RLIS_API int rlis_gemm_f32(const void* X_, const void* W_, void* Y_, int T, int 
   const int run = f32_run(K), cus = compute_units();
   RLIS_REQUIRE(cus > 0, "gemm_f32: cannot read the device properties");
   const int vec = ldy % 4 == 0 && (uintptr_t)Y % 16 == 0;
-  if (T <= 32) {
+  // Rows whose bytes a buffer's 32-bit offset reaches.  More than 4 rows bring half as much x as W
+  // into the rings and more: over more than eight tiles a compute unit the stream kernel, which
+  // keeps x of short runs in registers, is ahead (128256 x 2048 at 16 rows: 192 us against 242, at 8
+  // no slower than the 192; 16384 x 2048, four tiles, 16 rows: 33 against 27).
+  const bool ring = K % 1024 == 0 && 4 * (ldw * (N - 1) + K) < (1LL << 32) &&
+                    4 * (ldx * (T - 1) + K) < (1LL << 32) &&
+                    (T <= 4 || run > 128 || ceil_div(N, 16) <= 8 * cus);
+  if (T <= 16 && ring) {
+    // Tiles of 16 weight rows, or of 12 or 8 where that takes rows off the busiest compute unit
+    // (3072 x 2048 at 4 rows: 8.6 us with 12, 2048 x 2048: 7.9 with 8)
+    int rows = 16, most = ceil_div(ceil_div(N, 16), cus) * 16;
+    for (int c = 12; c >= 8; c -= 4) {
+      const int m = ceil_div(ceil_div(N, c), cus) * c;
+      if (m < most) { rows = c; most = m; }
+    }
+    int rc;
+#define GO(RW, XW) rc = launch_ring<RW, XW>(X, W, Y, T, N, run, cus, ldx, ldw, ldy, vec, stream)
+#define BY_X(RW)                        \
+  do {                                  \
+    if (T <= 4) GO(RW, 1);              \
+    else if (T <= 8) GO(RW, 2);         \
+    else GO(RW, 4);                     \
+  } while (0)
+    if (rows == 16) BY_X(4);
+    else if (rows == 12) BY_X(3);
+    else BY_X(2);
+#undef BY_X
+#undef GO
+    if (rc) return rc;
+  } else if (T <= 32) {
     if (T <= 16) launch_stream<1>(X, W, Y, T, N, K, run, cus, ldx, ldw, ldy, vec, stream);
     else launch_stream<2>(X, W, Y, T, N, K, run, cus, ldx, ldw, ldy, vec, stream);
   } else {

@@ -226,6 +226,29 @@ def test_linear_float32_same_bits_for_any_number_of_rows(ops, N, K):
     assert bool(torch.isnan(got[20]).all()) and not bool(torch.isfinite(got[3]).any())
 
 
+@pytest.mark.parametrize("N,K", [(1, 1024), (7, 3072), (2048, 1024), (2049, 2048), (3069, 1024), (4099, 1024),
+                                 (40, 14336), (33000, 1024)])
+def test_linear_float32_ring_kernel(ops, N, K):
+    """Up to 16 rows over whole 1024s of K (tiles of 8, 12 and 16 weight rows, the last one cut,
+    several and no tiles of a compute unit, 1 to 16 rows of x in places for 4, 8 and 16, x strided
+    or not): the bits of the same rows in a product of 40, which no ring takes."""
+    base = rnd(40, K + 8, seed=1)
+    x, w = base[:, :K], rnd(N, K + 4, seed=2)[:, :K]
+    full = ops.linear(x, w)
+    want = x.double() @ w.double().t()
+    bound = (K / 64 + 19) * 2.0 ** -24 * 4 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((full.double() - want).abs() <= bound).all())
+    for T in (1, 3, 4, 5, 8, 9, 16):
+        assert torch.equal(ops.linear(x[:T], w), full[:T]), T
+        assert torch.equal(ops.linear(x[:T].contiguous(), w.contiguous()), full[:T]), T
+    bad = x[:16].clone()
+    bad[3, K - 1], bad[10, 0] = float("inf"), float("nan")
+    got = ops.linear(bad, w)
+    keep = [i for i in range(16) if i not in (3, 10)]
+    assert torch.equal(got[keep], full[keep])
+    assert bool(torch.isnan(got[10]).all()) and not bool(torch.isfinite(got[3]).any())
+
+
 @pytest.mark.parametrize("out_dtype", DTYPES)
 @pytest.mark.parametrize("T,N,K", [(1, 2048, 2048), (1, 331, 104), (8, 3072, 2048), (16, 100, 64),
                                    (2, 2048, 8192), (7, 2049, 14336), (3, 128256, 2048), (4, 7, 520),
