@@ -27,11 +27,13 @@ SKINNY_MAX_ROWS = 64
 # ... and with at most this many rows the streaming kernel (16 at most; 0 switches it off).
 STREAM_MAX_ROWS = 16
 # ... and, where the rows are short enough for a wave to keep 32 of them in registers (k up to
-# 3072), with up to this many rows its form for 17 to 32 rows (0 switches that off: such steps
-# then take the library's products, the split-k kernel and the norm and SwiGLU kernels).
+# 3072), with up to this many rows its form for 17 to 32 rows (0 switches that off, and the kernel
+# for 17 to 64 rows with it: such steps then take the library's products, the split-k kernel and
+# the norm and SwiGLU kernels).
 STREAM_WIDE_MAX_ROWS = 32
-# A product whose result joins the residual stream as partial sums (``partials=True``) takes the
-# split-k kernel from 17 rows up to this many (64 at most; 0 switches it off).
+# A product whose result joins the residual stream as partial sums (``partials=True``) and whose
+# sizes ``_rows_kernel`` does not take goes to the split-k kernel from 17 rows up to this many
+# (64 at most; 0 switches it off).
 SPLITK_MAX_ROWS = 64
 # Single tokens in a batch that also holds portions of prompts take the decode attention kernel.
 SPLIT_MIXED_ATTENTION = True
@@ -653,9 +655,9 @@ def weighted_sum(x: torch.Tensor, a: float, y: Optional[torch.Tensor], b: float 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` stored in float32, for results that enter a recurrence.  From 17 to 64 rows of
-    bfloat16 it is the split-k kernel's partial sums added in order (the library's products with
-    a float32 result are slow at such row counts: 25 us against 6 + 3 for 64 x 2,048 x 2,048);
-    otherwise ``linear(x, w, float32)``."""
+    bfloat16 over sizes that ``_rows_kernel`` does not take it is the split-k kernel's partial sums
+    added in order (the library's products with a float32 result are slow at such row counts: 25 us
+    against 6 + 3 for 64 x 2,048 x 2,048); otherwise ``linear(x, w, float32)``."""
     if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and not _rows_kernel(x, w) \
             and STREAM_MAX_ROWS < x.shape[0] <= SPLITK_MAX_ROWS and x.shape[0] > stream_rows(x.shape[1]):
         y = linear(x, w, torch.float32, partials=True)
