@@ -131,10 +131,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((QB == 1 &&
   __shared__ __attribute__((aligned(16))) bf16_t Ks_all[kTileBufs * BN * KS];
   __shared__ __attribute__((aligned(16))) bf16_t Vs_all[kTileBufs * D * VS];
 
-  // The wave's number as a scalar: what a whole wave skips or masks is then a scalar branch, not a
-  // masked stretch (32 heads of 128, 8,192 tokens: 7 % of the kernel; the 8B shape's prefill of
-  // 8,192 tokens by eight layers 28.25 -> 27.79 ms).
-  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
   const int l16 = lane % 16, lq = lane / 16;
   // Blocks are numbered heads-fastest over the units of work, which arrive sorted by falling
   // work.  One round of blocks (tiles_per_round units x all heads) fills the compute units once;
