@@ -26,10 +26,13 @@
 //    wherever the long form runs, x is loaded as often as W, and a load of either takes its
 //    compute unit about 24 ns (56 clocks, sixteen row pieces of 64 bytes), which bounds it.
 //  * gemm_f32_tiles: more rows, bound by the matrix cores (154 TFLOP/s for a large library
-//    product here).  Tiles of x and W go through two LDS buffers taking turns, 32 k at a time,
-//    rows 160 bytes apart so that the 16-byte reads of a fragment are free of bank conflicts.
-//    384 rows of the 1B shape: q/k/v 310 -> 68 us (71 TFLOP/s; 288 tiles do not come out even
-//    over 256 compute units), output 300 -> 45, gate/up 461 -> 225 (114), down 1100 -> 162.
+//    product here).  Tiles of 16 to 80 rows of x, by what comes out even over the compute units.  384
+//    rows of the 1B shape, us, tiles of 64 x 64 or 64 x 32 with both operands through LDS -> this:
+//    q/k/v 68 -> 50 (98 TFLOP/s), output 45 -> 32 (100), gate/up 225 -> 214 (120), down 162 -> 112 (115).
+//
+// Gated (gate and up rows side by side in a tile, SwiGLU behind the sums): the same bits as the product
+// and the SwiGLU kernel, without the intermediate.  16384 x 2048 at 4 / 16 / 32 / 64 / 384 rows, us, product and
+// SwiGLU kernel -> gated: 27.7 -> 26.2, 30.9 -> 29.2, 39.1 -> 38.6, 48.1 -> 45.5, 221 -> 215.
 // The sums in parts also halve the error and more: 2.1e-7 of the result's norm against 64 bits at
 // K = 2048 (gemm_plain 8.1e-7), 4.1e-7 at 8192 (1.6e-6).
 #include "common.h"
@@ -61,53 +64,104 @@ __device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int k, int e
   return k < end ? v : z;
 }
 
+// silu(gate) * up in float32's own exponential and division, as the SwiGLU kernel has it.
+__device__ __forceinline__ float silu_times(float gate, float up) {
+  const float s = gate / (1.0f + expf(-gate));
+  return s * up;
+}
+
 // ------------------------------------------------------------------ up to 32 rows
-// The sum of a tile's runs, which lie in LDS as [run][group of rows][lane], for rows t * 16 .. + 15
-// of x: stored by one wave.
-template <int TG>
-__device__ __forceinline__ void store_tile(const float* red, int runs, int t, int tile, int rows,
-                                           float* Y, int T, int N, long long ldy, int vec_out) {
-  const int lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
-  f32x4 s;
-  for (int q0 = 0; q0 < runs; q0 += kPartRuns) {
-    f32x4 p = *(const f32x4*)(red + (q0 * TG + t) * 256 + lane * 4);
-    for (int q = q0 + 1; q < min(runs, q0 + kPartRuns); ++q)
-      p += *(const f32x4*)(red + (q * TG + t) * 256 + lane * 4);
-    s = q0 == 0 ? p : s + p;
-  }
-  const int token = t * 16 + r, n = tile * rows + 4 * g;
-  if (token >= T || 4 * g >= rows) return;
-  float* y = Y + token * ldy + n;
-  if (vec_out && n + 4 <= N) {
+// What a call computes: Y (T, N) = X W^T, or gated, with W (2 N, K) gate rows then up rows, Y =
+// silu(gate) * up.
+struct F32Args {
+  const float* X;
+  const float* W;
+  float* Y;
+  int T, N, K, run;
+  long long ldx, ldw, ldy;
+  int vec;                     // rows of Y lie on 16-byte boundaries
+};
+
+// The weight row that lane r of a tile's products holds; rows: weight rows of a tile (lanes beyond
+// hold a row twice), gated 8 gate rows and the 8 up rows of the same columns.
+template <bool GATED>
+__device__ __forceinline__ int weight_row(int tile, int r, int rows, int N) {
+  if (GATED) return min(tile * 8 + r % 8, N - 1) + (r < 8 ? 0 : N);
+  return min(tile * rows + (r < rows ? r : r - rows), N - 1);
+}
+
+// Columns n .. n + 3 of a token's row.
+__device__ __forceinline__ void store_four(const F32Args& a, f32x4 s, int token, int n) {
+  float* y = a.Y + token * a.ldy + n;
+  if (a.vec && n + 4 <= a.N) {
     *(f32x4*)y = s;
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (n + i < N) y[i] = s[i];
+      if (n + i < a.N) y[i] = s[i];
   }
+}
+
+// The gated results of a wave's 16 weight rows, columns n0 .. n0 + 7 of a lane's token.  Lanes below 32
+// hold the gates of four columns, lane + 32 the ups of the same: the lower takes the first two columns,
+// the upper the last two (half of the exponentials each).
+__device__ __forceinline__ void store_gated(const F32Args& a, f32x4 s, int token, int n0) {
+  const int lane = threadIdx.x % 64, g = lane / 16;
+  float o[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float other = __shfl_xor(lane < 32 ? s[2 + i] : s[i], 32, 64);
+    o[i] = silu_times(lane < 32 ? s[i] : other, lane < 32 ? other : s[2 + i]);
+  }
+  const int n = n0 + (g & 1) * 4 + (g >> 1) * 2;
+  if (token >= a.T) return;
+  float* y = a.Y + token * a.ldy + n;
+  if (n < a.N) y[0] = o[0];
+  if (n + 1 < a.N) y[1] = o[1];
+}
+
+// The sum of a tile's runs, which lie in LDS as [run][group of rows][lane], for rows t * 16 .. + 15
+// of x: stored by one wave.
+template <int TG, bool GATED>
+__device__ __forceinline__ void store_tile(const F32Args& a, const float* red, int runs, int t,
+                                           int tile, int rows) {
+  const int lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  f32x4 s;
+  for (int q0 = 0; q0 < runs; q0 += kPartRuns) {
+    f32x4 v[kPartRuns];
+#pragma unroll
+    for (int q = 0; q < kPartRuns; ++q)
+      v[q] = *(const f32x4*)(red + (min(q0 + q, runs - 1) * TG + t) * 256 + lane * 4);
+#pragma unroll
+    for (int q = 1; q < kPartRuns; ++q)
+      if (q0 + q < runs) v[0] += v[q];
+    s = q0 == 0 ? v[0] : s + v[0];
+  }
+  const int token = t * 16 + r;
+  if (GATED) store_gated(a, s, token, tile * 8);
+  else if (token < a.T && 4 * g < rows) store_four(a, s, token, tile * rows + 4 * g);
 }
 
 // Runs of at most 128 k: a wave per run, x in registers.  TG groups of 16 rows of x.  CUT: not
 // every run is 128 k.
-template <int TG, bool CUT>
+template <int TG, bool CUT, bool GATED>
 __global__ __launch_bounds__(kMaxRuns * 64) void gemm_f32_stream_kernel(
-    const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int T, int N,
-    int K, int run, int tiles, long long ldx, long long ldw, long long ldy, int vec_out) {
+    const F32Args a, int tiles) {
   extern __shared__ __attribute__((aligned(16))) float red[];   // [2][runs][TG][64 lanes][4]
   constexpr int J = 8;                                          // steps of 16 k
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, waves = blockDim.x / 64;
   const int r = lane % 16, g = lane / 16;
-  const int k0 = wave * run, k1 = min(K, k0 + run);             // this wave's run
+  const int run = a.run, k0 = wave * run, k1 = min(a.K, k0 + run);   // this wave's run
   f32x4 x[TG][J], w[2][J];
 #pragma unroll
   for (int t = 0; t < TG; ++t) {
-    const float* xr = X + (long long)min(t * 16 + r, T - 1) * ldx;
+    const float* xr = a.X + (long long)min(t * 16 + r, a.T - 1) * a.ldx;
 #pragma unroll
     for (int j = 0; j < J; ++j) x[t][j] = load4<CUT>(xr, k0 + 16 * j + 4 * g, k1);
   }
   const auto ask = [&](f32x4(&wn)[J], int tile) {
     // (past the last tile its last row is read again: no load under a condition)
-    const float* wr = W + (long long)min(tile * 16 + r, N - 1) * ldw;
+    const float* wr = a.W + (long long)weight_row<GATED>(tile, r, 16, a.N) * a.ldw;
 #pragma unroll
     for (int j = 0; j < J; ++j) wn[j] = load4<CUT>(wr, k0 + 16 * j + 4 * g, k1);
   };
@@ -139,31 +193,31 @@ __global__ __launch_bounds__(kMaxRuns * 64) void gemm_f32_stream_kernel(
     __syncthreads();
     // (the next tile writes the other buffer; this one is written again behind the barrier that
     // its readers reach only when they are done)
-    for (int t = wave; t < TG; t += waves) store_tile<TG>(part, waves, t, tile, 16, Y, T, N, ldy, vec_out);
+    for (int t = wave; t < TG; t += waves) store_tile<TG, GATED>(a, part, waves, t, tile, 16);
   }
 }
 
 // Longer runs: a wave per two runs (at most eight waves, so that a lane has 256 registers), each
 // walked in chunks of 64 k; a ring of RING chunks of weights and x keeps RING - 1 of them in
 // flight, over the ends of runs and tiles.  CUT: a run is no multiple of 64, or not all are whole.
-template <int TG, bool CUT>
-__global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(
-    const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int T, int N,
-    int K, int run, int runs, int tiles, long long ldx, long long ldw, long long ldy, int vec_out) {
+template <int TG, bool CUT, bool GATED>
+__global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(const F32Args a, int runs,
+                                                                             int tiles) {
   extern __shared__ __attribute__((aligned(16))) float red[];   // [2][runs][TG][64 lanes][4]
   constexpr int J = 4, RING = TG == 1 ? 5 : 4;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const int r = lane % 16, g = lane / 16;
+  const int run = a.run, K = a.K;
   const int chunks = (run + 16 * J - 1) / (16 * J);             // of a run
   const float* xr[TG];
 #pragma unroll
-  for (int t = 0; t < TG; ++t) xr[t] = X + (long long)min(t * 16 + r, T - 1) * ldx;
+  for (int t = 0; t < TG; ++t) xr[t] = a.X + (long long)min(t * 16 + r, a.T - 1) * a.ldx;
   f32x4 w[RING][J], x[RING][TG][J];
 
   // where the next chunk that is asked for lies
   int a_tile = blockIdx.x, a_run = 0, a_chunk = 0;
   const auto ask = [&](f32x4(&wn)[J], f32x4(&xn)[TG][J]) {
-    const float* wr = W + (long long)min(a_tile * 16 + r, N - 1) * ldw;
+    const float* wr = a.W + (long long)weight_row<GATED>(a_tile, r, 16, a.N) * a.ldw;
     const int k0 = (2 * wave + a_run) * run, k1 = min(K, k0 + run);
     // (a wave's second run may lie past K: the row's last elements are read and, cut, zeroed)
     const int at = k0 + a_chunk * 16 * J + 4 * g;
@@ -211,14 +265,15 @@ __global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(
         const int mine = 2 * wave + m_run;
         if (mine < runs) {
 #pragma unroll
-          for (int t = 0; t < TG; ++t) *(f32x4*)(part + (mine * TG + t) * 256 + lane * 4) = acc[t];
+          for (int t = 0; t < TG; ++t)
+            *(f32x4*)(part + (mine * TG + t) * 256 + lane * 4) = acc[t];
         }
 #pragma unroll
         for (int t = 0; t < TG; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (++m_run == 2) {                            // the end of a tile
           m_run = 0;
           __syncthreads();
-          if (wave < TG) store_tile<TG>(part, runs, wave, tile, 16, Y, T, N, ldy, vec_out);
+          if (wave < TG) store_tile<TG, GATED>(a, part, runs, wave, tile, 16);
           buf ^= 1;
           tile += gridDim.x;
           if (tile >= tiles) break;
@@ -239,30 +294,29 @@ template <int RW, int XW>
 __host__ __device__ constexpr int ring_chunks() {
   return std::min(6, 16384 / ((RW + XW) * 1024));
 }
-template <int RW, int XW>
-__global__ __launch_bounds__(512) void gemm_f32_ring_kernel(
-    const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int T, int N,
-    int run, int tiles, uint32_t ldx, uint32_t ldw, long long ldy, int vec_out) {
+template <int RW, int XW, bool GATED>
+__global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int tiles) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
   constexpr int PER = RW + XW, CHUNK = PER * 1024, NB = ring_chunks<RW, XW>();
   typedef __attribute__((address_space(3))) void* lds_ptr;
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring_smem[];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int r = lane % 16, g = lane / 16;
+  const uint32_t ldx = (uint32_t)a.ldx, ldw = (uint32_t)a.ldw;
   unsigned char* ring = ring_smem + wave * NB * CHUNK;
   float* red = (float*)(ring_smem + 8 * NB * CHUNK);            // [2][16 runs][64 lanes][4]
-  const int chunks = run / 64 * 2;                              // of this wave's two runs
-  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(X + 2 * wave * run), 0, 0xffffffff, 0x00027000);
-  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(W + 2 * wave * run), 0, 0xffffffff, 0x00027000);
+  const int chunks = a.run / 64 * 2;                            // of this wave's two runs
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + 2 * wave * a.run), 0, 0xffffffff, 0x00027000);
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + 2 * wave * a.run), 0, 0xffffffff, 0x00027000);
   // instruction i brings rows 4 i .. + 3 of a chunk, 16 lanes a row
   uint32_t src[PER];
   const auto place = [&](int row) { return (uint32_t)((r ^ (row & 15)) * 16); };
 #pragma unroll
-  for (int i = 0; i < XW; ++i) src[RW + i] = (uint32_t)min(4 * i + g, T - 1) * ldx * 4 + place(4 * i + g);
+  for (int i = 0; i < XW; ++i) src[RW + i] = (uint32_t)min(4 * i + g, a.T - 1) * ldx * 4 + place(4 * i + g);
   const auto weight_rows = [&](int tile) {
 #pragma unroll
     for (int i = 0; i < RW; ++i)
-      src[i] = (uint32_t)min(tile * 4 * RW + 4 * i + g, N - 1) * ldw * 4 + place(4 * i + g);
+      src[i] = (uint32_t)weight_row<GATED>(tile, 4 * i + g, 4 * RW, a.N) * ldw * 4 + place(4 * i + g);
   };
   int a_tile = blockIdx.x, a_chunk = 0;
   const auto ask = [&](int buf) {
@@ -285,7 +339,7 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(
 #pragma unroll
   for (int b = 0; b < NB; ++b) ask(b);
   const int w_row = r < 4 * RW ? r : r - 4 * RW, x_row = min(r, 4 * XW - 1);
-  int buf = 0, side = 0;
+  int buf = 0, side = 0, turn = 0;
   for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, side ^= 1) {
     float* part = red + side * 16 * 256;
 #pragma unroll 1
@@ -316,225 +370,269 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(
     __syncthreads();
     // (the next tile writes the other side; this one is written again behind the barrier that its
     // reader reaches only when it is done)
-    if (wave == 0) store_tile<1>(part, 16, 0, tile, 4 * RW, Y, T, N, ldy, vec_out);
+    // (the waves take turns: the one that stores is behind the others when the next tile ends)
+    if (wave == turn) store_tile<1, GATED>(a, part, 16, 0, tile, 4 * RW);
+    turn = (turn + 1) % 8;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // (loads past the last tile)
 #endif
 }
 
 // ------------------------------------------------------------------ more rows
-// Tile of BM rows of x and BN weight rows by G groups of four waves, each group with its own
-// LDS tiles and 1 / G of the parts of k; the waves of a group as 2 x 2, each BM / 2 x BN / 2.  At
-// the end the first group adds the parts of the others to its own, in order.  CUT: k does not
-// come out even (K no multiple of 32, the last run or the last parts not whole).
-template <int BM, int BN, int G, bool CUT>
-__global__ __launch_bounds__(256 * G) void gemm_f32_tiles_kernel(
-    const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int T, int N,
-    int K, int run, int tiles_m, int tiles, int share, long long ldx, long long ldw, long long ldy,
-    int vec_out) {
-  constexpr int BK = 32, STRIDE = BK + 8;            // floats; 160 bytes a row
-  constexpr int MI = BM / 32, NI = BN / 32;          // 16 x 16 blocks of a wave
-  constexpr int LOADS = (BM + BN) * (BK / 4) / 256;  // 16-byte pieces a thread stages
-  constexpr int TILE = (BM + BN) * STRIDE;
-  extern __shared__ __attribute__((aligned(16))) float smem[];   // [G][2][TILE]
+// Tile of 16 * MI rows of x and 64 weight rows by G groups of four waves, each group with 1 / G of
+// the parts of k, 32 k a step.  A wave takes all rows of x and 16 weight rows, which no other wave
+// needs: they go from memory into its registers, two steps ahead.  x goes through LDS (two buffers
+// taking turns, two more steps on their way; rows 160 bytes apart, so that the 16-byte reads of a
+// fragment are free of bank conflicts).  At the end the first group adds the parts of the others to its
+// own, in order.  CUT: K is not sixteen whole runs.  GATED: a wave's weight rows are 8 gate rows and the 8 up rows of the same columns.
+constexpr int kTileStride = 32 + 8;                  // floats
+template <int MI, int G>
+constexpr int tile_bytes() {
+  return G * 2 * 16 * MI * kTileStride * 4;
+}
+template <int MI, int G, bool CUT, bool GATED>
+__global__ __launch_bounds__(256 * G, 4) void gemm_f32_tiles_kernel(const F32Args a, int tiles_m,
+                                                                    int tiles, int share) {
+  constexpr int BM = 16 * MI, BK = 32, D = 2, COLS = GATED ? 32 : 64;
+  constexpr int LOADS = (MI + 1) / 2;                // 16-byte pieces of x a thread stages
+  extern __shared__ __attribute__((aligned(16))) float smem[];   // [G][2][BM][kTileStride]
   // workgroups of one die (blockIdx % 8) take neighbouring tiles, the tiles of x fastest, so
   // that its L2 serves the weight rows that they share
   const int tile = (int)(blockIdx.x % 8) * share + (int)(blockIdx.x / 8);
   if (tile >= tiles) return;
-  const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * BN;
-  const int group = G == 1 ? 0 : threadIdx.x / 256;
+  const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * COLS;
+  const int group = threadIdx.x / 256;
   const int tid = threadIdx.x % 256, lane = tid % 64, wave = tid / 64;
   const int r = lane % 16, g = lane / 16;
-  const int wm = wave / 2 * (BM / 2), wn = wave % 2 * (BN / 2);
-  float* lds = smem + group * 2 * TILE;
-  const int span = kMaxRuns / G * run;               // a multiple of 64
+  float* lds = smem + group * 2 * BM * kTileStride;
+  const int run = a.run, K = a.K;
+  const int span = kMaxRuns / G * run;
   const int k_begin = group * span;
-  const int k_count = G > 1 ? span : ((K + run - 1) / run * run + BK - 1) / BK * BK;
+  const int k_count = span;                          // (a multiple of 64)
 
+  const float* wr = a.W + (long long)weight_row<GATED>(tile / tiles_m * 4 + wave, r, 16, a.N) * a.ldw;
   const float* src[LOADS];
-  int dst[LOADS], kk[LOADS];
+  const int xk = k_begin + tid % 8 * 4;
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int p = tid + i * 256, rw = p / (BK / 4);  // rows of x first, then weight rows
-    kk[i] = k_begin + p % (BK / 4) * 4;
-    dst[i] = rw * STRIDE + p % (BK / 4) * 4;
-    src[i] = rw < BM ? X + (long long)min(m0 + rw, T - 1) * ldx
-                     : W + (long long)min(n0 + rw - BM, N - 1) * ldw;
-  }
+  for (int i = 0; i < LOADS; ++i)
+    src[i] = a.X + (long long)min(m0 + tid / 8 + i * 32, a.T - 1) * a.ldx;
   // acc: the run under way; part: its part so far; total: the parts (of the first group their
   // sum, of a later one the first of its two)
-  f32x4 total[NI][MI], part[NI][MI], acc[NI][MI], st[LOADS];
+  f32x4 total[MI], part[MI], acc[MI];
   int part_runs = 0, parts = 0;
 #pragma unroll
-  for (int a = 0; a < NI; ++a) {
-#pragma unroll
-    for (int b = 0; b < MI; ++b) total[a][b] = part[a][b] = acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int b = 0; b < MI; ++b) total[b] = part[b] = acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
   const auto end_part = [&]() {
-    if (group == 0 || parts == 0) {
+    if (G < 4 && (group == 0 || parts == 0)) {
 #pragma unroll
-      for (int a = 0; a < NI; ++a) {
-#pragma unroll
-        for (int b = 0; b < MI; ++b)
-          total[a][b] = parts == 0 ? part[a][b] : total[a][b] + part[a][b];
-      }
+      for (int b = 0; b < MI; ++b) total[b] = parts == 0 ? part[b] : total[b] + part[b];
     }
     part_runs = 0;
     ++parts;
   };
+  f32x4 w[D][2], x[D][LOADS];
+  const auto ask_x = [&](f32x4(&xn)[LOADS], int k0) {
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) st[i] = load4<CUT>(src[i], kk[i], K);
+    for (int i = 0; i < LOADS; ++i) xn[i] = load4<CUT>(src[i], xk + k0, K);
+  };
+  const auto keep_x = [&](const f32x4(&xn)[LOADS], int buf) {
 #pragma unroll
-  for (int i = 0; i < LOADS; ++i) *(f32x4*)(lds + dst[i]) = st[i];
-  __syncthreads();
-  int buf = 0, left = run;                           // k left of the run
-  for (int k0 = 0; k0 < k_count; k0 += BK, buf ^= 1) {
+    for (int i = 0; i < LOADS; ++i) {
+      if (MI % 2 == 0 || i + 1 < LOADS || tid < 128)
+        *(f32x4*)(lds + (buf * BM + tid / 8 + i * 32) * kTileStride + tid % 8 * 4) = xn[i];
+    }
+  };
+  int left = run;                                    // k left of the run
+  const auto step = [&](f32x4(&wn)[2], f32x4(&x_ask)[LOADS], const f32x4(&x_keep)[LOADS], int k0, int buf) {
+    ask_x(x_ask, k0 + D * BK);
+    const float* xs = lds + (buf * BM + r) * kTileStride + 4 * g;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) st[i] = load4<CUT>(src[i], k0 + BK + kk[i], K);
-    const float* xs = lds + buf * TILE + (wm + r) * STRIDE + 4 * g;
-    const float* ws = lds + buf * TILE + (BM + wn + r) * STRIDE + 4 * g;
+    for (int h = 0; h < 2; ++h) {
+      f32x4 xv[MI];
 #pragma unroll
-    for (int h = 0; h < BK; h += 16) {
-      f32x4 x[MI], w[NI];
-#pragma unroll
-      for (int b = 0; b < MI; ++b) x[b] = *(const f32x4*)(xs + b * 16 * STRIDE + h);
-#pragma unroll
-      for (int a = 0; a < NI; ++a) w[a] = *(const f32x4*)(ws + a * 16 * STRIDE + h);
+      for (int b = 0; b < MI; ++b) xv[b] = *(const f32x4*)(xs + b * 16 * kTileStride + h * 16);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int a = 0; a < NI; ++a) {
-#pragma unroll
-          for (int b = 0; b < MI; ++b) acc[a][b] = mfma_f32(w[a][i], x[b][i], acc[a][b]);
-        }
+        for (int b = 0; b < MI; ++b) acc[b] = mfma_f32(wn[h][i], xv[b][i], acc[b]);
       }
+      wn[h] = load4<CUT>(wr, k_begin + k0 + D * BK + h * 16 + 4 * g, K);
       left -= 16;
       if (left == 0) {                               // the end of a run
         left = run;
 #pragma unroll
-        for (int a = 0; a < NI; ++a) {
-#pragma unroll
-          for (int b = 0; b < MI; ++b) {
-            part[a][b] = part_runs == 0 ? acc[a][b] : part[a][b] + acc[a][b];
-            acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
+        for (int b = 0; b < MI; ++b) {
+          part[b] = part_runs == 0 ? acc[b] : part[b] + acc[b];
+          acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
         if (++part_runs == kPartRuns) end_part();
       }
     }
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) *(f32x4*)(lds + (buf ^ 1) * TILE + dst[i]) = st[i];
+    keep_x(x_keep, buf ^ 1);
     __syncthreads();
+  };
+#pragma unroll
+  for (int q = 0; q < D; ++q) {
+    ask_x(x[q], q * BK);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) w[q][h] = load4<CUT>(wr, k_begin + q * BK + h * 16 + 4 * g, K);
+  }
+  keep_x(x[0], 0);
+  __syncthreads();
+  for (int k0 = 0; k0 < k_count; k0 += D * BK) {
+#pragma unroll
+    for (int q = 0; q < D; ++q) step(w[q], x[q], x[(q + 1) % D], k0 + q * BK, q % 2);
   }
   if (part_runs > 0) end_part();
-  if (G > 1) {
-    // [group - 1][the group's part][wave][block][lane]
-    constexpr int EACH = 4 / G;
-    static_assert((G - 1) * EACH * BM * BN <= G * 2 * TILE, "the parts fit the tiles' LDS");
-    f32x4* hand = (f32x4*)smem;
-    const auto place = [&](int q, int a, int b) {
-      return hand + (((q * 4 + wave) * NI + a) * MI + b) * 64 + lane;
-    };
-    if (group > 0) {
+  if (G == 4) {
 #pragma unroll
-      for (int a = 0; a < NI; ++a) {
-#pragma unroll
-        for (int b = 0; b < MI; ++b) {
-          *place((group - 1) * EACH, a, b) = total[a][b];
-          if (EACH > 1) *place((group - 1) * EACH + 1, a, b) = part[a][b];
-        }
-      }
-    }
-    __syncthreads();
-    if (group > 0) return;
-#pragma unroll
-    for (int q = 0; q < (G - 1) * EACH; ++q) {
-#pragma unroll
-      for (int a = 0; a < NI; ++a) {
-#pragma unroll
-        for (int b = 0; b < MI; ++b) total[a][b] += *place(q, a, b);
-      }
-    }
+    for (int b = 0; b < MI; ++b) total[b] = part[b];
   }
-#pragma unroll
-  for (int a = 0; a < NI; ++a) {
+  // [group - 1][the group's part][wave][block][lane]
+  constexpr int EACH = 4 / G;
+  static_assert((G - 1) * EACH * 4 * MI * 1024 <= tile_bytes<MI, G>(), "the parts fit the tiles' LDS");
+  f32x4* hand = (f32x4*)smem;
+  const auto place = [&](int q, int b) { return hand + ((q * 4 + wave) * MI + b) * 64 + lane; };
+  if (group > 0) {
 #pragma unroll
     for (int b = 0; b < MI; ++b) {
-      const f32x4 s = total[a][b];
-      const int token = m0 + wm + b * 16 + r, n = n0 + wn + a * 16 + 4 * g;
-      if (token >= T) continue;
-      float* y = Y + token * ldy + n;
-      if (vec_out && n + 4 <= N) {
-        *(f32x4*)y = s;
-      } else {
+      *place((group - 1) * EACH, b) = total[b];
+      if (EACH > 1) *place((group - 1) * EACH + 1, b) = part[b];
+    }
+  }
+  __syncthreads();
+  if (group > 0) return;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (n + i < N) y[i] = s[i];
-      }
+  for (int q = 0; q < (G - 1) * EACH; ++q) {
+#pragma unroll
+    for (int b = 0; b < MI; ++b) total[b] += *place(q, b);
+  }
+#pragma unroll
+  for (int b = 0; b < MI; ++b) {
+    const int token = m0 + b * 16 + r;
+    if (GATED) {
+      store_gated(a, total[b], token, n0 + wave * 8);
+    } else if (token < a.T) {
+      store_four(a, total[b], token, n0 + wave * 16 + 4 * g);
     }
   }
 }
 
-template <int RW, int XW>
-int launch_ring(const float* X, const float* W, float* Y, int T, int N, int run, int cus, long long ldx,
-                long long ldw, long long ldy, int vec, hipStream_t stream) {
+template <int RW, int XW, bool GATED>
+int launch_ring(const F32Args& a, int cus, hipStream_t stream) {
   static LdsGrant grant;
   constexpr int bytes = 8 * ring_chunks<RW, XW>() * (RW + XW) * 1024 + 2 * 16 * 1024;
-  const auto kernel = gemm_f32_ring_kernel<RW, XW>;
+  const auto kernel = gemm_f32_ring_kernel<RW, XW, GATED>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_f32: %s", hipGetErrorString(e));
-  const int tiles = ceil_div(N, 4 * RW);
-  kernel<<<std::min(tiles, cus), 512, bytes, stream>>>(X, W, Y, T, N, run, tiles, (uint32_t)ldx,
-                                                       (uint32_t)ldw, ldy, vec);
+  const int tiles = ceil_div(a.N, GATED ? 8 : 4 * RW);
+  kernel<<<std::min(tiles, cus), 512, bytes, stream>>>(a, tiles);
   return 0;
 }
 
-template <int TG>
-void launch_stream(const float* X, const float* W, float* Y, int T, int N, int K, int run, int cus,
-                   long long ldx, long long ldw, long long ldy, int vec, hipStream_t stream) {
-  const int tiles = ceil_div(N, 16), runs = ceil_div(K, run), lds = 2 * runs * TG * 1024;
-  if (run <= 128) {
+template <int TG, bool GATED>
+void launch_stream(const F32Args& a, int cus, hipStream_t stream) {
+  const int tiles = ceil_div(a.N, GATED ? 8 : 16), runs = ceil_div(a.K, a.run), lds = 2 * runs * TG * 1024;
+  if (a.run <= 128) {
     // as many workgroups as the registers of a compute unit hold (128 a lane at 16 waves)
     const int grid = std::min(tiles, cus * std::max(1, kMaxRuns / runs));
-    const auto kernel = K % run || run != 128 ? gemm_f32_stream_kernel<TG, true>
-                                              : gemm_f32_stream_kernel<TG, false>;
-    kernel<<<grid, runs * 64, lds, stream>>>(X, W, Y, T, N, K, run, tiles, ldx, ldw, ldy, vec);
+    const auto kernel = a.K % a.run || a.run != 128 ? gemm_f32_stream_kernel<TG, true, GATED>
+                                                    : gemm_f32_stream_kernel<TG, false, GATED>;
+    kernel<<<grid, runs * 64, lds, stream>>>(a, tiles);
   } else {
-    const auto kernel = K % run || runs % 2 || run % 64 ? gemm_f32_stream_long_kernel<TG, true>
-                                                        : gemm_f32_stream_long_kernel<TG, false>;
-    kernel<<<std::min(tiles, cus), ceil_div(runs, 2) * 64, lds, stream>>>(
-        X, W, Y, T, N, K, run, runs, tiles, ldx, ldw, ldy, vec);
+    const auto kernel = a.K % a.run || runs % 2 || a.run % 64 ? gemm_f32_stream_long_kernel<TG, true, GATED>
+                                                              : gemm_f32_stream_long_kernel<TG, false, GATED>;
+    kernel<<<std::min(tiles, cus), ceil_div(runs, 2) * 64, lds, stream>>>(a, runs, tiles);
   }
 }
 
-template <int BM, int BN, int G, bool CUT>
-int launch_tiles_form(const float* X, const float* W, float* Y, int T, int N, int K, int run,
-                      long long ldx, long long ldw, long long ldy, int vec, hipStream_t stream) {
+template <int MI, int G, bool CUT, bool GATED>
+int launch_tiles_form(const F32Args& a, hipStream_t stream) {
   static LdsGrant grant;
-  constexpr int bytes = G * 2 * (BM + BN) * 40 * 4;
-  const auto kernel = gemm_f32_tiles_kernel<BM, BN, G, CUT>;
+  constexpr int bytes = tile_bytes<MI, G>();
+  const auto kernel = gemm_f32_tiles_kernel<MI, G, CUT, GATED>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_f32: %s", hipGetErrorString(e));
-  const int tm = ceil_div(T, BM), tiles = tm * ceil_div(N, BN), share = ceil_div(tiles, 8);
-  kernel<<<share * 8, 256 * G, bytes, stream>>>(X, W, Y, T, N, K, run, tm, tiles, share, ldx, ldw,
-                                                ldy, vec);
+  const int tm = ceil_div(a.T, 16 * MI), tiles = tm * ceil_div(a.N, GATED ? 32 : 64);
+  const int share = ceil_div(tiles, 8);
+  kernel<<<share * 8, 256 * G, bytes, stream>>>(a, tm, tiles, share);
   return 0;
 }
 
-template <int BM, int BN, int G>
-int launch_tiles(const float* X, const float* W, float* Y, int T, int N, int K, int run,
-                 long long ldx, long long ldw, long long ldy, int vec, hipStream_t stream) {
-  const bool cut = K % 32 || K % run || (G > 1 && kMaxRuns * run != K);
-  return cut ? launch_tiles_form<BM, BN, G, true>(X, W, Y, T, N, K, run, ldx, ldw, ldy, vec, stream)
-             : launch_tiles_form<BM, BN, G, false>(X, W, Y, T, N, K, run, ldx, ldw, ldy, vec, stream);
+template <int MI, int G, bool GATED>
+int launch_tiles(const F32Args& a, hipStream_t stream) {
+  return a.K == kMaxRuns * a.run ? launch_tiles_form<MI, G, false, GATED>(a, stream)
+                                 : launch_tiles_form<MI, G, true, GATED>(a, stream);
+}
+
+template <bool GATED>
+int by_rows(const F32Args& a, int cus, hipStream_t stream) {
+  const int T = a.T, rows_of_w = GATED ? 2 * a.N : a.N;
+  // Rows whose bytes a buffer's 32-bit offset reaches.  More than 4 rows bring half as much x as W
+  // into the rings and more: over more than eight tiles a compute unit the stream kernel, which
+  // keeps x of short runs in registers, is ahead (128256 x 2048 at 16 rows: 192 us against 242, at 8
+  // no slower than the 192; 16384 x 2048, four tiles, 16 rows: 33 against 27).
+  const bool ring = a.K % 1024 == 0 && 4 * (a.ldw * (rows_of_w - 1) + a.K) < (1LL << 32) &&
+                    4 * (a.ldx * (T - 1) + a.K) < (1LL << 32) &&
+                    (T <= 4 || a.run > 128 || ceil_div(rows_of_w, 16) <= 8 * cus);
+  if (T <= 16 && ring) {
+    if (GATED) {
+      if (T <= 4) return launch_ring<4, 1, GATED>(a, cus, stream);
+      if (T <= 8) return launch_ring<4, 2, GATED>(a, cus, stream);
+      return launch_ring<4, 4, GATED>(a, cus, stream);
+    }
+    // Tiles of 16 weight rows, or of 12 or 8 where that takes rows off the busiest compute unit
+    // (3072 x 2048 at 4 rows: 8.6 us with 12, 2048 x 2048: 7.9 with 8)
+    int rows = 16, most = ceil_div(ceil_div(a.N, 16), cus) * 16;
+    for (int c = 12; c >= 8; c -= 4) {
+      const int m = ceil_div(ceil_div(a.N, c), cus) * c;
+      if (m < most) { rows = c; most = m; }
+    }
+#define BY_X(RW)                                                     \
+  (T <= 4 ? launch_ring<RW, 1, false>(a, cus, stream)                \
+          : T <= 8 ? launch_ring<RW, 2, false>(a, cus, stream)       \
+                   : launch_ring<RW, 4, false>(a, cus, stream))
+    return rows == 16 ? BY_X(4) : rows == 12 ? BY_X(3) : BY_X(2);
+#undef BY_X
+  }
+  if (T <= 32) {
+    if (T <= 16) launch_stream<1, GATED>(a, cus, stream);
+    else launch_stream<2, GATED>(a, cus, stream);
+    return 0;
+  }
+  // Every tile and number of groups gives the same bits; the matrix cores bound them, so what counts is
+  // the blocks of 16 rows that the busiest compute unit works through: the height that makes least of
+  // rounds of tiles times the time of a round.  A round of 16, 32, ... 80 rows over K = 2048 takes 18, 20,
+  // 30, 38 and 48 us (one of 16 rows is bound by its loads of W, 56 clocks each).  384 rows, by height: 3072 x 2048
+  // 93 / 62 / 62 / 77 / 50 us, 2048 x 2048 58 / 43 / 33 / 40 / 49; 200 rows of 16384 x 2048 244 / 145 / 152 / 154 / 145.
+  // Four groups take a tile's k in quarters where no compute unit has a second tile (2048 x 2048, 384
+  // rows: 33 us against 34 with two, 2048 x 8192: 112 against 119); two otherwise, so that a second tile
+  // works through its first and last steps beside them (16384 x 2048, 384 rows: 212 against 231).
+  const int tn = ceil_div(a.N, GATED ? 32 : 64);
+  constexpr int kRound[] = {0, 18, 20, 30, 38, 48};
+  int mi = 1;
+  long long least = 1LL << 62;
+  for (int m = 5; m > 0; --m) {
+    const long long us = ceil_div_ll((long long)ceil_div(T, 16 * m) * tn, cus) * kRound[m];
+    if (us < least) { least = us; mi = m; }
+  }
+  const bool pairs = (long long)ceil_div(T, 16 * mi) * tn > cus;
+#define GO(M) \
+  case M: return pairs ? launch_tiles<M, 2, GATED>(a, stream) : launch_tiles<M, 4, GATED>(a, stream)
+  switch (mi) {
+    GO(1); GO(2); GO(3); GO(4);
+    default: return launch_tiles<5, 4, GATED>(a, stream);
+  }
+#undef GO
 }
 
 }  // namespace
 
 // Y (T,N) = X (T,K) * W (N,K)^T, float32, row strides in elements; K and the strides of X and W
-// multiples of 4, X and W on 16-byte boundaries.
+// multiples of 4, X and W on 16-byte boundaries.  gated: W (2 N,K) gate rows then up rows, Y =
+// silu(gate) * up.
 RLIS_API int rlis_gemm_f32(const void* X_, const void* W_, void* Y_, int T, int N, int K,
-                           long long ldx, long long ldw, long long ldy, hipStream_t stream) {
+                           long long ldx, long long ldw, long long ldy, int gated, hipStream_t stream) {
   const float *X = (const float*)X_, *W = (const float*)W_;
   float* Y = (float*)Y_;
   RLIS_REQUIRE(T >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes T=%d N=%d K=%d", T, N, K);
@@ -543,62 +641,14 @@ RLIS_API int rlis_gemm_f32(const void* X_, const void* W_, void* Y_, int T, int 
                    (uintptr_t)W % 16 == 0,
                "gemm_f32: K and the strides of x and W must be multiples of 4, x and W on 16-byte "
                "boundaries");
-  RLIS_REQUIRE(ceil_div(T, 64) <= 65535 && N <= (1 << 26), "gemm_f32: T=%d N=%d is too large", T, N);
+  RLIS_REQUIRE(ceil_div(T, 64) <= 65535 && N <= (1 << (gated ? 25 : 26)), "gemm_f32: T=%d N=%d is too large",
+               T, N);
   if (T == 0) return 0;
-  const int run = f32_run(K), cus = rlis_stream_compute_units();
+  const int cus = rlis_stream_compute_units();
   RLIS_REQUIRE(cus > 0, "gemm_f32: cannot read the device properties");
-  const int vec = ldy % 4 == 0 && (uintptr_t)Y % 16 == 0;
-  // Rows whose bytes a buffer's 32-bit offset reaches.  More than 4 rows bring half as much x as W
-  // into the rings and more: over more than eight tiles a compute unit the stream kernel, which
-  // keeps x of short runs in registers, is ahead (128256 x 2048 at 16 rows: 192 us against 242, at 8
-  // no slower than the 192; 16384 x 2048, four tiles, 16 rows: 33 against 27).
-  const bool ring = K % 1024 == 0 && 4 * (ldw * (N - 1) + K) < (1LL << 32) &&
-                    4 * (ldx * (T - 1) + K) < (1LL << 32) &&
-                    (T <= 4 || run > 128 || ceil_div(N, 16) <= 8 * cus);
-  if (T <= 16 && ring) {
-    // Tiles of 16 weight rows, or of 12 or 8 where that takes rows off the busiest compute unit
-    // (3072 x 2048 at 4 rows: 8.6 us with 12, 2048 x 2048: 7.9 with 8)
-    int rows = 16, most = ceil_div(ceil_div(N, 16), cus) * 16;
-    for (int c = 12; c >= 8; c -= 4) {
-      const int m = ceil_div(ceil_div(N, c), cus) * c;
-      if (m < most) { rows = c; most = m; }
-    }
-    int rc;
-#define GO(RW, XW) rc = launch_ring<RW, XW>(X, W, Y, T, N, run, cus, ldx, ldw, ldy, vec, stream)
-#define BY_X(RW)                        \
-  do {                                  \
-    if (T <= 4) GO(RW, 1);              \
-    else if (T <= 8) GO(RW, 2);         \
-    else GO(RW, 4);                     \
-  } while (0)
-    if (rows == 16) BY_X(4);
-    else if (rows == 12) BY_X(3);
-    else BY_X(2);
-#undef BY_X
-#undef GO
-    if (rc) return rc;
-  } else if (T <= 32) {
-    if (T <= 16) launch_stream<1>(X, W, Y, T, N, K, run, cus, ldx, ldw, ldy, vec, stream);
-    else launch_stream<2>(X, W, Y, T, N, K, run, cus, ldx, ldw, ldy, vec, stream);
-  } else {
-    // Every tile and number of groups gives the same bits; the matrix cores bound all of them,
-    // so the compute units should have the same work and four waves a SIMD.  Where half tiles
-    // number at most one a compute unit, four groups take a tile's k in quarters (1B output
-    // projection, 2048 x 2048, 128 rows: 30 us; one group 52); likewise whole tiles (384 rows:
-    // 45 us; one group 64).  Beyond that half tiles only where they save part of a round
-    // (3072 x 2048, 384 rows: 68 us against 77), and two groups up to two tiles a compute unit
-    // (16384 x 2048, 128 rows: 83 us against 89).
-    const int t64 = ceil_div(T, 64) * ceil_div(N, 64), t32 = ceil_div(T, 64) * ceil_div(N, 32);
-    int rc;
-#define GO(BN, G) rc = launch_tiles<64, BN, G>(X, W, Y, T, N, K, run, ldx, ldw, ldy, vec, stream)
-    if (t32 <= cus) GO(32, 4);
-    else if (t64 <= cus) GO(64, 4);
-    else if (ceil_div(t32, cus) < 2 * ceil_div(t64, cus) && t64 <= 2 * cus) GO(32, 1);
-    else if (t64 <= 2 * cus) GO(64, 2);
-    else GO(64, 1);
-#undef GO
-    if (rc) return rc;
-  }
+  const F32Args a = {X, W, Y, T, N, K, f32_run(K), ldx, ldw, ldy, ldy % 4 == 0 && (uintptr_t)Y % 16 == 0};
+  const int rc = gated ? by_rows<true>(a, cus, stream) : by_rows<false>(a, cus, stream);
+  if (rc) return rc;
   RLIS_LAUNCH_CHECK("gemm_f32");
   return 0;
 }

@@ -948,15 +948,20 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         name = "rlis_gemm_bf16_skinny" if T <= SKINNY_MAX_ROWS else "rlis_gemm_bf16_mfma"
         lib.call(name, x.data_ptr(), w.data_ptr(), y.data_ptr(), _DT[out_dtype], T, N, K, ldx,
                  ldw, N, stream)
-    elif (x.dtype == w.dtype == out_dtype == torch.float32 and K % 4 == 0 and ldx % 4 == 0
-          and ldw % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-          and T <= F32_MAX_ROWS and N <= F32_MAX_WEIGHT_ROWS):
-        lib.call("rlis_gemm_f32", x.data_ptr(), w.data_ptr(), y.data_ptr(), T, N, K, ldx, ldw, N,
+    elif out_dtype == torch.float32 and _f32_kernels(x, w, ldx, ldw):
+        lib.call("rlis_gemm_f32", x.data_ptr(), w.data_ptr(), y.data_ptr(), T, N, K, ldx, ldw, N, 0,
                  stream)
     else:
         lib.call("rlis_gemm_plain", x.data_ptr(), _dt(x), w.data_ptr(), _dt(w), y.data_ptr(),
                  _DT[out_dtype], T, N, K, ldx, ldw, N, stream)
     return y
+
+
+def _f32_kernels(x: torch.Tensor, w: torch.Tensor, ldx: int, ldw: int) -> bool:
+    """Whether the 32-bit kernels (gemm_f32.hip) take ``x @ w.T`` with rows ``ldx`` and ``ldw`` apart."""
+    return (x.dtype == w.dtype == torch.float32 and x.shape[1] % 4 == 0 and ldx % 4 == 0 and ldw % 4 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.shape[0] <= F32_MAX_ROWS and w.shape[0] <= F32_MAX_WEIGHT_ROWS)
 
 
 def can_fuse_norm_linear(resid: torch.Tensor, w: torch.Tensor, rows: Optional[int] = None
@@ -1115,9 +1120,9 @@ def linear_scaled(xw: torch.Tensor, ss: torch.Tensor, eps: float, w: torch.Tenso
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]`` of shape ``(2 I, K)``.
 
-    Up to 16 rows of bfloat16 (32 over short rows), and 17 to 64 of sizes that ``_rows_kernel`` takes,
-    go through one kernel that never stores the ``(T, 2 I)`` intermediate; everything else is the
-    product followed by the SwiGLU kernel."""
+    Up to 16 rows of bfloat16 (32 over short rows), 17 to 64 of sizes that ``_rows_kernel`` takes, and
+    float32 that ``_f32_kernels`` takes (the same bits) go through one kernel that never stores the
+    ``(T, 2 I)`` intermediate; everything else is the product followed by the SwiGLU kernel."""
     T, K = x.shape
     two_i = w_gate_up.shape[0]
     if two_i % 2:
@@ -1133,6 +1138,11 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
         (BF16_GEMM == "own" or T <= STREAM_MAX_ROWS)
     if fusable and not streamed and K == w_gate_up.shape[1] and _rows_kernel(x, w_gate_up, gated=True):
         return _rows_linear(x, w_gate_up, torch.bfloat16, gated=True)
+    if T > 0 and two_i > 0 and K == w_gate_up.shape[1] and _f32_kernels(x, w_gate_up, ldx, ldw):
+        y = torch.empty((T, two_i // 2), dtype=torch.float32, device=x.device)
+        lib.call("rlis_gemm_f32", x.data_ptr(), w_gate_up.data_ptr(), y.data_ptr(), T, two_i // 2, K, ldx,
+                 ldw, two_i // 2, 1, lib.stream_ptr())
+        return y
     if not (streamed or skinny):
         return swiglu(linear(x, w_gate_up, x.dtype))
     y = torch.empty((T, two_i // 2), dtype=torch.bfloat16, device=x.device)

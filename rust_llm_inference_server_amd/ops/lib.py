@@ -66,7 +66,7 @@ _SIGNATURES = {
     "rlis_norm_rope_kv_write": [P, I, L, I, I, I, I, I, I, I, I, F, P, P, P, P, P, P, I, I, I, P],
     "rlis_copy_pages": [P, I, I, L, L, P, P, I, P],
     "rlis_gemm_plain": [P, I, P, I, P, I, I, I, I, L, L, L, P],
-    "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, P],
+    "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, I, P],
     "rlis_gemm_bf16_rows": [P, P, P, I, I, I, I, I, L, L, L, L, P, I, I, F, I, P],
     "rlis_gemm_bf16_mfma": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny": [P, P, P, I, I, I, I, L, L, L, P],
