@@ -142,13 +142,14 @@ __device__ __forceinline__ void store_tile(const F32Args& a, const float* red, i
   else if (token < a.T && 4 * g < rows) store_four(a, s, token, tile * rows + 4 * g);
 }
 
-// Runs of at most 128 k: a wave per run, x in registers.  TG groups of 16 rows of x.  CUT: not
-// every run is 128 k.
-template <int TG, bool CUT, bool GATED>
+// Runs of at most 16 J k: a wave per run, x in registers.  TG groups of 16 rows of x.  CUT: not
+// every run is 16 J k.  J as small as holds a run: what a load of a place past it costs (56 clocks of its
+// compute unit) is most of a small model's product (192 and 640 x 192, 3 rows: 6.5 to 7 us with places for
+// 128 k, 3.3 to 4 with 16).
+template <int TG, int J, bool CUT, bool GATED>
 __global__ __launch_bounds__(kMaxRuns * 64) void gemm_f32_stream_kernel(
     const F32Args a, int tiles) {
   extern __shared__ __attribute__((aligned(16))) float red[];   // [2][runs][TG][64 lanes][4]
-  constexpr int J = 8;                                          // steps of 16 k
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, waves = blockDim.x / 64;
   const int r = lane % 16, g = lane / 16;
   const int run = a.run, k0 = wave * run, k1 = min(a.K, k0 + run);   // this wave's run
@@ -536,8 +537,11 @@ void launch_stream(const F32Args& a, int cus, hipStream_t stream) {
   if (a.run <= 128) {
     // as many workgroups as the registers of a compute unit hold (128 a lane at 16 waves)
     const int grid = std::min(tiles, cus * std::max(1, kMaxRuns / runs));
-    const auto kernel = a.K % a.run || a.run != 128 ? gemm_f32_stream_kernel<TG, true, GATED>
-                                                    : gemm_f32_stream_kernel<TG, false, GATED>;
+    const auto kernel = a.run == 16   ? gemm_f32_stream_kernel<TG, 1, true, GATED>
+                        : a.run == 32 ? gemm_f32_stream_kernel<TG, 2, true, GATED>
+                        : a.run <= 64 ? gemm_f32_stream_kernel<TG, 4, true, GATED>
+                        : a.K % a.run || a.run != 128 ? gemm_f32_stream_kernel<TG, 8, true, GATED>
+                                                      : gemm_f32_stream_kernel<TG, 8, false, GATED>;
     kernel<<<grid, runs * 64, lds, stream>>>(a, tiles);
   } else {
     const auto kernel = a.K % a.run || runs % 2 || a.run % 64 ? gemm_f32_stream_long_kernel<TG, true, GATED>
