@@ -87,20 +87,31 @@ __device__ __forceinline__ float xor32_max(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// The value of the lane N further on, round the row of sixteen.
+template <int N>
+__device__ __forceinline__ float row_turn(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+
+// Sum and maximum over a wave; every lane gets the result.  Behind the steps over 32, 16 and 8 lanes a
+// value repeats every 8 lanes of a row, and so on: the lane 4 (2, 1) further on holds what lane ^ 4 holds.
+// In the vector unit: a general shuffle goes through LDS, some 100 clocks a step.
 __device__ __forceinline__ float wave_sum(float v) {
   v = xor32_sum(v);
   v = xor16_sum(v);
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+  v += row_turn<8>(v);
+  v += row_turn<4>(v);
+  v += row_turn<2>(v);
+  return v + row_turn<1>(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
   v = xor32_max(v);
   v = xor16_max(v);
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+  v = fmaxf(v, row_turn<8>(v));
+  v = fmaxf(v, row_turn<4>(v));
+  v = fmaxf(v, row_turn<2>(v));
+  return fmaxf(v, row_turn<1>(v));
 }
 
 // Sum over a block of NT threads (NT a multiple of 64); every thread gets the result.  The
