@@ -25,6 +25,7 @@
 //    KV head, so K and V are read once per group; contexts are split into partitions.
 //  * attn_reduce: merges the partitions.
 #include "common.h"
+#include "gemm_stream.h"
 
 #include <float.h>
 #include <math.h>
@@ -387,12 +388,12 @@ template <> struct Vec16<bf16_t> {
 template <typename TX, int G, int DPL>
 __global__ __launch_bounds__(256) void attn_decode_kernel(
     const TX* __restrict__ q, long long q_stride, TX* __restrict__ out, long long out_stride,
-    float* __restrict__ part_ml, float* __restrict__ part_acc, const TX* __restrict__ k_pages,
-    const TX* __restrict__ v_pages, const int* __restrict__ block_tables, int max_pages,
+    float* __restrict__ part_ml, float* __restrict__ part_acc, const TX* k_pages,
+    const TX* v_pages, const int* __restrict__ block_tables, int max_pages,
     const int* __restrict__ ctx_lens, const int* __restrict__ token_rows, int nh, int nkv, int d,
     int page_size, float scale, int window, int splits, int chunks_per_kv, int part_keys,
     int max_parts, const float* __restrict__ slopes, const float* __restrict__ head_scales,
-    float softcap, const float* __restrict__ sinks, int keep_first, int chunk_len) {
+    float softcap, const float* __restrict__ sinks, int keep_first, int chunk_len, DecodeRope rope) {
   extern __shared__ float smem[];
   float* q_s = smem;                     // G * d
   float* p_s = q_s + G * d;              // 4 waves * G * 64
@@ -414,10 +415,32 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const int kbeg = lo + split * part;
   const int kend = min(ctx, kbeg + part);
 
+  // Dim j of a head turned by its position's angles (rotate-half).
+  const TX* qrow = q + (long long)row * q_stride;
+  const int half = rope.cos ? rope.rot / 2 : 0;
+  const long long angles = half ? (long long)rope.positions[seq] * half : 0;
+  const auto turned = [&](const TX* head, int j) {
+    const float x = ld(head + j);
+    if (j >= 2 * half) return x;
+    const int a = j < half ? j : j - half;
+    const float cc = rope.cos[angles + a], sn = rope.sin[angles + a];
+    const float other = ld(head + (j < half ? j + half : j - half));
+    return j < half ? x * cc - other * sn : x * cc + other * sn;
+  };
+  // The step's own key and value go to their page first, by every workgroup that reads them back (those
+  // of a KV head's other query heads store the same).
+  const int slot = rope.slots && kbeg < ctx && ctx <= kbeg + part ? rope.slots[seq] : -1;
+  if (slot >= 0 && tid < d) {
+    const long long page = slot / page_size;
+    const int off = slot - (int)page * page_size;
+    st((TX*)k_pages + ((page * nkv + kvh) * page_size + off) * d + tid,
+       turned(qrow + rope.k_off + kvh * d, tid));
+    ((TX*)v_pages)[((page * nkv + kvh) * (long long)d + tid) * page_size + off] =
+        qrow[rope.v_off + kvh * d + tid];
+  }
   for (int i = tid; i < G * d; i += 256) {
     const int hh = min(i / d, gn - 1), j = i % d;
-    q_s[i] = ld(q + (long long)row * q_stride + (h0 + hh) * d + j) * scale *
-             (head_scales ? head_scales[h0 + hh] : 1.0f);
+    q_s[i] = turned(qrow + (h0 + hh) * d, j) * scale * (head_scales ? head_scales[h0 + hh] : 1.0f);
   }
   __syncthreads();
 
@@ -444,10 +467,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   const int kept = split == 0 ? min(keep_first, lo) : 0;
   for (int run = kept > 0 ? 0 : 1; run < 2; ++run) {
   const int rbeg = run == 0 ? 0 : kbeg, rend = run == 0 ? kept : kend;
-  // Every wave runs the same number of rounds so that the block-wide barriers match.
-  const int rounds = rend > rbeg ? (rend - rbeg + 255) / 256 : 0;
-  for (int it = 0; it < rounds; ++it) {
-    const int k0 = rbeg + it * 256 + wave * 64;
+  for (int k0 = rbeg + wave * 64; k0 < rend; k0 += 256) {
     const int kpos = k0 + lane;
     const bool valid = kpos < rend;
     float s[G];
@@ -459,16 +479,30 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       const int off = kpos % page_size;
       const TX* kp = k_pages + ((page * nkv + kvh) * page_size + off) * d;
       vbase = (page * nkv + kvh) * (long long)d * page_size + off;
-      for (int j = 0; j < d; j += VN) {
-        float kv[VN];
-        Vec16<TX>::load(kp + j, kv);
+      // eight loads at once (d is a multiple of 8: what is left over are pairs)
+      constexpr int AT = 8;
+      float kv[AT][VN];
+      const auto dot = [&](int j, const float* kj) {
 #pragma unroll
         for (int hh = 0; hh < G; ++hh) {
           float a = s[hh];
 #pragma unroll
-          for (int e = 0; e < VN; ++e) a = fmaf(q_s[hh * d + j + e], kv[e], a);
+          for (int e = 0; e < VN; ++e) a = fmaf(q_s[hh * d + j + e], kj[e], a);
           s[hh] = a;
         }
+      };
+      int j = 0;
+#pragma unroll 1
+      for (; j + AT * VN <= d; j += AT * VN) {
+#pragma unroll
+        for (int b = 0; b < AT; ++b) Vec16<TX>::load(kp + j + b * VN, kv[b]);
+#pragma unroll
+        for (int b = 0; b < AT; ++b) dot(j + b * VN, kv[b]);
+      }
+#pragma unroll 1
+      for (; j < d; j += VN) {
+        Vec16<TX>::load(kp + j, kv[0]);
+        dot(j, kv[0]);
       }
     }
     float corr[G];
@@ -484,7 +518,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       my_p[hh * 64 + lane] = p;
     }
     my_vbase[lane] = vbase;
-    __syncthreads();
+    wave_lds_fence();                      // (a wave reads what its own lanes wrote)
     const int n = max(0, min(64, rend - k0));
     const bool vec_run = run == 0 ? (page_size % VN == 0) : vec_ok;
 #pragma unroll
@@ -496,13 +530,28 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       if (j < d) {
         int kk = 0;
         if (vec_run) {
-          for (; kk + VN <= n; kk += VN) {
-            float v[VN];
-            Vec16<TX>::load(v_pages + my_vbase[kk] + (long long)j * page_size, v);
+          constexpr int AT = 4;
+          float v[AT][VN];
+          const auto load = [&](int b, int k) {
+            Vec16<TX>::load(v_pages + my_vbase[k] + (long long)j * page_size, v[b]);
+          };
+          const auto add = [&](int b, int k) {
 #pragma unroll
             for (int e = 0; e < VN; ++e)
 #pragma unroll
-              for (int hh = 0; hh < G; ++hh) a[hh] = fmaf(my_p[hh * 64 + kk + e], v[e], a[hh]);
+              for (int hh = 0; hh < G; ++hh) a[hh] = fmaf(my_p[hh * 64 + k + e], v[b][e], a[hh]);
+          };
+#pragma unroll 1
+          for (; kk + AT * VN <= n; kk += AT * VN) {
+#pragma unroll
+            for (int b = 0; b < AT; ++b) load(b, kk + b * VN);
+#pragma unroll
+            for (int b = 0; b < AT; ++b) add(b, kk + b * VN);
+          }
+#pragma unroll 1
+          for (; kk + VN <= n; kk += VN) {
+            load(0, kk);
+            add(0, kk);
           }
         }
         for (; kk < n; ++kk) {
@@ -514,7 +563,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 #pragma unroll
       for (int hh = 0; hh < G; ++hh) acc[hh][i] = a[hh];
     }
-    __syncthreads();
+    wave_lds_fence();
   }
   }
 
@@ -754,7 +803,7 @@ static int launch_decode(const void* q, long long q_stride, void* out, long long
                          int page_size, float scale, int window, int splits, int part_keys,
                          int max_parts, const float* slopes, const float* head_scales,
                          float softcap, const float* sinks, int keep_first, int chunk_len,
-                         hipStream_t stream) {
+                         const DecodeRope& rope, hipStream_t stream) {
   const int g = nh / nkv;
   const int chunks = ceil_div(g, G);
   dim3 grid(nkv * chunks, S, splits);
@@ -767,7 +816,7 @@ static int launch_decode(const void* q, long long q_stride, void* out, long long
       (const TX*)q, q_stride, (TX*)out, out_stride, part_ml, part_acc, (const TX*)k_pages,     \
       (const TX*)v_pages, block_tables, max_pages, ctx_lens, token_rows, nh, nkv, d, page_size, \
       scale, window, splits, chunks, part_keys, max_parts, slopes, head_scales, softcap,       \
-      sinks, keep_first, chunk_len)
+      sinks, keep_first, chunk_len, rope)
   if (dpl <= 1) LAUNCH(1);
   else if (dpl <= 2) LAUNCH(2);
   else LAUNCH(4);
@@ -778,7 +827,13 @@ static int launch_decode(const void* q, long long q_stride, void* out, long long
 // q rows are token_rows[seq] (or seq when null) of a (T, q_stride) matrix, out likewise.
 // A sequence's visible keys are cut into partitions of decode_part_len(keys, part_keys,
 // max_parts); `splits` must be at least the live partitions of the longest context (at most
-// max_parts).  part_ml (S, nh, splits, 2) and part_acc (S, nh, splits, d) float32 are needed
+// max_parts).  cos, sin (rot / 2 angles a position; null: none): the queries come unrotated and are
+// turned as they are loaded (rotate-half, the first rot dims); slots (null: none): the step's own key
+// (turned likewise) and value, k_off and v_off into a row of q, are stored to their page first.
+// That is float32's, where it gives the bits of rope_kv_write in front: 4 requests at 100 positions, 32
+// heads of 64, rotation kernel and attention 4.7 + 11.3 us -> 9.7; 3 at 25, heads of 32, 4.4 + 7.5 -> 8.4
+// (eight keys' and four values' loads under way at once; all 64 keys' and values' in straight-line code
+// 14.2 and 12.2: a kernel this short waits for its instructions).  part_ml (S, nh, splits, 2) and part_acc (S, nh, splits, d) float32 are needed
 // when splits > 1.
 RLIS_API int rlis_attn_decode(const void* q, int dtype, long long q_stride, void* out,
                               long long out_stride, float* part_ml, float* part_acc,
@@ -787,8 +842,15 @@ RLIS_API int rlis_attn_decode(const void* q, int dtype, long long q_stride, void
                               int nh, int nkv, int d, int page_size, float scale, int window,
                               int splits, int part_keys, int max_parts, const float* slopes,
                               const float* head_scales, float softcap, const float* sinks,
-                              int keep_first, int chunk, hipStream_t stream) {
+                              int keep_first, int chunk, const float* cos, const float* sin, int rot,
+                              const int* positions, const int* slots, long long k_off,
+                              long long v_off, hipStream_t stream) {
   RLIS_REQUIRE(S >= 0 && nh > 0 && nkv > 0 && d > 0 && page_size > 0, "attn_decode: bad sizes");
+  RLIS_REQUIRE(!(cos || slots) || (dtype == RLIS_F32 && !token_rows),
+               "attn_decode: only float32 rows in the sequences' order are turned and stored here");
+  RLIS_REQUIRE((cos == nullptr) == (sin == nullptr) && (!cos || (positions && rot > 0 && rot % 2 == 0 && rot <= d)),
+               "attn_decode: cannot rotate %d of %d dims", rot, d);
+  const DecodeRope rope = {cos, sin, positions, slots, k_off, v_off, rot};
   RLIS_REQUIRE(chunk >= 0 && (chunk == 0 || (window == 0 && keep_first == 0)),
                "attn_decode: a window or chunks, not both");
   RLIS_REQUIRE(part_keys >= 64 && part_keys % 64 == 0 && max_parts >= 1 && splits <= max_parts,
@@ -809,22 +871,22 @@ RLIS_API int rlis_attn_decode(const void* q, int dtype, long long q_stride, void
       rc = launch_decode<TX, 1>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
                                 v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
                                 nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, stream); \
+                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
     else if (g == 2)                                                                             \
       rc = launch_decode<TX, 2>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
                                 v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
                                 nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, stream); \
+                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
     else if (g <= 4)                                                                             \
       rc = launch_decode<TX, 4>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
                                 v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
                                 nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, stream); \
+                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
     else                                                                                         \
       rc = launch_decode<TX, 8>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
                                 v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
                                 nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, stream); \
+                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
   } while (0)
   if (dtype == RLIS_F32) BY_G(float);
   else if (dtype == RLIS_BF16) BY_G(bf16_t);

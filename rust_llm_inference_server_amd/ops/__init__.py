@@ -49,7 +49,7 @@ FUSE_NORM_LINEAR = True
 # itself and hands the norm's sums over, so that the product behind the norm needs no pass over
 # whole rows (up to 16 rows, one k slice on both sides).
 JOIN_NORM_LINEAR = True
-# The matrix-core decode attention rotates q and k and stores the new k, v itself where it can.
+# The decode attention (matrix-core, and float32's) rotates q and k and stores the new k, v itself where it can.
 FUSE_ROPE_DECODE = True
 # The matrix-core prefill attention rotates its queries as it loads them where it can (the
 # rotation kernel then turns and stores the keys and values only).
@@ -1370,8 +1370,8 @@ def rope_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_di
     ``keep_first`` and ``chunk`` as there).  ``qkv`` may hold the queries alone (``(T, nh * d)``) when
     nothing is written to the cache.  A decode batch that takes the
     matrix-core decode kernel does both in that kernel when the whole head is rotated
-    (rotate-half) and is 64, 128 or 256 wide (or nothing is rotated); ``qkv`` is then left
-    unrotated.  Under the same conditions a batch with portions of prompts leaves the queries
+    (rotate-half) and is 64, 128 or 256 wide (or nothing is rotated), and so does one of float32
+    rotated in halves; ``qkv`` is then left unrotated.  Under the same conditions a batch with portions of prompts leaves the queries
     unrotated too: ``rope_kv_write`` turns and stores the keys and values alone, and the
     matrix-core kernels (prefill for the portions, decode for single tokens beside them) turn
     each query as they load it.  ``interleaved`` and ``bias_slopes`` as in ``rope_kv_write``
@@ -1395,12 +1395,15 @@ def rope_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_di
                                counters=counters, **more)
     fusable = cos is None or (2 * cos.shape[1] == d and d in (64, 128, 256) and not interleaved)
     whole_rows = qkv.shape[1] == (nh + 2 * nkv) * d
-    if cos is not None and fusable and whole_rows and (mfma or kind == "prefill"):
+    # float32's decode kernel turns heads of any width, the bits of rope_kv_write in front of it
+    vector = (kind == "decode" and qkv.dtype == torch.float32 and not interleaved
+              and (cos is None or cos.dim() == 2 and 2 * cos.shape[1] <= d))
+    if cos is not None and whole_rows and (fusable and (mfma or kind == "prefill") or vector):
         _check(cos, "cos", torch.float32, 2)
         _check(sin, "sin", torch.float32, 2)
         if cos.shape != sin.shape or not (cos.is_contiguous() and sin.is_contiguous()):
             raise KernelError("rope_attention: cos and sin must match and be contiguous")
-    if mfma and fusable and FUSE_ROPE_DECODE and whole_rows:
+    if (mfma and fusable or vector) and FUSE_ROPE_DECODE and whole_rows:
         if write_kv and slots is None:
             raise KernelError("rope_attention: a cache write needs slots")
         return paged_attention(qkv, nh, nkv, d, k_pages, v_pages, page_size, block_tables, step,
@@ -1483,7 +1486,7 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     sees the keys of its own chunk alone, those up to p with ``floor(key / c) = floor(p / c)``.
     ``force`` names one of 'generic', 'decode', 'prefill' for tests.  ``rope`` (from
     ``rope_attention`` only): ``(cos, sin, positions, slots)`` for the matrix-core decode kernel
-    to rotate and store the step's tokens itself; with portions of prompts in the batch
+    or float32's to rotate and store the step's tokens itself; with portions of prompts in the batch
     ``slots`` is None (the pages hold the step's keys and values already) and both matrix-core
     kernels turn the unrotated queries as they load them.  ``counters``: int32 zeros on the device, the
     caller's, in which the matrix-core decode kernel's workgroups count themselves in when they
@@ -1543,10 +1546,10 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
         raise KernelError("attention: the count of kept first keys must not be negative")
     kind, mfma = _attention_kernel(qkv, nh, nkv, d, page_size, step, force, slopes_ptr is not None,
                                    shaped, PLAIN_EXTRAS and (sinks_ptr is not None or kept > 0))
-    if rope is not None and not (mfma or (kind == "prefill" and rope[3] is None
-                                          and rope[0] is not None)):
-        raise KernelError("attention: only the matrix-core kernels rotate, and only the decode "
-                          "kernel stores")
+    if rope is not None and not (mfma or (kind == "decode" and qkv.dtype == torch.float32)
+                                 or (kind == "prefill" and rope[3] is None and rope[0] is not None)):
+        raise KernelError("attention: only the matrix-core kernels and float32's decode kernel rotate, "
+                          "and only the decode kernels store")
     if kind == "generic":
         seqs, poss = _i32(step.seq_of_token, "seq_of_token", T), _i32(step.positions, "positions", T)
         if (force is None and qkv.dtype == torch.float32 and d in (16, 32, 64, 128, 256) and not kept
@@ -1586,16 +1589,16 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
             part_acc = torch.empty((S, nh, depth, d), dtype=torch.float32, device=qkv.device)
         ml_ptr = None if part_ml is None else part_ml.data_ptr()
         acc_ptr = None if part_acc is None else part_acc.data_ptr()
+        cos_p = sin_p = pos_p = slots_p = None
+        rot = 0
+        if rope is not None:
+            cos, sin, positions, slots = rope
+            pos_p = _i32(positions, "positions", S)
+            slots_p = None if slots is None else _i32(slots, "slots", S)
+            if cos is not None:
+                cos_p, sin_p, rot = cos.data_ptr(), sin.data_ptr(), 2 * cos.shape[1]
         if matrix:
             lib.ensure_attention_unit(d)
-            cos_p = sin_p = pos_p = slots_p = None
-            rot = 0
-            if rope is not None:
-                cos, sin, positions, slots = rope
-                pos_p = _i32(positions, "positions", S)
-                slots_p = None if slots is None else _i32(slots, "slots", S)
-                if cos is not None:
-                    cos_p, sin_p, rot = cos.data_ptr(), sin.data_ptr(), 2 * cos.shape[1]
             if DECODE_WALK:
                 groups, cap = -(-depth // DECODE_WALK), DECODE_WALK
             else:
@@ -1622,7 +1625,7 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
                      block_tables.data_ptr(), max_pages, _i32(step.ctx_lens, "ctx_lens", S), None,
                      S, nh, nkv, d, page_size, float(scale), win, depth, ap.DECODE_PART_KEYS,
                      ap.DECODE_MAX_PARTS, slopes_ptr, scales_ptr, softcap, sinks_ptr, kept,
-                     span, stream)
+                     span, cos_p, sin_p, rot, pos_p, slots_p, nh * d, (nh + nkv) * d, stream)
 
     if kind == "decode":
         if not step.all_decode:

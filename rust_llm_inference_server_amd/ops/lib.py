@@ -79,7 +79,7 @@ _SIGNATURES = {
     "rlis_attn_generic": [P, I, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P, P, F, P, I, I, P],
     "rlis_attn_tiles_f32": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P, P, F, P, I, I, I, P],
     "rlis_attn_decode": [P, I, L, P, L, P, P, P, P, P, I, P, P, I, I, I, I, I, F, I, I, I, I, P, P, F,
-                         P, I, I, P],
+                         P, I, I, P, P, I, P, P, L, L, P],
     "rlis_attn_decode_mfma": [P, L, P, L, P, P, P, P, P, I, P, I, I, I, I, I, I, F, I, I, I, P, I, I, I,
                               P, P, I, P, P, L, L, P, P, F, P, I, I, I, P],
     "rlis_attn_prefill_mfma": [P, L, P, L, P, P, P, I, P, P, P, I, I, I, I, I, I, F, I, I, I, P, P,
