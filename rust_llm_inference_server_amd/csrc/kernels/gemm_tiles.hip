@@ -1,0 +1,369 @@
+// bfloat16 products y = x * W^T of more than 64 rows of x: portions of prompts, on the matrix cores.
+//
+// At these sizes what bounds a product is how fast a compute unit is fed, not the matrix cores: every
+// tile brings its rows of x and of W into LDS once per stage of 64 k (buffer_load ... lds, 128 bytes a
+// row), and what a die's 32 units ask for while a line is still on its way from memory is served at
+// about 60 bytes a nanosecond and unit, against 135 for lines that its L2 holds already (reads alone,
+// eight units to a line; the same with 32 or 160 KB under way).  So a tile starts its walk over k two
+// stages behind its neighbour along x and one behind its neighbour along W (gate/up of the 1B shape at
+// 2,048 rows: 139 -> 120 us): each line is asked for by one of them and found by the others.  Ids go
+// round the dies and each die takes a run of tiles, eight along x for each along W, so that those
+// that share a line share an L2.
+//
+// Each wave holds MI x NI blocks of 16 x 16 (v_mfma_f32_16x16x32_bf16).  One barrier a stage, in its
+// middle: behind it the stage to come is whole and the one before it free.  Reads of the next half
+// stage and loads of a later stage stand one by one between the products: issued in a row, a stage's
+// loads alone hold a wave for as long as its products take (512 x 3,072 x 2,048 in 128 x 128: 19 us,
+// then 16).  Piece c (16 bytes) of row r of a stage lies at c ^ (r / 2 % 8), which the load does by
+// choosing what a lane reads, so that fragments are read without bank conflicts.  Which weight rows
+// a group of 16 holds is chosen so that a lane stores 16 bytes of neighbouring columns; gated, gate
+// and up rows of the same columns lie in turn and a lane holds both.
+//
+// The order of a sum follows from the sizes and from where in x and W the tile lies.
+//
+// MI355X, us, weights cold, the library's product (with SwiGLU kernel; with the norm that adds
+// output's and down's partial sums) -> this, at 96 / 256 / 512 rows:
+//   1B  q/k/v 10.6 -> 9.1, 10.9 -> 9.6, 13.6 -> 12.9      output 12.0 -> 9.9, 13.6 -> 11.9, 15.9 -> 14.5
+//       gate/up 22.8 -> 20.0, 34.4 -> 27.8, 41.4 -> 39.7  down 24.5 -> 16.0, 30.8 -> 23.7, 38.7 -> 32.0
+//   3B  q/k/v 18.7 -> 16.7, 32.2 -> 24.9                  output 22.2 -> 14.8, 22.8 -> 19.8, 27.5 -> 26.9
+//       gate/up 29.7 -> 29.6, 46.7 -> 40.6, 59.1 -> 55.4  down 40.8 -> 21.7, 39.6 -> 34.9, 52.2 -> 44.3
+//   8B  q/k/v 23.9 -> 21.5, 40.9 -> 32.5                  output 26.9 -> 16.7, 28.5 -> 24.4, 37.0 -> 33.9
+//       gate/up 56.2 -> 50.6, 75.8 -> 70.3                down 69.9 -> 35.0, 69.0 -> 52.1, 99.0 -> 72.1
+#include "common.h"
+#include "gemm_stream.h"
+
+#include <algorithm>
+
+namespace {
+
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+constexpr int kBK = 64;                    // k of a stage: 128 bytes a row
+
+// Waits until at most N loads from memory, and no read from LDS, are under way.  The builtin, so that
+// the compiler, which places waits of its own before a fragment is used, knows that it has arrived.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | 7 << 4 | 0 << 8 | (N >> 4) << 14);
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+struct TilesArgs {
+  const bf16_t* X;
+  const bf16_t* W;
+  void* Y;
+  int T, N, steps;         // N: output columns; steps: stages of a slice of k
+  int mt, nt, slices;      // tiles along x's rows and W's, slices of k
+  int group;               // tiles of x's rows that are walked together
+  int ldx, ldw;            // elements
+  long long ldy, slice_stride;
+};
+
+enum { kOutBf16 = 0, kOutF32 = 1, kOutGated = 2 };
+
+// WM x WN waves, each MI groups of 16 rows of x by NI groups of 16 weight rows; BUFS stages in LDS.
+template <int MI, int NI, int WM, int WN, int BUFS, int OUT>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArgs p) {
+#ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
+  constexpr int WAVES = WM * WN, BM = 16 * MI * WM, BN = 16 * NI * WN;
+  constexpr int STAGE = (BM + BN) * kBK * 2;
+  constexpr int XI = BM / 8 / WAVES, WI = BN / 8 / WAVES, PER = XI + WI;
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "");
+  static_assert(NI % 2 == 0, "");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int r = lane % 16, g = lane / 16;
+  const int wm = wave % WM, wn = wave / WM;
+
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)p.X, 0, 0xffffffff, 0x00027000);
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00027000);
+
+  // Workgroup id -> tile.  Ids go round the eight dies; each die takes a run of the walk.
+  const int per_slice = p.mt * p.nt, total = per_slice * p.slices;
+  const auto place = [&](int id, int& m0, int& n0, int& slice) {
+    id = min(id, total - 1);
+    const int die = id & 7, at = id >> 3;
+    int lin = die * (total >> 3) + min(die, total & 7) + at;
+    slice = lin / per_slice;
+    lin -= slice * per_slice;
+    const int band = lin / (p.group * p.nt), rows = min(p.group, p.mt - band * p.group);
+    lin -= band * p.group * p.nt;
+    m0 = (band * p.group + lin % rows) * BM;
+    n0 = lin / rows * (OUT == kOutGated ? BN / 2 : BN);
+  };
+
+  // Instruction i of this wave brings rows (i * WAVES + wave) * 8 .. + 7 of a stage, x rows first;
+  // piece c of row q of the stage lies at c ^ (q / 2 % 8).
+  uint32_t src[PER];
+  int a_k = 0, a_from = 0;                 // bytes into a row: the stage to ask for, the slice's start
+  const auto sources = [&](int id) {
+    int m0, n0, slice;
+    place(id, m0, n0, slice);
+    const int q8 = lane / 8, c = lane % 8;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const int q = (i * WAVES + wave) * 8 + q8;
+      src[i] = ((uint32_t)min(m0 + q, p.T - 1) * p.ldx + (uint32_t)((c ^ (q / 2 % 8)) * 8)) * 2;
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+      const int q = (i * WAVES + wave) * 8 + q8;
+      const int b = q / 16, o = q % 16;
+      int n;
+      if (OUT == kOutGated) {
+        // groups of 16: gate and up rows in turn, of the same columns
+        const int pair = b / 2;
+        const int col = NI % 4 == 0 ? pair / 2 * 32 + o / 4 * 8 + pair % 2 * 4 + o % 4 : pair * 16 + o;
+        n = min(n0 + col, p.N - 1) + (b % 2 ? p.N : 0);
+      } else if (OUT == kOutBf16) {
+        // two groups of 16 share 32 columns so that a lane holds eight neighbours
+        n = min(n0 + b / 2 * 32 + o / 4 * 8 + b % 2 * 4 + o % 4, p.N - 1);
+      } else {
+        n = min(n0 + q, p.N - 1);
+      }
+      src[XI + i] = ((uint32_t)n * p.ldw + (uint32_t)((c ^ (q / 2 % 8)) * 8)) * 2;
+    }
+    a_from = slice * p.steps * (kBK * 2);
+    const int turn = m0 / BM * 2 + n0 / (OUT == kOutGated ? BN / 2 : BN);
+    a_k = a_from + turn % p.steps * (kBK * 2);
+  };
+  int a_id = blockIdx.x, a_left = p.steps, a_buf = 0;
+  const auto ask = [&](int i) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(i < XI ? xr : wr, (lds_ptr)(smem + a_buf + (i * WAVES + wave) * 1024),
+                                             16, src[i], a_k, 0, 0);
+  };
+  const auto asked = [&]() {               // the stage has been asked for, on to the next
+    a_buf = a_buf + STAGE == BUFS * STAGE ? 0 : a_buf + STAGE;
+    a_k += kBK * 2;
+    if (a_k == a_from + p.steps * (kBK * 2)) a_k = a_from;
+    if (--a_left == 0) {
+      // (past the last tile the last one is read again)
+      a_left = p.steps;
+      a_id += gridDim.x;
+      sources(a_id);
+    }
+  };
+
+  // fragments of a half stage (32 k)
+  const int x_at = (wm * 16 * MI + r) * 128 + ((g ^ (r / 2)) * 16);
+  const int w_at = (BM + wn * 16 * NI + r) * 128 + ((g ^ (r / 2)) * 16);
+  struct Half {
+    bf16x8 x[MI], w[NI];
+  };
+  const auto read = [&](Half& h, int buf, int ks, int i) {
+    if (i < MI) h.x[i] = *(const bf16x8*)(smem + buf + (x_at ^ (ks * 64)) + i * 2048);
+    else h.w[i - MI] = *(const bf16x8*)(smem + buf + (w_at ^ (ks * 64)) + (i - MI) * 2048);
+  };
+  f32x4 acc[NI][MI];
+  const auto clear = [&]() {
+#pragma unroll
+    for (int a = 0; a < NI; ++a)
+#pragma unroll
+      for (int m = 0; m < MI; ++m) acc[a][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  // The products of one half stage.  Between them, one at a time, so that neither the LDS nor the
+  // memory pipe makes a wave wait before its products: the reads of the half stage to come and half
+  // of the loads of the stage that takes the place of the last one.
+  constexpr int PRODUCTS = NI * MI, READS = MI + NI, LATE = PER / 2;
+  const auto half = [&](const Half& h, Half& next, int buf, int ks, int from, int loads) {
+#pragma unroll
+    for (int j = 0; j < PRODUCTS; ++j) {
+      const int a = j / MI, m = j % MI;
+      acc[a][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h.w[a], h.x[m], acc[a][m], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < READS; ++i)
+        if (i * 3 * PRODUCTS / (READS * 4) == j) read(next, buf, ks, i);
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (i < loads && i * PRODUCTS / loads == j) ask(from + i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  sources(a_id);
+#pragma unroll
+  for (int s = 0; s < BUFS - 1; ++s) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) ask(i);
+    asked();
+  }
+#pragma unroll
+  for (int i = 0; i < PER - LATE; ++i) ask(i);
+  Half h0, h1;
+  wait_loads<PER*(BUFS - 2) + PER - LATE>();
+  barrier();
+#pragma unroll
+  for (int i = 0; i < READS; ++i) read(h0, 0, 0, i);
+  wait_loads<63>();
+  int buf = 0;
+  for (int id = blockIdx.x; id < total; id += gridDim.x) {
+    clear();
+    for (int step = 0; step < p.steps; ++step) {
+      half(h0, h1, buf, 1, PER - LATE, LATE);
+      asked();
+      wait_loads<PER*(BUFS - 2)>();
+      barrier();                           // the next stage is whole, this one has been read
+      buf = buf + STAGE == BUFS * STAGE ? 0 : buf + STAGE;
+      half(h1, h0, buf, 0, 0, PER - LATE);
+      wait_loads<63>();                    // (of h0)
+    }
+    int m0, n0, slice;
+    place(id, m0, n0, slice);
+#pragma unroll
+    for (int m = 0; m < MI; ++m) {
+      const int token = m0 + (wm * MI + m) * 16 + r;
+      if (token >= p.T) continue;
+      if (OUT == kOutGated) {
+        bf16_t* row = (bf16_t*)p.Y + (long long)token * p.ldy;
+        constexpr int Q = NI % 4 == 0 ? 2 : 1;   // pairs of blocks whose columns are neighbours
+#pragma unroll
+        for (int a = 0; a < NI / 2; a += Q) {
+          uint32_t o[2 * Q];
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+              const f32x4 gate = acc[2 * (a + q)][m], up = acc[2 * (a + q) + 1][m];
+              o[q * 2 + i / 2] = f32_to_bf16(gated_result(gate[i], up[i], 0)) |
+                                 (uint32_t)f32_to_bf16(gated_result(gate[i + 1], up[i + 1], 0)) << 16;
+            }
+          const int n = n0 + wn * NI * 8 + a * 16 + g * 4 * Q;
+          if (n >= p.N) continue;
+          if (Q == 2) *(uint4*)(row + n) = make_uint4(o[0], o[1], o[2 * Q - 2], o[2 * Q - 1]);
+          else *(uint2*)(row + n) = make_uint2(o[0], o[1]);
+        }
+      } else if (OUT == kOutBf16) {
+        bf16_t* row = (bf16_t*)p.Y + (long long)token * p.ldy;
+#pragma unroll
+        for (int a = 0; a < NI; a += 2) {
+          const f32x4 u = acc[a][m], v = acc[a + 1][m];
+          const int n = n0 + (wn * NI + a) * 16 + g * 8;
+          if (n >= p.N) continue;
+          *(uint4*)(row + n) = make_uint4(f32_to_bf16(u[0]) | (uint32_t)f32_to_bf16(u[1]) << 16,
+                                          f32_to_bf16(u[2]) | (uint32_t)f32_to_bf16(u[3]) << 16,
+                                          f32_to_bf16(v[0]) | (uint32_t)f32_to_bf16(v[1]) << 16,
+                                          f32_to_bf16(v[2]) | (uint32_t)f32_to_bf16(v[3]) << 16);
+        }
+      } else {
+        float* row = (float*)p.Y + slice * p.slice_stride + (long long)token * p.ldy;
+#pragma unroll
+        for (int a = 0; a < NI; ++a) {
+          const int n = n0 + (wn * NI + a) * 16 + g * 4;
+          if (n < p.N) *(f32x4*)(row + n) = acc[a][m];
+        }
+      }
+    }
+  }
+  wait_loads<0>();                         // (loads past the last tile still write LDS)
+#endif
+}
+
+template <int MI, int NI, int WM, int WN, int BUFS, int OUT>
+int launch_tiles(TilesArgs a, hipStream_t stream) {
+  static LdsGrant grant;
+  constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN;
+  constexpr int bytes = BUFS * (BM + BN) * kBK * 2;
+  static_assert(bytes <= 160 * 1024, "");
+  const auto kernel = gemm_tiles_kernel<MI, NI, WM, WN, BUFS, OUT>;
+  const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
+  RLIS_REQUIRE(e == hipSuccess, "gemm_tiles: %s", hipGetErrorString(e));
+  a.mt = ceil_div(a.T, BM);
+  a.nt = ceil_div(a.N, OUT == kOutGated ? BN / 2 : BN);
+  a.group = std::min(a.mt, 8);
+  const int cus = rlis_stream_compute_units();
+  RLIS_REQUIRE(cus > 0, "gemm_tiles: cannot read the device properties");
+  const int resident = std::max(1, std::min(160 * 1024 / bytes, 8 / (WM * WN)));
+  const long long total = (long long)a.mt * a.nt * a.slices;
+  RLIS_REQUIRE(total < (1 << 30), "gemm_tiles: too many tiles");
+  kernel<<<dim3((int)std::min<long long>(total, (long long)cus * resident)), WM * WN * 64, bytes, stream>>>(a);
+  return 0;
+}
+
+template <int MI, int NI, int WM, int WN, int BUFS>
+int launch_out(const TilesArgs& a, int out, hipStream_t stream) {
+  if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16>(a, stream);
+  if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32>(a, stream);
+  return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated>(a, stream);
+}
+
+// The tiles: rows of x by weight rows, and how long a stage takes (us; where two workgroups share a
+// compute unit, half of what it takes both).  Fitted to some 1,200 products of the 1B, 3B and 8B shapes at 72
+// to 2,048 rows, which the sums below give to 8 %.
+struct TileForm {
+  int rows, cols;
+  float stage;
+};
+constexpr TileForm kForms[] = {{128, 256, 0.75f}, {128, 128, 0.48f}, {128, 64, 0.35f}, {64, 64, 0.215f}};
+constexpr int kUnits = 256;                // compute units of the chip
+constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
+
+}  // namespace
+
+// How the product of T rows with N weight rows (gated: gate and up rows together) is cut: the tile (an
+// index that rlis_gemm_bf16_tiles takes) + 16 times the slices of k, or -1 where the library should
+// have it.  partials: the result may come as `slices` partial sums (0: as many of 1, 2 and 4 as suit).
+//
+// The tile (and the number of slices) is what makes least of the rounds over the compute units times
+// a round's stages, with what partial sums cost.  The library has tiles of 256 x 256 at more flops a
+// byte, which win once they fill the chip: up to 256 rows this is ahead at every shape (0.43 to 1.01 of
+// its time); beyond that with partial sums up to 512 rows (0.73 to 1.01), over a k of 8,192 and more,
+// where the library's call over slices of k is at its worst, up to 1,024 (0.73 to 0.96) and up to
+// 2,048 where one round fills the chip (0.91, 0.96; else 1.0 to 1.1); gated, up to 512 rows, where the
+// rounds come out even (0.94, 0.96; else 1.01 to 1.3); plain, up to 1,024 rows over weights of up to
+// 16 MB (0.91 to 0.98; larger ones 0.98 to 1.15).
+RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices) {
+  if (T <= 0 || N <= 0 || K <= 0) return -1;
+  float least = 0.f;
+  int best = -1, best_rounds = 0, best_tiles = 0;
+  for (int s = slices > 0 ? slices : 1; s <= (slices > 0 ? slices : partials ? 4 : 1); s *= 2) {
+    if (K % (s * kBK) || (slices <= 0 && s > 1 && K / s < 512)) continue;
+    for (int f = 0; f < 4; ++f) {
+      const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
+      const long long rounds = (tiles + kUnits - 1) / kUnits;
+      if (rounds > 1 << 20) continue;
+      const float us = (float)rounds * (K / s / kBK) * kForms[f].stage +
+                       (s > 1 ? kPartial * s : kPartial / 2) * (float)T * N;
+      if (best < 0 || us < least) least = us, best = f + 16 * s, best_rounds = (int)rounds, best_tiles = (int)tiles;
+    }
+  }
+  if (best < 0) return -1;
+  const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL);
+  bool here = T <= 256;
+  if (partials) here = here || T <= 512 || (K >= 8192 && (T <= 1024 || (T <= 2048 && best_rounds == 1 && even)));
+  else if (gated) here = here || (T <= 512 && even);
+  else here = here || (T <= 1024 && (long long)N * K <= 1 << 23);
+  return here ? best : -1;
+}
+
+// Y (T,N) = X (T,K) * W (N,K)^T, N a multiple of 8, K of 64 times the slices.  out 0: bfloat16; 1:
+// float32, `slices` partial results slice_stride elements apart; 2: gated, W (2 N,K) gate rows then up
+// rows, Y = silu(gate) * up in bfloat16.  tile: as rlis_gemm_bf16_tiles_plan gives it.
+RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out, int T, int N, int K,
+                                  int slices, long long ldx, long long ldw, long long ldy,
+                                  long long slice_stride, int tile, hipStream_t stream) {
+  RLIS_REQUIRE(T > 0 && N > 0 && N % 8 == 0 && slices > 0 && K > 0 && K % (slices * kBK) == 0,
+               "gemm_tiles: bad sizes T=%d N=%d K=%d slices=%d", T, N, K, slices);
+  RLIS_REQUIRE(out >= 0 && out <= 2 && (slices == 1 || out == 1), "gemm_tiles: no such form");
+  RLIS_REQUIRE(ldx >= K && ldw >= K && ldy >= N && ldx % 8 == 0 && ldw % 8 == 0 && ldy % 8 == 0 &&
+                   slice_stride % 4 == 0 && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 &&
+                   (uintptr_t)Y % 16 == 0,
+               "gemm_tiles: rows must lie on 16-byte boundaries");
+  RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * N * (out == 2 ? 2 : 1) < (1LL << 32),
+               "gemm_tiles: x or W passes 4 GB");
+  const TilesArgs a = {(const bf16_t*)X, (const bf16_t*)W, Y, T, N, K / slices / kBK, 0, 0, slices, 0,
+                       (int)ldx, (int)ldw, ldy, slice_stride};
+  int rc = 1;
+  switch (tile) {
+    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, stream); break;   // 128 x 256, 144 KB of LDS
+    case 1: rc = launch_out<4, 2, 2, 4, 5>(a, out, stream); break;   // 128 x 128, 160 KB
+    case 2: rc = launch_out<4, 2, 2, 2, 3>(a, out, stream); break;   // 128 x 64, 72 KB: two to a compute unit
+    case 3: rc = launch_out<2, 2, 2, 2, 4>(a, out, stream); break;   // 64 x 64, 64 KB: two to a compute unit
+    default: RLIS_REQUIRE(false, "gemm_tiles: no tile %d", tile);
+  }
+  if (rc) return rc;
+  RLIS_LAUNCH_CHECK("gemm_tiles");
+  return 0;
+}

@@ -866,6 +866,49 @@ def _rows_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, slice
     return y
 
 
+TILES_MIN_ROWS = 65       # rows of x from which on the kernel in tiles may take a product
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles_plan(T: int, N: int, K: int, gated: bool, partials: bool, slices: int) -> int:
+    return lib.load().rlis_gemm_bf16_tiles_plan(T, N, K, int(gated), int(partials), slices)
+
+
+def _tiles(x: torch.Tensor, w: torch.Tensor, gated: bool = False, partials: bool = False) -> int:
+    """How the kernel for more than 64 rows (gemm_tiles.hip, whose rule says which products it is ahead
+    of the library at) cuts ``x @ w.T``, or -1: bfloat16, a k in 64s, weight rows in eights (``gated``
+    in sixteens), rows on 16-byte boundaries, x and W below 4 GB.  Over a k that goes to the library in
+    slices (``library_slices``) partial sums come in as many."""
+    T, K = x.shape
+    N = w.shape[0]
+    if not (T >= TILES_MIN_ROWS and BF16_GEMM == "library"
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and K > 0 and K % 64 == 0 and N > 0 and N % (16 if gated else 8) == 0
+            and x.stride(1) == 1 and w.stride(1) == 1
+            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.stride(0) >= K and w.stride(0) >= K
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and 2 * N * w.stride(0) < 1 << 32 and 2 * T * x.stride(0) < 1 << 32):
+        return -1
+    slices = library_slices(T, K) if partials else 1
+    if slices > 1 and K % (64 * slices):
+        return -1
+    return _tiles_plan(T, N, K, gated, partials, slices if slices > 1 or not partials else 0)
+
+
+def _tiles_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, plan: int,
+                  gated: bool = False) -> torch.Tensor:
+    T, K = x.shape
+    N = w.shape[0] // 2 if gated else w.shape[0]
+    slices = plan // 16
+    if slices > 1:
+        out_dtype = torch.float32
+    y = torch.empty((T, N) if slices == 1 else (slices, T, N), dtype=out_dtype, device=x.device)
+    lib.call("rlis_gemm_bf16_tiles", x.data_ptr(), w.data_ptr(), y.data_ptr(),
+             2 if gated else int(out_dtype == torch.float32), T, N, K, slices, x.stride(0), w.stride(0),
+             N, T * N, plan % 16, lib.stream_ptr())
+    return y
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
            partials: bool = False) -> torch.Tensor:
     """``x @ w.T`` for ``x (T, K)`` and ``w (N, K)``, float32 accumulation.
@@ -875,7 +918,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     float32 weight or ``x`` beside bfloat16, the plain FMA kernel.
     bfloat16 operands take the streaming kernel up to 16 rows (32 over short rows) and the kernel
     for 17 to 64 rows beyond (``_rows_kernel``; few weight rows over a long k only as partial sums,
-    ``_rows_in_one_slice``); more rows, and other sizes, go to the library's
+    ``_rows_in_one_slice``); from 65 rows on the kernel in tiles where it is ahead of the library
+    (``_tiles``); other products, and other sizes, go to the library's
     GEMM (hipBLASLt, through its own entry points), or with ``BF16_GEMM = "own"`` to the skinny
     kernel up to 64 rows and the hand-written matrix-core GEMM beyond.
 
@@ -912,6 +956,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         lib.call("rlis_gemm_bf16_splitk", x.data_ptr(), w.data_ptr(), y.data_ptr(), T, N, K, ldx,
                  ldw, T * N, stream)
         return y
+    if bf16 and T >= TILES_MIN_ROWS and out_dtype in (torch.bfloat16, torch.float32):
+        plan = _tiles(x, w, partials=partials)
+        if plan >= 0:
+            return _tiles_linear(x, w, out_dtype, plan)
     if bf16 and aligned and T > STREAM_MAX_ROWS and BF16_GEMM == "library":
         ws = lib.library_workspace(x.device) if LIBRARY_GEMM_DIRECT else None
         slices = library_slices(T, K) if partials and ws is not None else 1
@@ -1120,8 +1168,8 @@ def linear_scaled(xw: torch.Tensor, ss: torch.Tensor, eps: float, w: torch.Tenso
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]`` of shape ``(2 I, K)``.
 
-    Up to 16 rows of bfloat16 (32 over short rows), 17 to 64 of sizes that ``_rows_kernel`` takes, and
-    float32 that ``_f32_kernels`` takes (the same bits) go through one kernel that never stores the
+    Up to 16 rows of bfloat16 (32 over short rows), 17 to 64 of sizes that ``_rows_kernel`` takes, more
+    where ``_tiles`` is ahead, and float32 that ``_f32_kernels`` takes (the same bits) go through one kernel that never stores the
     ``(T, 2 I)`` intermediate; everything else is the product followed by the SwiGLU kernel."""
     T, K = x.shape
     two_i = w_gate_up.shape[0]
@@ -1138,6 +1186,10 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
         (BF16_GEMM == "own" or T <= STREAM_MAX_ROWS)
     if fusable and not streamed and K == w_gate_up.shape[1] and _rows_kernel(x, w_gate_up, gated=True):
         return _rows_linear(x, w_gate_up, torch.bfloat16, gated=True)
+    if fusable and not streamed and T >= TILES_MIN_ROWS:
+        plan = _tiles(x, w_gate_up, gated=True)
+        if plan >= 0:
+            return _tiles_linear(x, w_gate_up, torch.bfloat16, plan, gated=True)
     if T > 0 and two_i > 0 and K == w_gate_up.shape[1] and _f32_kernels(x, w_gate_up, ldx, ldw):
         y = torch.empty((T, two_i // 2), dtype=torch.float32, device=x.device)
         lib.call("rlis_gemm_f32", x.data_ptr(), w_gate_up.data_ptr(), y.data_ptr(), T, two_i // 2, K, ldx,

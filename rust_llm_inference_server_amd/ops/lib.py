@@ -68,6 +68,7 @@ _SIGNATURES = {
     "rlis_gemm_plain": [P, I, P, I, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, I, P],
     "rlis_gemm_bf16_rows": [P, P, P, I, I, I, I, I, L, L, L, L, P, I, I, F, I, P],
+    "rlis_gemm_bf16_tiles": [P, P, P, I, I, I, I, I, L, L, L, L, I, P],
     "rlis_gemm_bf16_mfma": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny_swiglu": [P, P, P, I, I, I, L, L, L, P],
@@ -122,6 +123,8 @@ def load() -> ctypes.CDLL:
     lib.rlis_gemm_bf16_stream_slices.argtypes = [I]
     lib.rlis_gemm_bf16_rows_slices.restype = c_int
     lib.rlis_gemm_bf16_rows_slices.argtypes = [I, I]
+    lib.rlis_gemm_bf16_tiles_plan.restype = c_int
+    lib.rlis_gemm_bf16_tiles_plan.argtypes = [I, I, I, I, I, I]
     lib.rlis_gemm_bf16_splitk_slices.restype = c_int
     lib.rlis_gemm_bf16_splitk_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_stream_join_tiles.restype = c_int
