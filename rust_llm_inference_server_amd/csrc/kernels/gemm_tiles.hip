@@ -21,6 +21,10 @@
 //
 // The order of a sum follows from the sizes and from where in x and W the tile lies.
 //
+// Tiles of 128 to 256 rows by 128, in steps of 32, so that a round comes out even over the compute units
+// (gate/up of the 1B shape at 381 rows: two of 192 31.9 us, three of 128 35.4, the library's with
+// the SwiGLU kernel 36.2).  More stages under way than the tiles have here change nothing.
+//
 // MI355X, us, weights cold, the library's product (with SwiGLU kernel; with the norm that adds
 // output's and down's partial sums) -> this, at 96 / 256 / 512 rows:
 //   1B  q/k/v 10.6 -> 9.1, 10.9 -> 9.6, 13.6 -> 12.9      output 12.0 -> 9.9, 13.6 -> 11.9, 15.9 -> 14.5
@@ -296,7 +300,9 @@ struct TileForm {
   int rows, cols;
   float stage;
 };
-constexpr TileForm kForms[] = {{128, 256, 0.75f}, {128, 128, 0.48f}, {128, 64, 0.35f}, {64, 64, 0.215f}};
+constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 0.66f}, {192, 128, 0.60f},
+                               {160, 128, 0.55f}, {128, 128, 0.48f}, {128, 64, 0.35f}, {64, 64, 0.215f}};
+constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
 constexpr int kUnits = 256;                // compute units of the chip
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
 
@@ -311,16 +317,16 @@ constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 pa
 // byte, which win once they fill the chip: up to 256 rows this is ahead at every shape (0.43 to 1.01 of
 // its time); beyond that with partial sums up to 512 rows (0.73 to 1.01), over a k of 8,192 and more,
 // where the library's call over slices of k is at its worst, up to 1,024 (0.73 to 0.96) and up to
-// 2,048 where one round fills the chip (0.91, 0.96; else 1.0 to 1.1); gated, up to 512 rows, where the
-// rounds come out even (0.94, 0.96; else 1.01 to 1.3); plain, up to 1,024 rows over weights of up to
-// 16 MB (0.91 to 0.98; larger ones 0.98 to 1.15).
+// 2,048 where one round fills the chip (0.86 to 0.96; else 1.0 to 1.1); gated, up to 512 rows, where the
+// rounds come out even or there is one (0.88 to 0.96; else 1.01 to 1.3); plain, up to 1,024 rows over
+// weights of up to 16 MB (0.91 to 0.98; larger ones 0.98 to 1.15).
 RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices) {
   if (T <= 0 || N <= 0 || K <= 0) return -1;
   float least = 0.f;
   int best = -1, best_rounds = 0, best_tiles = 0;
   for (int s = slices > 0 ? slices : 1; s <= (slices > 0 ? slices : partials ? 4 : 1); s *= 2) {
     if (K % (s * kBK) || (slices <= 0 && s > 1 && K / s < 512)) continue;
-    for (int f = 0; f < 4; ++f) {
+    for (int f = 0; f < kFormCount; ++f) {
       const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
       const long long rounds = (tiles + kUnits - 1) / kUnits;
       if (rounds > 1 << 20) continue;
@@ -332,8 +338,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   if (best < 0) return -1;
   const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL);
   bool here = T <= 256;
-  if (partials) here = here || T <= 512 || (K >= 8192 && (T <= 1024 || (T <= 2048 && best_rounds == 1 && even)));
-  else if (gated) here = here || (T <= 512 && even);
+  if (partials) here = here || T <= 512 || (K >= 8192 && T <= 1024) || (T <= 2048 && best_rounds == 1 && even);
+  else if (gated) here = here || (T <= 512 && (even || best_rounds == 1));
   else here = here || (T <= 1024 && (long long)N * K <= 1 << 23);
   return here ? best : -1;
 }
@@ -357,10 +363,14 @@ RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out
                        (int)ldx, (int)ldw, ldy, slice_stride};
   int rc = 1;
   switch (tile) {
-    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, stream); break;   // 128 x 256, 144 KB of LDS
-    case 1: rc = launch_out<4, 2, 2, 4, 5>(a, out, stream); break;   // 128 x 128, 160 KB
-    case 2: rc = launch_out<4, 2, 2, 2, 3>(a, out, stream); break;   // 128 x 64, 72 KB: two to a compute unit
-    case 3: rc = launch_out<2, 2, 2, 2, 4>(a, out, stream); break;   // 64 x 64, 64 KB: two to a compute unit
+    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, stream); break;   // 128 x 256
+    case 1: rc = launch_out<4, 4, 4, 2, 3>(a, out, stream); break;   // 256 x 128
+    case 2: rc = launch_out<7, 4, 2, 2, 3>(a, out, stream); break;   // 224 x 128
+    case 3: rc = launch_out<6, 4, 2, 2, 3>(a, out, stream); break;   // 192 x 128
+    case 4: rc = launch_out<5, 4, 2, 2, 4>(a, out, stream); break;   // 160 x 128
+    case 5: rc = launch_out<4, 2, 2, 4, 5>(a, out, stream); break;   // 128 x 128
+    case 6: rc = launch_out<4, 2, 2, 2, 3>(a, out, stream); break;   // 128 x 64, two to a compute unit
+    case 7: rc = launch_out<2, 2, 2, 2, 4>(a, out, stream); break;   // 64 x 64, two to a compute unit
     default: RLIS_REQUIRE(false, "gemm_tiles: no tile %d", tile);
   }
   if (rc) return rc;
