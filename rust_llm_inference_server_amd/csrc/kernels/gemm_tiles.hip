@@ -21,6 +21,10 @@
 //
 // The order of a sum follows from the sizes and from where in x and W the tile lies.
 //
+// 33 to 64 rows take it too where there is much of W (gate/up, the output head): one row of tiles, each
+// line of W read once and non-temporally.  64 rows, us: head 1B 117 (library) -> 88, 3B 164 -> 130; gate/up
+// against gemm_rows.hip 1B 16.5 -> 15.1, 3B 22.5 -> 22.1, 8B 51.4 -> 43.5.
+//
 // Tiles of 128 to 256 rows by 128, in steps of 32, so that a round comes out even over the compute units
 // (gate/up of the 1B shape at 381 rows: two of 192 31.9 us, three of 128 35.4, the library's with
 // the SwiGLU kernel 36.2).  More stages under way than the tiles have here change nothing.
@@ -68,7 +72,7 @@ struct TilesArgs {
 enum { kOutBf16 = 0, kOutF32 = 1, kOutGated = 2 };
 
 // WM x WN waves, each MI groups of 16 rows of x by NI groups of 16 weight rows; BUFS stages in LDS.
-template <int MI, int NI, int WM, int WN, int BUFS, int OUT>
+template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArgs p) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
   constexpr int WAVES = WM * WN, BM = 16 * MI * WM, BN = 16 * NI * WN;
@@ -135,8 +139,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
   };
   int a_id = blockIdx.x, a_left = p.steps, a_buf = 0;
   const auto ask = [&](int i) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(i < XI ? xr : wr, (lds_ptr)(smem + a_buf + (i * WAVES + wave) * 1024),
-                                             16, src[i], a_k, 0, 0);
+    const lds_ptr to = (lds_ptr)(smem + a_buf + (i * WAVES + wave) * 1024);
+    if (i < XI) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, to, 16, src[i], a_k, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, src[i], a_k, 0, NT ? 2 : 0);
   };
   const auto asked = [&]() {               // the stage has been asked for, on to the next
     a_buf = a_buf + STAGE == BUFS * STAGE ? 0 : a_buf + STAGE;
@@ -265,13 +270,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
 #endif
 }
 
-template <int MI, int NI, int WM, int WN, int BUFS, int OUT>
+template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT>
 int launch_tiles(TilesArgs a, hipStream_t stream) {
   static LdsGrant grant;
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN;
   constexpr int bytes = BUFS * (BM + BN) * kBK * 2;
   static_assert(bytes <= 160 * 1024, "");
-  const auto kernel = gemm_tiles_kernel<MI, NI, WM, WN, BUFS, OUT>;
+  const auto kernel = gemm_tiles_kernel<MI, NI, WM, WN, BUFS, OUT, NT>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_tiles: %s", hipGetErrorString(e));
   a.mt = ceil_div(a.T, BM);
@@ -287,10 +292,16 @@ int launch_tiles(TilesArgs a, hipStream_t stream) {
 }
 
 template <int MI, int NI, int WM, int WN, int BUFS>
-int launch_out(const TilesArgs& a, int out, hipStream_t stream) {
-  if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16>(a, stream);
-  if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32>(a, stream);
-  return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated>(a, stream);
+int launch_out(const TilesArgs& a, int out, int nt, hipStream_t stream) {
+  // (rows of W that a second tile reads too must stay in the caches: gate/up of 256 rows 137 -> 174 us)
+  if (nt && a.T <= 16 * MI * WM) {
+    if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16, true>(a, stream);
+    if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32, true>(a, stream);
+    return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated, true>(a, stream);
+  }
+  if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16, false>(a, stream);
+  if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32, false>(a, stream);
+  return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated, false>(a, stream);
 }
 
 // The tiles: rows of x by weight rows, and how long a stage takes (us; where two workgroups share a
@@ -301,8 +312,10 @@ struct TileForm {
   float stage;
 };
 constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 0.66f}, {192, 128, 0.60f},
-                               {160, 128, 0.55f}, {128, 128, 0.48f}, {128, 64, 0.35f}, {64, 64, 0.215f}};
+                               {160, 128, 0.55f}, {128, 128, 0.48f}, {128, 64, 0.35f}, {64, 64, 0.215f},
+                               {64, 128, 0.33f}, {64, 256, 0.46f}};
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
+constexpr int kWideForms = 8;              // those that products of more than 64 rows choose from
 constexpr int kUnits = 256;                // compute units of the chip
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
 
@@ -326,7 +339,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   int best = -1, best_rounds = 0, best_tiles = 0;
   for (int s = slices > 0 ? slices : 1; s <= (slices > 0 ? slices : partials ? 4 : 1); s *= 2) {
     if (K % (s * kBK) || (slices <= 0 && s > 1 && K / s < 512)) continue;
-    for (int f = 0; f < kFormCount; ++f) {
+    for (int f = 0; f < (T <= 64 ? kFormCount : kWideForms); ++f) {
+      if (T <= 64 && kForms[f].rows > 64) continue;
       const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
       const long long rounds = (tiles + kUnits - 1) / kUnits;
       if (rounds > 1 << 20) continue;
@@ -337,7 +351,7 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   }
   if (best < 0) return -1;
   const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL);
-  bool here = T <= 256;
+  bool here = T <= 256;                    // (up to 64 rows the caller knows which)
   if (partials) here = here || T <= 512 || (K >= 8192 && T <= 1024) || (T <= 2048 && best_rounds == 1 && even);
   else if (gated) here = here || (T <= 512 && (even || best_rounds == 1));
   else here = here || (T <= 1024 && (long long)N * K <= 1 << 23);
@@ -346,10 +360,11 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
 
 // Y (T,N) = X (T,K) * W (N,K)^T, N a multiple of 8, K of 64 times the slices.  out 0: bfloat16; 1:
 // float32, `slices` partial results slice_stride elements apart; 2: gated, W (2 N,K) gate rows then up
-// rows, Y = silu(gate) * up in bfloat16.  tile: as rlis_gemm_bf16_tiles_plan gives it.
+// rows, Y = silu(gate) * up in bfloat16.  tile: as rlis_gemm_bf16_tiles_plan gives it.  nt: W is loaded
+// non-temporally (load_weights) where one row of tiles holds all of x.
 RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out, int T, int N, int K,
                                   int slices, long long ldx, long long ldw, long long ldy,
-                                  long long slice_stride, int tile, hipStream_t stream) {
+                                  long long slice_stride, int tile, int nt, hipStream_t stream) {
   RLIS_REQUIRE(T > 0 && N > 0 && N % 8 == 0 && slices > 0 && K > 0 && K % (slices * kBK) == 0,
                "gemm_tiles: bad sizes T=%d N=%d K=%d slices=%d", T, N, K, slices);
   RLIS_REQUIRE(out >= 0 && out <= 2 && (slices == 1 || out == 1), "gemm_tiles: no such form");
@@ -363,14 +378,16 @@ RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out
                        (int)ldx, (int)ldw, ldy, slice_stride};
   int rc = 1;
   switch (tile) {
-    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, stream); break;   // 128 x 256
-    case 1: rc = launch_out<4, 4, 4, 2, 3>(a, out, stream); break;   // 256 x 128
-    case 2: rc = launch_out<7, 4, 2, 2, 3>(a, out, stream); break;   // 224 x 128
-    case 3: rc = launch_out<6, 4, 2, 2, 3>(a, out, stream); break;   // 192 x 128
-    case 4: rc = launch_out<5, 4, 2, 2, 4>(a, out, stream); break;   // 160 x 128
-    case 5: rc = launch_out<4, 2, 2, 4, 5>(a, out, stream); break;   // 128 x 128
-    case 6: rc = launch_out<4, 2, 2, 2, 3>(a, out, stream); break;   // 128 x 64, two to a compute unit
-    case 7: rc = launch_out<2, 2, 2, 2, 4>(a, out, stream); break;   // 64 x 64, two to a compute unit
+    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, nt, stream); break;   // 128 x 256
+    case 1: rc = launch_out<4, 4, 4, 2, 3>(a, out, nt, stream); break;   // 256 x 128
+    case 2: rc = launch_out<7, 4, 2, 2, 3>(a, out, nt, stream); break;   // 224 x 128
+    case 3: rc = launch_out<6, 4, 2, 2, 3>(a, out, nt, stream); break;   // 192 x 128
+    case 4: rc = launch_out<5, 4, 2, 2, 4>(a, out, nt, stream); break;   // 160 x 128
+    case 5: rc = launch_out<4, 2, 2, 4, 5>(a, out, nt, stream); break;   // 128 x 128
+    case 6: rc = launch_out<4, 2, 2, 2, 3>(a, out, nt, stream); break;   // 128 x 64, two to a compute unit
+    case 7: rc = launch_out<2, 2, 2, 2, 4>(a, out, nt, stream); break;   // 64 x 64, two to a compute unit
+    case 8: rc = launch_out<4, 2, 1, 4, 3>(a, out, nt, stream); break;   // 64 x 128, two to a compute unit
+    case 9: rc = launch_out<4, 4, 1, 4, 2>(a, out, nt, stream); break;   // 64 x 256, two to a compute unit
     default: RLIS_REQUIRE(false, "gemm_tiles: no tile %d", tile);
   }
   if (rc) return rc;

@@ -866,7 +866,13 @@ def _rows_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, slice
     return y
 
 
-TILES_MIN_ROWS = 65       # rows of x from which on the kernel in tiles may take a product
+# Rows of x from which on the kernel in tiles may take a product.  From the second on those that would
+# go to the library for their many weight rows (the output head: 64 rows, 117 -> 88 us), and gate/up
+# whose tiles of 64 weight rows fill the compute units and that has at least this many elements (64 rows, kernel for 17 to 64 rows -> tiles: 16384 x 2048 16.4 -> 15.0 us,
+# 28672 x 4096 50.0 -> 42.6; 5632 x 2048 11.8 -> 13.5, 4096 x 1024 6.4 -> 9.1, which stay there).
+TILES_MIN_ROWS = 65
+TILES_MIN_ROWS_WIDE = 33
+TILES_WIDE_GATED = 1 << 25
 
 
 @functools.lru_cache(maxsize=4096)
@@ -875,13 +881,18 @@ def _tiles_plan(T: int, N: int, K: int, gated: bool, partials: bool, slices: int
 
 
 def _tiles(x: torch.Tensor, w: torch.Tensor, gated: bool = False, partials: bool = False) -> int:
-    """How the kernel for more than 64 rows (gemm_tiles.hip, whose rule says which products it is ahead
-    of the library at) cuts ``x @ w.T``, or -1: bfloat16, a k in 64s, weight rows in eights (``gated``
+    """How the kernel in tiles (gemm_tiles.hip, whose rule says which products of more than 64 rows it is
+    ahead of the library at) cuts ``x @ w.T``, or -1: bfloat16, a k in 64s, weight rows in eights (``gated``
     in sixteens), rows on 16-byte boundaries, x and W below 4 GB.  Over a k that goes to the library in
     slices (``library_slices``) partial sums come in as many."""
     T, K = x.shape
     N = w.shape[0]
-    if not (T >= TILES_MIN_ROWS and BF16_GEMM == "library"
+    if T < TILES_MIN_ROWS and not (T >= TILES_MIN_ROWS_WIDE and ROWS_MAX_ROWS >= 64
+                                   and STREAM_WIDE_MAX_ROWS > STREAM_MAX_ROWS
+                                   and (N >= 64 * 256 and N * K >= TILES_WIDE_GATED if gated
+                                        else N > ROWS_LIBRARY_N)):
+        return -1
+    if not (BF16_GEMM == "library"
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and K > 0 and K % 64 == 0 and N > 0 and N % (16 if gated else 8) == 0
             and x.stride(1) == 1 and w.stride(1) == 1
@@ -905,7 +916,7 @@ def _tiles_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, plan
     y = torch.empty((T, N) if slices == 1 else (slices, T, N), dtype=out_dtype, device=x.device)
     lib.call("rlis_gemm_bf16_tiles", x.data_ptr(), w.data_ptr(), y.data_ptr(),
              2 if gated else int(out_dtype == torch.float32), T, N, K, slices, x.stride(0), w.stride(0),
-             N, T * N, plan % 16, lib.stream_ptr())
+             N, T * N, plan % 16, _streamed.nt, lib.stream_ptr())
     return y
 
 
@@ -956,7 +967,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         lib.call("rlis_gemm_bf16_splitk", x.data_ptr(), w.data_ptr(), y.data_ptr(), T, N, K, ldx,
                  ldw, T * N, stream)
         return y
-    if bf16 and T >= TILES_MIN_ROWS and out_dtype in (torch.bfloat16, torch.float32):
+    if bf16 and T >= TILES_MIN_ROWS_WIDE and out_dtype in (torch.bfloat16, torch.float32):
         plan = _tiles(x, w, partials=partials)
         if plan >= 0:
             return _tiles_linear(x, w, out_dtype, plan)
@@ -1184,12 +1195,12 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     streamed = fusable and T <= stream_rows(K) and _one_item_per_wave(K)
     skinny = fusable and not streamed and T <= SKINNY_MAX_ROWS and \
         (BF16_GEMM == "own" or T <= STREAM_MAX_ROWS)
-    if fusable and not streamed and K == w_gate_up.shape[1] and _rows_kernel(x, w_gate_up, gated=True):
-        return _rows_linear(x, w_gate_up, torch.bfloat16, gated=True)
-    if fusable and not streamed and T >= TILES_MIN_ROWS:
+    if fusable and not streamed and T >= TILES_MIN_ROWS_WIDE:
         plan = _tiles(x, w_gate_up, gated=True)
         if plan >= 0:
             return _tiles_linear(x, w_gate_up, torch.bfloat16, plan, gated=True)
+    if fusable and not streamed and K == w_gate_up.shape[1] and _rows_kernel(x, w_gate_up, gated=True):
+        return _rows_linear(x, w_gate_up, torch.bfloat16, gated=True)
     if T > 0 and two_i > 0 and K == w_gate_up.shape[1] and _f32_kernels(x, w_gate_up, ldx, ldw):
         y = torch.empty((T, two_i // 2), dtype=torch.float32, device=x.device)
         lib.call("rlis_gemm_f32", x.data_ptr(), w_gate_up.data_ptr(), y.data_ptr(), T, two_i // 2, K, ldx,

@@ -68,7 +68,7 @@ _SIGNATURES = {
     "rlis_gemm_plain": [P, I, P, I, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, I, P],
     "rlis_gemm_bf16_rows": [P, P, P, I, I, I, I, I, L, L, L, L, P, I, I, F, I, P],
-    "rlis_gemm_bf16_tiles": [P, P, P, I, I, I, I, I, L, L, L, L, I, P],
+    "rlis_gemm_bf16_tiles": [P, P, P, I, I, I, I, I, L, L, L, L, I, I, P],
     "rlis_gemm_bf16_mfma": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny_swiglu": [P, P, P, I, I, I, L, L, L, P],
