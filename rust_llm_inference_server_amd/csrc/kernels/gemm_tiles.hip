@@ -328,11 +328,12 @@ constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 pa
 // The tile (and the number of slices) is what makes least of the rounds over the compute units times
 // a round's stages, with what partial sums cost.  The library has tiles of 256 x 256 at more flops a
 // byte, which win once they fill the chip: up to 256 rows this is ahead at every shape (0.43 to 1.01 of
-// its time); beyond that with partial sums up to 512 rows (0.73 to 1.01), over a k of 8,192 and more,
-// where the library's call over slices of k is at its worst, up to 1,024 (0.73 to 0.96) and up to
-// 2,048 where one round fills the chip (0.86 to 0.96; else 1.0 to 1.1); gated, up to 512 rows, where the
-// rounds come out even or there is one (0.88 to 0.96; else 1.01 to 1.3); plain, up to 1,024 rows over
-// weights of up to 16 MB (0.91 to 0.98; larger ones 0.98 to 1.15).
+// its time).  Beyond that, with partial sums: up to 512 rows (0.73 to 1.01), but over a k of 8,192 and
+// more, which the library has in slices too, where the rounds come out even, then up to 1,024 rows
+// (in a step 1B 512 rows 33.9 -> 31.7 us with the norm; uneven 381 rows 27.5 -> 29.9, 3B 512 rows 41.4 ->
+// 43.9), and up to 2,048 where one even round fills the chip (0.86 to 0.96; else 1.0 to 1.1).  Gated, up
+// to 512 rows, where the rounds come out even or there is one (0.88 to 0.96; else 1.01 to 1.3).  Plain,
+// up to 1,024 rows over weights of up to 16 MB (0.91 to 0.98; larger ones 0.98 to 1.15).
 RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices) {
   if (T <= 0 || N <= 0 || K <= 0) return -1;
   float least = 0.f;
@@ -352,7 +353,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   if (best < 0) return -1;
   const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL);
   bool here = T <= 256;                    // (up to 64 rows the caller knows which)
-  if (partials) here = here || T <= 512 || (K >= 8192 && T <= 1024) || (T <= 2048 && best_rounds == 1 && even);
+  if (partials)
+    here = here || (K < 8192 ? T <= 512 : T <= 1024 && even) || (T <= 2048 && best_rounds == 1 && even);
   else if (gated) here = here || (T <= 512 && (even || best_rounds == 1));
   else here = here || (T <= 1024 && (long long)N * K <= 1 << 23);
   return here ? best : -1;
