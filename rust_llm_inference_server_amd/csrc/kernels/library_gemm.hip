@@ -1,5 +1,5 @@
-// bfloat16 products with more than 64 rows (and the ones of 17 to 64 rows that do not join the
-// residual stream) are the library's: hipBLASLt, called here directly.  The reference uses a
+// bfloat16 products of many rows that gemm_tiles.hip is not ahead at, and sizes that no kernel of the
+// package takes, are the library's: hipBLASLt, called here directly.  The reference uses a
 // library matmul for every projection (crates/model/src/layers.rs:30-46, candle's matmul).
 //
 // Why not through the tensor library's matmul: a step that mixes a portion of a prompt with

@@ -816,9 +816,9 @@ def _try_out(x, w, y, out_f32, T, N, K, ldx, ldw, slices, ws, stream, partial=Fa
 
 # The kernel for 17 to 64 rows (gemm_rows.hip; ``STREAM_WIDE_MAX_ROWS`` up to 16 switches it off
 # with the streaming kernel's form for 17 to 32 rows).  Beyond 32 rows a product of more than this
-# many weight rows goes to the library: x is read as often as W there, and tiles of 64 rows read
-# it more often than the library's (1B output head, 128,256 rows, 64 rows of x: 130 against 120 us;
-# 32 rows of x 108 against 113; gate/up of the 8B shape, 28,672: 53 against 56).
+# many weight rows is not this kernel's: x is read as often as W there, and tiles of 64 rows read
+# it more often than larger ones (1B output head, 128,256 rows, 64 rows of x: 130 against the library's 120 us
+# and 88 in tiles of 64 x 256; 32 rows of x 108 against the library's 113).
 ROWS_MAX_ROWS = 64
 ROWS_LIBRARY_N = 32768
 
