@@ -385,31 +385,39 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
 // needs: they go from memory into its registers, two steps ahead.  x goes through LDS (two buffers
 // taking turns, two more steps on their way; rows 160 bytes apart, so that the 16-byte reads of a
 // fragment are free of bank conflicts).  At the end the first group adds the parts of the others to its
-// own, in order.  CUT: K is not sixteen whole runs.  GATED: a wave's weight rows are 8 gate rows and the 8 up rows of the same columns.
+// own, in order.  ENDS: where K ends.  GATED: a wave's weight rows are 8 gate rows and the 8 up rows of the
+// same columns.
+//
+// A K that is no sixteen whole runs: groups that would hold none are not launched and steps past K are not
+// multiplied, and where K ends with a step no load is selected (2,048 x 8,192 over 64 / 320 us: sixteen runs walked
+// 106 / 179, no others 36 / 108, no selects 35 / 106).
+enum { kWholeRuns = 0, kWholeSteps = 1, kAnywhere = 2 };
 constexpr int kTileStride = 32 + 8;                  // floats
-template <int MI, int G>
-constexpr int tile_bytes() {
-  return G * 2 * 16 * MI * kTileStride * 4;
+template <int MI>
+constexpr int tile_bytes(int groups) {
+  return groups * 2 * 16 * MI * kTileStride * 4;
 }
-template <int MI, int G, bool CUT, bool GATED>
+template <int MI, int G, int ENDS, bool GATED>
 __global__ __launch_bounds__(256 * G, 4) void gemm_f32_tiles_kernel(const F32Args a, int tiles_m,
                                                                     int tiles, int share) {
   constexpr int BM = 16 * MI, BK = 32, D = 2, COLS = GATED ? 32 : 64;
+  constexpr bool CUT = ENDS == kAnywhere, SHORT = ENDS != kWholeRuns;
   constexpr int LOADS = (MI + 1) / 2;                // 16-byte pieces of x a thread stages
-  extern __shared__ __attribute__((aligned(16))) float smem[];   // [G][2][BM][kTileStride]
+  extern __shared__ __attribute__((aligned(16))) float smem[];   // [groups][2][BM][kTileStride]
   // workgroups of one die (blockIdx % 8) take neighbouring tiles, the tiles of x fastest, so
   // that its L2 serves the weight rows that they share
   const int tile = (int)(blockIdx.x % 8) * share + (int)(blockIdx.x / 8);
   if (tile >= tiles) return;
   const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * COLS;
-  const int group = threadIdx.x / 256;
+  const int groups = blockDim.x / 256, group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256);
   const int tid = threadIdx.x % 256, lane = tid % 64, wave = tid / 64;
   const int r = lane % 16, g = lane / 16;
   float* lds = smem + group * 2 * BM * kTileStride;
   const int run = a.run, K = a.K;
   const int span = kMaxRuns / G * run;
   const int k_begin = group * span;
-  const int k_count = span;                          // (a multiple of 64)
+  // (in 64s; every group walks as many steps: they share the barriers)
+  const int k_count = SHORT ? min(span, (K + D * BK - 1) / (D * BK) * (D * BK)) : span;
 
   const float* wr = a.W + (long long)weight_row<GATED>(tile / tiles_m * 4 + wave, r, 16, a.N) * a.ldw;
   const float* src[LOADS];
@@ -447,15 +455,18 @@ __global__ __launch_bounds__(256 * G, 4) void gemm_f32_tiles_kernel(const F32Arg
   const auto step = [&](f32x4(&wn)[2], f32x4(&x_ask)[LOADS], const f32x4(&x_keep)[LOADS], int k0, int buf) {
     ask_x(x_ask, k0 + D * BK);
     const float* xs = lds + (buf * BM + r) * kTileStride + 4 * g;
+    const bool live = !SHORT || k_begin + k0 < K;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      f32x4 xv[MI];
+      if (live) {
+        f32x4 xv[MI];
 #pragma unroll
-      for (int b = 0; b < MI; ++b) xv[b] = *(const f32x4*)(xs + b * 16 * kTileStride + h * 16);
+        for (int b = 0; b < MI; ++b) xv[b] = *(const f32x4*)(xs + b * 16 * kTileStride + h * 16);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int b = 0; b < MI; ++b) acc[b] = mfma_f32(wn[h][i], xv[b][i], acc[b]);
+          for (int b = 0; b < MI; ++b) acc[b] = mfma_f32(wn[h][i], xv[b][i], acc[b]);
+        }
       }
       wn[h] = load4<CUT>(wr, k_begin + k0 + D * BK + h * 16 + 4 * g, K);
       left -= 16;
@@ -484,14 +495,18 @@ __global__ __launch_bounds__(256 * G, 4) void gemm_f32_tiles_kernel(const F32Arg
 #pragma unroll
     for (int q = 0; q < D; ++q) step(w[q], x[q], x[(q + 1) % D], k0 + q * BK, q % 2);
   }
-  if (part_runs > 0) end_part();
+  if (G == 1 && SHORT && (left < run || part_runs > 0)) {   // K ended inside a part
+#pragma unroll
+    for (int b = 0; b < MI; ++b) part[b] = part_runs == 0 ? acc[b] : part[b] + acc[b];
+    end_part();
+  }
   if (G == 4) {
 #pragma unroll
     for (int b = 0; b < MI; ++b) total[b] = part[b];
   }
   // [group - 1][the group's part][wave][block][lane]
   constexpr int EACH = 4 / G;
-  static_assert((G - 1) * EACH * 4 * MI * 1024 <= tile_bytes<MI, G>(), "the parts fit the tiles' LDS");
+  static_assert((G - 1) * EACH * 4 * MI * 1024 <= tile_bytes<MI>(G), "the parts fit the tiles' LDS");
   f32x4* hand = (f32x4*)smem;
   const auto place = [&](int q, int b) { return hand + ((q * 4 + wave) * MI + b) * 64 + lane; };
   if (group > 0) {
@@ -505,6 +520,7 @@ __global__ __launch_bounds__(256 * G, 4) void gemm_f32_tiles_kernel(const F32Arg
   if (group > 0) return;
 #pragma unroll
   for (int q = 0; q < (G - 1) * EACH; ++q) {
+    if (SHORT && q >= (groups - 1) * EACH) break;
 #pragma unroll
     for (int b = 0; b < MI; ++b) total[b] += *place(q, b);
   }
@@ -550,23 +566,24 @@ void launch_stream(const F32Args& a, int cus, hipStream_t stream) {
   }
 }
 
-template <int MI, int G, bool CUT, bool GATED>
+template <int MI, int G, int ENDS, bool GATED>
 int launch_tiles_form(const F32Args& a, hipStream_t stream) {
   static LdsGrant grant;
-  constexpr int bytes = tile_bytes<MI, G>();
-  const auto kernel = gemm_f32_tiles_kernel<MI, G, CUT, GATED>;
-  const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
+  const auto kernel = gemm_f32_tiles_kernel<MI, G, ENDS, GATED>;
+  const hipError_t e = grant_lds(grant, (const void*)kernel, tile_bytes<MI>(G));
   RLIS_REQUIRE(e == hipSuccess, "gemm_f32: %s", hipGetErrorString(e));
+  const int groups = ceil_div(a.K, kMaxRuns / G * a.run);   // (no more than have a part)
   const int tm = ceil_div(a.T, 16 * MI), tiles = tm * ceil_div(a.N, GATED ? 32 : 64);
   const int share = ceil_div(tiles, 8);
-  kernel<<<share * 8, 256 * G, bytes, stream>>>(a, tm, tiles, share);
+  kernel<<<share * 8, 256 * groups, tile_bytes<MI>(groups), stream>>>(a, tm, tiles, share);
   return 0;
 }
 
 template <int MI, int G, bool GATED>
 int launch_tiles(const F32Args& a, hipStream_t stream) {
-  return a.K == kMaxRuns * a.run ? launch_tiles_form<MI, G, false, GATED>(a, stream)
-                                 : launch_tiles_form<MI, G, true, GATED>(a, stream);
+  if (a.K == kMaxRuns * a.run) return launch_tiles_form<MI, G, kWholeRuns, GATED>(a, stream);
+  return a.K % 32 == 0 ? launch_tiles_form<MI, G, kWholeSteps, GATED>(a, stream)
+                       : launch_tiles_form<MI, G, kAnywhere, GATED>(a, stream);
 }
 
 template <bool GATED>
@@ -611,7 +628,12 @@ int by_rows(const F32Args& a, int cus, hipStream_t stream) {
   // 93 / 62 / 62 / 77 / 50 us, 2048 x 2048 58 / 43 / 33 / 40 / 49; 200 rows of 16384 x 2048 244 / 145 / 152 / 154 / 145.
   // Four groups take a tile's k in quarters where no compute unit has a second tile (2048 x 2048, 384
   // rows: 33 us against 34 with two, 2048 x 8192: 112 against 119); two otherwise, so that a second tile
-  // works through its first and last steps beside them (16384 x 2048, 384 rows: 212 against 231).
+  // works through its first and last steps beside them (16384 x 2048, 384 rows: 212 against 231), but
+  // 80 rows, whose sums leave no room for a second tile (3072 x 2048, 384 rows: 49 us against 53 with two).
+  // Over a short k a group is soon done and one does with the fewest steps for nothing (8192 x 192, 768 rows: 37 us
+  // with two, 33 with one; x 384 59 and 52; x 768 88 and 86; x 1024 equal), two where all four
+  // would have a part to do (640 x 256, 512 rows: 7.3 us with four, 6.6).  16 rows take two always:
+  // their loads of W bound them, whoever waits (640 x 512, 64 rows: 8.0 us with four, 7.1).
   const int tn = ceil_div(a.N, GATED ? 32 : 64);
   constexpr int kRound[] = {0, 18, 20, 30, 38, 48};
   int mi = 1;
@@ -621,10 +643,15 @@ int by_rows(const F32Args& a, int cus, hipStream_t stream) {
     if (us < least) { least = us; mi = m; }
   }
   const bool pairs = (long long)ceil_div(T, 16 * mi) * tn > cus;
-#define GO(M) \
-  case M: return pairs ? launch_tiles<M, 2, GATED>(a, stream) : launch_tiles<M, 4, GATED>(a, stream)
+  const bool halves = pairs || (a.K <= 512 && a.K == kMaxRuns * a.run);
+#define GO(M)                                                                      \
+  case M:                                                                          \
+    return pairs && a.K <= 768 ? launch_tiles<M, 1, GATED>(a, stream)              \
+                               : halves ? launch_tiles<M, 2, GATED>(a, stream)     \
+                                        : launch_tiles<M, 4, GATED>(a, stream)
   switch (mi) {
-    GO(1); GO(2); GO(3); GO(4);
+    case 1: return launch_tiles<1, 2, GATED>(a, stream);
+    GO(2); GO(3); GO(4);
     default: return launch_tiles<5, 4, GATED>(a, stream);
   }
 #undef GO
