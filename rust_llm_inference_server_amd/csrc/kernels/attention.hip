@@ -376,6 +376,21 @@ template <> struct Vec16<bf16_t> {
   }
 };
 
+// Loads of a key (and runs of a dim's values) that the decode kernel has under way at once; 1: as the
+// compiler orders them.  Few requests wait for these loads, so as many as the registers beside G heads'
+// sums take, and not fewer for heads of 256 dims, whose key is 64 loads.  One request of 600 keys, us, eight and four for every
+// form -> these (before there were any, with the rotation kernel): float32 8 heads of 256 on one KV head 154 -> 73 (110), bfloat16
+// 32 of 128 on 8 40.4 -> 32.4 (35.0), 32 of 64 on 8 26.0 -> 21.7 (24.8), 16 of 80 on 2 64.3 -> 48.5 (76).
+template <typename TX, int G, int DPL>
+constexpr int keys_ahead() {
+  if (sizeof(TX) == 2) return G == 8 && DPL < 4 ? 1 : 4;
+  return G * DPL >= 32 ? 32 : 8;
+}
+template <typename TX, int G>
+constexpr int values_ahead() {
+  return sizeof(TX) == 2 && G >= 4 ? 1 : 4;
+}
+
 // Grid (kv head * head chunks, sequence, split); 256 threads.  Head chunk c serves query
 // heads kvh * g + c * G + [0, G) (those beyond the group are computed on a clamped head and
 // dropped).  Partition `split` of a sequence with n visible keys covers
@@ -479,9 +494,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       const int off = kpos % page_size;
       const TX* kp = k_pages + ((page * nkv + kvh) * page_size + off) * d;
       vbase = (page * nkv + kvh) * (long long)d * page_size + off;
-      // eight loads at once (d is a multiple of 8: what is left over are pairs)
-      constexpr int AT = 8;
-      float kv[AT][VN];
+      constexpr int AT = keys_ahead<TX, G, DPL>();
       const auto dot = [&](int j, const float* kj) {
 #pragma unroll
         for (int hh = 0; hh < G; ++hh) {
@@ -492,17 +505,26 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
         }
       };
       int j = 0;
+      if constexpr (AT > 1) {
+        float kv[AT][VN];
 #pragma unroll 1
-      for (; j + AT * VN <= d; j += AT * VN) {
+        for (; j + AT * VN <= d; j += AT * VN) {
 #pragma unroll
-        for (int b = 0; b < AT; ++b) Vec16<TX>::load(kp + j + b * VN, kv[b]);
+          for (int b = 0; b < AT; ++b) Vec16<TX>::load(kp + j + b * VN, kv[b]);
 #pragma unroll
-        for (int b = 0; b < AT; ++b) dot(j + b * VN, kv[b]);
-      }
+          for (int b = 0; b < AT; ++b) dot(j + b * VN, kv[b]);
+        }
 #pragma unroll 1
-      for (; j < d; j += VN) {
-        Vec16<TX>::load(kp + j, kv[0]);
-        dot(j, kv[0]);
+        for (; j < d; j += VN) {
+          Vec16<TX>::load(kp + j, kv[0]);
+          dot(j, kv[0]);
+        }
+      } else {
+        for (; j < d; j += VN) {
+          float kv[VN];
+          Vec16<TX>::load(kp + j, kv);
+          dot(j, kv);
+        }
       }
     }
     float corr[G];
@@ -530,7 +552,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
       if (j < d) {
         int kk = 0;
         if (vec_run) {
-          constexpr int AT = 4;
+          constexpr int AT = values_ahead<TX, G>();
           float v[AT][VN];
           const auto load = [&](int b, int k) {
             Vec16<TX>::load(v_pages + my_vbase[k] + (long long)j * page_size, v[b]);
@@ -541,17 +563,24 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 #pragma unroll
               for (int hh = 0; hh < G; ++hh) a[hh] = fmaf(my_p[hh * 64 + k + e], v[b][e], a[hh]);
           };
+          if constexpr (AT > 1) {
 #pragma unroll 1
-          for (; kk + AT * VN <= n; kk += AT * VN) {
+            for (; kk + AT * VN <= n; kk += AT * VN) {
 #pragma unroll
-            for (int b = 0; b < AT; ++b) load(b, kk + b * VN);
+              for (int b = 0; b < AT; ++b) load(b, kk + b * VN);
 #pragma unroll
-            for (int b = 0; b < AT; ++b) add(b, kk + b * VN);
-          }
+              for (int b = 0; b < AT; ++b) add(b, kk + b * VN);
+            }
 #pragma unroll 1
-          for (; kk + VN <= n; kk += VN) {
-            load(0, kk);
-            add(0, kk);
+            for (; kk + VN <= n; kk += VN) {
+              load(0, kk);
+              add(0, kk);
+            }
+          } else {
+            for (; kk + VN <= n; kk += VN) {
+              load(0, kk);
+              add(0, kk);
+            }
           }
         }
         for (; kk < n; ++kk) {
