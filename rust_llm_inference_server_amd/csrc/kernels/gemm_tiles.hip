@@ -329,14 +329,25 @@ constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 pa
 // have it.  partials: the result may come as `slices` partial sums (0: as many of 1, 2 and 4 as suit).
 //
 // The tile (and the number of slices) is what makes least of the rounds over the compute units times
-// a round's stages, with what partial sums cost.  The library has tiles of 256 x 256 at more flops a
-// byte, which win once they fill the chip: up to 256 rows this is ahead at every shape (0.43 to 1.01 of
-// its time).  Beyond that, with partial sums: up to 512 rows (0.73 to 1.01), but over a k of 8,192 and
-// more, which the library has in slices too, where the rounds come out even, then up to 1,024 rows
-// (in a step 1B 512 rows 33.9 -> 31.7 us with the norm; uneven 381 rows 27.5 -> 29.9, 3B 512 rows 41.4 ->
-// 43.9), and up to 2,048 where one even round fills the chip (0.86 to 0.96; else 1.0 to 1.1).  Gated, up
-// to 512 rows, where the rounds come out even or there is one (0.88 to 0.96; else 1.01 to 1.3).  Plain,
-// up to 1,024 rows over weights of up to 16 MB (0.91 to 0.98; larger ones 0.98 to 1.15).
+// a round's stages, with what partial sums cost.  Which products are taken is measured against the library's, tried
+// out as it is, with weights that no cache holds: 64 to 57,344 weight rows over a k of 64 to 28,672, 65 to
+// 2,048 rows.  In one slice a tile walks all of k, which the library cuts where there are few tiles (160 x
+// 4096 at 128 rows 13.9 us against its 6.4, 1024 x 8192 35 against 15, 3072 x 4096 22 against 17), so:
+//
+//   plain    k of 256 to 512, and to 1,024 from 1,024 weight rows on: up to 256 rows, to 1,024 over up to
+//            8,192 weight rows (0.27 to 1.06 of the library's time); k up to 2,048 from 1,024 weight rows on while
+//            tiles of 64 x 64 make one round with at least 3/16 of the units in it (0.75 to 1.06; two rounds 0.9 to
+//            1.15); 16,384 weight rows and more (there are tiles enough): up to 128 rows at any k (0.56 to 1.09), to
+//            256 over up to 32,768 (0.65 to 1.06), beyond where rounds come out even (else up to 1.5).
+//   partials k below 8,192: up to 512 rows (0.49 to 1.08; over 1,024 < k <= 2,048 and more than 2,048 weight rows
+//            beyond 256 rows only where the rounds come out even: else up to 1.1), to 2,048 where one even round
+//            fills the chip.  k from 8,192 on, which the library has in slices too: where one even round fills
+//            the chip, to 2,048 rows, and up to 192 rows over up to 1,024 weight rows (0.7 to 1.08; uneven 0.86
+//            to 1.19, two rounds 1.06 to 1.26), over more than 4,096 weight rows up to 128 rows of a k of 16,384
+//            and more (0.64 to 1.02; else up to 1.25).
+//   gated    k up to 1,024, and to 2,048 from 1,024 weight rows on: up to 256 rows, to 512 where the rounds come out
+//            even or there is one (0.36 to 1.03).  Longer k from 5,632 weight rows on: up to 192 rows, beyond where
+//            rounds come out nearly even (0.66 to 1.1; fewer weight rows up to 2.0).
 RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices) {
   if (T <= 0 || N <= 0 || K <= 0) return -1;
   float least = 0.f;
@@ -354,12 +365,32 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     }
   }
   if (best < 0) return -1;
-  const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL);
-  bool here = T <= 256;                    // (up to 64 rows the caller knows which)
-  if (partials)
-    here = here || (K < 8192 ? T <= 512 : T <= 1024 && even) || (T <= 2048 && best_rounds == 1 && even);
-  else if (gated) here = here || (T <= 512 && (even || best_rounds == 1));
-  else here = here || (T <= 1024 && (long long)N * K <= 1 << 23);
+  // (nine in ten places of the rounds have a tile)
+  const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL), one = best_rounds == 1;
+  bool here;
+  if (T <= 64) {
+    here = true;                           // (the caller knows which)
+  } else if (partials) {
+    if (K < 8192) {
+      here = T <= 256 || (T <= 512 && (K <= 1024 || K > 2048 || N <= 2048 || even)) || (T <= 2048 && one && even);
+    } else if (N > 4096) {
+      here = T <= 128 && K >= 16384;
+    } else {
+      here = (T <= 192 && N <= 1024) || (T <= 2048 && one && even && (T <= 512 || N >= 1024));
+    }
+  } else if (gated) {
+    if (K > 2048)
+      here = N >= 5632 && (T <= 192 || (T <= 256 && best_tiles * 20LL >= best_rounds * (kUnits * 17LL)) || (T <= 512 && even));
+    else
+      here = (K <= 1024 || N >= 1024) && (T <= 256 || (T <= 512 && (even || one)));
+  } else if (N >= 64 * kUnits) {
+    here = T <= 128 || (T <= 256 && (N <= 128 * kUnits || (even && K >= 2048)));
+  } else if (K <= 1024) {
+    here = (K <= 512 ? K >= 256 : N >= 1024) && (T <= 256 || (T <= 1024 && N <= 8192));
+  } else {
+    const long long tiles = (long long)ceil_div(T, 64) * ceil_div(N, 64);
+    here = K <= 2048 && N >= 1024 && tiles <= kUnits && tiles >= kUnits * 3 / 16;
+  }
   return here ? best : -1;
 }
 

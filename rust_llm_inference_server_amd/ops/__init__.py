@@ -818,7 +818,7 @@ def _try_out(x, w, y, out_f32, T, N, K, ldx, ldw, slices, ws, stream, partial=Fa
 # with the streaming kernel's form for 17 to 32 rows).  Beyond 32 rows a product of more than this
 # many weight rows is not this kernel's: x is read as often as W there, and tiles of 64 rows read
 # it more often than larger ones (1B output head, 128,256 rows, 64 rows of x: 130 against the library's 120 us
-# and 88 in tiles of 64 x 256; 32 rows of x 108 against the library's 113).
+# and 88 in tiles of 64 x 256, see TILES_WIDE_N; 32 rows of x 108 against the library's 113).
 ROWS_MAX_ROWS = 64
 ROWS_LIBRARY_N = 32768
 
@@ -866,12 +866,15 @@ def _rows_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, slice
     return y
 
 
-# Rows of x from which on the kernel in tiles may take a product.  From the second on those that would
-# go to the library for their many weight rows (the output head: 64 rows, 117 -> 88 us), and gate/up
-# whose tiles of 64 weight rows fill the compute units and that has at least this many elements (64 rows, kernel for 17 to 64 rows -> tiles: 16384 x 2048 16.4 -> 15.0 us,
-# 28672 x 4096 50.0 -> 42.6; 5632 x 2048 11.8 -> 13.5, 4096 x 1024 6.4 -> 9.1, which stay there).
+# Rows of x from which on the kernel in tiles may take a product; from 33 to 64 those of so much of W that
+# one row of tiles fills the compute units: the output head (64 rows: 128256 x 2048 117 -> 88 us, 65536 x
+# 2048 72 -> 46; 50000 x 1024 24 -> 27 and 32776 x 3072 44 -> 65, which stay the library's), and gate/up of at least
+# this many elements (kernel for 17 to 64 rows -> tiles: 16384 x 2048 16.4 -> 15.0, 28672 x 4096 50 -> 43, 57344 x
+# 8192 198 -> 162; 5632 x 2048 11.8 -> 13.5, and over a longer k with just one tile a unit, 16384 x
+# 4096, 27 -> 33, which stay there).
 TILES_MIN_ROWS = 65
 TILES_MIN_ROWS_WIDE = 33
+TILES_WIDE_N = 256 * 256
 TILES_WIDE_GATED = 1 << 25
 
 
@@ -889,8 +892,8 @@ def _tiles(x: torch.Tensor, w: torch.Tensor, gated: bool = False, partials: bool
     N = w.shape[0]
     if T < TILES_MIN_ROWS and not (T >= TILES_MIN_ROWS_WIDE and ROWS_MAX_ROWS >= 64
                                    and STREAM_WIDE_MAX_ROWS > STREAM_MAX_ROWS
-                                   and (N >= 64 * 256 and N * K >= TILES_WIDE_GATED if gated
-                                        else N > ROWS_LIBRARY_N)):
+                                   and (N >= (64 if K <= 3072 else 80) * 256 and N * K >= TILES_WIDE_GATED
+                                        if gated else N >= TILES_WIDE_N)):
         return -1
     if not (BF16_GEMM == "library"
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
