@@ -319,7 +319,6 @@ constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 
                                {64, 128, 0.33f}, {64, 256, 0.46f}};
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
 constexpr int kWideForms = 8;              // those that products of more than 64 rows choose from
-constexpr int kUnits = 256;                // compute units of the chip
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
 
 }  // namespace
@@ -327,6 +326,7 @@ constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 pa
 // How the product of T rows with N weight rows (gated: gate and up rows together) is cut: the tile (an
 // index that rlis_gemm_bf16_tiles takes) + 16 times the slices of k, or -1 where the library should
 // have it.  partials: the result may come as `slices` partial sums (0: as many of 1, 2 and 4 as suit).
+// units: the device's compute units (the figures are those of 256).
 //
 // The tile (and the number of slices) is what makes least of the rounds over the compute units times
 // a round's stages, with what partial sums cost.  Which products are taken is measured against the library's, tried
@@ -348,8 +348,8 @@ constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 pa
 //   gated    k up to 1,024, and to 2,048 from 1,024 weight rows on: up to 256 rows, to 512 where the rounds come out
 //            even or there is one (0.36 to 1.03).  Longer k from 5,632 weight rows on: up to 192 rows, beyond where
 //            rounds come out nearly even (0.66 to 1.1; fewer weight rows up to 2.0).
-RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices) {
-  if (T <= 0 || N <= 0 || K <= 0) return -1;
+RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices, int units) {
+  if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
   float least = 0.f;
   int best = -1, best_rounds = 0, best_tiles = 0;
   for (int s = slices > 0 ? slices : 1; s <= (slices > 0 ? slices : partials ? 4 : 1); s *= 2) {
@@ -357,7 +357,7 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     for (int f = 0; f < (T <= 64 ? kFormCount : kWideForms); ++f) {
       if (T <= 64 && kForms[f].rows > 64) continue;
       const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
-      const long long rounds = (tiles + kUnits - 1) / kUnits;
+      const long long rounds = (tiles + units - 1) / units;
       if (rounds > 1 << 20) continue;
       const float us = (float)rounds * (K / s / kBK) * kForms[f].stage +
                        (s > 1 ? kPartial * s : kPartial / 2) * (float)T * N;
@@ -366,7 +366,7 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   }
   if (best < 0) return -1;
   // (nine in ten places of the rounds have a tile)
-  const bool even = best_tiles * 10LL >= best_rounds * (kUnits * 9LL), one = best_rounds == 1;
+  const bool even = best_tiles * 10LL >= best_rounds * (units * 9LL), one = best_rounds == 1;
   bool here;
   if (T <= 64) {
     here = true;                           // (the caller knows which)
@@ -380,16 +380,16 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     }
   } else if (gated) {
     if (K > 2048)
-      here = N >= 5632 && (T <= 192 || (T <= 256 && best_tiles * 20LL >= best_rounds * (kUnits * 17LL)) || (T <= 512 && even));
+      here = N >= 5632 && (T <= 192 || (T <= 256 && best_tiles * 20LL >= best_rounds * (units * 17LL)) || (T <= 512 && even));
     else
       here = (K <= 1024 || N >= 1024) && (T <= 256 || (T <= 512 && (even || one)));
-  } else if (N >= 64 * kUnits) {
-    here = T <= 128 || (T <= 256 && (N <= 128 * kUnits || (even && K >= 2048)));
+  } else if (N >= 64 * units) {
+    here = T <= 128 || (T <= 256 && (N <= 128 * units || (even && K >= 2048)));
   } else if (K <= 1024) {
     here = (K <= 512 ? K >= 256 : N >= 1024) && (T <= 256 || (T <= 1024 && N <= 8192));
   } else {
     const long long tiles = (long long)ceil_div(T, 64) * ceil_div(N, 64);
-    here = K <= 2048 && N >= 1024 && tiles <= kUnits && tiles >= kUnits * 3 / 16;
+    here = K <= 2048 && N >= 1024 && tiles <= units && tiles >= units * 3 / 16;
   }
   return here ? best : -1;
 }

@@ -818,7 +818,7 @@ def _try_out(x, w, y, out_f32, T, N, K, ldx, ldw, slices, ws, stream, partial=Fa
 # with the streaming kernel's form for 17 to 32 rows).  Beyond 32 rows a product of more than this
 # many weight rows is not this kernel's: x is read as often as W there, and tiles of 64 rows read
 # it more often than larger ones (1B output head, 128,256 rows, 64 rows of x: 130 against the library's 120 us
-# and 88 in tiles of 64 x 256, see TILES_WIDE_N; 32 rows of x 108 against the library's 113).
+# and 88 in tiles of 64 x 256, see TILES_WIDE_ROWS; 32 rows of x 108 against the library's 113).
 ROWS_MAX_ROWS = 64
 ROWS_LIBRARY_N = 32768
 
@@ -874,7 +874,7 @@ def _rows_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, slice
 # 4096, 27 -> 33, which stay there).
 TILES_MIN_ROWS = 65
 TILES_MIN_ROWS_WIDE = 33
-TILES_WIDE_N = 256 * 256
+TILES_WIDE_ROWS = 256                      # weight rows a compute unit
 TILES_WIDE_GATED = 1 << 25
 
 
@@ -890,10 +890,11 @@ def _tiles(x: torch.Tensor, w: torch.Tensor, gated: bool = False, partials: bool
     slices (``library_slices``) partial sums come in as many."""
     T, K = x.shape
     N = w.shape[0]
+    units = _compute_units(x.device)
     if T < TILES_MIN_ROWS and not (T >= TILES_MIN_ROWS_WIDE and ROWS_MAX_ROWS >= 64
                                    and STREAM_WIDE_MAX_ROWS > STREAM_MAX_ROWS
-                                   and (N >= (64 if K <= 3072 else 80) * 256 and N * K >= TILES_WIDE_GATED
-                                        if gated else N >= TILES_WIDE_N)):
+                                   and (N >= (64 if K <= 3072 else 80) * units and N * K >= TILES_WIDE_GATED
+                                        if gated else N >= TILES_WIDE_ROWS * units)):
         return -1
     if not (BF16_GEMM == "library"
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16

@@ -124,7 +124,7 @@ def load() -> ctypes.CDLL:
     lib.rlis_gemm_bf16_rows_slices.restype = c_int
     lib.rlis_gemm_bf16_rows_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_tiles_plan.restype = c_int
-    lib.rlis_gemm_bf16_tiles_plan.argtypes = [I, I, I, I, I, I]
+    lib.rlis_gemm_bf16_tiles_plan.argtypes = [I, I, I, I, I, I, I]
     lib.rlis_gemm_bf16_splitk_slices.restype = c_int
     lib.rlis_gemm_bf16_splitk_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_stream_join_tiles.restype = c_int

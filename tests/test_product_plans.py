@@ -10,8 +10,8 @@ from rust_llm_inference_server_amd.csrc import build
 @pytest.fixture(scope="module")
 def plan():
     fn = ctypes.CDLL(build.ensure("kernels")).rlis_gemm_bf16_tiles_plan
-    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] * 6
-    return fn
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] * 7
+    return lambda *sizes, units=256: fn(*sizes, units)
 
 
 @pytest.mark.parametrize("T,N,K", [(96, 160, 4096), (65, 1024, 8192), (256, 2304, 9216), (1000, 64, 14336), (128, 64, 4096),
@@ -40,3 +40,12 @@ def test_plain_products_that_fill_the_units_are_taken(plan, T, N, K):
 def test_partial_sums_and_gate_up(plan, T, N, K, gated, slices, taken):
     """Products handed over as partial sums (``slices``: as many as the library cuts k into), and gate/up."""
     assert (plan(T, N, K, gated, 1 - gated, slices) >= 0) == taken
+
+
+def test_rounds_are_those_of_the_device(plan):
+    """A partition of a quarter of the compute units has four times the rounds: what fills the chip in one round there
+    is a quarter of the tiles, and larger tiles pay earlier."""
+    assert plan(512, 2048, 2048, 0, 0, 1) >= 0 and plan(512, 2048, 2048, 0, 0, 1, units=64) == -1
+    assert plan(128, 2048, 2048, 0, 0, 1, units=64) >= 0
+    assert plan(96, 6144, 512, 0, 0, 1, units=64) % 16 != plan(96, 6144, 512, 0, 0, 1) % 16
+    assert plan(96, 2048, 2048, 0, 0, 1, units=0) == -1
