@@ -879,8 +879,8 @@ TILES_WIDE_GATED = 1 << 25
 
 
 @functools.lru_cache(maxsize=4096)
-def _tiles_plan(T: int, N: int, K: int, gated: bool, partials: bool, slices: int) -> int:
-    return lib.load().rlis_gemm_bf16_tiles_plan(T, N, K, int(gated), int(partials), slices)
+def _tiles_plan(T: int, N: int, K: int, gated: bool, partials: bool, slices: int, units: int) -> int:
+    return lib.load().rlis_gemm_bf16_tiles_plan(T, N, K, int(gated), int(partials), slices, units)
 
 
 def _tiles(x: torch.Tensor, w: torch.Tensor, gated: bool = False, partials: bool = False) -> int:
@@ -907,7 +907,7 @@ def _tiles(x: torch.Tensor, w: torch.Tensor, gated: bool = False, partials: bool
     slices = library_slices(T, K) if partials else 1
     if slices > 1 and K % (64 * slices):
         return -1
-    return _tiles_plan(T, N, K, gated, partials, slices if slices > 1 or not partials else 0)
+    return _tiles_plan(T, N, K, gated, partials, slices if slices > 1 or not partials else 0, units)
 
 
 def _tiles_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, plan: int,
