@@ -337,14 +337,17 @@ constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 pa
 //   plain    k of 256 to 512, and to 1,024 from 1,024 weight rows on: up to 256 rows, to 1,024 over up to
 //            8,192 weight rows (0.27 to 1.06 of the library's time); k up to 2,048 from 1,024 weight rows on while
 //            tiles of 64 x 64 make one round with at least 3/16 of the units in it (0.75 to 1.06; two rounds 0.9 to
-//            1.15); 16,384 weight rows and more (there are tiles enough): up to 128 rows at any k (0.56 to 1.09), to
+//            1.15), k up to 4,096 up to 160 rows while that round has 3/4 of the units, from 97 rows on, where the
+//            library takes a step, 5/8 (0.81 to 1.03; else 0.94 to 1.3, but 6,144 weight rows at 136 rows 0.75);
+//            16,384 weight rows and more (there are tiles enough): up to 128 rows at any k (0.56 to 1.09), to
 //            256 over up to 32,768 (0.65 to 1.06), beyond where rounds come out even (else up to 1.5).
 //   partials k below 8,192: up to 512 rows (0.49 to 1.08; over 1,024 < k <= 2,048 and more than 2,048 weight rows
 //            beyond 256 rows only where the rounds come out even: else up to 1.1), to 2,048 where one even round
-//            fills the chip.  k from 8,192 on, which the library has in slices too: where one even round fills
-//            the chip, to 2,048 rows, and up to 192 rows over up to 1,024 weight rows (0.7 to 1.08; uneven 0.86
-//            to 1.19, two rounds 1.06 to 1.26), over more than 4,096 weight rows up to 128 rows of a k of 16,384
-//            and more (0.64 to 1.02; else up to 1.25).
+//            fills the chip.  k from 8,192 on, which the library has in slices too: up to 192 rows (0.67 to 1.15
+//            alone; down in a step of the 3B shape, where the library's algorithm is another row count's, 4 us ahead
+//            at 66 to 152 rows), to 2,048 where one even round fills the chip (0.9 to 1.04; uneven up to 1.26,
+//            two rounds of 768 to 2,048 rows 1.06 to 1.26); over more than 4,096 weight rows up to 128 rows of a
+//            k of 16,384 and more (0.64 to 1.02; else up to 1.25).
 //   gated    k up to 1,024, and to 2,048 from 1,024 weight rows on: up to 256 rows, to 512 where the rounds come out
 //            even or there is one (0.36 to 1.03).  Longer k from 5,632 weight rows on: up to 192 rows, beyond where
 //            rounds come out nearly even (0.66 to 1.1; fewer weight rows up to 2.0).
@@ -376,7 +379,7 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     } else if (N > 4096) {
       here = T <= 128 && K >= 16384;
     } else {
-      here = (T <= 192 && N <= 1024) || (T <= 2048 && one && even && (T <= 512 || N >= 1024));
+      here = T <= 192 || (T <= 2048 && one && even && (T <= 512 || N >= 1024));
     }
   } else if (gated) {
     if (K > 2048)
@@ -389,7 +392,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     here = (K <= 512 ? K >= 256 : N >= 1024) && (T <= 256 || (T <= 1024 && N <= 8192));
   } else {
     const long long tiles = (long long)ceil_div(T, 64) * ceil_div(N, 64);
-    here = K <= 2048 && N >= 1024 && tiles <= units && tiles >= units * 3 / 16;
+    here = tiles <= units && (K <= 2048 ? N >= 1024 && tiles >= units * 3 / 16
+                                        : K <= 4096 && T <= 160 && tiles >= units * (T <= 96 ? 6 : 5) / 8);
   }
   return here ? best : -1;
 }
