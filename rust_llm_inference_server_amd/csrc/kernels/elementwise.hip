@@ -252,8 +252,9 @@ static bool launch_add_rmsnorm_bf16x8(float* resid, const void* delta, const voi
 
 // The delta as a stack of float32 partial sums (what the split-k and the streaming products
 // leave for their consumer), rows of a multiple of 4 and at most NT * 4 * CH elements: four
-// elements per thread and chunk, 16-byte accesses.  Such stacks come with few rows (64 at most)
-// and up to dozens of parts, so a row gets a wide workgroup (NT threads, as many as the row has
+// elements per thread and chunk, 16-byte accesses.  Such stacks come with few rows (up to 64) and
+// up to dozens of parts, or with up to 2,048 rows and up to eight (products in tiles, the library's in slices;
+// 512 rows of 2048 with four 6.4 us, 2,048 with two 13.3), so a row gets a wide workgroup (NT threads, as many as the row has
 // groups of four, up to 1024) and every thread keeps up to eight parts of its chunk in flight (four
 // of each where it has several chunks; no more than there are, which the launch chooses); the parts
 // are added in order and their sum rounded to bfloat16 when round_parts is set.  One part: a float32

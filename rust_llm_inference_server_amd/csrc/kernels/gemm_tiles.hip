@@ -1,4 +1,5 @@
-// bfloat16 products y = x * W^T of more than 64 rows of x: portions of prompts, on the matrix cores.
+// bfloat16 products y = x * W^T of more than 64 rows of x (portions of prompts; of 33 on over many weight
+// rows), on the matrix cores.
 //
 // At these sizes what bounds a product is how fast a compute unit is fed, not the matrix cores: every
 // tile brings its rows of x and of W into LDS once per stage of 64 k (buffer_load ... lds, 128 bytes a
@@ -25,20 +26,23 @@
 //
 // 33 to 64 rows take it too where there is much of W (gate/up, the output head): one row of tiles, each
 // line of W read once and non-temporally.  64 rows, us: head 1B 117 (library) -> 88, 3B 164 -> 130; gate/up
-// against gemm_rows.hip 1B 16.5 -> 15.1, 3B 22.5 -> 22.1, 8B 51.4 -> 43.5.
+// against gemm_rows.hip 1B 16.4 -> 15.0, 3B 22.5 -> 22.1, 8B 50.0 -> 42.6.
 //
 // Tiles of 128 to 256 rows by 128, in steps of 32, so that a round comes out even over the compute units
-// (gate/up of the 1B shape at 381 rows: two of 192 31.9 us, three of 128 35.4, the library's with
-// the SwiGLU kernel 36.2).  More stages under way than the tiles have here change nothing.
+// (gate/up of the 1B shape at 381 rows in a step: two of 192 31.3 us, three of 128 35.4, the library's with
+// the SwiGLU kernel 36.7).  More stages under way than the tiles have here change nothing.
 //
-// MI355X, us, weights cold, the library's product (with SwiGLU kernel; with the norm that adds
-// output's and down's partial sums) -> this, at 96 / 256 / 512 rows:
-//   1B  q/k/v 10.6 -> 9.1, 10.9 -> 9.6, 13.6 -> 12.9      output 12.0 -> 9.9, 13.6 -> 11.9, 15.9 -> 14.5
-//       gate/up 22.8 -> 20.0, 34.4 -> 27.8, 41.4 -> 39.7  down 24.5 -> 16.0, 30.8 -> 23.7, 38.7 -> 32.0
-//   3B  q/k/v 18.7 -> 16.7, 32.2 -> 24.9                  output 22.2 -> 14.8, 22.8 -> 19.8, 27.5 -> 26.9
-//       gate/up 29.7 -> 29.6, 46.7 -> 40.6, 59.1 -> 55.4  down 40.8 -> 21.7, 39.6 -> 34.9, 52.2 -> 44.3
-//   8B  q/k/v 23.9 -> 21.5, 40.9 -> 32.5                  output 26.9 -> 16.7, 28.5 -> 24.4, 37.0 -> 33.9
-//       gate/up 56.2 -> 50.6, 75.8 -> 70.3                down 69.9 -> 35.0, 69.0 -> 52.1, 99.0 -> 72.1
+// MI355X, us, weights cold, the library's product, tried out (with SwiGLU kernel; with the norm that adds
+// output's and down's partial sums) -> this, at 96 / 256 / 512 rows (-: the library's):
+//   1B  q/k/v 13.0 -> 12.0, 14.1 -> 12.7, -               output 15.6 -> 10.4, 16.1 -> 13.2, 18.0 -> 16.7
+//       gate/up 23.5 -> 20.0, 31.3 -> 27.1, 42.2 -> 36.6  down 16.3 -> 16.0, 24.8 -> 23.2, 33.0 -> 31.6
+//   3B  q/k/v -, at 112 rows 19.1 -> 17.4                 output 17.9 -> 14.3, 21.7 -> 22.5, 27.4 -> 27.6
+//       gate/up 30.4 -> 29.5, 41.8 -> 40.1, 60.7 -> 51.4  down 22.6 -> 22.0, -, -
+//   8B  q/k/v 20.6 -> 21.3, at 112 rows 25.9 -> 22.2      output 20.8 -> 16.6, 26.1 -> 26.9, 36.7 -> 32.9
+//       gate/up 62.2 -> 55.4, 77.1 -> 70.2, -             down 36.0 -> 35.2, 47.6 -> 46.7, 71.4 -> 69.3
+// In a step, where a row count between those tried out takes another's algorithm, the library is further behind
+// (prompts of 72 / 128 / 200 tokens, twelve layers, us: 1B 1,204 -> 1,037, 1,232 -> 1,099, 1,429 -> 1,248; 8B 2,107 ->
+// 1,824, 2,334 -> 2,043, 2,666 -> 2,342).
 #include "common.h"
 #include "gemm_stream.h"
 

@@ -933,8 +933,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     float32 weight or ``x`` beside bfloat16, the plain FMA kernel.
     bfloat16 operands take the streaming kernel up to 16 rows (32 over short rows) and the kernel
     for 17 to 64 rows beyond (``_rows_kernel``; few weight rows over a long k only as partial sums,
-    ``_rows_in_one_slice``); from 65 rows on the kernel in tiles where it is ahead of the library
-    (``_tiles``); other products, and other sizes, go to the library's
+    ``_rows_in_one_slice``); from 65 rows on, over many weight rows from 33 on, the kernel in tiles where it
+    is ahead of the library (``_tiles``); other products, and other sizes, go to the library's
     GEMM (hipBLASLt, through its own entry points), or with ``BF16_GEMM = "own"`` to the skinny
     kernel up to 64 rows and the hand-written matrix-core GEMM beyond.
 
@@ -1183,8 +1183,9 @@ def linear_scaled(xw: torch.Tensor, ss: torch.Tensor, eps: float, w: torch.Tenso
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]`` of shape ``(2 I, K)``.
 
-    Up to 16 rows of bfloat16 (32 over short rows), 17 to 64 of sizes that ``_rows_kernel`` takes, more
-    where ``_tiles`` is ahead, and float32 that ``_f32_kernels`` takes (the same bits) go through one kernel that never stores the
+    Up to 16 rows of bfloat16 (32 over short rows), 17 to 64 of sizes that ``_rows_kernel`` takes, 33 and more
+    where ``_tiles`` is ahead, and float32 that ``_f32_kernels`` takes (the same bits; but 5 to 16 rows of few
+    weight rows over a long k) go through one kernel that never stores the
     ``(T, 2 I)`` intermediate; everything else is the product followed by the SwiGLU kernel."""
     T, K = x.shape
     two_i = w_gate_up.shape[0]
