@@ -378,9 +378,10 @@ template <> struct Vec16<bf16_t> {
 
 // Loads of a key (and runs of a dim's values) that the decode kernel has under way at once; 1: as the
 // compiler orders them.  Few requests wait for these loads, so as many as the registers beside G heads'
-// sums take, and not fewer for heads of 256 dims, whose key is 64 loads.  One request of 600 keys, us, eight and four for every
-// form -> these (before there were any, with the rotation kernel): float32 8 heads of 256 on one KV head 154 -> 73 (110), bfloat16
-// 32 of 128 on 8 40.4 -> 32.4 (35.0), 32 of 64 on 8 26.0 -> 21.7 (24.8), 16 of 80 on 2 64.3 -> 48.5 (76).
+// sums take, and not fewer for heads of 256 dims, whose key is 64 loads.  One request of 600 keys, us,
+// eight and four for every form -> these (before there were any, with the rotation kernel): float32 8 heads
+// of 256 on one KV head 154 -> 73 (110), bfloat16 32 of 128 on 8 40.4 -> 32.4 (35.0), 32 of 64 on 8 26.0 ->
+// 21.7 (24.8), 16 of 80 on 2 64.3 -> 48.5 (76).
 template <typename TX, int G, int DPL>
 constexpr int keys_ahead() {
   if (sizeof(TX) == 2) return G == 8 && DPL < 4 ? 1 : 4;
