@@ -28,6 +28,16 @@
 // line of W read once and non-temporally.  64 rows, us: head 1B 117 (library) -> 88, 3B 164 -> 130; gate/up
 // against gemm_rows.hip 1B 16.4 -> 15.0, 3B 22.5 -> 22.1, 8B 50.0 -> 42.6.
 //
+// q, k and v (kOutHeads): the weight rows of dims j and j + d / 2 of a head lie in turn like gate and up, so a lane
+// holds both halves of what a rotation turns; it turns the keys and stores keys and values to the cache's pages, and
+// the queries stay as they are for the attention kernels to turn.  In place of the library's product and a pass of
+// 6 to 8 us over its rows (elementwise.hip); weights cold, us: 1B 128 / 512 / 1,024 / 2,048 rows 16.3 -> 10.5, 21.8 ->
+// 16.8, 27.7 -> 23.9, 36.8 -> 34.7; 3B 24.3 -> 19.5, 32.7 -> 33.1, 46.2 -> 42.0, - ; 8B 29.2 -> 23.9, 42.9 -> 39.1, 59.6
+// -> 57.3, - .  Tiles 96 wide make even rounds of 3,072 and 6,144 weight rows.  Values are stored two bytes
+// at a time, sixteen tokens side by side: the tiles that hold them end a microsecond later than the others.
+//
+// 256 x 256 has the most operations to a byte that is fed (the accumulators fill half of a wave's registers).
+//
 // Tiles of 128 to 256 rows by 128, in steps of 32, so that a round comes out even over the compute units
 // (gate/up of the 1B shape at 381 rows in a step: two of 192 31.3 us, three of 128 35.4, the library's with
 // the SwiGLU kernel 36.7).  More stages under way than the tiles have here change nothing.
@@ -64,6 +74,18 @@ __device__ __forceinline__ void wait_loads() {
 }
 __device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// The step's q, k and v rows on their way out (kOutHeads): q as it is, k turned by its position and v into
+// the cache's pages.
+struct HeadsArgs {
+  const float* cos;        // (positions, d / 2) float32; null: nothing is turned
+  const float* sin;
+  const int* positions;    // (T)
+  const int* slots;        // (T) page * page size + offset; below 0: not stored
+  bf16_t* k_pages;         // (pages, nkv, page size, d)
+  bf16_t* v_pages;         // (pages, nkv, d, page size)
+  int nh, nkv, half_shift, page_shift;   // d / 2 and the page size are powers of two
+};
+
 struct TilesArgs {
   const bf16_t* X;
   const bf16_t* W;
@@ -73,9 +95,79 @@ struct TilesArgs {
   int group;               // tiles of x's rows that are walked together
   int ldx, ldw;            // elements
   long long ldy, slice_stride;
+  HeadsArgs heads;
 };
 
-enum { kOutBf16 = 0, kOutF32 = 1, kOutGated = 2 };
+// (kOutGated, kOutHeads: N counts pairs of weight rows whose products meet in a lane)
+enum { kOutBf16 = 0, kOutF32 = 1, kOutGated = 2, kOutHeads = 3 };
+constexpr bool in_pairs(int out) { return out >= kOutGated; }
+
+// Four or eight neighbouring dims of a head.
+template <int Q>
+__device__ __forceinline__ void store_dims(bf16_t* to, const float (&v)[4 * Q]) {
+  uint32_t o[2 * Q];
+#pragma unroll
+  for (int i = 0; i < 2 * Q; ++i) o[i] = f32_to_bf16(v[2 * i]) | (uint32_t)f32_to_bf16(v[2 * i + 1]) << 16;
+  if (Q == 2) *(uint4*)to = make_uint4(o[0], o[1], o[2 * Q - 2], o[2 * Q - 1]);
+  else *(uint2*)to = make_uint2(o[0], o[1]);
+}
+
+// The sums that a lane holds of one token: dims j .. and j + d / 2 .. of whichever heads its columns are.
+template <int MI, int NI>
+__device__ __forceinline__ void store_heads(const TilesArgs& p, const f32x4 (&acc)[NI][MI], int m, int token,
+                                            int first, int g) {
+  constexpr int Q = NI % 4 == 0 ? 2 : 1;   // pairs of blocks whose dims are neighbours
+  const HeadsArgs& h = p.heads;
+  const int half = 1 << h.half_shift, d = 2 * half;
+#pragma unroll
+  for (int a = 0; a < NI / 2; a += Q) {
+    const int n = first + a * 16 + g * 4 * Q;
+    if (n >= p.N) continue;
+    const int head = n >> h.half_shift, j = n & (half - 1);
+    float lo[4 * Q], hi[4 * Q];
+#pragma unroll
+    for (int e = 0; e < 4 * Q; ++e) {
+      lo[e] = acc[2 * (a + e / 4)][m][e % 4];
+      hi[e] = acc[2 * (a + e / 4) + 1][m][e % 4];
+    }
+    if (head < h.nh) {
+      bf16_t* to = (bf16_t*)p.Y + (long long)token * p.ldy + head * d + j;
+      store_dims<Q>(to, lo);
+      store_dims<Q>(to + half, hi);
+      continue;
+    }
+    const int slot = h.slots[token];
+    if (slot < 0) continue;
+    const long long page = slot >> h.page_shift;
+    const int off = slot & ((1 << h.page_shift) - 1);
+    if (head < h.nh + h.nkv) {
+      bf16_t* to = h.k_pages + (((page * h.nkv + head - h.nh) << h.page_shift) + off) * d + j;
+      if (h.cos) {
+        const long long at = (long long)h.positions[token] * half + j;
+#pragma unroll
+        for (int e = 0; e < 4 * Q; e += 4) {
+          const f32x4 c = *(const f32x4*)(h.cos + at + e), s = *(const f32x4*)(h.sin + at + e);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            // (the product is rounded first, as one that goes through memory is)
+            const float x = bf16_to_f32(f32_to_bf16(lo[e + i])), y = bf16_to_f32(f32_to_bf16(hi[e + i]));
+            lo[e + i] = x * c[i] - y * s[i];
+            hi[e + i] = y * c[i] + x * s[i];
+          }
+        }
+      }
+      store_dims<Q>(to, lo);
+      store_dims<Q>(to + half, hi);
+    } else {
+      bf16_t* to = h.v_pages + ((((page * h.nkv + head - h.nh - h.nkv) * d + j) << h.page_shift) + off);
+#pragma unroll
+      for (int e = 0; e < 4 * Q; ++e) {
+        to[(long long)e << h.page_shift] = f32_to_bf16(lo[e]);
+        to[(long long)(e + half) << h.page_shift] = f32_to_bf16(hi[e]);
+      }
+    }
+  }
+}
 
 // WM x WN waves, each MI groups of 16 rows of x by NI groups of 16 weight rows; BUFS stages in LDS.
 template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT>
@@ -86,6 +178,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
   constexpr int XI = BM / 8 / WAVES, WI = BN / 8 / WAVES, PER = XI + WI;
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "");
   static_assert(NI % 2 == 0, "");
+  // The largest tile has room for two stages and a half: its ring is one of quarter stages (half of x's
+  // rows, half of W's), ten of them, and a stage's x is asked for half a stage ahead of its W.
+  constexpr bool QUARTERS = BUFS == 2 && WAVES == 8;
+  static_assert(!QUARTERS || (BM == BN && WM == 2 && WN % 2 == 0), "");
+  constexpr int RING = QUARTERS ? STAGE / 2 * 5 : STAGE * BUFS;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int r = lane % 16, g = lane / 16;
@@ -105,7 +202,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
     const int band = lin / (p.group * p.nt), rows = min(p.group, p.mt - band * p.group);
     lin -= band * p.group * p.nt;
     m0 = (band * p.group + lin % rows) * BM;
-    n0 = lin / rows * (OUT == kOutGated ? BN / 2 : BN);
+    n0 = lin / rows * (in_pairs(OUT) ? BN / 2 : BN);
   };
 
   // Instruction i of this wave brings rows (i * WAVES + wave) * 8 .. + 7 of a stage, x rows first;
@@ -126,11 +223,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
       const int q = (i * WAVES + wave) * 8 + q8;
       const int b = q / 16, o = q % 16;
       int n;
-      if (OUT == kOutGated) {
-        // groups of 16: gate and up rows in turn, of the same columns
+      if (in_pairs(OUT)) {
+        // groups of 16 in turn: gate and up rows of the same columns, or dims j and j + d / 2 of a head
         const int pair = b / 2;
         const int col = NI % 4 == 0 ? pair / 2 * 32 + o / 4 * 8 + pair % 2 * 4 + o % 4 : pair * 16 + o;
-        n = min(n0 + col, p.N - 1) + (b % 2 ? p.N : 0);
+        n = min(n0 + col, p.N - 1);
+        if (OUT == kOutGated) n += b % 2 ? p.N : 0;
+        else n += (n >> p.heads.half_shift << p.heads.half_shift) + (b % 2 << p.heads.half_shift);
       } else if (OUT == kOutBf16) {
         // two groups of 16 share 32 columns so that a lane holds eight neighbours
         n = min(n0 + b / 2 * 32 + o / 4 * 8 + b % 2 * 4 + o % 4, p.N - 1);
@@ -140,17 +239,19 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
       src[XI + i] = ((uint32_t)n * p.ldw + (uint32_t)((c ^ (q / 2 % 8)) * 8)) * 2;
     }
     a_from = slice * p.steps * (kBK * 2);
-    const int turn = n0 / (OUT == kOutGated ? BN / 2 : BN);   // (of the weight rows alone)
+    const int turn = n0 / (in_pairs(OUT) ? BN / 2 : BN);   // (of the weight rows alone)
     a_k = a_from + turn % p.steps * (kBK * 2);
   };
   int a_id = blockIdx.x, a_left = p.steps, a_buf = 0;
   const auto ask = [&](int i) {
-    const lds_ptr to = (lds_ptr)(smem + a_buf + (i * WAVES + wave) * 1024);
+    int at = a_buf;
+    if (QUARTERS && i * 4 / PER * (STAGE / 4) + at >= RING) at -= RING;
+    const lds_ptr to = (lds_ptr)(smem + at + (i * WAVES + wave) * 1024);
     if (i < XI) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, to, 16, src[i], a_k, 0, 0);
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, src[i], a_k, 0, NT ? 2 : 0);
   };
   const auto asked = [&]() {               // the stage has been asked for, on to the next
-    a_buf = a_buf + STAGE == BUFS * STAGE ? 0 : a_buf + STAGE;
+    a_buf = a_buf + STAGE >= RING ? a_buf + STAGE - RING : a_buf + STAGE;
     a_k += kBK * 2;
     if (a_k == a_from + p.steps * (kBK * 2)) a_k = a_from;
     if (--a_left == 0) {
@@ -162,14 +263,21 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
   };
 
   // fragments of a half stage (32 k)
-  const int x_at = (wm * 16 * MI + r) * 128 + ((g ^ (r / 2)) * 16);
-  const int w_at = (BM + wn * 16 * NI + r) * 128 + ((g ^ (r / 2)) * 16);
+  constexpr int X_PART = QUARTERS ? 16 * MI : BM;  // rows of a part of the ring
+  const int x_at = (wm * 16 * MI % X_PART + r) * 128 + ((g ^ (r / 2)) * 16);
+  const int w_at = ((QUARTERS ? 0 : BM) + wn * 16 * NI % (QUARTERS ? BN / 2 : BN) + r) * 128 + ((g ^ (r / 2)) * 16);
+  const int w_part = QUARTERS ? (2 + wn / (WN / 2)) * (STAGE / 4) : 0, x_part = QUARTERS ? wm * (STAGE / 4) : 0;
+  int x_buf = x_part, w_buf = w_part;
+  const auto onward = [&]() {              // to the next stage's parts
+    x_buf = x_buf + STAGE >= RING ? x_buf + STAGE - RING : x_buf + STAGE;
+    w_buf = w_buf + STAGE >= RING ? w_buf + STAGE - RING : w_buf + STAGE;
+  };
   struct Half {
     bf16x8 x[MI], w[NI];
   };
-  const auto read = [&](Half& h, int buf, int ks, int i) {
-    if (i < MI) h.x[i] = *(const bf16x8*)(smem + buf + (x_at ^ (ks * 64)) + i * 2048);
-    else h.w[i - MI] = *(const bf16x8*)(smem + buf + (w_at ^ (ks * 64)) + (i - MI) * 2048);
+  const auto read = [&](Half& h, int ks, int i) {
+    if (i < MI) h.x[i] = *(const bf16x8*)(smem + x_buf + (x_at ^ (ks * 64)) + i * 2048);
+    else h.w[i - MI] = *(const bf16x8*)(smem + w_buf + (w_at ^ (ks * 64)) + (i - MI) * 2048);
   };
   f32x4 acc[NI][MI];
   const auto clear = [&]() {
@@ -179,10 +287,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
       for (int m = 0; m < MI; ++m) acc[a][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
   // The products of one half stage.  Between them, one at a time, so that neither the LDS nor the
-  // memory pipe makes a wave wait before its products: the reads of the half stage to come and half
-  // of the loads of the stage that takes the place of the last one.
+  // memory pipe makes a wave wait before its products: the reads of the half stage to come and loads of
+  // later stages.
   constexpr int PRODUCTS = NI * MI, READS = MI + NI, LATE = PER / 2;
-  const auto half = [&](const Half& h, Half& next, int buf, int ks, int from, int loads) {
+  const auto half = [&](const Half& h, Half& next, int ks, auto loads) {
 #pragma unroll
     for (int j = 0; j < PRODUCTS; ++j) {
       const int a = j / MI, m = j % MI;
@@ -190,17 +298,39 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < READS; ++i)
-        if (i * 3 * PRODUCTS / (READS * 4) == j) read(next, buf, ks, i);
-#pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if (i < loads && i * PRODUCTS / loads == j) ask(from + i);
+        if (i * 3 * PRODUCTS / (READS * 4) == j) read(next, ks, i);
+      loads(j);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // loads from .. from + count - 1 of the stage to ask for, spread over `places` products from `first` on
+  const auto some = [&](int j, int from, int count, int first, int places) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (i < count && first + i * places / count == j) ask(from + i);
+  };
+  // Beside a stage's earlier half the later loads of the stage that takes the place of the last one,
+  // beside its later half the first ones of the next.  In quarters all of a stage beside its later half: the W
+  // that the ring has room for now, then the next stage's x (gate/up of 2,048 rows of the 1B shape 116 us with x beside
+  // the earlier half, 110 so).
+  const auto early = [&](int j) {
+    if (!QUARTERS) some(j, PER - LATE, LATE, 0, PRODUCTS);
+  };
+  const auto late = [&](int j) {
+    if (!QUARTERS) {
+      some(j, 0, PER - LATE, 0, PRODUCTS);
+    } else {
+      some(j, PER / 2, PER / 2, 0, PRODUCTS / 2);
+      if (j == PRODUCTS / 2 - 1) asked();
+      some(j, 0, PER / 2, PRODUCTS / 2, PRODUCTS / 2);
+    }
+  };
+  // (loads that may still be under way when a stage must be whole)
+  constexpr int AHEAD = QUARTERS ? PER / 2 : PER * (BUFS - 2);
 
   sources(a_id);
 #pragma unroll
-  for (int s = 0; s < BUFS - 1; ++s) {
+  for (int s = 0; s < (QUARTERS ? BUFS : BUFS - 1); ++s) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) ask(i);
     asked();
@@ -208,21 +338,20 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
 #pragma unroll
   for (int i = 0; i < PER - LATE; ++i) ask(i);
   Half h0, h1;
-  wait_loads<PER*(BUFS - 2) + PER - LATE>();
+  wait_loads<PER*(QUARTERS ? 1 : BUFS - 2) + PER - LATE>();
   barrier();
 #pragma unroll
-  for (int i = 0; i < READS; ++i) read(h0, 0, 0, i);
+  for (int i = 0; i < READS; ++i) read(h0, 0, i);
   wait_loads<63>();
-  int buf = 0;
   for (int id = blockIdx.x; id < total; id += gridDim.x) {
     clear();
     for (int step = 0; step < p.steps; ++step) {
-      half(h0, h1, buf, 1, PER - LATE, LATE);
-      asked();
-      wait_loads<PER*(BUFS - 2)>();
+      half(h0, h1, 1, early);
+      if (!QUARTERS) asked();
+      wait_loads<AHEAD>();
       barrier();                           // the next stage is whole, this one has been read
-      buf = buf + STAGE == BUFS * STAGE ? 0 : buf + STAGE;
-      half(h1, h0, buf, 0, 0, PER - LATE);
+      onward();
+      half(h1, h0, 0, late);
       wait_loads<63>();                    // (of h0)
     }
     int m0, n0, slice;
@@ -250,6 +379,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
           if (Q == 2) *(uint4*)(row + n) = make_uint4(o[0], o[1], o[2 * Q - 2], o[2 * Q - 1]);
           else *(uint2*)(row + n) = make_uint2(o[0], o[1]);
         }
+      } else if (OUT == kOutHeads) {
+        store_heads<MI, NI>(p, acc, m, token, n0 + wn * NI * 8, g);
       } else if (OUT == kOutBf16) {
         bf16_t* row = (bf16_t*)p.Y + (long long)token * p.ldy;
 #pragma unroll
@@ -280,13 +411,13 @@ template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT>
 int launch_tiles(TilesArgs a, hipStream_t stream) {
   static LdsGrant grant;
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN;
-  constexpr int bytes = BUFS * (BM + BN) * kBK * 2;
+  constexpr int bytes = (BUFS * 2 + (BUFS == 2 && WM * WN == 8)) * (BM + BN) * kBK;
   static_assert(bytes <= 160 * 1024, "");
   const auto kernel = gemm_tiles_kernel<MI, NI, WM, WN, BUFS, OUT, NT>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_tiles: %s", hipGetErrorString(e));
   a.mt = ceil_div(a.T, BM);
-  a.nt = ceil_div(a.N, OUT == kOutGated ? BN / 2 : BN);
+  a.nt = ceil_div(a.N, in_pairs(OUT) ? BN / 2 : BN);
   a.group = std::min(a.mt, 8);
   const int cus = rlis_stream_compute_units();
   RLIS_REQUIRE(cus > 0, "gemm_tiles: cannot read the device properties");
@@ -301,14 +432,50 @@ template <int MI, int NI, int WM, int WN, int BUFS>
 int launch_out(const TilesArgs& a, int out, int nt, hipStream_t stream) {
   // (rows of W that a second tile reads too must stay in the caches: the output head of the 1B shape at 96
   // rows in tiles of 64 x 256 132 us, non-temporally 178)
-  if (nt && a.T <= 16 * MI * WM) {
+  if (nt && a.T <= 16 * MI * WM && out != kOutHeads) {
     if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16, true>(a, stream);
     if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32, true>(a, stream);
     return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated, true>(a, stream);
   }
+  if (out == kOutHeads) return launch_tiles<MI, NI, WM, WN, BUFS, kOutHeads, false>(a, stream);
   if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16, false>(a, stream);
   if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32, false>(a, stream);
   return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated, false>(a, stream);
+}
+
+// Tiles of which a compute unit holds two, unless there are not that many: a unit with one has all of the LDS
+// for its ring (q/k/v, cold weights, us: 200 x 5,120 x 3,072 in 128 x 64 26.2 with three stages, 23.8 with six; 65 x
+// 6,144 x 4,096 in 64 x 64 22.0 with four, 19.5 with nine; output of 512 rows of the 1B shape no faster).
+template <int MI, int NI, int WM, int WN, int BUFS, int ALONE>
+int launch_deep(const TilesArgs& a, int out, int nt, hipStream_t stream) {
+  const long long tiles = (long long)ceil_div(a.T, 16 * MI * WM) * ceil_div(a.N, 8 * NI * WN);
+  if (out == kOutHeads && tiles <= rlis_stream_compute_units())
+    return launch_tiles<MI, NI, WM, WN, ALONE, kOutHeads, false>(a, stream);
+  return launch_out<MI, NI, WM, WN, BUFS>(a, out, nt, stream);
+}
+
+int launch_form(const TilesArgs& a, int out, int tile, int nt, hipStream_t stream) {
+  int rc = -1;
+  switch (tile) {
+    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, nt, stream); break;   // 128 x 256
+    case 1: rc = launch_out<4, 4, 4, 2, 3>(a, out, nt, stream); break;   // 256 x 128
+    case 2: rc = launch_out<7, 4, 2, 2, 3>(a, out, nt, stream); break;   // 224 x 128
+    case 3: rc = launch_out<6, 4, 2, 2, 3>(a, out, nt, stream); break;   // 192 x 128
+    case 4: rc = launch_out<5, 4, 2, 2, 4>(a, out, nt, stream); break;   // 160 x 128
+    case 5: rc = launch_out<4, 2, 2, 4, 5>(a, out, nt, stream); break;   // 128 x 128
+    case 6: rc = launch_deep<4, 2, 2, 2, 3, 6>(a, out, nt, stream); break;  // 128 x 64, two to a compute unit
+    case 7: rc = launch_deep<2, 2, 2, 2, 4, 9>(a, out, nt, stream); break;  // 64 x 64, two to a compute unit
+    case 8: rc = launch_out<4, 2, 1, 4, 3>(a, out, nt, stream); break;   // 64 x 128, two to a compute unit
+    case 9: rc = launch_out<4, 4, 1, 4, 2>(a, out, nt, stream); break;   // 64 x 256, two to a compute unit
+    case 10: rc = launch_out<8, 4, 2, 4, 2>(a, out, nt, stream); break;  // 256 x 256
+    case 11: if (out == kOutHeads) rc = launch_tiles<2, 6, 4, 1, 5, kOutHeads, false>(a, stream); break;  // 128 x 96
+    case 12: if (out == kOutHeads) rc = launch_tiles<1, 6, 4, 1, 4, kOutHeads, false>(a, stream); break;  // 64 x 96, two to a unit
+    default: RLIS_REQUIRE(false, "gemm_tiles: no tile %d", tile);
+  }
+  RLIS_REQUIRE(rc >= 0, "gemm_tiles: tile %d is of q, k and v alone", tile);
+  if (rc) return rc;
+  RLIS_LAUNCH_CHECK("gemm_tiles");
+  return 0;
 }
 
 // The tiles: rows of x by weight rows, and how long a stage takes (us; where two workgroups share a
@@ -324,6 +491,19 @@ constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
 constexpr int kWideForms = 8;              // those that products of more than 64 rows choose from
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
+
+// The same for q, k and v on their way to the cache: a stage's time with two workgroups to a compute unit and
+// alone (where there is no more than one tile a unit), and what ends a round (us).
+struct HeadsForm {
+  int tile, rows, cols;
+  float stage, alone, end;
+};
+constexpr HeadsForm kHeadsForms[] = {
+    {0, 128, 256, 0.73f, 0.73f, 2.7f}, {1, 256, 128, 0.67f, 0.67f, 3.6f}, {3, 192, 128, 0.545f, 0.545f, 5.1f},
+    {4, 160, 128, 0.48f, 0.48f, 3.9f}, {5, 128, 128, 0.47f, 0.47f, 1.4f}, {6, 128, 64, 0.32f, 0.36f, 0.f},
+    {7, 64, 64, 0.204f, 0.215f, 0.f},  {10, 256, 256, 1.17f, 1.17f, 8.6f}, {11, 128, 96, 0.40f, 0.40f, 2.4f},
+    {12, 64, 96, 0.27f, 0.30f, 0.f}};
+constexpr int kHeadsFormCount = sizeof(kHeadsForms) / sizeof(kHeadsForms[0]);
 
 }  // namespace
 
@@ -402,6 +582,30 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   return here ? best : -1;
 }
 
+// The tile that rlis_gemm_bf16_tiles_heads should take for T rows and N weight rows, or -1 where the library's
+// product and the kernel that turns and stores (elementwise.hip) are ahead.  Both sides are estimated: a tile's
+// stages, what ends a round and what is fixed; the library's from the bytes of W, the operations and the rows that
+// pass through memory.  Fitted to 65 to 8,192 rows of ten shapes, 1,536 to 12,288 weight rows over a k of 512 to
+// 8,192, weights cold (tiles to 10 %; the library, whose algorithms are a clock's choice, to 15 %).  Of 136 products
+// the rule takes 120, 0.55 to 1.02 of the library's time; beyond 8,192 weight rows the tiles have to be ahead by a
+// fifteenth (12,288 x 4,096 at 768 and 1,024 rows would be taken at 1.05 to 1.1).  Figures are those of 256 units.
+RLIS_API int rlis_gemm_bf16_tiles_heads_plan(int T, int N, int K, int units) {
+  if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
+  float least = 0.f;
+  int best = -1;
+  for (int f = 0; f < kHeadsFormCount; ++f) {
+    const HeadsForm& form = kHeadsForms[f];
+    const long long tiles = (long long)ceil_div(T, form.rows) * ceil_div(N, form.cols);
+    const long long rounds = (tiles + units - 1) / units;
+    const float us = (float)rounds * (K / kBK * (rounds == 1 ? form.alone : form.stage) + form.end);
+    if (best < 0 || us < least) least = us, best = form.tile;
+  }
+  const float share = 256.f / units;
+  const float here = least + 4.9f + (0.095e-6f * K + 0.6e-6f * T) * N;
+  const float library = 12.f + 0.454e-6f * N * K + (1.19e-9f * T * K + 1.05e-6f * T) * N * share;
+  return here < library * (N > 32 * units ? 0.93f : 1.f) ? best : -1;
+}
+
 // Y (T,N) = X (T,K) * W (N,K)^T, N a multiple of 8, K of 64 times the slices.  out 0: bfloat16; 1:
 // float32, `slices` partial results slice_stride elements apart; 2: gated, W (2 N,K) gate rows then up
 // rows, Y = silu(gate) * up in bfloat16.  tile: as rlis_gemm_bf16_tiles_plan gives it.  nt: W is loaded
@@ -419,22 +623,37 @@ RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out
   RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * N * (out == 2 ? 2 : 1) < (1LL << 32),
                "gemm_tiles: x or W passes 4 GB");
   const TilesArgs a = {(const bf16_t*)X, (const bf16_t*)W, Y, T, N, K / slices / kBK, 0, 0, slices, 0,
-                       (int)ldx, (int)ldw, ldy, slice_stride};
-  int rc = 1;
-  switch (tile) {
-    case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, nt, stream); break;   // 128 x 256
-    case 1: rc = launch_out<4, 4, 4, 2, 3>(a, out, nt, stream); break;   // 256 x 128
-    case 2: rc = launch_out<7, 4, 2, 2, 3>(a, out, nt, stream); break;   // 224 x 128
-    case 3: rc = launch_out<6, 4, 2, 2, 3>(a, out, nt, stream); break;   // 192 x 128
-    case 4: rc = launch_out<5, 4, 2, 2, 4>(a, out, nt, stream); break;   // 160 x 128
-    case 5: rc = launch_out<4, 2, 2, 4, 5>(a, out, nt, stream); break;   // 128 x 128
-    case 6: rc = launch_out<4, 2, 2, 2, 3>(a, out, nt, stream); break;   // 128 x 64, two to a compute unit
-    case 7: rc = launch_out<2, 2, 2, 2, 4>(a, out, nt, stream); break;   // 64 x 64, two to a compute unit
-    case 8: rc = launch_out<4, 2, 1, 4, 3>(a, out, nt, stream); break;   // 64 x 128, two to a compute unit
-    case 9: rc = launch_out<4, 4, 1, 4, 2>(a, out, nt, stream); break;   // 64 x 256, two to a compute unit
-    default: RLIS_REQUIRE(false, "gemm_tiles: no tile %d", tile);
-  }
-  if (rc) return rc;
-  RLIS_LAUNCH_CHECK("gemm_tiles");
-  return 0;
+                       (int)ldx, (int)ldw, ldy, slice_stride, {}};
+  return launch_form(a, out, tile, nt, stream);
+}
+
+// Q, and the cache's pages, from X (T,K) * W ((nh + 2 nkv) d,K)^T, W's rows the query, key and value heads: Q
+// (T, nh d) holds the query heads as they come, keys go to k_pages (pages, nkv, page_size, d) turned by
+// positions (rotate-half over the whole head, cos and sin (positions, d / 2); null: as they come), values to
+// v_pages (pages, nkv, d, page_size), at slots (below 0: not stored).  d 64, 128 or 256, page_size a power of two.
+// Products are rounded to bfloat16 before they are turned: the bits of rlis_gemm_bf16_tiles and rlis_rope_kv_write.
+RLIS_API int rlis_gemm_bf16_tiles_heads(const void* X, const void* W, void* Q, int T, int nh, int nkv, int d, int K,
+                                        long long ldx, long long ldw, long long ldq, const float* cos,
+                                        const float* sin, const int* positions, const int* slots, void* k_pages,
+                                        void* v_pages, int page_size, int tile, hipStream_t stream) {
+  RLIS_REQUIRE(T > 0 && nh > 0 && nkv > 0 && K > 0 && K % kBK == 0, "gemm_tiles_heads: bad sizes T=%d nh=%d nkv=%d K=%d",
+               T, nh, nkv, K);
+  RLIS_REQUIRE(d == 64 || d == 128 || d == 256, "gemm_tiles_heads: heads of %d, 64, 128 or 256 only", d);
+  RLIS_REQUIRE(page_size > 0 && (page_size & (page_size - 1)) == 0, "gemm_tiles_heads: page size %d must be a power of two",
+               page_size);
+  const long long rows = (nh + 2LL * nkv) * d;
+  RLIS_REQUIRE(ldx >= K && ldw >= K && ldq >= (long long)nh * d && ldx % 8 == 0 && ldw % 8 == 0 && ldq % 8 == 0 &&
+                   (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)Q % 16 == 0 &&
+                   (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0,
+               "gemm_tiles_heads: rows must lie on 16-byte boundaries");
+  RLIS_REQUIRE(positions && slots && k_pages && v_pages && !cos == !sin && (uintptr_t)cos % 16 == 0 &&
+                   (uintptr_t)sin % 16 == 0,
+               "gemm_tiles_heads: pages, slots, positions and both tables of angles are needed");
+  RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * rows < (1LL << 32), "gemm_tiles_heads: x or W passes 4 GB");
+  TilesArgs a = {(const bf16_t*)X, (const bf16_t*)W, Q, T, (int)(rows / 2), K / kBK, 0, 0, 1, 0,
+                 (int)ldx, (int)ldw, ldq, 0, {}};
+  a.heads = {cos, sin, positions, slots, (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, 0, 0};
+  while (2 << a.heads.half_shift < d) ++a.heads.half_shift;
+  while (1 << a.heads.page_shift < page_size) ++a.heads.page_shift;
+  return launch_form(a, kOutHeads, tile, 0, stream);
 }

@@ -1496,6 +1496,81 @@ def rope_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_di
                            **more)
 
 
+@functools.lru_cache(maxsize=4096)
+def _tiles_heads_plan(T: int, N: int, K: int, units: int) -> int:
+    return lib.load().rlis_gemm_bf16_tiles_heads_plan(T, N, K, units)
+
+
+def project_heads_plan(T: int, w: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int) -> int:
+    """The tile that ``project_rope_attention`` takes for ``T`` rows of x, or -1 where the product, the
+    kernel that turns and stores, and the attention are to run one by one: up to ``TILES_MIN_ROWS`` - 1 rows, where
+    decode kernels store by themselves; weights that are no bfloat16 rows of heads of 64, 128 or 256 over a k in
+    64s; and where the library is ahead (gemm_tiles.hip)."""
+    if not (T >= TILES_MIN_ROWS and BF16_GEMM == "library" and FUSE_ROPE_PREFILL and w.dtype == torch.bfloat16
+            and head_dim in (64, 128, 256) and w.dim() == 2
+            and w.shape[0] == (num_heads + 2 * num_kv_heads) * head_dim and w.shape[1] > 0 and w.shape[1] % 64 == 0
+            and w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.stride(0) >= w.shape[1]
+            and w.data_ptr() % 16 == 0 and 2 * w.shape[0] * w.stride(0) < 1 << 32):
+        return -1
+    return _tiles_heads_plan(T, w.shape[0], w.shape[1], _compute_units(w.device))
+
+
+def _project_heads(x: torch.Tensor, w: torch.Tensor, tile: int, num_heads: int, num_kv_heads: int, head_dim: int,
+                   cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], positions: torch.Tensor,
+                   slots: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, page_size: int) -> torch.Tensor:
+    """The query heads of ``x @ w.T``, unrotated, in rows ``(T, nh * d)``; its key heads, turned, and its value heads go
+    to the pages: what ``linear`` and ``rope_kv_write`` without ``rotate_q`` leave."""
+    T, K = x.shape
+    nh, nkv, d = num_heads, num_kv_heads, head_dim
+    for t, name, shape in ((k_pages, "k_pages", (nkv, page_size, d)), (v_pages, "v_pages", (nkv, d, page_size))):
+        _check(t, name, x.dtype, 4)
+        if tuple(t.shape[1:]) != shape or not t.is_contiguous():
+            raise KernelError(f"project_heads: {name} has shape {tuple(t.shape)}, expected "
+                              f"(pages, {shape[0]}, {shape[1]}, {shape[2]}) contiguous")
+    q = torch.empty((T, nh * d), dtype=x.dtype, device=x.device)
+    lib.call("rlis_gemm_bf16_tiles_heads", x.data_ptr(), w.data_ptr(), q.data_ptr(), T, nh, nkv, d, K, x.stride(0),
+             w.stride(0), nh * d, None if cos is None else cos.data_ptr(), None if sin is None else sin.data_ptr(),
+             _i32(positions, "positions", T), _i32(slots, "slots", T), k_pages.data_ptr(), v_pages.data_ptr(),
+             page_size, tile, lib.stream_ptr())
+    return q
+
+
+def project_rope_attention(x: torch.Tensor, w: torch.Tensor, tile: int, num_heads: int, num_kv_heads: int,
+                           head_dim: int, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor],
+                           positions: torch.Tensor, slots: Optional[torch.Tensor], k_pages: torch.Tensor,
+                           v_pages: torch.Tensor, page_size: int, block_tables: torch.Tensor, step, scale: float,
+                           window: Optional[int] = None, plan: Optional[StepPlan] = None,
+                           interleaved: bool = False, bias_slopes: Optional[torch.Tensor] = None,
+                           counters: Optional[torch.Tensor] = None, head_scales: Optional[torch.Tensor] = None,
+                           softcap: float = 0.0, sinks: Optional[torch.Tensor] = None, keep_first: int = 0,
+                           chunk: Optional[int] = None) -> Optional[torch.Tensor]:
+    """``rope_attention`` of ``linear(x, w)`` with the cache written by the product itself (``tile``:
+    ``project_heads_plan``), for steps with portions of prompts that take the matrix-core kernels and that turn
+    nothing, or whole heads in halves.  None: those two have to run, and nothing has happened."""
+    nh, nkv, d = num_heads, num_kv_heads, head_dim
+    shaped = head_scales is not None or softcap > 0
+    if not (tile >= 0 and x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == w.shape[1] and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and x.stride(0) >= x.shape[1] and x.data_ptr() % 16 == 0
+            and 2 * x.shape[0] * x.stride(0) < 1 << 32 and slots is not None):
+        return None
+    rows = x.new_empty((0, nh * d))               # (as the query rows will lie)
+    kind, _ = _attention_kernel(rows, nh, nkv, d, page_size, step, None, bias_slopes is not None, shaped,
+                                PLAIN_EXTRAS and (sinks is not None or bool(keep_first and window)))
+    if kind != "prefill" or not (_decode_mfma_ok(rows, nh, nkv, d, page_size)
+                                 or (plan is not None and not plan.value("num_decode"))):
+        return None
+    if cos is not None and not (not interleaved and sin is not None and cos.dtype == sin.dtype == torch.float32
+                                and cos.dim() == 2 and cos.shape == sin.shape and 2 * cos.shape[1] == d
+                                and cos.is_contiguous() and sin.is_contiguous()
+                                and cos.data_ptr() % 16 == 0 and sin.data_ptr() % 16 == 0):
+        return None
+    q = _project_heads(x, w, tile, nh, nkv, d, cos, sin, positions, slots, k_pages, v_pages, page_size)
+    return paged_attention(q, nh, nkv, d, k_pages, v_pages, page_size, block_tables, step, scale, window, plan=plan,
+                           bias_slopes=bias_slopes, counters=counters, head_scales=head_scales, softcap=softcap,
+                           sinks=sinks, keep_first=keep_first, chunk=chunk,
+                           rope=None if cos is None else (cos, sin, positions, None))
+
+
 def norm_rope_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
                         real_dim: int, eps: float, cos: Optional[torch.Tensor],
                         sin: Optional[torch.Tensor], positions: torch.Tensor,

@@ -69,6 +69,7 @@ _SIGNATURES = {
     "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, I, P],
     "rlis_gemm_bf16_rows": [P, P, P, I, I, I, I, I, L, L, L, L, P, I, I, F, I, P],
     "rlis_gemm_bf16_tiles": [P, P, P, I, I, I, I, I, L, L, L, L, I, I, P],
+    "rlis_gemm_bf16_tiles_heads": [P, P, P, I, I, I, I, I, L, L, L, P, P, P, P, P, P, I, I, P],
     "rlis_gemm_bf16_mfma": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny": [P, P, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_bf16_skinny_swiglu": [P, P, P, I, I, I, L, L, L, P],
@@ -125,6 +126,8 @@ def load() -> ctypes.CDLL:
     lib.rlis_gemm_bf16_rows_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_tiles_plan.restype = c_int
     lib.rlis_gemm_bf16_tiles_plan.argtypes = [I, I, I, I, I, I, I]
+    lib.rlis_gemm_bf16_tiles_heads_plan.restype = c_int
+    lib.rlis_gemm_bf16_tiles_heads_plan.argtypes = [I, I, I, I]
     lib.rlis_gemm_bf16_splitk_slices.restype = c_int
     lib.rlis_gemm_bf16_splitk_slices.argtypes = [I, I]
     lib.rlis_gemm_bf16_stream_join_tiles.restype = c_int

@@ -290,6 +290,11 @@ class PagedAttention(Mixer):
             # (one number, read once while the model is built)
             self.mix_weight = float(ctx.take(join(prefix, mix["name"])).to(torch.float32).item())
 
+        # queries, keys and values are what the one product gives: nothing stands between it and the rotation
+        self.plain_heads = not (self.taps or self.bias is not None or self.q_norm is not None or self.temp_every
+                                or self.gated or self.prepared or self.turned_norm or self.shared_kv
+                                or self.mix_key is not None)
+
         self.planner = ops.attention_planner(
             self.num_heads, self.num_kv_heads, self.head_dim, self.act_dtype,
             biased=getattr(self.position, "bias_slopes", None) is not None,
@@ -373,6 +378,14 @@ class PagedAttention(Mixer):
                              f"{self.position.max_positions}")
         if self.prepared:
             return self._forward_prepared(x, step, binding, group)
+        if self.plain_heads and binding.writes and not step.all_decode:
+            tile = ops.project_heads_plan(step.num_tokens, self.w_qkv, self.num_heads, self.num_kv_heads,
+                                          self.head_dim)
+            if tile >= 0:
+                x = x.tensor() if isinstance(x, NormedInput) else x
+                out = self._project_and_attend(x, tile, step, binding, group)
+                if out is not None:
+                    return ops.pending_linear(out, self.w_o, self.act_dtype)
         rows = self._project(x, step, binding)
         qkv = rows[:, :self.qkv_cols] if self.gated else rows
         if self.turned_norm:
@@ -402,17 +415,28 @@ class PagedAttention(Mixer):
 
     def _attend(self, qkv: torch.Tensor, step: Any, binding: CacheBinding, group: Any
                 ) -> torch.Tensor:
-        return ops.rope_attention(qkv, self.num_heads, self.num_kv_heads, self.head_dim,
-                                  self.position.cos, self.position.sin, step.positions,
-                                  group.slots, binding.k_pages, binding.v_pages, group.page_size,
-                                  group.block_tables, step, self.scale, self.window,
+        return ops.rope_attention(qkv, *self._attention_args(step, binding, group),
                                   write_kv=binding.writes and not self.shared_kv,
-                                  plan=step.plans.get(self.planner.key()),
-                                  interleaved=bool(getattr(self.position, "interleaved", False)),
-                                  bias_slopes=getattr(self.position, "bias_slopes", None),
-                                  counters=binding.counters, head_scales=self.head_scales,
-                                  softcap=self.softcap, sinks=self.sinks,
-                                  keep_first=self.keep_first, chunk=self.chunk)
+                                  **self._attention_options(step, binding))
+
+    def _project_and_attend(self, x: torch.Tensor, tile: int, step: Any, binding: CacheBinding, group: Any
+                            ) -> Optional[torch.Tensor]:
+        """Queries, keys and values from one product that writes the cache itself; None: not of this step."""
+        return ops.project_rope_attention(x, self.w_qkv, tile, *self._attention_args(step, binding, group),
+                                          **self._attention_options(step, binding))
+
+    def _attention_args(self, step: Any, binding: CacheBinding, group: Any) -> tuple:
+        return (self.num_heads, self.num_kv_heads, self.head_dim, self.position.cos, self.position.sin,
+                step.positions, group.slots, binding.k_pages, binding.v_pages, group.page_size,
+                group.block_tables, step, self.scale, self.window)
+
+    def _attention_options(self, step: Any, binding: CacheBinding) -> Dict[str, Any]:
+        return dict(plan=step.plans.get(self.planner.key()),
+                    interleaved=bool(getattr(self.position, "interleaved", False)),
+                    bias_slopes=getattr(self.position, "bias_slopes", None),
+                    counters=binding.counters, head_scales=self.head_scales,
+                    softcap=self.softcap, sinks=self.sinks,
+                    keep_first=self.keep_first, chunk=self.chunk)
 
     def _forward_prepared(self, x: Any, step: Any, binding: CacheBinding, group: Any) -> Any:
         """Layers whose keys serve as values behind norms over whole rows: one kernel adds the

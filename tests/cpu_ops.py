@@ -633,6 +633,10 @@ def rope_attention(qkv, num_heads, num_kv_heads, head_dim, cos, sin, positions, 
                            softcap=softcap, sinks=sinks, keep_first=keep_first, chunk=chunk)
 
 
+def project_heads_plan(T, w, num_heads, num_kv_heads, head_dim):
+    return -1                         # (product, rotation and attention one by one)
+
+
 def _lowbias32(x):
     x ^= x >> 16
     x = (x * 0x7FEB352D) & 0xFFFFFFFF
@@ -667,7 +671,7 @@ def install(monkeypatch) -> None:
     for name in ("embed", "add_residual", "add_rmsnorm", "swiglu", "linear", "linear_swiglu",
                  "pending_linear", "can_fuse_norm_linear", "rope_kv_write", "norm_rope_kv_write",
                  "norm_rope_attention",
-                 "rope_attention",
+                 "rope_attention", "project_heads_plan",
                  "copy_pages", "attention_planner", "paged_attention", "sample_rows",
                  "clamped_glu", "weighted_sum", "linear_f32", "soft_cap_", "shift_mix", "tail_update",
                  "causal_conv", "delta_scan", "decay_scan", "head_norm_gate", "selective_scan",

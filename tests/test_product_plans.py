@@ -50,3 +50,16 @@ def test_rounds_are_those_of_the_device(plan):
     assert plan(128, 2048, 2048, 0, 0, 1, units=64) >= 0
     assert plan(96, 6144, 512, 0, 0, 1, units=64) % 16 != plan(96, 6144, 512, 0, 0, 1) % 16
     assert plan(96, 2048, 2048, 0, 0, 1, units=0) == -1
+
+
+@pytest.mark.parametrize("T,N,K,taken", [
+    (65, 3072, 2048, True), (381, 3072, 2048, True), (512, 3072, 2048, True), (2048, 3072, 2048, True), (8192, 5120, 3072, True),
+    (256, 5120, 3072, True), (256, 6144, 4096, True), (1024, 6144, 4096, True), (4096, 1536, 1024, True),
+    (2048, 5120, 3072, False), (2048, 6144, 4096, False), (1300, 6144, 4096, False), (2048, 10240, 8192, False),
+    (768, 12288, 4096, False), (65, 0, 64, False)])
+def test_products_that_write_the_cache(T, N, K, taken):
+    """q, k and v: against the library's product and the kernel that turns and stores."""
+    fn = ctypes.CDLL(build.ensure("kernels")).rlis_gemm_bf16_tiles_heads_plan
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] * 4
+    assert (fn(T, N, K, 256) >= 0) == taken
+    assert not taken or fn(T, N, K, 256) in (0, 1, 3, 4, 5, 6, 7, 10, 11, 12)
