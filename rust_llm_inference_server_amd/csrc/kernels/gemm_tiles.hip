@@ -48,6 +48,8 @@
 //       gate/up 23.5 -> 20.0, 31.3 -> 27.1, 42.2 -> 36.6  down 16.3 -> 16.0, 24.8 -> 23.2, 33.0 -> 31.6
 //   3B  q/k/v -, at 112 rows 19.1 -> 17.4                 output 17.9 -> 14.3, 21.7 -> 22.5, 27.4 -> 27.6
 //       gate/up 30.4 -> 29.5, 41.8 -> 40.1, 60.7 -> 51.4  down 22.6 -> 22.0, -, -
+//   (gate/up 1,024 / 2,048 / 8,192 rows in 256 x 256: 1B 67.8 -> 61.4, 120.8 -> 115.7, 453 -> 434; 3B 91.8 -> 84.1, 169.3 ->
+//   160.7, 635 -> 607; down of 2,048 rows of the 1B shape 76.6 -> 75.2)
 //   8B  q/k/v 20.6 -> 21.3, at 112 rows 25.9 -> 22.2      output 20.8 -> 16.6, 26.1 -> 26.9, 36.7 -> 32.9
 //       gate/up 62.2 -> 55.4, 77.1 -> 70.2, -             down 36.0 -> 35.2, 47.6 -> 46.7, 71.4 -> 69.3
 // In a step, where a row count between those tried out takes another's algorithm, the library is further behind
@@ -487,9 +489,11 @@ struct TileForm {
 };
 constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 0.66f}, {192, 128, 0.60f},
                                {160, 128, 0.55f}, {128, 128, 0.48f}, {128, 64, 0.35f}, {64, 64, 0.215f},
-                               {64, 128, 0.33f}, {64, 256, 0.46f}};
+                               {64, 128, 0.33f}, {64, 256, 0.46f}, {256, 256, 1.38f}};
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
 constexpr int kWideForms = 8;              // those that products of more than 64 rows choose from
+constexpr int kLargest = 10;               // and gate/up beyond 512 rows
+constexpr float kPartialStage = 0.71f;     // of tiles of 128 x 256 that store partial sums: ahead of 256 x 128 there
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
 
 // The same for q, k and v on their way to the cache: a stage's time with two workgroups to a compute unit and
@@ -534,19 +538,22 @@ constexpr int kHeadsFormCount = sizeof(kHeadsForms) / sizeof(kHeadsForms[0]);
 //            k of 16,384 and more (0.64 to 1.02; else up to 1.25).
 //   gated    k up to 1,024, and to 2,048 from 1,024 weight rows on: up to 256 rows, to 512 where the rounds come out
 //            even or there is one (0.36 to 1.03).  Longer k from 5,632 weight rows on: up to 192 rows, beyond where
-//            rounds come out nearly even (0.66 to 1.1; fewer weight rows up to 2.0).
+//            rounds come out nearly even (0.66 to 1.1; fewer weight rows up to 2.0).  From 1,024 rows on (over a k of
+//            1,024 beyond 512) where rounds come out even, k of 1,024 to 3,072 from 8,192 weight rows on (0.78 to 1.0, most in
+//            tiles of 256 x 256; uneven rounds up to 1.12, 640 and 768 rows 1.05 to 1.14; over a k of 4,096 and 8,192 0.97 to
+//            1.06).
 RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices, int units) {
   if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
   float least = 0.f;
   int best = -1, best_rounds = 0, best_tiles = 0;
   for (int s = slices > 0 ? slices : 1; s <= (slices > 0 ? slices : partials ? 4 : 1); s *= 2) {
     if (K % (s * kBK) || (slices <= 0 && s > 1 && K / s < 512)) continue;
-    for (int f = 0; f < (T <= 64 ? kFormCount : kWideForms); ++f) {
-      if (T <= 64 && kForms[f].rows > 64) continue;
+    for (int f = 0; f < kFormCount; ++f) {
+      if (T <= 64 ? kForms[f].rows > 64 : f >= kWideForms && !(f == kLargest && gated && T > 512)) continue;
       const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
       const long long rounds = (tiles + units - 1) / units;
       if (rounds > 1 << 20) continue;
-      const float us = (float)rounds * (K / s / kBK) * kForms[f].stage +
+      const float us = (float)rounds * (K / s / kBK) * (f == 0 && partials ? kPartialStage : kForms[f].stage) +
                        (s > 1 ? kPartial * s : kPartial / 2) * (float)T * N;
       if (best < 0 || us < least) least = us, best = f + 16 * s, best_rounds = (int)rounds, best_tiles = (int)tiles;
     }
@@ -565,6 +572,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     } else {
       here = T <= 192 || (T <= 2048 && one && even && (T <= 512 || N >= 1024));
     }
+  } else if (gated && T > 512) {
+    here = even && K >= 1024 && K <= 3072 && N >= 8192 && (T >= 1024 || K == 1024);
   } else if (gated) {
     if (K > 2048)
       here = N >= 5632 && (T <= 192 || (T <= 256 && best_tiles * 20LL >= best_rounds * (units * 17LL)) || (T <= 512 && even));
@@ -588,7 +597,9 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
 // pass through memory.  Fitted to 65 to 8,192 rows of ten shapes, 1,536 to 12,288 weight rows over a k of 512 to
 // 8,192, weights cold (tiles to 10 %; the library, whose algorithms are a clock's choice, to 15 %).  Of 136 products
 // the rule takes 120, 0.55 to 1.02 of the library's time; beyond 8,192 weight rows the tiles have to be ahead by a
-// fifteenth (12,288 x 4,096 at 768 and 1,024 rows would be taken at 1.05 to 1.1).  Figures are those of 256 units.
+// fifteenth (12,288 x 4,096 at 768 and 1,024 rows would be taken at 1.05 to 1.1), and by a seventh from 4,096 rows on
+// over a k of 4,096 and more, where the library reaches 1.5 PFLOP/s (8,192 rows of the 8B shape in a step 312 us against its
+// 295).  Figures are those of 256 units.
 RLIS_API int rlis_gemm_bf16_tiles_heads_plan(int T, int N, int K, int units) {
   if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
   float least = 0.f;
@@ -603,7 +614,7 @@ RLIS_API int rlis_gemm_bf16_tiles_heads_plan(int T, int N, int K, int units) {
   const float share = 256.f / units;
   const float here = least + 4.9f + (0.095e-6f * K + 0.6e-6f * T) * N;
   const float library = 12.f + 0.454e-6f * N * K + (1.19e-9f * T * K + 1.05e-6f * T) * N * share;
-  return here < library * (N > 32 * units ? 0.93f : 1.f) ? best : -1;
+  return here < library * (T >= 4096 && K >= 4096 ? 0.85f : N > 32 * units ? 0.93f : 1.f) ? best : -1;
 }
 
 // Y (T,N) = X (T,K) * W (N,K)^T, N a multiple of 8, K of 64 times the slices.  out 0: bfloat16; 1:

@@ -293,7 +293,7 @@ class PagedAttention(Mixer):
         # queries, keys and values are what the one product gives: nothing stands between it and the rotation
         self.plain_heads = not (self.taps or self.bias is not None or self.q_norm is not None or self.temp_every
                                 or self.gated or self.prepared or self.turned_norm or self.shared_kv
-                                or self.mix_key is not None)
+                                or self.mix_key is not None or self.w_qkv.dtype != torch.bfloat16)
 
         self.planner = ops.attention_planner(
             self.num_heads, self.num_kv_heads, self.head_dim, self.act_dtype,

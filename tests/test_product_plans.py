@@ -43,6 +43,14 @@ def test_partial_sums_and_gate_up(plan, T, N, K, gated, slices, taken):
     assert (plan(T, N, K, gated, 1 - gated, slices) >= 0) == taken
 
 
+@pytest.mark.parametrize("T,N,K,taken", [
+    (1024, 16384, 2048, 10), (2048, 16384, 2048, 10), (8192, 16384, 3072, 10), (1536, 16384, 2048, 1), (2048, 8192, 1024, 10),
+    (640, 16384, 2048, None), (768, 16384, 3072, None), (2048, 28672, 4096, None), (2048, 4096, 2048, None), (4096, 16384, 512, None)])
+def test_gate_up_of_prompts(plan, T, N, K, taken):
+    """gate/up of more than 512 rows: even rounds alone, most in the largest tile."""
+    assert plan(T, N, K, 1, 0, 1) == (-1 if taken is None else 16 + taken)
+
+
 def test_rounds_are_those_of_the_device(plan):
     """A partition of a quarter of the compute units has four times the rounds: what fills the chip in one round there
     is a quarter of the tiles, and larger tiles pay earlier."""
@@ -55,7 +63,7 @@ def test_rounds_are_those_of_the_device(plan):
 @pytest.mark.parametrize("T,N,K,taken", [
     (65, 3072, 2048, True), (381, 3072, 2048, True), (512, 3072, 2048, True), (2048, 3072, 2048, True), (8192, 5120, 3072, True),
     (256, 5120, 3072, True), (256, 6144, 4096, True), (1024, 6144, 4096, True), (4096, 1536, 1024, True),
-    (2048, 5120, 3072, False), (2048, 6144, 4096, False), (1300, 6144, 4096, False), (2048, 10240, 8192, False),
+    (2048, 5120, 3072, False), (2048, 6144, 4096, False), (8192, 6144, 4096, False), (1300, 6144, 4096, False), (2048, 10240, 8192, False),
     (768, 12288, 4096, False), (65, 0, 64, False)])
 def test_products_that_write_the_cache(T, N, K, taken):
     """q, k and v: against the library's product and the kernel that turns and stores."""
