@@ -14,6 +14,10 @@
 // non-temporally where the model is larger than the memory-side cache (64 rows, gate/up with the
 // SwiGLU, 1B: 20.1 -> 19.0 us; 32 rows, 8B: 52 -> 46).
 // The order of a sum follows from N and K alone: a row's bits do not depend on the rows beside it.
+// What ends a slice: with the join, the last of a tile's slices to store its sum (past the die's cache, then an
+// atomic count) adds all of them to the residual; the sums of squares that scale the rows of the product behind
+// are asked for in front of its first stages, not behind them (the wait for them is in order: q/k/v of 27 rows of
+// the 3B shape 11.6 -> 10.8 us, gate/up 21.8 -> 21.3).
 // Weights loaded straight into registers instead (16 rows x 64 bytes an instruction, more bytes
 // under way): 10 to 20 % slower.
 //
@@ -41,6 +45,16 @@ __device__ __forceinline__ void wait_loads() {
 }
 __device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// What the last of a tile's slices to finish does with their sum (JOINS).
+struct RowsJoin {
+  float* resid;           // (T,N): the sum is added to it
+  const void* weight;     // (N) the next norm's, bfloat16 or float32
+  bf16_t* xw;             // (T,N): resid times the weight
+  float* ss;              // (T, ss_stride): a tile's sums of resid squared
+  unsigned* arrivals;     // one a tile, zero before and after
+  int ss_stride, weight_f32, round_sum;
+};
+
 struct RowsArgs {
   const bf16_t* X;
   const bf16_t* W;
@@ -51,10 +65,75 @@ struct RowsArgs {
   const float* ss;        // scaled: (T, ss_stride) partial sums of squares, ss_count a row
   int ss_count, ss_stride;
   float eps;
+  RowsJoin join;
 };
 
+// Sums that workgroups of one launch hand to each other, 16 bytes at a time, past the caches that only one die
+// sees (device scope: what an atomic of that scope does, see attention_mfma.hip).
+constexpr int kDeviceScope = 16;           // (sc1)
+
+// The sum of a tile's slices joins the residual, and the rows that the next product reads are made of it.
+// Slices are added in order and, with round_sum, rounded once to bfloat16: the floats of the norm kernel that
+// adds a stack of partial sums (elementwise.hip).
+template <int NI>
+__device__ __forceinline__ void join_tile(const RowsArgs& p, const RowsJoin& j, int slices, int tile) {
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int LANES = 4 * NI;            // lanes a row, four columns each
+  const auto parts = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, 0xffffffff, 0x00027000);
+  const int c = threadIdx.x % LANES * 4, n = tile * 16 * NI + c;
+  const bool inside = n < p.N;
+  f32x4 weight{0.f, 0.f, 0.f, 0.f};
+  if (inside) {
+    if (j.weight_f32) {
+      weight = *(const f32x4*)((const float*)j.weight + n);
+    } else {
+      const uint2 u = *(const uint2*)((const bf16_t*)j.weight + n);
+      weight = f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                     __uint_as_float(u.y & 0xffff0000u)};
+    }
+  }
+  constexpr int kRows = kWaves * 64 / LANES;     // rows at a time
+  for (int t0 = 0; t0 < p.T; t0 += kRows) {
+    const int token = t0 + threadIdx.x / LANES;
+    const bool live = inside && token < p.T;
+    const long long at = live ? (long long)token * p.ldy + n : 0;
+    f32x4 part[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long long from = at + (q < slices ? q : 0) * p.slice_stride;
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(parts, (int)(from * 4), 0, kDeviceScope);
+      part[q] = __builtin_bit_cast(f32x4, v);
+    }
+    f32x4 r = *(const f32x4*)(j.resid + (live ? (long long)token * p.N + n : 0));
+    float squares = 0.f;
+    uint32_t o[2];
+    float scaled[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float sum = part[0][e];
+#pragma unroll
+      for (int q = 1; q < 4; ++q) sum = q < slices ? sum + part[q][e] : sum;
+      if (j.round_sum) sum = bf16_to_f32(f32_to_bf16(sum));
+      r[e] += sum;
+      squares += r[e] * r[e];
+      scaled[e] = r[e] * weight[e];
+    }
+    o[0] = f32_to_bf16(scaled[0]) | (uint32_t)f32_to_bf16(scaled[1]) << 16;
+    o[1] = f32_to_bf16(scaled[2]) | (uint32_t)f32_to_bf16(scaled[3]) << 16;
+    if (!live) squares = 0.f;
+#pragma unroll
+    for (int d = 1; d < LANES; d *= 2) squares += __shfl_xor(squares, d, 64);
+    if (live) {
+      *(f32x4*)(j.resid + (long long)token * p.N + n) = r;
+      *(uint2*)(j.xw + (long long)token * p.N + n) = make_uint2(o[0], o[1]);
+      if (c == 0) j.ss[(long long)token * j.ss_stride + tile] = squares;
+    }
+  }
+#endif
+}
+
 // MI groups of 16 rows of x, NI groups of 16 weight rows, BUFS stages in LDS.
-template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, typename TY>
+template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, bool JOINS, typename TY>
 __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
   constexpr int ROWS = 16 * (MI + NI), STAGE = ROWS * kBK * 2;
@@ -114,27 +193,38 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
       weight_rows(a_tile);
     }
   };
+  // The rows' sums of squares, a quarter of a row's partial sums per lane: the first 64 are asked for in front of the
+  // stages, behind which they would be waited for.
+  constexpr int kFirst = 4;
+  f32x4 first_sums[SCALED ? kFirst : 1];
+  const int ss_token = threadIdx.x / 4, ss_q = threadIdx.x % 4;
+  const float* ss_row = SCALED ? p.ss + (long long)min(ss_token, p.T - 1) * p.ss_stride : nullptr;
+  if (SCALED) {
+#pragma unroll
+    for (int k = 0; k < kFirst; ++k) first_sums[k] = *(const f32x4*)(ss_row + min(ss_q * 4 + 16 * k, (p.ss_count - 1) & ~3));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   weight_rows(a_tile);
 #pragma unroll
   for (int s = 0; s < BUFS - 1; ++s) ask();
 
   if (SCALED) {
-    // the rows' sums of squares, a quarter of a row's partial sums per lane
-    const int token = threadIdx.x / 4, q = threadIdx.x % 4;
     float s = 0.f;
-    if (token < 16 * MI) {
-      const float* row = p.ss + (long long)min(token, p.T - 1) * p.ss_stride;
-      for (int i = q * 4; i < p.ss_count; i += 16) {
-        const f32x4 v = *(const f32x4*)(row + i);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s += i + e < p.ss_count ? v[e] : 0.f;
-      }
+    for (int k = 0; k < kFirst; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += ss_q * 4 + 16 * k + e < p.ss_count ? first_sums[k][e] : 0.f;
+    for (int i = ss_q * 4 + 16 * kFirst; i < p.ss_count; i += 16) {
+      const f32x4 v = *(const f32x4*)(ss_row + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += i + e < p.ss_count ? v[e] : 0.f;
     }
     s += __shfl_xor(s, 1, 64);
     s += __shfl_xor(s, 2, 64);
-    if (token < 16 * MI && q == 0)
-      ((float*)red)[token] = rsqrtf(s / (float)(p.steps * kBK) + p.eps);
-    __syncthreads();
+    if (ss_token < 16 * MI && ss_q == 0)
+      ((float*)red)[ss_token] = rsqrtf(s / (float)(p.steps * kBK) + p.eps);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();                             // (the stages stay under way)
   }
   // (a wave stores the rows of one group of x: blocks are dealt out in fours, MI is 2 or 4)
   static_assert(MI == 2 || MI == 4, "");
@@ -202,7 +292,12 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
         }
         const int n = tile * 16 * NI + a * 16 + 4 * g;
         if (!live || n >= p.N) continue;
-        if (sizeof(TY) == 4) {
+        if (JOINS) {
+          const auto parts = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, 0xffffffff, 0x00027000);
+          const long long to = blockIdx.y * p.slice_stride + (long long)token * p.ldy + n;
+          typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), parts, (int)(to * 4), 0, kDeviceScope);
+        } else if (sizeof(TY) == 4) {
           *(f32x4*)((float*)p.Y + blockIdx.y * p.slice_stride + (long long)token * p.ldy + n) = v;
         } else {
           uint2 o;
@@ -212,17 +307,31 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
         }
       }
     }
+    if (JOINS) {
+      // The last of the tile's slices to get here joins them: everybody's stores have arrived before it is counted in.
+      int& last = *(int*)red;              // (behind the barrier nobody reads sums)
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        unsigned* slot = p.join.arrivals + tile;
+        const bool end = __hip_atomic_fetch_add(slot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.y - 1;
+        last = end;
+        if (end) __hip_atomic_store(slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      if (last) join_tile<NI>(p, p.join, gridDim.y, tile);
+    }
   }
   wait_loads<0>();                         // (loads past the last tile still write LDS)
 #endif
 }
 
-template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, typename TY>
+template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, bool JOINS, typename TY>
 int launch_form(const RowsArgs& a, int slices, hipStream_t stream) {
   static LdsGrant grant;
   constexpr int bytes = BUFS * 16 * (MI + NI) * kBK * 2 + kWaves * (NI * MI < 8 ? NI * MI : 8) * 1024;
   static_assert(bytes <= 160 * 1024, "");
-  const auto kernel = gemm_rows_kernel<MI, NI, BUFS, SCALED, GATED, NT, TY>;
+  const auto kernel = gemm_rows_kernel<MI, NI, BUFS, SCALED, GATED, NT, JOINS, TY>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_rows: %s", hipGetErrorString(e));
   RowsArgs b = a;
@@ -233,10 +342,10 @@ int launch_form(const RowsArgs& a, int slices, hipStream_t stream) {
   return 0;
 }
 
-template <int MI, int NI, int BUFS, bool SCALED, bool GATED, typename TY>
+template <int MI, int NI, int BUFS, bool SCALED, bool GATED, typename TY, bool JOINS = false>
 int launch(const RowsArgs& a, int slices, int nt, hipStream_t stream) {
-  return nt ? launch_form<MI, NI, BUFS, SCALED, GATED, true, TY>(a, slices, stream)
-            : launch_form<MI, NI, BUFS, SCALED, GATED, false, TY>(a, slices, stream);
+  return nt ? launch_form<MI, NI, BUFS, SCALED, GATED, true, JOINS, TY>(a, slices, stream)
+            : launch_form<MI, NI, BUFS, SCALED, GATED, false, JOINS, TY>(a, slices, stream);
 }
 
 // out: 0 bfloat16, 1 float32 (slices of k, slice_stride apart), 2 gated
@@ -247,6 +356,7 @@ int form(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
     if (out == 1) return launch<MI, NI, BUFS, true, false, float>(a, slices, nt, stream);
     return launch<MI, NI, BUFS, true, true, bf16_t>(a, slices, nt, stream);
   }
+  if (a.join.resid) return launch<MI, NI, BUFS, false, false, float, true>(a, slices, nt, stream);
   if (out == 0) return launch<MI, NI, BUFS, false, false, bf16_t>(a, slices, nt, stream);
   if (out == 1) return launch<MI, NI, BUFS, false, false, float>(a, slices, nt, stream);
   return launch<MI, NI, BUFS, false, true, bf16_t>(a, slices, nt, stream);
@@ -269,6 +379,21 @@ int slices_of(int N, int K) {
   int s = 4;
   while (s > 1 && (steps % s || steps / s < 4 || ceil_div(N, 64) * s > kUnits)) s /= 2;
   return s;
+}
+
+int dispatch(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
+  const int ni = row_groups(out == 2 ? 2 * a.N : a.N, slices);
+  int rc;
+  if (a.T <= 32) {
+    rc = ni == 1 ? form<2, 1, 8>(a, out, slices, nt, stream) : ni == 2 ? form<2, 2, 8>(a, out, slices, nt, stream)
+                                                                   : form<2, 4, 5>(a, out, slices, nt, stream);
+  } else {
+    rc = ni == 1 ? form<4, 1, 6>(a, out, slices, nt, stream) : ni == 2 ? form<4, 2, 5>(a, out, slices, nt, stream)
+                                                                   : form<4, 4, 4>(a, out, slices, nt, stream);
+  }
+  if (rc) return rc;
+  RLIS_LAUNCH_CHECK("gemm_rows");
+  return 0;
 }
 
 }  // namespace
@@ -297,17 +422,41 @@ RLIS_API int rlis_gemm_bf16_rows(const void* X, const void* W, void* Y, int out,
   RLIS_REQUIRE(!ss || (ss_count > 0 && ss_stride >= ss_count && ss_stride % 4 == 0 && (uintptr_t)ss % 16 == 0),
                "gemm_rows: the sums of squares must be rows on 16-byte boundaries");
   const RowsArgs a = {(const bf16_t*)X, (const bf16_t*)W, Y, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw,
-                      ldy, slice_stride, ss, ss_count, ss_stride, eps};
-  const int ni = row_groups(out == 2 ? 2 * N : N, slices);
-  int rc;
-  if (T <= 32) {
-    rc = ni == 1 ? form<2, 1, 8>(a, out, slices, nt, stream) : ni == 2 ? form<2, 2, 8>(a, out, slices, nt, stream)
-                                                                   : form<2, 4, 5>(a, out, slices, nt, stream);
-  } else {
-    rc = ni == 1 ? form<4, 1, 6>(a, out, slices, nt, stream) : ni == 2 ? form<4, 2, 5>(a, out, slices, nt, stream)
-                                                                   : form<4, 4, 4>(a, out, slices, nt, stream);
-  }
-  if (rc) return rc;
-  RLIS_LAUNCH_CHECK("gemm_rows");
-  return 0;
+                      ldy, slice_stride, ss, ss_count, ss_stride, eps, {}};
+  return dispatch(a, out, slices, nt, stream);
+}
+
+// Tiles of weight rows of a product with `slices` partial sums: sums of squares a row, and arrival counters.
+RLIS_API int rlis_gemm_bf16_rows_join_tiles(int N, int slices) {
+  return N > 0 && slices > 0 ? ceil_div(N, 16 * row_groups(N, slices)) : 0;
+}
+
+// resid (T,N) += X (T,K) * W (N,K)^T for 17 to 64 rows over two or four slices of k, the sum of the slices rounded to
+// bfloat16 first with round_sum; xw (T,N) = resid * weight in bfloat16, ss (T, ss_stride) the sums of resid squared over
+// each of rlis_gemm_bf16_rows_join_tiles(N, slices) tiles of columns.  parts: (slices,T,N) float32 of scratch.  arrivals:
+// a counter a tile, all zero before the launch and again after it; launches that overlap in time must not share
+// them.  In place of the partial sums and the norm that adds them: down of the 3B shape at 27 rows in a step 11.6 + 4.8 ->
+// 15.6 us, and the q/k/v product behind it, scaled here, 12.6 -> 10.8.  At 64 rows of the 1B shape output and down got 3.5
+// us slower for a norm of 5.0 less, the scaled gate/up and q/k/v took 1.2 us more, and the step as a whole 1 %
+// more.
+RLIS_API int rlis_gemm_bf16_rows_join(const void* X, const void* W, float* parts, int T, int N, int K, int slices,
+                                      long long ldx, long long ldw, float* resid, const void* weight, int weight_dtype,
+                                      int round_sum, void* xw, float* ss, int ss_stride, unsigned* arrivals, int arrival_slots,
+                                      int nt, hipStream_t stream) {
+  RLIS_REQUIRE(T > 0 && T <= 64 && N > 0 && N % 8 == 0 && (slices == 2 || slices == 4) && K > 0 && K % (slices * kBK) == 0,
+               "gemm_rows_join: bad sizes T=%d N=%d K=%d slices=%d", T, N, K, slices);
+  const int tiles = rlis_gemm_bf16_rows_join_tiles(N, slices);
+  RLIS_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 &&
+                   (uintptr_t)parts % 16 == 0 && (uintptr_t)resid % 16 == 0 && (uintptr_t)xw % 16 == 0 &&
+                   (uintptr_t)weight % 16 == 0,
+               "gemm_rows_join: rows must lie on 16-byte boundaries");
+  RLIS_REQUIRE(parts && resid && weight && xw && ss && ss_stride >= tiles && arrivals && arrival_slots >= tiles,
+               "gemm_rows_join: an operand is missing or too short for %d tiles", tiles);
+  RLIS_REQUIRE(weight_dtype == RLIS_F32 || weight_dtype == RLIS_BF16, "gemm_rows_join: unknown weight dtype %d", weight_dtype);
+  RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * N < (1LL << 32) && 4LL * slices * T * N < (1LL << 31),
+               "gemm_rows_join: x or W passes 4 GB, or the partial sums 2 GB");
+  RowsArgs a = {(const bf16_t*)X, (const bf16_t*)W, parts, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw,
+                N, (long long)T * N, nullptr, 0, 0, 0.f, {}};
+  a.join = {resid, weight, (bf16_t*)xw, ss, arrivals, ss_stride, weight_dtype == RLIS_F32, round_sum};
+  return dispatch(a, 1, slices, nt, stream);
 }

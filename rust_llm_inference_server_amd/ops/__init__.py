@@ -108,6 +108,7 @@ def _counters_for(device: torch.device) -> torch.Tensor:
 class _Streamed(threading.local):
     nt = 0                # weights of the model under way are loaded non-temporally
     cache_layers = 0      # its layers that keep keys and values
+    counters = None       # int32 zeros of its runner's, for kernels whose workgroups count themselves in
 
 
 _streamed = _Streamed()
@@ -119,16 +120,19 @@ MEMORY_SIDE_CACHE_BYTES = 256 << 20
 
 
 @contextlib.contextmanager
-def weights_of(nbytes: int, cache_layers: int = 0):
+def weights_of(nbytes: int, cache_layers: int = 0, counters: Optional[torch.Tensor] = None):
     """Inside the block, what this thread launches is a model's that holds ``nbytes`` of weights and
     reads all of them in a step, and that keeps keys and values in ``cache_layers`` layers.  (It moves no
-    bit of a result; a captured step keeps what held at its capture.)"""
-    old = _streamed.nt, _streamed.cache_layers
-    _streamed.nt, _streamed.cache_layers = int(nbytes > MEMORY_SIDE_CACHE_BYTES), cache_layers
+    bit of a result; a captured step keeps what held at its capture.)  ``counters``: int32 zeros on the device
+    that belong to the step's runner, whose launches do not overlap in time; products of 17 to 32 rows in slices of
+    k join the residual (``linear_join_norm``) where there are some."""
+    old = _streamed.nt, _streamed.cache_layers, _streamed.counters
+    _streamed.nt, _streamed.cache_layers, _streamed.counters = \
+        int(nbytes > MEMORY_SIDE_CACHE_BYTES), cache_layers, counters
     try:
         yield
     finally:
-        _streamed.nt, _streamed.cache_layers = old
+        _streamed.nt, _streamed.cache_layers, _streamed.counters = old
 
 
 def _streamed_values(partitions: int, nkv: int, d: int) -> int:
@@ -1107,13 +1111,33 @@ def _streams_in_one_slice(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def _rows_join_slices(x: torch.Tensor, w: torch.Tensor) -> int:
+    """Slices of k (two or four) in which the kernel for 17 to 64 rows has ``x @ w.T`` join the residual, or 0:
+    17 to 32 rows and weights that it takes (``_rows_kernel``), more than one slice, counters for its tiles.  (With
+    the product behind scaled, against partial sums and the norm kernel: 27 requests of the 3B shape, down, a step
+    2.866 -> 2.799 ms; 64 requests of the 1B shape, output and down, 1.246 -> 1.258, which stay with the norm.)"""
+    counters = _streamed.counters
+    if counters is None or not (JOIN_NORM_LINEAR and x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1]
+                                and STREAM_MAX_ROWS < x.shape[0] <= min(32, STREAM_WIDE_MAX_ROWS)
+                                and x.device == counters.device and _rows_kernel(x, w)):
+        return 0
+    T, K = x.shape
+    N = w.shape[0]
+    slices = lib.load().rlis_gemm_bf16_rows_slices(N, K)
+    if slices < 2 or 4 * slices * T * N >= 1 << 31 \
+            or lib.load().rlis_gemm_bf16_rows_join_tiles(N, slices) > min(256, counters.numel()):
+        return 0
+    return slices
+
+
 def pending_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None):
     """The projection whose result joins the residual stream: ``linear(x, w, out_dtype,
     partials=True)``, or where the norm behind it may take it in (``JOIN_NORM_LINEAR``; up to 16
     rows of bfloat16, 32 over short rows, one k slice, an output width that the next product can
-    read as its rows)
+    read as its rows; 17 to 32 rows in slices, ``_rows_join_slices``)
     a ``PendingProduct`` that has not run."""
-    if JOIN_NORM_LINEAR and _streams_in_one_slice(x, w) and w.shape[0] % 8 == 0:
+    if JOIN_NORM_LINEAR and _streams_in_one_slice(x, w) and w.shape[0] % 8 == 0 \
+            or x.dim() == 2 and x.shape[0] > STREAM_MAX_ROWS and _rows_join_slices(x, w):
         return PendingProduct(x, w, out_dtype)
     return linear(x, w, out_dtype, partials=True)
 
@@ -1122,6 +1146,13 @@ def can_join_norm_linear(product: PendingProduct, resid: torch.Tensor, w: torch.
     """Whether ``linear_join_norm`` and ``linear_scaled`` take this product, residual and the
     weight of the product behind the norm."""
     T, H = resid.shape
+    if T > STREAM_MAX_ROWS and not _streams_in_one_slice(product.x, product.w):
+        # (the product behind has to be the same kernel's, scaled)
+        return (resid.dtype == torch.float32 and resid.is_contiguous() and product.shape == (T, H)
+                and resid.data_ptr() % 16 == 0 and w.dim() == 2 and w.dtype == torch.bfloat16 and w.shape[1] == H
+                and w.shape[0] % 16 == 0 and H % 128 == 0 and T <= stream_rows(H) and w.stride(1) == 1
+                and w.stride(0) % 8 == 0 and w.stride(0) >= H and w.data_ptr() % 16 == 0
+                and 2 * w.shape[0] * w.stride(0) < 1 << 32 and _rows_join_slices(product.x, product.w) > 0)
     return (JOIN_NORM_LINEAR and resid.dtype == torch.float32 and resid.is_contiguous()
             and product.shape == (T, H) and w.dim() == 2 and w.shape[1] == H
             and w.dtype == torch.bfloat16 and w.stride(1) == 1 and w.stride(0) % 8 == 0
@@ -1144,6 +1175,19 @@ def linear_join_norm(product: PendingProduct, resid: torch.Tensor, norm_weight: 
     if norm_weight.numel() != N or not norm_weight.is_contiguous():
         raise KernelError(f"linear_join_norm: norm weight has {norm_weight.numel()} entries, "
                           f"rows have {N}")
+    slices = _rows_join_slices(x, w) if T > STREAM_MAX_ROWS and not _streams_in_one_slice(x, w) else 0
+    if slices:
+        tiles = lib.load().rlis_gemm_bf16_rows_join_tiles(N, slices)
+        stride = -(-tiles // 4) * 4
+        xw = torch.empty((T, N), dtype=torch.bfloat16, device=x.device)
+        ss = torch.empty((T, stride), dtype=torch.float32, device=x.device)[:, :tiles]
+        parts = torch.empty((slices, T, N), dtype=torch.float32, device=x.device)
+        counters = _streamed.counters
+        lib.call("rlis_gemm_bf16_rows_join", x.data_ptr(), w.data_ptr(), parts.data_ptr(), T, N, K, slices, x.stride(0),
+                 w.stride(0), resid.data_ptr(), norm_weight.data_ptr(), _dt(norm_weight), int(bool(round_sum)),
+                 xw.data_ptr(), ss.data_ptr(), stride, _i32(counters, "counters", 1), counters.numel(), _streamed.nt,
+                 lib.stream_ptr())
+        return xw, ss
     tiles = lib.load().rlis_gemm_bf16_stream_join_tiles(N, K)
     if tiles <= 0:
         raise KernelError("linear_join_norm: cannot read the device properties")

@@ -68,6 +68,7 @@ _SIGNATURES = {
     "rlis_gemm_plain": [P, I, P, I, P, I, I, I, I, L, L, L, P],
     "rlis_gemm_f32": [P, P, P, I, I, I, L, L, L, I, P],
     "rlis_gemm_bf16_rows": [P, P, P, I, I, I, I, I, L, L, L, L, P, I, I, F, I, P],
+    "rlis_gemm_bf16_rows_join": [P, P, P, I, I, I, I, L, L, P, P, I, I, P, P, I, P, I, I, P],
     "rlis_gemm_bf16_tiles": [P, P, P, I, I, I, I, I, L, L, L, L, I, I, P],
     "rlis_gemm_bf16_tiles_heads": [P, P, P, I, I, I, I, I, L, L, L, P, P, P, P, P, P, I, I, P],
     "rlis_gemm_bf16_mfma": [P, P, P, I, I, I, I, L, L, L, P],
@@ -124,6 +125,8 @@ def load() -> ctypes.CDLL:
     lib.rlis_gemm_bf16_stream_slices.argtypes = [I]
     lib.rlis_gemm_bf16_rows_slices.restype = c_int
     lib.rlis_gemm_bf16_rows_slices.argtypes = [I, I]
+    lib.rlis_gemm_bf16_rows_join_tiles.restype = c_int
+    lib.rlis_gemm_bf16_rows_join_tiles.argtypes = [I, I]
     lib.rlis_gemm_bf16_tiles_plan.restype = c_int
     lib.rlis_gemm_bf16_tiles_plan.argtypes = [I, I, I, I, I, I, I]
     lib.rlis_gemm_bf16_tiles_heads_plan.restype = c_int
