@@ -378,10 +378,10 @@ template <> struct Vec16<bf16_t> {
 
 // Loads of a key (and runs of a dim's values) that the decode kernel has under way at once; 1: as the
 // compiler orders them.  Few requests wait for these loads, so as many as the registers beside G heads'
-// sums take, and not fewer for heads of 256 dims, whose key is 64 loads.  One request of 600 keys, us,
-// eight and four for every form -> these (before there were any, with the rotation kernel): float32 8 heads
-// of 256 on one KV head 154 -> 73 (110), bfloat16 32 of 128 on 8 40.4 -> 32.4 (35.0), 32 of 64 on 8 26.0 ->
-// 21.7 (24.8), 16 of 80 on 2 64.3 -> 48.5 (76).
+// sums take, and not fewer for heads of 256 dims, whose key is 64 loads.  One request of 600 keys, us, a KV
+// head's heads together, eight and four for every form -> these: float32 8 heads of 256 on one KV head 154 ->
+// 73, bfloat16 32 of 128 on 8 40.4 -> 32.4, 32 of 64 on 8 26.0 -> 21.7, 16 of 80 on 2 64.3 -> 48.5.  A head or
+// two of float32, four -> eight runs of values: 32 of 64 on 8 15.9 -> 13.9, 8 of 256 on one 43 -> 36.
 template <typename TX, int G, int DPL>
 constexpr int keys_ahead() {
   if (sizeof(TX) == 2) return G == 8 && DPL < 4 ? 1 : 4;
@@ -389,7 +389,14 @@ constexpr int keys_ahead() {
 }
 template <typename TX, int G>
 constexpr int values_ahead() {
-  return sizeof(TX) == 2 && G >= 4 ? 1 : 4;
+  if (sizeof(TX) == 2) return G >= 4 ? 1 : 4;
+  return G <= 2 ? 8 : 4;
+}
+// A wave's loops over its keys counted in scalar registers.  float32 at 24 heads of 128 on 8, 32 requests of 500
+// keys 52.4 -> 46.8 us; 32 of 64 on 8, 16 requests of 4,000 keys, four heads a workgroup, 71 -> 80.
+template <typename TX, int G, int DPL>
+constexpr bool scalar_loops() {
+  return sizeof(TX) == 4 && (G <= 2 || (G == 4 && DPL == 2));
 }
 
 // Grid (kv head * head chunks, sequence, split); 256 threads.  Head chunk c serves query
@@ -416,7 +423,8 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
   float* ml_s = p_s + 4 * G * 64;        // 4 waves * G * 2
   float* acc_s = ml_s + 4 * G * 2;       // 4 waves * G * d
   long long* vbase_s = (long long*)(acc_s + 4 * G * d);  // 4 waves * 64
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = scalar_loops<TX, G, DPL>() ? __builtin_amdgcn_readfirstlane(tid / 64) : tid / 64;
   const int kvh = blockIdx.x / chunks_per_kv, chunk = blockIdx.x % chunks_per_kv;
   const int seq = blockIdx.y, split = blockIdx.z;
   const int g = nh / nkv;
@@ -571,6 +579,15 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
               for (int b = 0; b < AT; ++b) load(b, kk + b * VN);
 #pragma unroll
               for (int b = 0; b < AT; ++b) add(b, kk + b * VN);
+            }
+            if constexpr (AT > 4) {
+#pragma unroll 1
+              for (; kk + 4 * VN <= n; kk += 4 * VN) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) load(b, kk + b * VN);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) add(b, kk + b * VN);
+              }
             }
 #pragma unroll 1
             for (; kk + VN <= n; kk += VN) {
@@ -861,10 +878,10 @@ static int launch_decode(const void* q, long long q_stride, void* out, long long
 // turned as they are loaded (rotate-half, the first rot dims); slots (null: none): the step's own key
 // (turned likewise) and value, k_off and v_off into a row of q, are stored to their page first.
 // That is float32's, where it gives the bits of rope_kv_write in front: 4 requests at 100 positions, 32
-// heads of 64, rotation kernel and attention 4.7 + 11.3 us -> 9.7; 3 at 25, heads of 32, 4.4 + 7.5 -> 8.4
-// (eight keys' and four values' loads under way at once; all 64 keys' and values' in straight-line code
-// 14.2 and 12.2: a kernel this short waits for its instructions).  part_ml (S, nh, splits, 2) and part_acc (S, nh, splits, d) float32 are needed
-// when splits > 1.
+// heads of 64, rotation kernel and attention 4.7 + 11.3 us -> 9.7; 3 at 25, heads of 32, 4.4 + 7.5 -> 8.4, both
+// with a KV head's query heads together (eight keys' and four values' loads under way at once; all 64 keys' and
+// values' in straight-line code 14.2 and 12.2: a kernel this short waits for its instructions).  part_ml (S, nh,
+// splits, 2) and part_acc (S, nh, splits, d) float32 are needed when splits > 1.
 RLIS_API int rlis_attn_decode(const void* q, int dtype, long long q_stride, void* out,
                               long long out_stride, float* part_ml, float* part_acc,
                               const void* k_pages, const void* v_pages, const int* block_tables,
@@ -893,35 +910,33 @@ RLIS_API int rlis_attn_decode(const void* q, int dtype, long long q_stride, void
   RLIS_REQUIRE(splits >= 1 && splits <= 8192 && S <= 65535, "attn_decode: bad grid");
   RLIS_REQUIRE(splits == 1 || (part_ml && part_acc), "attn_decode: partitions need a workspace");
   if (S == 0) return 0;
+  // Query heads a workgroup: as few as the units have room for at one workgroup each.  A head's sums are the same
+  // in any; keys and values of a KV head are read once per workgroup, out of the caches.  float32, us, all heads of
+  // a KV head together -> this: 32 heads of 64 on 8, 3 requests of 25 keys 7.7 -> 5.8, 4 of 100 9.4 -> 7.5, 4 of
+  // 1,000 33 -> 24, 16 of 200 10.7 -> 9.9; 24 of 128 on 8, 4 of 1,000 68 -> 39; 8 of 256 on one, 1 of 600 83 -> 36.
+  // Past one a unit the shared reads are ahead: 32 of 64 on 8, 64 of 200 18.4, two heads 23.3, one 38.6.
   const int g = nh / nkv;
+  const long long units = rlis_stream_compute_units();
+  int heads = 1;
+  while (heads < 8 && heads < g && (long long)nkv * ceil_div(g, heads) * S * splits > units) heads *= 2;
   int rc = 0;
+#define LAUNCH(TX, G)                                                                            \
+  rc = launch_decode<TX, G>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages, v_pages,   \
+                            block_tables, max_pages, ctx_lens, token_rows, S, nh, nkv, d,        \
+                            page_size, scale, window, splits, part_keys, max_parts, slopes,      \
+                            head_scales, softcap, sinks, keep_first, chunk, rope, stream)
 #define BY_G(TX)                                                                                 \
   do {                                                                                           \
-    if (g == 1)                                                                                  \
-      rc = launch_decode<TX, 1>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
-                                v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
-                                nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
-    else if (g == 2)                                                                             \
-      rc = launch_decode<TX, 2>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
-                                v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
-                                nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
-    else if (g <= 4)                                                                             \
-      rc = launch_decode<TX, 4>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
-                                v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
-                                nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
-    else                                                                                         \
-      rc = launch_decode<TX, 8>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages,        \
-                                v_pages, block_tables, max_pages, ctx_lens, token_rows, S, nh,   \
-                                nkv, d, page_size, scale, window, splits, part_keys, max_parts,       \
-                                slopes, head_scales, softcap, sinks, keep_first, chunk, rope, stream); \
+    if (heads == 1) LAUNCH(TX, 1);                                                               \
+    else if (heads == 2) LAUNCH(TX, 2);                                                          \
+    else if (heads == 4) LAUNCH(TX, 4);                                                          \
+    else LAUNCH(TX, 8);                                                                          \
   } while (0)
   if (dtype == RLIS_F32) BY_G(float);
   else if (dtype == RLIS_BF16) BY_G(bf16_t);
   else RLIS_REQUIRE(false, "attn_decode: unknown dtype %d", dtype);
 #undef BY_G
+#undef LAUNCH
   if (rc) return rc;
   RLIS_LAUNCH_CHECK("attn_decode");
   if (splits > 1) {
