@@ -208,7 +208,7 @@ class Model:
         """Logits float32 ``(R, V)`` at ``step.logit_rows``; K, V and state of the step's
         tokens are left in ``pools``."""
         from .. import ops
-        with ops.weights_of(self.weight_bytes, self.cache_layers, pools.counters):
+        with ops.weights_of(self.weight_bytes, self.cache_layers, getattr(pools, "counters", None)):
             return self._forward(step, pools)
 
     def _forward(self, step: Any, pools: Any) -> torch.Tensor:
