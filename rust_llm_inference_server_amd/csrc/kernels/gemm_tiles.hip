@@ -492,7 +492,7 @@ constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 
                                {64, 128, 0.33f}, {64, 256, 0.46f}, {256, 256, 1.38f}};
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
 constexpr int kWideForms = 8;              // those that products of more than 64 rows choose from
-constexpr int kLargest = 10;               // and gate/up beyond 512 rows
+constexpr int kLargest = 10;               // and gate/up beyond 512 rows, output heads beyond 128
 constexpr float kPartialStage = 0.71f;     // of tiles of 128 x 256 that store partial sums: ahead of 256 x 128 there
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
 
@@ -528,7 +528,11 @@ constexpr int kHeadsFormCount = sizeof(kHeadsForms) / sizeof(kHeadsForms[0]);
 //            1.15), k up to 4,096 up to 160 rows while that round has 3/4 of the units, from 97 rows on, where the
 //            library takes a step, 5/8 (0.81 to 1.03; else 0.94 to 1.3, but 6,144 weight rows at 136 rows 0.75);
 //            16,384 weight rows and more (there are tiles enough): up to 128 rows at any k (0.56 to 1.09), to
-//            256 over up to 32,768 (0.65 to 1.06), beyond where rounds come out even (else up to 1.5).
+//            256 over up to 32,768 (0.65 to 1.06), beyond where rounds come out even (else up to 1.5).  There
+//            tiles of 256 x 256 pay from some 200 rows on (128,256 x 2,048 at 256 rows, float32, us: library 182,
+//            256 x 128 154, these 139; 65,536 x 4,096 156, 136, 127).  From 98,304 weight rows on also up to 512
+//            rows where rounds come out even (0.82 to 1.01, 128,256 x 2,048 at 384 and 512 rows 268 -> 224 and
+//            308 -> 253; 65,536 x 2,048 0.99 to 1.06, 40,960 up to 1.13, more rows 0.88 to 1.04).
 //   partials k below 8,192: up to 512 rows (0.49 to 1.08; over 1,024 < k <= 2,048 and more than 2,048 weight rows
 //            beyond 256 rows only where the rounds come out even: else up to 1.1), to 2,048 where one even round
 //            fills the chip.  k from 8,192 on, which the library has in slices too: up to 192 rows (0.67 to 1.15
@@ -549,7 +553,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
   for (int s = slices > 0 ? slices : 1; s <= (slices > 0 ? slices : partials ? 4 : 1); s *= 2) {
     if (K % (s * kBK) || (slices <= 0 && s > 1 && K / s < 512)) continue;
     for (int f = 0; f < kFormCount; ++f) {
-      if (T <= 64 ? kForms[f].rows > 64 : f >= kWideForms && !(f == kLargest && gated && T > 512)) continue;
+      const bool largest = f == kLargest && (gated ? T > 512 : !partials && T > 128 && N >= 64 * units);
+      if (T <= 64 ? kForms[f].rows > 64 : f >= kWideForms && !largest) continue;
       const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
       const long long rounds = (tiles + units - 1) / units;
       if (rounds > 1 << 20) continue;
@@ -580,7 +585,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     else
       here = (K <= 1024 || N >= 1024) && (T <= 256 || (T <= 512 && (even || one)));
   } else if (N >= 64 * units) {
-    here = T <= 128 || (T <= 256 && (N <= 128 * units || (even && K >= 2048)));
+    here = T <= 128 || (T <= 256 && (N <= 128 * units || (even && K >= 1024))) ||
+           (T <= 512 && N >= 384 * units && even && K >= 1024);
   } else if (K <= 1024) {
     here = (K <= 512 ? K >= 256 : N >= 1024) && (T <= 256 || (T <= 1024 && N <= 8192));
   } else {

@@ -51,6 +51,15 @@ def test_gate_up_of_prompts(plan, T, N, K, taken):
     assert plan(T, N, K, 1, 0, 1) == (-1 if taken is None else 16 + taken)
 
 
+@pytest.mark.parametrize("T,N,K,taken", [
+    (128, 128256, 2048, 0), (200, 128256, 2048, 2), (256, 128256, 2048, 10), (256, 65536, 4096, 10), (256, 151936, 2048, 1),
+    (256, 128256, 1024, 10), (256, 128256, 512, None), (256, 100352, 2048, None), (256, 28672, 4096, 1), (384, 128256, 2048, 0),
+    (512, 128256, 4096, 10), (512, 100352, 2048, None), (384, 65536, 2048, None), (512, 40960, 2048, None), (513, 128256, 2048, None)])
+def test_output_heads(plan, T, N, K, taken):
+    """Many weight rows: even rounds alone beyond 128 rows, up to 512 over the widest."""
+    assert plan(T, N, K, 0, 0, 1) == (-1 if taken is None else 16 + taken)
+
+
 def test_rounds_are_those_of_the_device(plan):
     """A partition of a quarter of the compute units has four times the rounds: what fills the chip in one round there
     is a quarter of the tiles, and larger tiles pay earlier."""
