@@ -146,8 +146,6 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
   const int r = lane % 16, g = lane / 16;
   const long long k_slice = (long long)blockIdx.y * p.steps * kBK;
 
-  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.X + k_slice), 0, 0xffffffff, 0x00027000);
-  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + k_slice), 0, 0xffffffff, 0x00027000);
   // instruction i of this wave brings rows (i * 4 + wave) * 4 .. + 3 of a stage, x rows first
   uint32_t src[PER];
 #pragma unroll
@@ -172,6 +170,10 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
   const auto first = [&](int tile) { return (int)((uint32_t)(tile + blockIdx.y) % (uint32_t)p.steps); };
   int a_left = p.steps, a_tile = blockIdx.x, a_buf = 0, a_step = first(a_tile);
   const auto ask = [&]() {
+    // (past the last tile nothing is read: a buffer of no bytes gives zeros without asking memory)
+    const int bytes = __builtin_amdgcn_readfirstlane(a_tile < p.tiles ? -1 : 0);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.X + k_slice), 0, bytes, 0x00027000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + k_slice), 0, bytes, 0x00027000);
     unsigned char* base = smem + a_buf * STAGE;
     const int at = a_step * kBK * 2;
 #pragma unroll
@@ -186,7 +188,6 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
     a_buf = a_buf + 1 == BUFS ? 0 : a_buf + 1;
     a_step = a_step + 1 == p.steps ? 0 : a_step + 1;
     if (--a_left == 0) {
-      // (past the last tile its last row is read again)
       a_left = p.steps;
       a_tile += gridDim.x;
       a_step = first(a_tile);

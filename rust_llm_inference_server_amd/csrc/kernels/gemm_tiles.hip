@@ -190,9 +190,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
   const int r = lane % 16, g = lane / 16;
   const int wm = wave % WM, wn = wave / WM;
 
-  const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)p.X, 0, 0xffffffff, 0x00027000);
-  const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, 0xffffffff, 0x00027000);
-
   // Workgroup id -> tile.  Ids go round the eight dies; each die takes a run of the walk.
   const int per_slice = p.mt * p.nt, total = per_slice * p.slices;
   const auto place = [&](int id, int& m0, int& n0, int& slice) {
@@ -249,6 +246,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
     int at = a_buf;
     if (QUARTERS && i * 4 / PER * (STAGE / 4) + at >= RING) at -= RING;
     const lds_ptr to = (lds_ptr)(smem + at + (i * WAVES + wave) * 1024);
+    // (past the last tile nothing is read: a buffer of no bytes gives zeros without asking memory)
+    const int bytes = __builtin_amdgcn_readfirstlane(a_id < total ? -1 : 0);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)p.X, 0, bytes, 0x00027000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, bytes, 0x00027000);
     if (i < XI) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, to, 16, src[i], a_k, 0, 0);
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, src[i], a_k, 0, NT ? 2 : 0);
   };
@@ -257,7 +258,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
     a_k += kBK * 2;
     if (a_k == a_from + p.steps * (kBK * 2)) a_k = a_from;
     if (--a_left == 0) {
-      // (past the last tile the last one is read again)
       a_left = p.steps;
       a_id += gridDim.x;
       sources(a_id);
