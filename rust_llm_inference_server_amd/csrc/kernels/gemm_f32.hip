@@ -15,8 +15,8 @@
 //    into LDS by direct loads that leave a wave 16 KB ahead of its products, with no registers held
 //    for them and whole lines (256 bytes of a row) per load.  At 4 rows, weights cold (MI355X, us,
 //    stream kernel -> this): 3072 x 2048 10.8 -> 8.3, 2048 x 2048 10.2 -> 7.4, 16384 x 2048 30.2 ->
-//    25.4 (5.3 TB/s), 2048 x 8192 30 -> 21, 128256 x 2048 182 -> 171 (6.2 TB/s), 4096 x 14336 39
-//    (6.0 TB/s); at 16 rows 2048 x 8192 37 -> 23.
+//    25.4 (5.3 TB/s), 2048 x 8192 30 -> 18, 128256 x 2048 182 -> 171 (6.2 TB/s), 4096 x 14336 39
+//    (6.0 TB/s); at 16 rows 2048 x 8192 37 -> 21.
 //  * gemm_f32_stream: other K, 17 to 32 rows, and 5 to 16 over short runs and many tiles (see the
 //    dispatch).  A workgroup takes 16 weight rows
 //    at a time, one wave per run of k, so a wave's loads of a tile are all in flight at once
@@ -293,7 +293,9 @@ __global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(con
 // a row twice).  The chunks a wave asks for ahead of its last products do not exist; they are asked of a buffer of no
 // bytes, so that the counts of loads under way stay what they are and memory is not asked (the last row read again
 // instead, up to as many bytes as a short tile's own: four tokens of the 1B shape behind prompts of 96, a pass 14,672 ->
-// 14,526 us).
+// 14,526 us).  Every other workgroup takes its waves' runs the other way round: rows a power of two apart, walked in
+// step by all workgroups, meet on the same few channels (2048 x 8192 at 4 rows 21.5 -> 17.8 us, 17 with the rows 1 KB
+// further apart; 3072 x 8192 28.0 -> 24.0; 4096 x 14336 41 either way).
 template <int RW, int XW>
 __host__ __device__ constexpr int ring_chunks() {
   return std::min(6, 16384 / ((RW + XW) * 1024));
@@ -310,6 +312,7 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
   unsigned char* ring = ring_smem + wave * NB * CHUNK;
   float* red = (float*)(ring_smem + 8 * NB * CHUNK);            // [2][16 runs][64 lanes][4]
   const int chunks = a.run / 64 * 2;                            // of this wave's two runs
+  const int flip = blockIdx.x & 1, turned = flip * (chunks / 2);  // (odd workgroups: the later run first)
   // instruction i brings rows 4 i .. + 3 of a chunk, 16 lanes a row
   uint32_t src[PER];
   const auto place = [&](int row) { return (uint32_t)((r ^ (row & 15)) * 16); };
@@ -327,7 +330,7 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
     const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + 2 * wave * a.run), 0, bytes, 0x00027000);
     const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + 2 * wave * a.run), 0, bytes, 0x00027000);
     unsigned char* base = ring + buf * CHUNK;
-    const int at = a_chunk * 256;
+    const int at = (a_chunk + turned < chunks ? a_chunk + turned : a_chunk + turned - chunks) * 256;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       if (i < RW)
@@ -371,7 +374,7 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
         }
         buf = buf + 1 == NB ? 0 : buf + 1;
       }
-      *(f32x4*)(part + (2 * wave + half) * 256 + lane * 4) = acc;
+      *(f32x4*)(part + (2 * wave + (half ^ flip)) * 256 + lane * 4) = acc;
     }
     __syncthreads();
     // (the next tile writes the other side; this one is written again behind the barrier that its
