@@ -82,16 +82,10 @@ __device__ __forceinline__ void join_tile(const RowsArgs& p, const RowsJoin& j, 
   const auto parts = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, 0xffffffff, 0x00027000);
   const int c = threadIdx.x % LANES * 4, n = tile * 16 * NI + c;
   const bool inside = n < p.N;
-  f32x4 weight{0.f, 0.f, 0.f, 0.f};
-  if (inside) {
-    if (j.weight_f32) {
-      weight = *(const f32x4*)((const float*)j.weight + n);
-    } else {
-      const uint2 u = *(const uint2*)((const bf16_t*)j.weight + n);
-      weight = f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                     __uint_as_float(u.y & 0xffff0000u)};
-    }
-  }
+  f32x4 weight{0.f, 0.f, 0.f, 0.f};        // (one by one: the norm's weight lies where its model has it)
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (inside) weight[e] = j.weight_f32 ? ((const float*)j.weight)[n + e] : bf16_to_f32(((const bf16_t*)j.weight)[n + e]);
   constexpr int kRows = kWaves * 64 / LANES;     // rows at a time
   for (int t0 = 0; t0 < p.T; t0 += kRows) {
     const int token = t0 + threadIdx.x / LANES;
@@ -448,8 +442,7 @@ RLIS_API int rlis_gemm_bf16_rows_join(const void* X, const void* W, float* parts
                "gemm_rows_join: bad sizes T=%d N=%d K=%d slices=%d", T, N, K, slices);
   const int tiles = rlis_gemm_bf16_rows_join_tiles(N, slices);
   RLIS_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 &&
-                   (uintptr_t)parts % 16 == 0 && (uintptr_t)resid % 16 == 0 && (uintptr_t)xw % 16 == 0 &&
-                   (uintptr_t)weight % 16 == 0,
+                   (uintptr_t)parts % 16 == 0 && (uintptr_t)resid % 16 == 0 && (uintptr_t)xw % 16 == 0,
                "gemm_rows_join: rows must lie on 16-byte boundaries");
   RLIS_REQUIRE(parts && resid && weight && xw && ss && ss_stride >= tiles && arrivals && arrival_slots >= tiles,
                "gemm_rows_join: an operand is missing or too short for %d tiles", tiles);
