@@ -59,6 +59,7 @@
 #include "gemm_stream.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -96,13 +97,20 @@ struct TilesArgs {
   int mt, nt, slices;      // tiles along x's rows and W's, slices of k
   int group;               // tiles of x's rows that are walked together
   int ldx, ldw;            // elements
+  int grid;                // workgroups
   long long ldy, slice_stride;
+};
+
+// (apart: handed to every kernel they made 1,024 x 1,024 products of 4.8 us 0.25 us longer)
+struct HeadsTilesArgs : TilesArgs {
   HeadsArgs heads;
 };
 
 // (kOutGated, kOutHeads: N counts pairs of weight rows whose products meet in a lane)
 enum { kOutBf16 = 0, kOutF32 = 1, kOutGated = 2, kOutHeads = 3 };
 constexpr bool in_pairs(int out) { return out >= kOutGated; }
+template <int OUT>
+using ArgsOf = std::conditional_t<OUT == kOutHeads, HeadsTilesArgs, TilesArgs>;
 
 // Four or eight neighbouring dims of a head.
 template <int Q>
@@ -116,7 +124,7 @@ __device__ __forceinline__ void store_dims(bf16_t* to, const float (&v)[4 * Q]) 
 
 // The sums that a lane holds of one token: dims j .. and j + d / 2 .. of whichever heads its columns are.
 template <int MI, int NI>
-__device__ __forceinline__ void store_heads(const TilesArgs& p, const f32x4 (&acc)[NI][MI], int m, int token,
+__device__ __forceinline__ void store_heads(const HeadsTilesArgs& p, const f32x4 (&acc)[NI][MI], int m, int token,
                                             int first, int g) {
   constexpr int Q = NI % 4 == 0 ? 2 : 1;   // pairs of blocks whose dims are neighbours
   const HeadsArgs& h = p.heads;
@@ -172,8 +180,8 @@ __device__ __forceinline__ void store_heads(const TilesArgs& p, const f32x4 (&ac
 }
 
 // WM x WN waves, each MI groups of 16 rows of x by NI groups of 16 weight rows; BUFS stages in LDS.
-template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArgs p) {
+template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT, typename Args>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const Args p) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
   constexpr int WAVES = WM * WN, BM = 16 * MI * WM, BN = 16 * NI * WN;
   constexpr int STAGE = (BM + BN) * kBK * 2;
@@ -227,8 +235,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
         const int pair = b / 2;
         const int col = NI % 4 == 0 ? pair / 2 * 32 + o / 4 * 8 + pair % 2 * 4 + o % 4 : pair * 16 + o;
         n = min(n0 + col, p.N - 1);
-        if (OUT == kOutGated) n += b % 2 ? p.N : 0;
-        else n += (n >> p.heads.half_shift << p.heads.half_shift) + (b % 2 << p.heads.half_shift);
+        if constexpr (OUT == kOutHeads)
+          n += (n >> p.heads.half_shift << p.heads.half_shift) + (b % 2 << p.heads.half_shift);
+        else
+          n += b % 2 ? p.N : 0;
       } else if (OUT == kOutBf16) {
         // two groups of 16 share 32 columns so that a lane holds eight neighbours
         n = min(n0 + b / 2 * 32 + o / 4 * 8 + b % 2 * 4 + o % 4, p.N - 1);
@@ -242,14 +252,17 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
     a_k = a_from + turn % p.steps * (kBK * 2);
   };
   int a_id = blockIdx.x, a_left = p.steps, a_buf = 0;
+  // x and W end 16 bytes below 4 GB at most.  Past the last tile nothing is read: a buffer of no bytes gives zeros
+  // without asking memory.  (All ones or none, chosen at each load, went through the vector unit between the products:
+  // 2,048 x 2,048 at 512 rows 12.0 -> 12.4 us.)
+  constexpr uint32_t kWhole = 0xfffffff0u;
+  uint32_t a_bytes = kWhole;
   const auto ask = [&](int i) {
     int at = a_buf;
     if (QUARTERS && i * 4 / PER * (STAGE / 4) + at >= RING) at -= RING;
     const lds_ptr to = (lds_ptr)(smem + at + (i * WAVES + wave) * 1024);
-    // (past the last tile nothing is read: a buffer of no bytes gives zeros without asking memory)
-    const int bytes = __builtin_amdgcn_readfirstlane(a_id < total ? -1 : 0);
-    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)p.X, 0, bytes, 0x00027000);
-    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, bytes, 0x00027000);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)p.X, 0, a_bytes, 0x00027000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, a_bytes, 0x00027000);
     if (i < XI) __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, to, 16, src[i], a_k, 0, 0);
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, src[i], a_k, 0, NT ? 2 : 0);
   };
@@ -259,7 +272,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
     if (a_k == a_from + p.steps * (kBK * 2)) a_k = a_from;
     if (--a_left == 0) {
       a_left = p.steps;
-      a_id += gridDim.x;
+      a_id += p.grid;
+      a_bytes = a_id < total ? kWhole : 0;
       sources(a_id);
     }
   };
@@ -272,14 +286,14 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
   int x_buf = x_part, w_buf = w_part;
   const auto onward = [&]() {              // to the next stage's parts
     x_buf = x_buf + STAGE >= RING ? x_buf + STAGE - RING : x_buf + STAGE;
-    w_buf = w_buf + STAGE >= RING ? w_buf + STAGE - RING : w_buf + STAGE;
+    if (QUARTERS) w_buf = w_buf + STAGE >= RING ? w_buf + STAGE - RING : w_buf + STAGE;
   };
   struct Half {
     bf16x8 x[MI], w[NI];
   };
   const auto read = [&](Half& h, int ks, int i) {
     if (i < MI) h.x[i] = *(const bf16x8*)(smem + x_buf + (x_at ^ (ks * 64)) + i * 2048);
-    else h.w[i - MI] = *(const bf16x8*)(smem + w_buf + (w_at ^ (ks * 64)) + (i - MI) * 2048);
+    else h.w[i - MI] = *(const bf16x8*)(smem + (QUARTERS ? w_buf : x_buf) + (w_at ^ (ks * 64)) + (i - MI) * 2048);
   };
   f32x4 acc[NI][MI];
   const auto clear = [&]() {
@@ -345,7 +359,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
 #pragma unroll
   for (int i = 0; i < READS; ++i) read(h0, 0, i);
   wait_loads<63>();
-  for (int id = blockIdx.x; id < total; id += gridDim.x) {
+  for (int id = blockIdx.x; id < total; id += p.grid) {
     clear();
     for (int step = 0; step < p.steps; ++step) {
       half(h0, h1, 1, early);
@@ -381,7 +395,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
           if (Q == 2) *(uint4*)(row + n) = make_uint4(o[0], o[1], o[2 * Q - 2], o[2 * Q - 1]);
           else *(uint2*)(row + n) = make_uint2(o[0], o[1]);
         }
-      } else if (OUT == kOutHeads) {
+      } else if constexpr (OUT == kOutHeads) {
         store_heads<MI, NI>(p, acc, m, token, n0 + wn * NI * 8, g);
       } else if (OUT == kOutBf16) {
         bf16_t* row = (bf16_t*)p.Y + (long long)token * p.ldy;
@@ -410,12 +424,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tiles_kernel(const TilesArg
 }
 
 template <int MI, int NI, int WM, int WN, int BUFS, int OUT, bool NT>
-int launch_tiles(TilesArgs a, hipStream_t stream) {
+int launch_tiles(ArgsOf<OUT> a, hipStream_t stream) {
   static LdsGrant grant;
   constexpr int BM = 16 * MI * WM, BN = 16 * NI * WN;
   constexpr int bytes = (BUFS * 2 + (BUFS == 2 && WM * WN == 8)) * (BM + BN) * kBK;
   static_assert(bytes <= 160 * 1024, "");
-  const auto kernel = gemm_tiles_kernel<MI, NI, WM, WN, BUFS, OUT, NT>;
+  const auto kernel = gemm_tiles_kernel<MI, NI, WM, WN, BUFS, OUT, NT, ArgsOf<OUT>>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_tiles: %s", hipGetErrorString(e));
   a.mt = ceil_div(a.T, BM);
@@ -426,7 +440,8 @@ int launch_tiles(TilesArgs a, hipStream_t stream) {
   const int resident = std::max(1, std::min(160 * 1024 / bytes, 8 / (WM * WN)));
   const long long total = (long long)a.mt * a.nt * a.slices;
   RLIS_REQUIRE(total < (1 << 30), "gemm_tiles: too many tiles");
-  kernel<<<dim3((int)std::min<long long>(total, (long long)cus * resident)), WM * WN * 64, bytes, stream>>>(a);
+  a.grid = (int)std::min<long long>(total, (long long)cus * resident);
+  kernel<<<dim3(a.grid), WM * WN * 64, bytes, stream>>>(a);
   return 0;
 }
 
@@ -434,30 +449,18 @@ template <int MI, int NI, int WM, int WN, int BUFS>
 int launch_out(const TilesArgs& a, int out, int nt, hipStream_t stream) {
   // (rows of W that a second tile reads too must stay in the caches: the output head of the 1B shape at 96
   // rows in tiles of 64 x 256 132 us, non-temporally 178)
-  if (nt && a.T <= 16 * MI * WM && out != kOutHeads) {
+  if (nt && a.T <= 16 * MI * WM) {
     if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16, true>(a, stream);
     if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32, true>(a, stream);
     return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated, true>(a, stream);
   }
-  if (out == kOutHeads) return launch_tiles<MI, NI, WM, WN, BUFS, kOutHeads, false>(a, stream);
   if (out == kOutBf16) return launch_tiles<MI, NI, WM, WN, BUFS, kOutBf16, false>(a, stream);
   if (out == kOutF32) return launch_tiles<MI, NI, WM, WN, BUFS, kOutF32, false>(a, stream);
   return launch_tiles<MI, NI, WM, WN, BUFS, kOutGated, false>(a, stream);
 }
 
-// Tiles of which a compute unit holds two, unless there are not that many: a unit with one has all of the LDS
-// for its ring (q/k/v, cold weights, us: 200 x 5,120 x 3,072 in 128 x 64 26.2 with three stages, 23.8 with six; 65 x
-// 6,144 x 4,096 in 64 x 64 22.0 with four, 19.5 with nine; output of 512 rows of the 1B shape no faster).
-template <int MI, int NI, int WM, int WN, int BUFS, int ALONE>
-int launch_deep(const TilesArgs& a, int out, int nt, hipStream_t stream) {
-  const long long tiles = (long long)ceil_div(a.T, 16 * MI * WM) * ceil_div(a.N, 8 * NI * WN);
-  if (out == kOutHeads && tiles <= rlis_stream_compute_units())
-    return launch_tiles<MI, NI, WM, WN, ALONE, kOutHeads, false>(a, stream);
-  return launch_out<MI, NI, WM, WN, BUFS>(a, out, nt, stream);
-}
-
 int launch_form(const TilesArgs& a, int out, int tile, int nt, hipStream_t stream) {
-  int rc = -1;
+  int rc = 0;
   switch (tile) {
     case 0: rc = launch_out<4, 4, 2, 4, 3>(a, out, nt, stream); break;   // 128 x 256
     case 1: rc = launch_out<4, 4, 4, 2, 3>(a, out, nt, stream); break;   // 256 x 128
@@ -465,18 +468,46 @@ int launch_form(const TilesArgs& a, int out, int tile, int nt, hipStream_t strea
     case 3: rc = launch_out<6, 4, 2, 2, 3>(a, out, nt, stream); break;   // 192 x 128
     case 4: rc = launch_out<5, 4, 2, 2, 4>(a, out, nt, stream); break;   // 160 x 128
     case 5: rc = launch_out<4, 2, 2, 4, 5>(a, out, nt, stream); break;   // 128 x 128
-    case 6: rc = launch_deep<4, 2, 2, 2, 3, 6>(a, out, nt, stream); break;  // 128 x 64, two to a compute unit
-    case 7: rc = launch_deep<2, 2, 2, 2, 4, 9>(a, out, nt, stream); break;  // 64 x 64, two to a compute unit
+    case 6: rc = launch_out<4, 2, 2, 2, 3>(a, out, nt, stream); break;   // 128 x 64, two to a compute unit
+    case 7: rc = launch_out<2, 2, 2, 2, 4>(a, out, nt, stream); break;   // 64 x 64, two to a compute unit
     case 8: rc = launch_out<4, 2, 1, 4, 3>(a, out, nt, stream); break;   // 64 x 128, two to a compute unit
     case 9: rc = launch_out<4, 4, 1, 4, 2>(a, out, nt, stream); break;   // 64 x 256, two to a compute unit
     case 10: rc = launch_out<8, 4, 2, 4, 2>(a, out, nt, stream); break;  // 256 x 256
-    case 11: if (out == kOutHeads) rc = launch_tiles<2, 6, 4, 1, 5, kOutHeads, false>(a, stream); break;  // 128 x 96
-    case 12: if (out == kOutHeads) rc = launch_tiles<1, 6, 4, 1, 4, kOutHeads, false>(a, stream); break;  // 64 x 96, two to a unit
     default: RLIS_REQUIRE(false, "gemm_tiles: no tile %d", tile);
   }
-  RLIS_REQUIRE(rc >= 0, "gemm_tiles: tile %d is of q, k and v alone", tile);
   if (rc) return rc;
   RLIS_LAUNCH_CHECK("gemm_tiles");
+  return 0;
+}
+
+// Tiles of which a compute unit holds two, unless there are not that many: a unit with one has all of the LDS
+// for its ring (q/k/v, cold weights, us: 200 x 5,120 x 3,072 in 128 x 64 26.2 with three stages, 23.8 with six; 65 x
+// 6,144 x 4,096 in 64 x 64 22.0 with four, 19.5 with nine; output of 512 rows of the 1B shape no faster).
+template <int MI, int NI, int WM, int WN, int BUFS, int ALONE>
+int launch_deep(const HeadsTilesArgs& a, hipStream_t stream) {
+  const long long tiles = (long long)ceil_div(a.T, 16 * MI * WM) * ceil_div(a.N, 8 * NI * WN);
+  if (tiles <= rlis_stream_compute_units()) return launch_tiles<MI, NI, WM, WN, ALONE, kOutHeads, false>(a, stream);
+  return launch_tiles<MI, NI, WM, WN, BUFS, kOutHeads, false>(a, stream);
+}
+
+// (the numbers of the tiles above, and two of their own)
+int launch_heads(const HeadsTilesArgs& a, int tile, hipStream_t stream) {
+  int rc = 0;
+  switch (tile) {
+    case 0: rc = launch_tiles<4, 4, 2, 4, 3, kOutHeads, false>(a, stream); break;
+    case 1: rc = launch_tiles<4, 4, 4, 2, 3, kOutHeads, false>(a, stream); break;
+    case 3: rc = launch_tiles<6, 4, 2, 2, 3, kOutHeads, false>(a, stream); break;
+    case 4: rc = launch_tiles<5, 4, 2, 2, 4, kOutHeads, false>(a, stream); break;
+    case 5: rc = launch_tiles<4, 2, 2, 4, 5, kOutHeads, false>(a, stream); break;
+    case 6: rc = launch_deep<4, 2, 2, 2, 3, 6>(a, stream); break;
+    case 7: rc = launch_deep<2, 2, 2, 2, 4, 9>(a, stream); break;
+    case 10: rc = launch_tiles<8, 4, 2, 4, 2, kOutHeads, false>(a, stream); break;
+    case 11: rc = launch_tiles<2, 6, 4, 1, 5, kOutHeads, false>(a, stream); break;  // 128 x 96
+    case 12: rc = launch_tiles<1, 6, 4, 1, 4, kOutHeads, false>(a, stream); break;  // 64 x 96, two to a compute unit
+    default: RLIS_REQUIRE(false, "gemm_tiles_heads: no tile %d", tile);
+  }
+  if (rc) return rc;
+  RLIS_LAUNCH_CHECK("gemm_tiles_heads");
   return 0;
 }
 
@@ -640,7 +671,7 @@ RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out
   RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * N * (out == 2 ? 2 : 1) < (1LL << 32),
                "gemm_tiles: x or W passes 4 GB");
   const TilesArgs a = {(const bf16_t*)X, (const bf16_t*)W, Y, T, N, K / slices / kBK, 0, 0, slices, 0,
-                       (int)ldx, (int)ldw, ldy, slice_stride, {}};
+                       (int)ldx, (int)ldw, 0, ldy, slice_stride};
   return launch_form(a, out, tile, nt, stream);
 }
 
@@ -667,10 +698,10 @@ RLIS_API int rlis_gemm_bf16_tiles_heads(const void* X, const void* W, void* Q, i
                    (uintptr_t)sin % 16 == 0,
                "gemm_tiles_heads: pages, slots, positions and both tables of angles are needed");
   RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * rows < (1LL << 32), "gemm_tiles_heads: x or W passes 4 GB");
-  TilesArgs a = {(const bf16_t*)X, (const bf16_t*)W, Q, T, (int)(rows / 2), K / kBK, 0, 0, 1, 0,
-                 (int)ldx, (int)ldw, ldq, 0, {}};
+  HeadsTilesArgs a = {{(const bf16_t*)X, (const bf16_t*)W, Q, T, (int)(rows / 2), K / kBK, 0, 0, 1, 0,
+                       (int)ldx, (int)ldw, 0, ldq, 0}, {}};
   a.heads = {cos, sin, positions, slots, (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, 0, 0};
   while (2 << a.heads.half_shift < d) ++a.heads.half_shift;
   while (1 << a.heads.page_shift < page_size) ++a.heads.page_shift;
-  return launch_form(a, kOutHeads, tile, 0, stream);
+  return launch_heads(a, tile, stream);
 }
