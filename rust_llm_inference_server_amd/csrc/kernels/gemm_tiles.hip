@@ -540,6 +540,10 @@ constexpr HeadsForm kHeadsForms[] = {
     {12, 64, 96, 0.27f, 0.30f, 0.f}};
 constexpr int kHeadsFormCount = sizeof(kHeadsForms) / sizeof(kHeadsForms[0]);
 
+// The library's: tiles that explain its times, whose rounds cost it as the rounds here do, and a stage's time.
+constexpr TileForm kLibraryForms[] = {{256, 256, 0.985f}, {256, 128, 0.563f}, {128, 256, 0.605f}, {128, 128, 0.40f},
+                                      {192, 256, 0.818f}, {256, 192, 0.845f}, {64, 128, 0.276f}};
+
 }  // namespace
 
 // How the product of T rows with N weight rows (gated: gate and up rows together) is cut: the tile (an
@@ -629,29 +633,36 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
 }
 
 // The tile that rlis_gemm_bf16_tiles_heads should take for T rows and N weight rows, or -1 where the library's
-// product and the kernel that turns and stores (elementwise.hip) are ahead.  Both sides are estimated: a tile's
-// stages, what ends a round and what is fixed; the library's from the bytes of W, the operations and the rows that
-// pass through memory.  Fitted to 65 to 8,192 rows of ten shapes, 1,536 to 12,288 weight rows over a k of 512 to
-// 8,192, weights cold (tiles to 10 %; the library, whose algorithms are a clock's choice, to 15 %).  Of 136 products
-// the rule takes 120, 0.55 to 1.02 of the library's time; beyond 8,192 weight rows the tiles have to be ahead by a
-// fifteenth (12,288 x 4,096 at 768 and 1,024 rows would be taken at 1.05 to 1.1), and by a seventh from 4,096 rows on
-// over a k of 4,096 and more, where the library reaches 1.5 PFLOP/s (8,192 rows of the 8B shape in a step 312 us against its
-// 295).  Figures are those of 256 units.
+// product and the kernel that turns and stores (elementwise.hip) are ahead.  Both sides are estimated: a tile's stages,
+// what ends a round and what is fixed; the library's as rounds of tiles too, with the rows that pass through memory.
+// 529 products of 20 shapes, 1,536 to 12,288 weight rows over a k of 512 to 8,192, at 65 to 8,192 rows, weights cold:
+// tiles 0.95 to 1.06 of what they take in half of all cases, 0.88 to 1.14 in nine of ten; the library 0.95 to 1.05 and
+// 0.89 to 1.12.  So the tiles have to be ahead by an estimated 2 to 7 %, the more rows the more (above 1,024 rows the
+// library runs its heuristics' first algorithm: 2,560 rows of 6,144 x 4,096 97 us, 2,800 160), past 4,096 rows by 14 %
+// but for many weight rows over a short k, where the tiles were behind nowhere (0.71 to 0.98).  Of the 529 this takes
+// 398, 0.53 to 1.07 of the library's time, 0.81 on average; the tiles are behind at 1,600 rows of 6,144 x 2,048
+// (1.07), 512 of 4,608 x 3,584 (1.03), 505 and 512 of 5,120 x 3,072 and 333 of 8,192 x 6,144 (1.02).
+// Figures are those of 256 units.
 RLIS_API int rlis_gemm_bf16_tiles_heads_plan(int T, int N, int K, int units) {
   if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
+  const auto rounds_of = [&](int rows, int cols) {
+    const long long tiles = (long long)ceil_div(T, rows) * ceil_div(N, cols);
+    return (float)((tiles + units - 1) / units);
+  };
   float least = 0.f;
   int best = -1;
   for (int f = 0; f < kHeadsFormCount; ++f) {
     const HeadsForm& form = kHeadsForms[f];
-    const long long tiles = (long long)ceil_div(T, form.rows) * ceil_div(N, form.cols);
-    const long long rounds = (tiles + units - 1) / units;
-    const float us = (float)rounds * (K / kBK * (rounds == 1 ? form.alone : form.stage) + form.end);
+    const float rounds = rounds_of(form.rows, form.cols);
+    const float us = rounds * (K / kBK * (rounds == 1.f ? form.alone : form.stage) + form.end);
     if (best < 0 || us < least) least = us, best = form.tile;
   }
-  const float share = 256.f / units;
   const float here = least + 4.9f + (0.095e-6f * K + 0.6e-6f * T) * N;
-  const float library = 12.f + 0.454e-6f * N * K + (1.19e-9f * T * K + 1.05e-6f * T) * N * share;
-  return here < library * (T >= 4096 && K >= 4096 ? 0.85f : N > 32 * units ? 0.93f : 1.f) ? best : -1;
+  float stages = rounds_of(kLibraryForms[0].rows, kLibraryForms[0].cols) * kLibraryForms[0].stage;
+  for (const TileForm& form : kLibraryForms) stages = std::min(stages, rounds_of(form.rows, form.cols) * form.stage);
+  const float library = 7.9f + stages * (K / kBK) + (0.2e-6f * K + 1.65e-6f * T) * N;
+  const float margin = T <= 4096 ? 0.99f - 1.9e-5f * T : N >= 5120 && K <= 3072 ? 1.f : 0.86f;
+  return here < library * margin ? best : -1;
 }
 
 // Y (T,N) = X (T,K) * W (N,K)^T, N a multiple of 8, K of 64 times the slices.  out 0: bfloat16; 1:
