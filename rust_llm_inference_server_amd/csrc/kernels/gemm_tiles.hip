@@ -565,9 +565,11 @@ constexpr TileForm kLibraryForms[] = {{256, 256, 0.985f}, {256, 128, 0.563f}, {1
 //            16,384 weight rows and more (there are tiles enough): up to 128 rows at any k (0.56 to 1.09), to
 //            256 over up to 32,768 (0.65 to 1.06), beyond where rounds come out even (else up to 1.5).  There
 //            tiles of 256 x 256 pay from some 200 rows on (128,256 x 2,048 at 256 rows, float32, us: library 182,
-//            256 x 128 154, these 139; 65,536 x 4,096 156, 136, 127).  From 98,304 weight rows on also up to 512
-//            rows where rounds come out even (0.82 to 1.01, 128,256 x 2,048 at 384 and 512 rows 268 -> 224 and
-//            308 -> 253; 65,536 x 2,048 0.99 to 1.06, 40,960 up to 1.13, more rows 0.88 to 1.04).
+//            256 x 128 154, these 139; 65,536 x 4,096 156, 136, 127).  Even rounds beyond 32,768 over a k of 2,048 and
+//            more: 0.81 to 1.03, but 1.0 to 1.14 over a k of 3,072 where weight rows come in 4,096s; over 1,024 and
+//            1,536 0.90 to 1.16.  More rows of x are the library's: at 257 to 512 rows the tiles take 0.8 to 0.95 of its
+//            time over 128,256 and 151,936 weight rows, which leave it with broken tiles, and 1.0 to 1.2 of it over
+//            126,976, 131,072, 160,000 and most others.
 //   partials k below 8,192: up to 512 rows (0.49 to 1.08; over 1,024 < k <= 2,048 and more than 2,048 weight rows
 //            beyond 256 rows only where the rounds come out even: else up to 1.1), to 2,048 where one even round
 //            fills the chip.  k from 8,192 on, which the library has in slices too: up to 192 rows (0.67 to 1.15
@@ -620,8 +622,7 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     else
       here = (K <= 1024 || N >= 1024) && (T <= 256 || (T <= 512 && (even || one)));
   } else if (N >= 64 * units) {
-    here = T <= 128 || (T <= 256 && (N <= 128 * units || (even && K >= 1024))) ||
-           (T <= 512 && N >= 384 * units && even && K >= 1024);
+    here = T <= 128 || (T <= 256 && (N <= 128 * units || (even && K >= 2048)));
   } else if (K <= 1024) {
     here = (K <= 512 ? K >= 256 : N >= 1024) && (T <= 256 || (T <= 1024 && N <= 8192));
   } else {

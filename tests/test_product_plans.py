@@ -53,10 +53,13 @@ def test_gate_up_of_prompts(plan, T, N, K, taken):
 
 @pytest.mark.parametrize("T,N,K,taken", [
     (128, 128256, 2048, 0), (200, 128256, 2048, 2), (256, 128256, 2048, 10), (256, 65536, 4096, 10), (256, 151936, 2048, 1),
-    (256, 128256, 1024, 10), (256, 128256, 512, None), (256, 100352, 2048, None), (256, 28672, 4096, 1), (384, 128256, 2048, 0),
-    (512, 128256, 4096, 10), (512, 100352, 2048, None), (384, 65536, 2048, None), (512, 40960, 2048, None), (513, 128256, 2048, None)])
+    (256, 128256, 512, None), (256, 100352, 2048, None), (256, 28672, 4096, 1), (512, 100352, 2048, None), (384, 65536, 2048, None),
+    (512, 40960, 2048, None), (513, 128256, 2048, None),
+    # (in tiles 1.03 to 1.2 of the library's time, but 0.84 to 0.97 over 128,256 weight rows alone)
+    (256, 65536, 1024, None), (256, 128256, 1024, None), (192, 128256, 1536, None), (320, 131072, 4096, None), (320, 256000, 3072, None),
+    (384, 160000, 3072, None), (384, 128256, 2048, None), (512, 128256, 4096, None)])
 def test_output_heads(plan, T, N, K, taken):
-    """Many weight rows: even rounds alone beyond 128 rows, up to 512 over the widest."""
+    """Many weight rows: even rounds alone beyond 128 rows, the library's beyond 256."""
     assert plan(T, N, K, 0, 0, 1) == (-1 if taken is None else 16 + taken)
 
 
