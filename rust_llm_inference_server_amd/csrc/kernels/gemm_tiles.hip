@@ -580,9 +580,11 @@ constexpr TileForm kLibraryForms[] = {{256, 256, 0.985f}, {256, 128, 0.563f}, {1
 //   gated    k up to 1,024, and to 2,048 from 1,024 weight rows on: up to 256 rows, to 512 where the rounds come out
 //            even or there is one (0.36 to 1.03).  Longer k from 5,632 weight rows on: up to 192 rows, beyond where
 //            rounds come out nearly even (0.66 to 1.1; fewer weight rows up to 2.0).  From 1,024 rows on (over a k of
-//            1,024 beyond 512) where rounds come out even, k of 1,024 to 3,072 from 8,192 weight rows on (0.78 to 1.0, most in
-//            tiles of 256 x 256; uneven rounds up to 1.12, 640 and 768 rows 1.05 to 1.14; over a k of 4,096 and 8,192 0.97 to
-//            1.06).
+//            1,024 beyond 512) where rounds come out even, k of 1,024 to 3,072 from 8,192 weight rows on: k of 1,024 as it is
+//            (0.78 to 1.01); longer ones in tiles of 256 x 256 where their last round is nearly full, in 256 x 128 and
+//            128 x 256 where it is full (334 products of 16 shapes at 1,024 to 8,192 rows: 220 taken, up to 1.02, 0.92 on
+//            average, 0.67 where the library has a broken round more; the smaller tiles up to 1.15; uneven rounds up to 1.12, 640 and 768 rows 1.05 to 1.14; over a k of
+//            4,096 and 8,192 0.97 to 1.06).
 RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices, int units) {
   if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
   float least = 0.f;
@@ -616,6 +618,13 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
     }
   } else if (gated && T > 512) {
     here = even && K >= 1024 && K <= 3072 && N >= 8192 && (T >= 1024 || K == 1024);
+    if (here && K > 1024) {
+      const int most = ceil_div(T, kForms[kLargest].rows) * ceil_div(N, kForms[kLargest].cols);
+      if (most * 20LL >= ceil_div(most, units) * (units * 17LL))
+        best = kLargest + 16;
+      else
+        here = best % 16 <= 1 && best_tiles * 20LL >= best_rounds * (units * 19LL);
+    }
   } else if (gated) {
     if (K > 2048)
       here = N >= 5632 && (T <= 192 || (T <= 256 && best_tiles * 20LL >= best_rounds * (units * 17LL)) || (T <= 512 && even));

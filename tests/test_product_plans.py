@@ -45,7 +45,12 @@ def test_partial_sums_and_gate_up(plan, T, N, K, gated, slices, taken):
 
 @pytest.mark.parametrize("T,N,K,taken", [
     (1024, 16384, 2048, 10), (2048, 16384, 2048, 10), (8192, 16384, 3072, 10), (1536, 16384, 2048, 1), (2048, 8192, 1024, 10),
-    (640, 16384, 2048, None), (768, 16384, 3072, None), (2048, 28672, 4096, None), (2048, 4096, 2048, None), (4096, 16384, 512, None)])
+    (640, 16384, 2048, None), (768, 16384, 3072, None), (2048, 28672, 4096, None), (2048, 4096, 2048, None), (4096, 16384, 512, None),
+    (1280, 8192, 1024, 4), (2560, 16384, 2048, 1), (2800, 16384, 2048, 10), (4096, 13824, 2560, 1),
+    # (in smaller tiles, or uneven, measured 1.03 to 1.15 of the library's time)
+    (1280, 8192, 2048, None), (3000, 13824, 2560, None), (1700, 14336, 3072, None), (1152, 20480, 2560, None),
+    (1344, 17920, 1536, None), (2304, 16384, 2048, None), (1536, 24576, 3072, None)])
+
 def test_gate_up_of_prompts(plan, T, N, K, taken):
     """gate/up of more than 512 rows: even rounds alone, most in the largest tile."""
     assert plan(T, N, K, 1, 0, 1) == (-1 if taken is None else 16 + taken)
