@@ -524,7 +524,9 @@ constexpr TileForm kForms[] = {{128, 256, 0.75f}, {256, 128, 0.72f}, {224, 128, 
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]);
 constexpr int kWideForms = 8;              // those that products of more than 64 rows choose from
 constexpr int kLargest = 10;               // and gate/up beyond 512 rows, output heads beyond 128
-constexpr float kPartialStage = 0.71f;     // of tiles of 128 x 256 that store partial sums: ahead of 256 x 128 there
+// of tiles of 128 x 256 that store partial sums over a k in 8,192s for weight rows in 2,048s, ahead of 256 x 128 there
+// (2,048 x 8,192 at 2,048 rows 62.0 against 64.0 us; else up to 8 % behind: 1,536 rows of 2,560 x 6,912 57.1 against 52.8)
+constexpr float kPartialStage = 0.71f;
 constexpr float kPartial = 1.75e-6f;       // us to write and add one float32 partial sum
 
 // The same for q, k and v on their way to the cache: a stage's time with two workgroups to a compute unit and
@@ -597,7 +599,8 @@ RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int parti
       const long long tiles = (long long)ceil_div(T, kForms[f].rows) * ceil_div(N, kForms[f].cols) * s;
       const long long rounds = (tiles + units - 1) / units;
       if (rounds > 1 << 20) continue;
-      const float us = (float)rounds * (K / s / kBK) * (f == 0 && partials ? kPartialStage : kForms[f].stage) +
+      const float stage = f == 0 && partials && K % 8192 == 0 && N % 2048 == 0 ? kPartialStage : kForms[f].stage;
+      const float us = (float)rounds * (K / s / kBK) * stage +
                        (s > 1 ? kPartial * s : kPartial / 2) * (float)T * N;
       if (best < 0 || us < least) least = us, best = f + 16 * s, best_rounds = (int)rounds, best_tiles = (int)tiles;
     }

@@ -43,6 +43,14 @@ def test_partial_sums_and_gate_up(plan, T, N, K, gated, slices, taken):
     assert (plan(T, N, K, gated, 1 - gated, slices) >= 0) == taken
 
 
+@pytest.mark.parametrize("T,N,K,slices,tile", [
+    (2048, 2048, 8192, 2, 0), (512, 4096, 8192, 4, 0), (256, 5120, 5120, 0, 1), (1536, 2560, 6912, 0, 1), (1280, 6144, 6144, 0, 1),
+    (512, 4096, 14336, 4, 1), (2048, 4096, 4096, 0, 1), (1280, 3072, 8192, 2, 1)])
+def test_partial_sums_in_the_flatter_tile(plan, T, N, K, slices, tile):
+    """128 x 256 for a k in 8,192s and weight rows in 2,048s; elsewhere 256 x 128 is up to 8 % ahead of it."""
+    assert plan(T, N, K, 0, 1, slices) % 16 == tile
+
+
 @pytest.mark.parametrize("T,N,K,taken", [
     (1024, 16384, 2048, 10), (2048, 16384, 2048, 10), (8192, 16384, 3072, 10), (1536, 16384, 2048, 1), (2048, 8192, 1024, 10),
     (640, 16384, 2048, None), (768, 16384, 3072, None), (2048, 28672, 4096, None), (2048, 4096, 2048, None), (4096, 16384, 512, None),
