@@ -1134,10 +1134,13 @@ def pending_linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.d
     """The projection whose result joins the residual stream: ``linear(x, w, out_dtype,
     partials=True)``, or where the norm behind it may take it in (``JOIN_NORM_LINEAR``; up to 16
     rows of bfloat16, 32 over short rows, one k slice, an output width that the next product can
-    read as its rows; 17 to 32 rows in slices, ``_rows_join_slices``)
+    read as its rows; 17 to 32 rows in slices, ``_rows_join_slices``, where that product takes as many rows
+    scaled; a residual of up to 1,024 only behind weights that no cache holds: 24 rows of 1,024 x 4,096 with q/k/v of
+    3,072 behind 13.5 -> 13.1 us, of a model that the memory-side cache holds 13.0 -> 13.5)
     a ``PendingProduct`` that has not run."""
     if JOIN_NORM_LINEAR and _streams_in_one_slice(x, w) and w.shape[0] % 8 == 0 \
-            or x.dim() == 2 and x.shape[0] > STREAM_MAX_ROWS and _rows_join_slices(x, w):
+            or (x.dim() == 2 and x.shape[0] > STREAM_MAX_ROWS and w.dim() == 2 and (w.shape[0] > 1024 or _streamed.nt)
+                and x.shape[0] <= stream_rows(w.shape[0]) and _rows_join_slices(x, w)):
         return PendingProduct(x, w, out_dtype)
     return linear(x, w, out_dtype, partials=True)
 
