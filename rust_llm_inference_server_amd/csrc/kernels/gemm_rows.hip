@@ -31,6 +31,7 @@
 #include "gemm_stream.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -61,12 +62,18 @@ struct RowsArgs {
   void* Y;
   int T, N, steps, tiles; // N: output columns; steps: stages of a tile (of its slice of k)
   int ldx, ldw;           // elements
+  int grid;               // workgroups a slice
   long long ldy, slice_stride;
   const float* ss;        // scaled: (T, ss_stride) partial sums of squares, ss_count a row
   int ss_count, ss_stride;
   float eps;
+};
+
+struct RowsJoinArgs : RowsArgs {
   RowsJoin join;
 };
+template <bool JOINS>
+using ArgsOf = std::conditional_t<JOINS, RowsJoinArgs, RowsArgs>;
 
 // Sums that workgroups of one launch hand to each other, 16 bytes at a time, past the caches that only one die
 // sees (device scope: what an atomic of that scope does, see attention_mfma.hip).
@@ -127,8 +134,8 @@ __device__ __forceinline__ void join_tile(const RowsArgs& p, const RowsJoin& j, 
 }
 
 // MI groups of 16 rows of x, NI groups of 16 weight rows, BUFS stages in LDS.
-template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, bool JOINS, typename TY>
-__global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p) {
+template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, bool JOINS, typename TY, typename Args>
+__global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const Args p) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
   constexpr int ROWS = 16 * (MI + NI), STAGE = ROWS * kBK * 2;
   constexpr int PER = MI + NI;             // load instructions of a wave and stage, 4 rows each
@@ -163,11 +170,14 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
   };
   const auto first = [&](int tile) { return (int)((uint32_t)(tile + blockIdx.y) % (uint32_t)p.steps); };
   int a_left = p.steps, a_tile = blockIdx.x, a_buf = 0, a_step = first(a_tile);
+  // x and W end 16 bytes below 4 GB at most.  Past the last tile nothing is read: a buffer of no bytes gives zeros
+  // without asking memory.  (All ones or none, chosen at each load, went through the vector unit: 64 rows of 512 x 1,024 in
+  // two slices 3.9 -> 4.2 us.)
+  constexpr uint32_t kWhole = 0xfffffff0u;
+  uint32_t a_bytes = kWhole;
   const auto ask = [&]() {
-    // (past the last tile nothing is read: a buffer of no bytes gives zeros without asking memory)
-    const int bytes = __builtin_amdgcn_readfirstlane(a_tile < p.tiles ? -1 : 0);
-    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.X + k_slice), 0, bytes, 0x00027000);
-    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + k_slice), 0, bytes, 0x00027000);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.X + k_slice), 0, a_bytes, 0x00027000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + k_slice), 0, a_bytes, 0x00027000);
     unsigned char* base = smem + a_buf * STAGE;
     const int at = a_step * kBK * 2;
 #pragma unroll
@@ -183,7 +193,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
     a_step = a_step + 1 == p.steps ? 0 : a_step + 1;
     if (--a_left == 0) {
       a_left = p.steps;
-      a_tile += gridDim.x;
+      a_tile += p.grid;
+      a_bytes = a_tile < p.tiles ? kWhole : 0;
       a_step = first(a_tile);
       weight_rows(a_tile);
     }
@@ -228,7 +239,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
   const float scale = SCALED ? ((float*)red)[token] : 1.f;
 
   int buf = 0;
-  for (int tile = blockIdx.x; tile < p.tiles; tile += gridDim.x) {
+  for (int tile = blockIdx.x; tile < p.tiles; tile += p.grid) {
     f32x4 acc[NI][MI];
 #pragma unroll
     for (int a = 0; a < NI; ++a)
@@ -287,7 +298,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
         }
         const int n = tile * 16 * NI + a * 16 + 4 * g;
         if (!live || n >= p.N) continue;
-        if (JOINS) {
+        if constexpr (JOINS) {
           const auto parts = __builtin_amdgcn_make_buffer_rsrc(p.Y, 0, 0xffffffff, 0x00027000);
           const long long to = blockIdx.y * p.slice_stride + (long long)token * p.ldy + n;
           typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -302,7 +313,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
         }
       }
     }
-    if (JOINS) {
+    if constexpr (JOINS) {
       // The last of the tile's slices to get here joins them: everybody's stores have arrived before it is counted in.
       int& last = *(int*)red;              // (behind the barrier nobody reads sums)
       __builtin_amdgcn_s_waitcnt(0);
@@ -322,28 +333,32 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs p
 }
 
 template <int MI, int NI, int BUFS, bool SCALED, bool GATED, bool NT, bool JOINS, typename TY>
-int launch_form(const RowsArgs& a, int slices, hipStream_t stream) {
+int launch_form(ArgsOf<JOINS> a, int slices, hipStream_t stream) {
   static LdsGrant grant;
   constexpr int bytes = BUFS * 16 * (MI + NI) * kBK * 2 + kWaves * (NI * MI < 8 ? NI * MI : 8) * 1024;
   static_assert(bytes <= 160 * 1024, "");
-  const auto kernel = gemm_rows_kernel<MI, NI, BUFS, SCALED, GATED, NT, JOINS, TY>;
+  const auto kernel = gemm_rows_kernel<MI, NI, BUFS, SCALED, GATED, NT, JOINS, TY, ArgsOf<JOINS>>;
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_rows: %s", hipGetErrorString(e));
-  RowsArgs b = a;
-  b.tiles = ceil_div(a.N, (GATED ? 8 : 16) * NI);
+  a.tiles = ceil_div(a.N, (GATED ? 8 : 16) * NI);
   const int cus = rlis_stream_compute_units();
   RLIS_REQUIRE(cus > 0, "gemm_rows: cannot read the device properties");
-  kernel<<<dim3(std::min(b.tiles, cus), slices), kWaves * 64, bytes, stream>>>(b);
+  a.grid = std::min(a.tiles, cus);
+  kernel<<<dim3(a.grid, slices), kWaves * 64, bytes, stream>>>(a);
   return 0;
 }
 
 template <int MI, int NI, int BUFS, bool SCALED, bool GATED, typename TY, bool JOINS = false>
-int launch(const RowsArgs& a, int slices, int nt, hipStream_t stream) {
+int launch(const ArgsOf<JOINS>& a, int slices, int nt, hipStream_t stream) {
   return nt ? launch_form<MI, NI, BUFS, SCALED, GATED, true, JOINS, TY>(a, slices, stream)
             : launch_form<MI, NI, BUFS, SCALED, GATED, false, JOINS, TY>(a, slices, stream);
 }
 
 // out: 0 bfloat16, 1 float32 (slices of k, slice_stride apart), 2 gated
+template <int MI, int NI, int BUFS>
+int form(const RowsJoinArgs& a, int, int slices, int nt, hipStream_t stream) {
+  return launch<MI, NI, BUFS, false, false, float, true>(a, slices, nt, stream);
+}
 template <int MI, int NI, int BUFS>
 int form(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
   if (a.ss) {
@@ -351,7 +366,6 @@ int form(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
     if (out == 1) return launch<MI, NI, BUFS, true, false, float>(a, slices, nt, stream);
     return launch<MI, NI, BUFS, true, true, bf16_t>(a, slices, nt, stream);
   }
-  if (a.join.resid) return launch<MI, NI, BUFS, false, false, float, true>(a, slices, nt, stream);
   if (out == 0) return launch<MI, NI, BUFS, false, false, bf16_t>(a, slices, nt, stream);
   if (out == 1) return launch<MI, NI, BUFS, false, false, float>(a, slices, nt, stream);
   return launch<MI, NI, BUFS, false, true, bf16_t>(a, slices, nt, stream);
@@ -376,7 +390,8 @@ int slices_of(int N, int K) {
   return s;
 }
 
-int dispatch(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
+template <typename Args>
+int dispatch(const Args& a, int out, int slices, int nt, hipStream_t stream) {
   const int ni = row_groups(out == 2 ? 2 * a.N : a.N, slices);
   int rc;
   if (a.T <= 32) {
@@ -416,8 +431,8 @@ RLIS_API int rlis_gemm_bf16_rows(const void* X, const void* W, void* Y, int out,
                "gemm_rows: x or W passes 4 GB");
   RLIS_REQUIRE(!ss || (ss_count > 0 && ss_stride >= ss_count && ss_stride % 4 == 0 && (uintptr_t)ss % 16 == 0),
                "gemm_rows: the sums of squares must be rows on 16-byte boundaries");
-  const RowsArgs a = {(const bf16_t*)X, (const bf16_t*)W, Y, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw,
-                      ldy, slice_stride, ss, ss_count, ss_stride, eps, {}};
+  const RowsArgs a = {(const bf16_t*)X, (const bf16_t*)W, Y, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw, 0,
+                      ldy, slice_stride, ss, ss_count, ss_stride, eps};
   return dispatch(a, out, slices, nt, stream);
 }
 
@@ -449,8 +464,8 @@ RLIS_API int rlis_gemm_bf16_rows_join(const void* X, const void* W, float* parts
   RLIS_REQUIRE(weight_dtype == RLIS_F32 || weight_dtype == RLIS_BF16, "gemm_rows_join: unknown weight dtype %d", weight_dtype);
   RLIS_REQUIRE(ldx * 2 * T < (1LL << 32) && ldw * 2 * N < (1LL << 32) && 4LL * slices * T * N < (1LL << 31),
                "gemm_rows_join: x or W passes 4 GB, or the partial sums 2 GB");
-  RowsArgs a = {(const bf16_t*)X, (const bf16_t*)W, parts, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw,
-                N, (long long)T * N, nullptr, 0, 0, 0.f, {}};
-  a.join = {resid, weight, (bf16_t*)xw, ss, arrivals, ss_stride, weight_dtype == RLIS_F32, round_sum};
+  const RowsJoinArgs a = {{(const bf16_t*)X, (const bf16_t*)W, parts, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw, 0,
+                           N, (long long)T * N, nullptr, 0, 0, 0.f},
+                          {resid, weight, (bf16_t*)xw, ss, arrivals, ss_stride, weight_dtype == RLIS_F32, round_sum}};
   return dispatch(a, 1, slices, nt, stream);
 }
