@@ -293,15 +293,14 @@ __global__ __launch_bounds__(kMaxRuns * 32) void gemm_f32_stream_long_kernel(con
 // a row twice).  The chunks a wave asks for ahead of its last products do not exist; they are asked of a buffer of no
 // bytes, so that the counts of loads under way stay what they are and memory is not asked (the last row read again
 // instead, up to as many bytes as a short tile's own: four tokens of the 1B shape behind prompts of 96, a pass 14,672 ->
-// 14,526 us).  Every other workgroup takes its waves' runs the other way round: rows a power of two apart, walked in
-// step by all workgroups, meet on the same few channels (2048 x 8192 at 4 rows 21.5 -> 17.8 us, 17 with the rows 1 KB
-// further apart; 3072 x 8192 28.0 -> 24.0; 4096 x 14336 41 either way).
+// 14,526 us).  Where the waves' runs start an odd number of 4 KB apart or nearly so (ring_turns), every other workgroup
+// takes them the other way round: walked in step by all workgroups they meet on the same few channels.
 template <int RW, int XW>
 __host__ __device__ constexpr int ring_chunks() {
   return std::min(6, 16384 / ((RW + XW) * 1024));
 }
 template <int RW, int XW, bool GATED>
-__global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int tiles) {
+__global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int tiles, int grid, int turns) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass knows no buffer resources)
   constexpr int PER = RW + XW, CHUNK = PER * 1024, NB = ring_chunks<RW, XW>();
   typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -312,7 +311,7 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
   unsigned char* ring = ring_smem + wave * NB * CHUNK;
   float* red = (float*)(ring_smem + 8 * NB * CHUNK);            // [2][16 runs][64 lanes][4]
   const int chunks = a.run / 64 * 2;                            // of this wave's two runs
-  const int flip = blockIdx.x & 1, turned = flip * (chunks / 2);  // (odd workgroups: the later run first)
+  const int flip = blockIdx.x & turns, turned = flip * (chunks / 2);  // (turns: odd workgroups take the later run first)
   // instruction i brings rows 4 i .. + 3 of a chunk, 16 lanes a row
   uint32_t src[PER];
   const auto place = [&](int row) { return (uint32_t)((r ^ (row & 15)) * 16); };
@@ -324,11 +323,11 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
       src[i] = (uint32_t)weight_row<GATED>(tile, 4 * i + g, 4 * RW, a.N) * ldw * 4 + place(4 * i + g);
   };
   int a_tile = blockIdx.x, a_chunk = 0;
+  constexpr uint32_t kWhole = 0xfffffff0u;   // (x and W end there at most; past the last tile nothing is read)
+  uint32_t a_bytes = kWhole;
   const auto ask = [&](int buf) {
-    // (past the last tile nothing is read)
-    const int bytes = __builtin_amdgcn_readfirstlane(a_tile < tiles ? -1 : 0);
-    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + 2 * wave * a.run), 0, bytes, 0x00027000);
-    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + 2 * wave * a.run), 0, bytes, 0x00027000);
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.X + 2 * wave * a.run), 0, a_bytes, 0x00027000);
+    const auto wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.W + 2 * wave * a.run), 0, a_bytes, 0x00027000);
     unsigned char* base = ring + buf * CHUNK;
     const int at = (a_chunk + turned < chunks ? a_chunk + turned : a_chunk + turned - chunks) * 256;
 #pragma unroll
@@ -340,7 +339,8 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
     }
     if (++a_chunk == chunks) {
       a_chunk = 0;
-      a_tile += gridDim.x;
+      a_tile += grid;
+      a_bytes = a_tile < tiles ? kWhole : 0;
       weight_rows(a_tile);
     }
   };
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(512) void gemm_f32_ring_kernel(const F32Args a, int
   for (int b = 0; b < NB; ++b) ask(b);
   const int w_row = r < 4 * RW ? r : r - 4 * RW, x_row = min(r, 4 * XW - 1);
   int buf = 0, side = 0, turn = 0;
-  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, side ^= 1) {
+  for (int tile = blockIdx.x; tile < tiles; tile += grid, side ^= 1) {
     float* part = red + side * 16 * 256;
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
@@ -543,6 +543,15 @@ __global__ __launch_bounds__(256 * G, 4) void gemm_f32_tiles_kernel(const F32Arg
   }
 }
 
+// Whether odd workgroups of the rings take their waves' runs the other way round (1) or all go in step (0); the same
+// bits.  At 4 rows, us, in step -> turned: 1,536 x 8,192 16.7 -> 15.6, 2,048 x 8,192 20.1 -> 16.1, 4,096 x 8,192 36.9 ->
+// 24.4, 16,384 x 8,192 113 -> 88, 4,096 x 24,576 71.7 -> 61.5, 4,096 x 9,216 27.6 -> 25.3, 3,072 x 7,168 18.4 -> 18.1;
+// 1,024 x 8,192 14.7 -> 15.4, 2,048 x 7,168 14.9 -> 15.9, and 0.97 to 1.06 of the time over every other k in 1,024s up to
+// 32,768 (6,144 x 4,096 19.3 -> 19.8, 3,072 x 16,384 35.9 -> 37.1).
+int ring_turns(int rows_of_w, int K) {
+  return (K % 16384 == 8192 && rows_of_w > 1024) || (K >= 7168 && K <= 9216 && rows_of_w >= 2560);
+}
+
 template <int RW, int XW, bool GATED>
 int launch_ring(const F32Args& a, int cus, hipStream_t stream) {
   static LdsGrant grant;
@@ -551,7 +560,8 @@ int launch_ring(const F32Args& a, int cus, hipStream_t stream) {
   const hipError_t e = grant_lds(grant, (const void*)kernel, bytes);
   RLIS_REQUIRE(e == hipSuccess, "gemm_f32: %s", hipGetErrorString(e));
   const int tiles = ceil_div(a.N, GATED ? 8 : 4 * RW);
-  kernel<<<std::min(tiles, cus), 512, bytes, stream>>>(a, tiles);
+  const int grid = std::min(tiles, cus);
+  kernel<<<grid, 512, bytes, stream>>>(a, tiles, grid, ring_turns(GATED ? 2 * a.N : a.N, a.K));
   return 0;
 }
 
