@@ -356,10 +356,6 @@ int launch(const ArgsOf<JOINS>& a, int slices, int nt, hipStream_t stream) {
 
 // out: 0 bfloat16, 1 float32 (slices of k, slice_stride apart), 2 gated
 template <int MI, int NI, int BUFS>
-int form(const RowsJoinArgs& a, int, int slices, int nt, hipStream_t stream) {
-  return launch<MI, NI, BUFS, false, false, float, true>(a, slices, nt, stream);
-}
-template <int MI, int NI, int BUFS>
 int form(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
   if (a.ss) {
     if (out == 0) return launch<MI, NI, BUFS, true, false, bf16_t>(a, slices, nt, stream);
@@ -390,8 +386,7 @@ int slices_of(int N, int K) {
   return s;
 }
 
-template <typename Args>
-int dispatch(const Args& a, int out, int slices, int nt, hipStream_t stream) {
+int dispatch(const RowsArgs& a, int out, int slices, int nt, hipStream_t stream) {
   const int ni = row_groups(out == 2 ? 2 * a.N : a.N, slices);
   int rc;
   if (a.T <= 32) {
@@ -403,6 +398,16 @@ int dispatch(const Args& a, int out, int slices, int nt, hipStream_t stream) {
   }
   if (rc) return rc;
   RLIS_LAUNCH_CHECK("gemm_rows");
+  return 0;
+}
+
+int dispatch_join(const RowsJoinArgs& a, int slices, int nt, hipStream_t stream) {
+  const int ni = row_groups(a.N, slices);
+  const int rc = ni == 1   ? launch<2, 1, 8, false, false, float, true>(a, slices, nt, stream)
+                 : ni == 2 ? launch<2, 2, 8, false, false, float, true>(a, slices, nt, stream)
+                           : launch<2, 4, 5, false, false, float, true>(a, slices, nt, stream);
+  if (rc) return rc;
+  RLIS_LAUNCH_CHECK("gemm_rows_join");
   return 0;
 }
 
@@ -441,7 +446,7 @@ RLIS_API int rlis_gemm_bf16_rows_join_tiles(int N, int slices) {
   return N > 0 && slices > 0 ? ceil_div(N, 16 * row_groups(N, slices)) : 0;
 }
 
-// resid (T,N) += X (T,K) * W (N,K)^T for 17 to 64 rows over two or four slices of k, the sum of the slices rounded to
+// resid (T,N) += X (T,K) * W (N,K)^T for up to 32 rows over two or four slices of k, the sum of the slices rounded to
 // bfloat16 first with round_sum; xw (T,N) = resid * weight in bfloat16, ss (T, ss_stride) the sums of resid squared over
 // each of rlis_gemm_bf16_rows_join_tiles(N, slices) tiles of columns.  parts: (slices,T,N) float32 of scratch.  arrivals:
 // a counter a tile, all zero before the launch and again after it; launches that overlap in time must not share
@@ -453,7 +458,7 @@ RLIS_API int rlis_gemm_bf16_rows_join(const void* X, const void* W, float* parts
                                       long long ldx, long long ldw, float* resid, const void* weight, int weight_dtype,
                                       int round_sum, void* xw, float* ss, int ss_stride, unsigned* arrivals, int arrival_slots,
                                       int nt, hipStream_t stream) {
-  RLIS_REQUIRE(T > 0 && T <= 64 && N > 0 && N % 8 == 0 && (slices == 2 || slices == 4) && K > 0 && K % (slices * kBK) == 0,
+  RLIS_REQUIRE(T > 0 && T <= 32 && N > 0 && N % 8 == 0 && (slices == 2 || slices == 4) && K > 0 && K % (slices * kBK) == 0,
                "gemm_rows_join: bad sizes T=%d N=%d K=%d slices=%d", T, N, K, slices);
   const int tiles = rlis_gemm_bf16_rows_join_tiles(N, slices);
   RLIS_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 &&
@@ -467,5 +472,5 @@ RLIS_API int rlis_gemm_bf16_rows_join(const void* X, const void* W, float* parts
   const RowsJoinArgs a = {{(const bf16_t*)X, (const bf16_t*)W, parts, T, N, K / slices / kBK, 0, (int)ldx, (int)ldw, 0,
                            N, (long long)T * N, nullptr, 0, 0, 0.f},
                           {resid, weight, (bf16_t*)xw, ss, arrivals, ss_stride, weight_dtype == RLIS_F32, round_sum}};
-  return dispatch(a, 1, slices, nt, stream);
+  return dispatch_join(a, slices, nt, stream);
 }

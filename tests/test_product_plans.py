@@ -58,7 +58,6 @@ def test_partial_sums_in_the_flatter_tile(plan, T, N, K, slices, tile):
     # (in smaller tiles, or uneven, measured 1.03 to 1.15 of the library's time)
     (1280, 8192, 2048, None), (3000, 13824, 2560, None), (1700, 14336, 3072, None), (1152, 20480, 2560, None),
     (1344, 17920, 1536, None), (2304, 16384, 2048, None), (1536, 24576, 3072, None)])
-
 def test_gate_up_of_prompts(plan, T, N, K, taken):
     """gate/up of more than 512 rows: even rounds alone, most in the largest tile."""
     assert plan(T, N, K, 1, 0, 1) == (-1 if taken is None else 16 + taken)
@@ -109,3 +108,33 @@ def test_products_that_write_the_cache_keep_their_side(N, K, most):
     fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] * 4
     sides = [fn(T, N, K, 256) >= 0 for T in range(65, 8193)]
     assert sum(a != b for a, b in zip(sides, sides[1:])) <= most
+
+
+@pytest.fixture(scope="module")
+def refusal():
+    """What an entry point says of arguments that it refuses before it asks the device for anything."""
+    from rust_llm_inference_server_amd.ops import lib as kernels
+    lib = ctypes.CDLL(build.ensure("kernels"))
+    lib.rlis_last_error.restype = ctypes.c_char_p
+
+    def call(name, *args):
+        fn = getattr(lib, name)
+        fn.restype, fn.argtypes = ctypes.c_int, kernels._SIGNATURES[name]
+        assert fn(*args) != 0
+        return lib.rlis_last_error().decode()
+    return call
+
+
+@pytest.mark.parametrize("T,said", [(32, "operand is missing"), (33, "bad sizes"), (64, "bad sizes"), (0, "bad sizes")])
+def test_the_join_in_slices_takes_up_to_32_rows(refusal, T, said):
+    """No step takes it beyond; nothing is compiled for more."""
+    assert said in refusal("rlis_gemm_bf16_rows_join", None, None, None, T, 2048, 8192, 4, 8192, 8192, None, None, 1, 1, None,
+                           None, 64, None, 0, 0, None)
+
+
+@pytest.mark.parametrize("tile", [2, 8, 9, 13, -1])
+def test_products_that_write_the_cache_have_tiles_of_their_own(refusal, tile):
+    """Tiles that the plan of q, k and v never names are refused (the operands are never looked at)."""
+    at = 4096
+    assert f"no tile {tile}" in refusal("rlis_gemm_bf16_tiles_heads", at, at, at, 128, 8, 2, 64, 256, 256, 256, 512, at, at, at, at,
+                                        at, at, 16, tile, None)
