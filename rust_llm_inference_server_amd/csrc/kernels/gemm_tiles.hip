@@ -161,8 +161,8 @@ __device__ __forceinline__ void store_heads(const HeadsTilesArgs& p, const f32x4
           for (int i = 0; i < 4; ++i) {
             // (the product is rounded first, as one that goes through memory is)
             const float x = bf16_to_f32(f32_to_bf16(lo[e + i])), y = bf16_to_f32(f32_to_bf16(hi[e + i]));
-            lo[e + i] = x * c[i] - y * s[i];
-            hi[e + i] = y * c[i] + x * s[i];
+            lo[e + i] = fmaf(x, c[i], -(y * s[i]));
+            hi[e + i] = fmaf(y, c[i], x * s[i]);
           }
         }
       }
@@ -703,7 +703,9 @@ RLIS_API int rlis_gemm_bf16_tiles(const void* X, const void* W, void* Y, int out
 // (T, nh d) holds the query heads as they come, keys go to k_pages (pages, nkv, page_size, d) turned by
 // positions (rotate-half over the whole head, cos and sin (positions, d / 2); null: as they come), values to
 // v_pages (pages, nkv, d, page_size), at slots (below 0: not stored).  d 64, 128 or 256, page_size a power of two.
-// Products are rounded to bfloat16 before they are turned: the bits of rlis_gemm_bf16_tiles and rlis_rope_kv_write.
+// Products are rounded to bfloat16 before they are turned.  Where a tile holds whole heads (weight rows in ds) the bits
+// are those of rlis_gemm_bf16_tiles in the same tile and rlis_rope_kv_write; elsewhere some dims of a head lie in another
+// tile than there and start their walk over k at another stage.
 RLIS_API int rlis_gemm_bf16_tiles_heads(const void* X, const void* W, void* Q, int T, int nh, int nkv, int d, int K,
                                         long long ldx, long long ldw, long long ldq, const float* cos,
                                         const float* sin, const int* positions, const int* slots, void* k_pages,
