@@ -122,10 +122,11 @@ MEMORY_SIDE_CACHE_BYTES = 256 << 20
 @contextlib.contextmanager
 def weights_of(nbytes: int, cache_layers: int = 0, counters: Optional[torch.Tensor] = None):
     """Inside the block, what this thread launches is a model's that holds ``nbytes`` of weights and
-    reads all of them in a step, and that keeps keys and values in ``cache_layers`` layers.  (It moves no
+    reads all of them in a step, and that keeps keys and values in ``cache_layers`` layers.  (Neither moves a
     bit of a result; a captured step keeps what held at its capture.)  ``counters``: int32 zeros on the device
-    that belong to the step's runner, whose launches do not overlap in time; products of 17 to 32 rows in slices of
-    k join the residual (``linear_join_norm``) where there are some."""
+    that belong to the step's runner, whose launches do not overlap in time; where there are some, products of 17 to
+    32 rows in slices of k join the residual (``linear_join_norm``), which rounds in another order than the norm kernel
+    does: the residual times the norm's weight to bfloat16, 1 / rms behind the next product's sums."""
     old = _streamed.nt, _streamed.cache_layers, _streamed.counters
     _streamed.nt, _streamed.cache_layers, _streamed.counters = \
         int(nbytes > MEMORY_SIDE_CACHE_BYTES), cache_layers, counters
@@ -1168,9 +1169,9 @@ def linear_join_norm(product: PendingProduct, resid: torch.Tensor, norm_weight: 
                      round_sum: bool) -> Tuple[torch.Tensor, torch.Tensor]:
     """Runs the product with what follows it inside: ``resid += x @ w.T`` (the product rounded
     to bfloat16 first with ``round_sum``, as a bfloat16 model's block output is), in place.
-    Returns ``(xw, ss)``: ``resid * norm_weight`` in bfloat16 and, ``(16, tiles)`` float32, per
-    row and tile of columns the sum of ``resid ** 2`` (rows from ``T`` on are not meant), for
-    ``linear_scaled``."""
+    Returns ``(xw, ss)``: ``resid * norm_weight`` in bfloat16 and, float32, per row and tile of
+    columns the sum of ``resid ** 2``, for ``linear_scaled``; ``ss`` has ``T`` rows of products in
+    slices of k, else 16 or 32 (rows from ``T`` on are not meant)."""
     x, w = product.x, product.w
     T, K = x.shape
     N = w.shape[0]
