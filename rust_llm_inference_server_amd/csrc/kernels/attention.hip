@@ -915,10 +915,18 @@ RLIS_API int rlis_attn_decode(const void* q, int dtype, long long q_stride, void
   // a KV head together -> this: 32 heads of 64 on 8, 3 requests of 25 keys 7.7 -> 5.8, 4 of 100 9.4 -> 7.5, 4 of
   // 1,000 33 -> 24, 16 of 200 10.7 -> 9.9; 24 of 128 on 8, 4 of 1,000 68 -> 39; 8 of 256 on one, 1 of 600 83 -> 36.
   // Past one a unit the shared reads are ahead: 32 of 64 on 8, 64 of 200 18.4, two heads 23.3, one 38.6.
+  // float32 heads of up to 128 dims go in twos from five workgroups to eight units on: there one by one, each with
+  // its own reads of the KV head's keys, takes up to 1.7 of two's time and 1.3 of all together's (8 requests of 1,024,
+  // one, two, four: 32 of 64 on 8 31.7, 19.6, 25.5, of 128 57.1, 33.6, 42.6; 40 keys of 64 dims 4.8, 5.2, 6.7), below
+  // 0.85 to 1.06 (32 heads at 1,024 keys 1.05 to 1.23) and nowhere more than all together.  bfloat16 heads and float32
+  // heads of 256 dims stay ahead one by one (32 of 72 on 8, 8 of 1,024 21.3 against 28.8; 8 of 256 on one, 24 of 800
+  // 53.0 against 58.6).
   const int g = nh / nkv;
   const long long units = rlis_stream_compute_units();
   int heads = 1;
-  while (heads < 8 && heads < g && (long long)nkv * ceil_div(g, heads) * S * splits > units) heads *= 2;
+  const auto groups = [&](int n) { return (long long)nkv * ceil_div(g, n) * S * splits; };
+  if (dtype == RLIS_F32 && d <= 128 && g > 1 && groups(1) * 8 > units * 5) heads = 2;
+  while (heads < 8 && heads < g && groups(heads) > units) heads *= 2;
   int rc = 0;
 #define LAUNCH(TX, G)                                                                            \
   rc = launch_decode<TX, G>(q, q_stride, out, out_stride, part_ml, part_acc, k_pages, v_pages,   \
