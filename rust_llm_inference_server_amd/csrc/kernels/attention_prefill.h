@@ -255,19 +255,19 @@ void WHOLE_KERNEL_NAME(
           for (int v = 0; v < 16; ++v) o[db][v] *= corr;
       }
       bf16x8 p[NB * 2];
-      float sum = 0.f;
+      float sum[2] = {0.f, 0.f};
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int v = 0; v < 16; v += 2) {
           const float a = __builtin_amdgcn_exp2f(fmaf(s[nb][v], in_exp, -m_use));
           const float b = __builtin_amdgcn_exp2f(fmaf(s[nb][v + 1], in_exp, -m_use));
-          const Bf16Pair ab = {(__bf16)a, (__bf16)b};
-          sum = __builtin_amdgcn_fdot2_f32_bf16(ab, Bf16Pair{(__bf16)1.f, (__bf16)1.f}, sum, false);
-          p[nb * 2 + v / 8][v % 8] = ab[0];
-          p[nb * 2 + v / 8][v % 8 + 1] = ab[1];
+          sum[0] += a;
+          sum[1] += b;
+          p[nb * 2 + v / 8][v % 8] = (__bf16)a;
+          p[nb * 2 + v / 8][v % 8 + 1] = (__bf16)b;
         }
-      l_run += sum;                                    // (the two lanes of a query are added at the end)
+      l_run += sum[0] + sum[1];                                  // (the two lanes of a query are added at the end)
 #pragma unroll
       for (int st = 0; st < NB * 2; ++st)
 #pragma unroll
