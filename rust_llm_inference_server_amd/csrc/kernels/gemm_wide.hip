@@ -29,10 +29,7 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
   static_assert(!(JOIN && GATED), "a product that joins the residual has no gate");
   constexpr int kTileBytes = TR * kStreamItem * 2;
   constexpr int kRed = TG * 256;                           // floats a wave hands over per tile
-  asm volatile("" ::"s"(X), "s"(W), "s"(Y), "s"(sh.T), "s"(sh.N), "s"(sh.K), "s"(sh.ldx), "s"(sh.ldw), "s"(sh.ldy),
-               "s"(sh.num_tiles), "s"(sh.nwaves), "s"(sh.groups));   // (in one go, see gemm_bf16_stream_kernel)
-  const int tid = threadIdx.x, lane = tid % 64, nwaves = sh.nwaves;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, nwaves = blockDim.x / 64;
   unsigned char* tile_s = wide_smem + wave * kTileBytes;
   float* red = (float*)(wide_smem + nwaves * kTileBytes);  // [2][nwaves][TG][16 tokens][16 rows]
   float* inv_s = red + 2 * nwaves * kRed;                  // [TG * 16]: the rows' scales
@@ -95,7 +92,7 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
   // not for the second tile as well.
   if constexpr (AHEAD == 2) {
     asm volatile("" ::: "memory");
-    RLIS_WIDE_LOAD_TILE(a1, tile + sh.groups);
+    RLIS_WIDE_LOAD_TILE(a1, tile + (int)gridDim.x);
   }
 
   // SCALED: the rows' scales come as partial sums of squares, scale_count a token.  A wave
@@ -130,7 +127,7 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
         *(uint4*)(tile_s + r * (kStreamItem * 2) + ((l32 ^ r) * 16)) = A_[p];
       }
     }
-    RLIS_WIDE_LOAD_TILE(A_, tile + AHEAD * sh.groups);   /* on its way during the arithmetic */
+    RLIS_WIDE_LOAD_TILE(A_, tile + AHEAD * (int)gridDim.x);   /* on its way during the arithmetic */
     if (has_item) {
       wave_lds_fence();
 #pragma unroll
@@ -185,7 +182,7 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
     __syncthreads();
     // 256 threads store a group of 16 tokens: thread (token t, row i); the groups are dealt
     // out to the workgroup's sets of 256 threads.
-    const int sets = nwaves / 4;
+    const int sets = blockDim.x / 256;
     for (int g = tid < sets * 256 ? tid / 256 : TG; g < TG; g += sets) {
       const int t = (tid % 256) / 16, i = tid % 16;
       const int tok = 16 * g + t;
@@ -235,11 +232,11 @@ __global__ __launch_bounds__(AHEAD == 2 ? 512 : (TG == 2 ? 768 : 512)) void gemm
   for (;;) {
     if (tile >= sh.num_tiles) break;
     one_tile(a0);
-    tile += sh.groups;
+    tile += gridDim.x;
     if constexpr (AHEAD == 2) {
       if (tile >= sh.num_tiles) break;
       one_tile(a1);
-      tile += sh.groups;
+      tile += gridDim.x;
     }
   }
 #undef RLIS_WIDE_LOAD_TILE
@@ -271,8 +268,6 @@ int launch_form(const void* X, const void* W, void* Y, StreamShape sh, const Str
   sh.num_tiles = (int)tiles;
   const long long cap = (long long)num_cus * per_cu;
   const long long groups = tiles < cap ? tiles : cap;
-  sh.nwaves = nwaves;
-  sh.groups = (int)groups;
   gemm_bf16_stream_wide_kernel<TC, GATED, TR, MODE, TG, AHEAD, NT>
       <<<(int)groups, nwaves * 64, smem, stream>>>((const bf16_t*)X, (const bf16_t*)W, (TC*)Y, sh,
                                                    nm);
@@ -331,7 +326,7 @@ int rlis_launch_stream_wide(const char* name, int mode, const void* X, const voi
   sh.T = T; sh.N = N; sh.K = K; sh.ldx = ldx; sh.ldw = ldw; sh.ldy = ldy;
   sh.part_stride = 0;
   sh.num_slices = 1;
-  sh.num_tiles = sh.nwaves = sh.groups = 0;
+  sh.num_tiles = 0;
   const int nwaves = max(4, K / kStreamItem);
   int rc = 1;
   if (mode == kStreamJoin) {
