@@ -650,7 +650,8 @@ __device__ __forceinline__ void load8(const bf16_t* p, float (&v)[8]) {
 }
 
 template <typename TC, bool GATED, int TR /* weight rows per tile: 16, 12 or 8 */, int MODE,
-          int IPW /* k items per wave: 1 or 4 */, bool PACK /* see below */, bool NT /* load_weights */>
+          int IPW /* k items per wave: 1 or 4 */, bool PACK /* see below */, bool NT /* load_weights */,
+          bool ONE /* no workgroup has a second tile */>
 __global__ __launch_bounds__(IPW == 1 ? 1024 : 512) void gemm_bf16_stream_kernel(const bf16_t* __restrict__ X,
                                                                 const bf16_t* __restrict__ W,
                                                                 TC* __restrict__ Y,
@@ -719,9 +720,13 @@ __global__ __launch_bounds__(IPW == 1 ? 1024 : 512) void gemm_bf16_stream_kernel
   // half of a tile's rows are the gate rows of consecutive columns and the second half their
   // up rows, N further down.  Everything but `half` and the lane's k is uniform over the wave.
   constexpr int cols_per_tile = GATED ? TR / 2 : TR;
-  // Tiles of 12 and 8 rows: all addresses, then the loads, in a row (q/k/v 6.36 -> 5.98 us at 8 rows of the 1B shape); with
-  // eight loads or more the first ones leave while the addresses of the others are made (gate/up 14.1 against 14.7).
-  constexpr bool kRowsFirst = !GATED && IPW == 1 && TR < 16;
+  // Tiles of 12 and 8 rows, one a workgroup: all addresses, then the loads, in a row (scaled, 1 / 8 / 16 rows, us: 3,072 x
+  // 2,048 5.92 / 6.43 / 7.08 -> 5.76 / 5.98 / 6.39, 2,048 x 2,048 4.84 / 5.47 / 6.15 -> 4.73 / 5.02 / 5.73).  With several
+  // tiles, whose workgroups have 12 and 16 waves or walk far, and with eight loads or more, the first ones leave while the
+  // addresses of the others are made (6,144 x 4,096 12.0 / 11.9 / 12.9 against 12.7 / 12.8 / 13.5; 128,256 x 2,048 85.5 /
+  // 92.7 / 97.3 against 86.0 / 94.0 / 98.4; gate/up 14.1 against 14.7).
+  static_assert(!ONE || (!GATED && IPW == 1 && TR < 16), "one tile a workgroup: tiles of 12 and 8 rows");
+  constexpr bool kRowsFirst = ONE;
 #define RLIS_STREAM_LOAD_TILE(a, tile_)                                                         \
   {                                                                                             \
     const int tl_ = (tile_);                                                                    \
@@ -1072,18 +1077,28 @@ static int stream_slices(int K) {
 // scaled form.
 constexpr int kStreamNormMaxK = kStreamMaxWaves * kStreamItem;
 
-template <typename TC, bool GATED, int TR, int MODE, int IPW, bool PACK, bool NT>
-static int launch_stream_form(const void* X, const void* W, void* Y, StreamShape sh,
-                              const StreamNorm& nm, int nwaves, int num_cus, hipStream_t stream) {
-  constexpr int kTileBytes = IPW * (MODE == kStreamNorm ? kStreamTileBytes : TR * kStreamItem * 2);
+template <typename TC, bool GATED, int TR, int MODE, int IPW, bool PACK, bool NT, bool ONE>
+static int launch_stream_form(const void* X, const void* W, void* Y, const StreamShape& sh,
+                              const StreamNorm& nm, size_t smem, hipStream_t stream) {
   static LdsGrant lds_raised;
   {
     hipError_t e = grant_lds(
-        lds_raised, (const void*)gemm_bf16_stream_kernel<TC, GATED, TR, MODE, IPW, PACK, NT>,
-        (IPW == 1 ? kStreamMaxWaves : 2 * kStreamMaxWaves / IPW) * (kTileBytes + 2048));
+        lds_raised, (const void*)gemm_bf16_stream_kernel<TC, GATED, TR, MODE, IPW, PACK, NT, ONE>,
+        (IPW == 1 ? kStreamMaxWaves : 2 * kStreamMaxWaves / IPW) * (int)(smem / sh.nwaves));
     RLIS_REQUIRE(e == hipSuccess, "gemm_bf16_stream: cannot raise the LDS limit: %s",
                  hipGetErrorString(e));
   }
+  gemm_bf16_stream_kernel<TC, GATED, TR, MODE, IPW, PACK, NT, ONE>
+      <<<sh.groups * sh.num_slices, sh.nwaves * 64, smem, stream>>>(
+          (const bf16_t*)X, (const bf16_t*)W, (TC*)Y, sh, nm);
+  return 0;
+}
+
+template <typename TC, bool GATED, int TR, int MODE, int IPW = 1, bool PACK = false>
+static int launch_stream_tiles(const void* X, const void* W, void* Y, StreamShape sh,
+                               const StreamNorm& nm, int nwaves, int num_cus,
+                               hipStream_t stream) {
+  constexpr int kTileBytes = IPW * (MODE == kStreamNorm ? kStreamTileBytes : TR * kStreamItem * 2);
   const size_t smem = (size_t)nwaves * (kTileBytes + 2048);
   const int per_cu = max(1, (int)((160 * 1024) / smem));
   const long long tiles = ceil_div_ll(sh.N, GATED ? TR / 2 : TR);
@@ -1094,18 +1109,13 @@ static int launch_stream_form(const void* X, const void* W, void* Y, StreamShape
   if (groups > cap) groups = cap;
   sh.nwaves = nwaves;
   sh.groups = (int)groups;
-  gemm_bf16_stream_kernel<TC, GATED, TR, MODE, IPW, PACK, NT>
-      <<<(int)(groups * sh.num_slices), nwaves * 64, smem, stream>>>(
-          (const bf16_t*)X, (const bf16_t*)W, (TC*)Y, sh, nm);
-  return 0;
-}
-
-template <typename TC, bool GATED, int TR, int MODE, int IPW = 1, bool PACK = false>
-static int launch_stream_tiles(const void* X, const void* W, void* Y, const StreamShape& sh,
-                               const StreamNorm& nm, int nwaves, int num_cus,
-                               hipStream_t stream) {
-  return nm.nt ? launch_stream_form<TC, GATED, TR, MODE, IPW, PACK, true>(X, W, Y, sh, nm, nwaves, num_cus, stream)
-               : launch_stream_form<TC, GATED, TR, MODE, IPW, PACK, false>(X, W, Y, sh, nm, nwaves, num_cus, stream);
+  if constexpr (!GATED && IPW == 1 && TR < 16) {
+    if (groups == tiles)
+      return nm.nt ? launch_stream_form<TC, GATED, TR, MODE, IPW, PACK, true, true>(X, W, Y, sh, nm, smem, stream)
+                   : launch_stream_form<TC, GATED, TR, MODE, IPW, PACK, false, true>(X, W, Y, sh, nm, smem, stream);
+  }
+  return nm.nt ? launch_stream_form<TC, GATED, TR, MODE, IPW, PACK, true, false>(X, W, Y, sh, nm, smem, stream)
+               : launch_stream_form<TC, GATED, TR, MODE, IPW, PACK, false, false>(X, W, Y, sh, nm, smem, stream);
 }
 
 int rlis_stream_compute_units() {
