@@ -46,10 +46,12 @@ constexpr int kHalfBytes = 16 * D * 2;             // of K, and of V
 constexpr int kTileBytes = 2 * kWholeHalves * kHalfBytes;
 constexpr int whole_lds(int groups) { return groups * 2 * kTileBytes; }
 
-template <int N>
-__device__ __forceinline__ void whole_wait_loads() {
+// In front of the barrier behind which a tile's place is filled anew: this wave's own part of the next tile has come, and
+// its reads of the last one have returned (the barrier is an asm statement, which does not hold back the products that
+// would otherwise wait for them).
+__device__ __forceinline__ void whole_wait_tile() {
   asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((N & 15) | 7 << 4 | 15 << 8 | (N >> 4) << 14);
+  __builtin_amdgcn_s_waitcnt(0 | 7 << 4 | 0 << 8);     // vmcnt(0) lgkmcnt(0)
   asm volatile("" ::: "memory");
 }
 }  // namespace
@@ -204,7 +206,7 @@ void WHOLE_KERNEL_NAME(
   for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks].v));
   for (int t = group; t < tiles + group; t += G) {
     const int k0 = kt0 + t * kWholeTile;
-    whole_wait_loads<0>();
+    whole_wait_tile();
     asm volatile("s_barrier" ::: "memory");            // the tile is whole, the one before it has been read
     if (t + G < tiles) ask();
     if (wave_q < n_new && t < tiles && k0 <= wave_last) {
