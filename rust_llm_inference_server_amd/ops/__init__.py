@@ -1776,6 +1776,8 @@ def paged_attention(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
         planner = AttentionPlanner(nh, nkv, d, matrix=qkv.dtype == torch.bfloat16,
                                    singles_apart=force is None and SPLIT_MIXED_ATTENTION
                                    and DECODE_ATTENTION != "vector", span=span)
+        # (as a mixer of such layers says: the same tiles, hence the same bits, as with its plan)
+        planner.whole_heads = not (win or span or slopes_ptr is not None or shaped)
         plan = _plan_now(step, planner, qkv.device)
 
     def decode(S: int, depth: int, matrix: bool) -> None:
