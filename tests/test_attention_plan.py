@@ -135,3 +135,67 @@ def test_layouts_the_matrix_kernels_do_not_take_plan_no_tiles():
     plan = wide_group.plan(lengths([5, 0], [1, 40]))
     assert plan.values["num_decode"] == 0 and plan.values["num_units64"] == 2
     assert plan.values["tile_row0"] == 0
+
+
+WHOLE = ("units64", "units128", "units128x2")
+
+
+def whole_planner(nh, nkv, d, **more):
+    planner = ap.AttentionPlanner(nh, nkv, d, **more)
+    planner.whole_heads = True
+    return planner
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(32, 8, 64), (24, 8, 128), (6, 2, 32)])
+@pytest.mark.parametrize("page", [8, 16, 64])
+def test_tiles_of_whole_heads_are_listed_once_per_run_and_alike_among_neighbours(nh, nkv, d, page):
+    """Layers whose queries see every earlier key: every tile of every portion once per run, in one list, longest first;
+    tiles of 128 alone where the kernel for whole heads takes them (heads of 64 and 128, pages from 16 on); and the same
+    for a sequence alone."""
+    planner = whole_planner(nh, nkv, d)
+    cached, new = [10, 300, 0, 40, 3000, 100, 7000], [1, 1, 300, 70, 200, 5000, 33]
+    plan = planner.plan(lengths(cached, new, page))
+    runs, seen = plan.arrays["seq_runs"].tolist(), {}
+    for name in WHOLE:
+        units = units_of(plan, name)
+        assert len(units) == plan.values["num_" + name]
+        tile, work = 64 if name == "units64" else 128, []
+        for s, qb, r, nr in units:
+            assert s >= 2 and nr == runs[s] and qb % tile == 0 and qb < new[s]
+            assert planner.tile_queries(cached[s], new[s], page) == tile
+            assert (planner.key_groups(new[s], cached[s] + new[s], nr, page) == 2) == (name == "units128x2") or tile == 64
+            seen.setdefault((s, qb, tile), []).append(r)
+            work.append(-(-(cached[s] + min(new[s], qb + tile)) // nr))
+        assert work == sorted(work, reverse=True)
+    for s in range(2, len(new)):
+        tile = planner.tile_queries(cached[s], new[s], page)
+        for qb in range(0, new[s], tile):
+            assert sorted(seen.pop((s, qb, tile))) == list(range(runs[s]))
+        one = planner.plan(lengths([cached[s]], [new[s]], page))
+        assert one.arrays["seq_runs"].tolist() == [runs[s]]
+        for name in WHOLE:
+            mine = sorted(u[1:] for u in units_of(plan, name) if u[0] == s)
+            assert mine == sorted(u[1:] for u in units_of(one, name))
+    assert not seen
+    taken = d in ap.WHOLE_HEADS and page >= 16
+    assert (plan.values["num_units64"] == 0) == taken
+    assert (plan.values["num_units128x2"] > 0) == taken
+    assert planner.key() != ap.AttentionPlanner(nh, nkv, d).key()
+
+
+def test_keys_are_shared_by_two_groups_of_waves_where_a_sequence_makes_few_workgroups():
+    """Both sides of the rule: workgroups (tiles x heads x runs), positions, head size, page, chunks."""
+    for d, most in ((64, 512), (128, 256)):
+        planner = whole_planner(32, 8, d)
+        tiles = most // 32
+        assert planner.key_groups(128 * tiles, 4096, 1, 16) == 2
+        assert planner.key_groups(128 * tiles + 1, 4096, 1, 16) == 1
+        assert planner.key_groups(128, 4096, tiles, 16) == 2 and planner.key_groups(128, 4096, tiles + 1, 16) == 1
+        assert planner.key_groups(100, 256, 1, 16) == 2 and planner.key_groups(100, 255, 1, 16) == 1
+        assert planner.key_groups(128, 4096, 1, 8) == 1
+        assert planner.tile_queries(0, 2, 16) == 128 and planner.tile_queries(0, 2, 8) == 64
+        assert ap.AttentionPlanner(32, 8, d).key_groups(128, 4096, 1, 16) == 1
+        chunked = whole_planner(32, 8, d, span=512)
+        assert chunked.key_groups(128, 4096, 1, 16) == 1 and chunked.tile_queries(0, 2, 16) == 64
+    assert whole_planner(32, 8, 96).key_groups(128, 4096, 1, 16) == 1
+    assert whole_planner(32, 8, 96).tile_queries(0, 2, 16) == 64
