@@ -17,20 +17,23 @@
 // G groups of four waves take a workgroup's tiles of keys in turn, each with LDS of its own, and the first adds up: a
 // walk of half the length where few workgroups leave the units to it (ops/attention_plan.py says where).
 //
-// The denominator is the sum of the probabilities as the second product takes them, rounded (one instruction for two):
-// what rounding did to a large one cancels.  Error against 64 bits, of the result's norm, form with two blocks of 16
-// queries a wave -> this: 1,024 tokens at head size 64 1.985e-3 -> 1.977e-3, 464 on 1,000 at 128 2.221e-3 -> 2.219e-3,
-// scores six times as wide 1.686e-3 -> 1.685e-3.  (A maximum that follows the true one only by steps of 2^8 spares the
-// rescaling and 3 to 10 % of the time, but puts the largest probabilities anywhere between powers of two: 5 % more error.)
+// The denominator is the float32 sum of the float32 probabilities, as in the other form: the sum of the rounded ones, as the
+// second product takes them, is one instruction for two and no faster (8,192 tokens of 32 heads of 128 549 us either way,
+// 2,048 of 32 heads of 64 30.7), and a row whose probabilities round one way is off by up to 2^-8 with it.  Error against 64
+// bits, of the result's norm, other form -> this: 1,024 tokens at head size 64 2.009e-3 -> 1.992e-3, 464 on 2,000 at 128
+// 2.230e-3 -> 2.196e-3, scores six times as wide 1.682e-3 -> 1.670e-3; where the other form has blocks of 16 queries and tiles
+// of 32 keys as before, 8,192 tokens 2.061e-3 -> 2.068e-3 (84 inputs: 0.977 to 1.004 times as much, the worst row 0.88 to
+// 1.06).  (A maximum that follows the true one only by steps of 2^8 spares the rescaling and 3 to 10 % of the time, but puts
+// the largest probabilities anywhere between powers of two: 5 % more error.)
 //
-// What bounds it is the vector unit beside the matrix cores: some 190 instructions and 33 exponentials a wave and tile at
-// head size 128, against 32 products; both are busy half of the time (counters), and a loop that issues the next tile's
-// products between this one's exponentials is slower (8,192 tokens of 32 heads of 128 595 us for 545).  Tiles of 32 keys
-// 598, three places 709 (one workgroup a unit).
+// What bounds it is the vector unit beside the matrix cores: 210 instructions and 33 exponentials a wave and tile at head size
+// 128, against 32 products; the vector unit is busy 48 % of 8,192 tokens' time and the matrix cores 40 % (counters; at head
+// size 64, 2,048 tokens, 60 and 23 %), and a loop that issues the next tile's products between this one's exponentials is
+// slower (8,192 tokens of 32 heads of 128 595 us for 545).  Tiles of 32 keys 598, three places 709 (one workgroup a unit).
 //
-// MI355X, us, 64 queries -> 128 in blocks of 16 -> this: 32 heads of 128, 8,192 tokens 867 -> 703 -> 536 (1.03 PFLOP/s),
-// 2,048 on 30,000 1,616 -> 1,263 -> 972, 512 on 8,192 134 -> 118 -> 94, 24 heads, 464 on 2,000 50.7 -> 58.2 -> 39; 32 heads of
-// 64, 2,048 tokens 45.3 -> 55.9 -> 31, 512 12.7 -> 18.4 -> 10.0, 8,192 426 -> 398 -> 307.
+// MI355X, us, the other form in the tiles that it took -> this, in turn: 32 heads of 128, 8,192 tokens 699 -> 549 (1.0 PFLOP/s),
+// 2,048 on 30,000 1,250 -> 993, 512 on 8,192 116 -> 90, 24 heads, 464 on 2,000 49.0 -> 34.7; 32 heads of 64, 2,048 tokens
+// 42.3 -> 30.6, 512 12.2 -> 9.3, 8,192 409 -> 317.
 #pragma once
 
 #if RLIS_HEAD_DIM == 64 || RLIS_HEAD_DIM == 128
@@ -131,7 +134,7 @@ void WHOLE_KERNEL_NAME(
   int ids = table[min(page_base + lane, last_page)], ids_next = table[min(page_base + 64 + lane, last_page)];
   const auto ask = [&]() {
     if ((min(a_key + kWholeTile - 1, khi - 1) >> page_shift) - page_base >= 64) {
-      // (a tile of 64 keys in pages of 16 holds four: ids move on by 60 so that none is split)
+      // (by the page that the tile starts in: all 64, or, where a run starts inside pages of 64 and more, 63 of them)
       const int by = (a_key >> page_shift) - page_base;
       if (by >= 64) {
         ids = ids_next;

@@ -584,10 +584,10 @@ constexpr TileForm kLibraryForms[] = {{256, 256, 0.985f}, {256, 128, 0.563f}, {1
 //            128 x 256 where it is full (334 products of 16 shapes at 1,024 to 8,192 rows: 220 taken, up to 1.02, 0.92 on
 //            average, 0.67 where the library has a broken round more; the smaller tiles up to 1.15; uneven rounds up to 1.12, 640 and 768 rows 1.05 to 1.14).  Where tiles of
 //            256 x 256 waste less than a tenth of their rounds, over a k of up to 5,120 and from 513 rows on (the product
-//            alone, us: 28,672 x 4,096 at 2,304 / 4,096 / 8,192 rows 411 -> 383, 705 -> 656, 1,406 -> 1,295; 22,016 x
-//            4,096 at 8,192 1,223 -> 1,015; 37,888 x 3,584 at 1,280 / 2,048 385 -> 256, 547 -> 408; 27,648 x 5,120 at
-//            4,096 1,053 -> 810; 16,384 x 2,048 and 3,072 at 1,000 66 -> 55, 94 -> 84: 37 products 0.65 to 0.95; with up to a
-//            quarter wasted 0.65 to 1.03, 57,344 x 8,192 0.94 to 1.0).
+//            alone, us: 28,672 x 4,096 at 2,304 / 4,096 / 8,192 rows 402 -> 393, 691 -> 674, 1,368 -> 1,326; 22,016 x
+//            4,096 at 8,192 1,211 -> 1,037; 37,888 x 3,584 at 1,280 / 2,048 386 -> 255, 544 -> 417; 27,648 x 5,120 at
+//            4,096 1,046 -> 819; 16,384 x 2,048 and 3,072 at 1,000 68 -> 59, 94 -> 85: 110 products 0.63 to 1.0, those of
+//            24,576 x 4,096 and 36,864 x 4,608 the closest, 0.96 to 1.0).
 RLIS_API int rlis_gemm_bf16_tiles_plan(int T, int N, int K, int gated, int partials, int slices, int units) {
   if (T <= 0 || N <= 0 || K <= 0 || units <= 0) return -1;
   float least = 0.f;

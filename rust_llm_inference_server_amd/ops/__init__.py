@@ -1181,7 +1181,9 @@ def linear_join_norm(product: PendingProduct, resid: torch.Tensor, norm_weight: 
                           f"rows have {N}")
     # 17 to 32 rows in slices of k wherever that kernel has them, also where the streaming kernel could (every one of its
     # workgroups reads all of x: output of the 3B shape at 27 rows 11.4 -> 7.3 us; decode steps, 27 requests of the 3B shape
-    # 2.773 -> 2.662 ms, 18 2.263 -> 2.188, 24 / 32 of the 1B shape 1.014 / 1.081 -> 0.963 / 1.020)
+    # 2.773 -> 2.662 ms, 18 2.263 -> 2.188, 24 / 32 of the 1B shape 1.014 / 1.081 -> 0.963 / 1.020.  At 17 to 22 rows the join
+    # alone is 2 to 12 % behind, 2,048 x 2,048 at 20 rows 7.45 -> 7.76 us, and with gate/up behind it, which has fewer sums
+    # of squares to add, 2.7 us ahead; so at all widths over 1,024)
     slices = _rows_join_slices(x, w) if T > STREAM_MAX_ROWS and resid.data_ptr() % 16 == 0 \
         and (not _streams_in_one_slice(x, w) or N > 1024 or _streamed.nt) else 0
     if slices:

@@ -30,15 +30,17 @@ from ..stepplan import HostPlan, StepLengths, StepPlanner
 DECODE_PART_KEYS = 1024
 DECODE_MAX_PARTS = 16
 PREFILL_TILE = 64     # new tokens per workgroup of the matrix-core prefill attention
-WIDE_TILE = 128       # ... of its form with two query blocks per wave
+WIDE_TILE = 128       # ... of its form with two query blocks per wave, and of the kernel for whole heads
 # Tiles of 128 queries of whole heads of these sizes (attention_prefill.h) are ahead of tiles of 64 at every length (us, 64
-# -> 128: 1B shape 63 to 190 new tokens 8.2 -> 6.6, 512 12.6 -> 10.0, 2,048 45 -> 31, 100 on 300 cached 11.5 -> 9.5; 3B
-# shape 1,024 28.7 -> 22.5, 464 on 2,000 50.7 -> 39).
+# -> 128: 1B shape 2 new tokens 4.7 -> 3.7, on 1,000 cached 18.8 -> 12.5, 17 on 8,000 23.8 -> 20.1, 512 12.2 -> 9.3, 2,048 42
+# -> 31; 3B shape 1,024 31.8 -> 24.7, 464 on 2,000 49 -> 34.7; one portion of 2 to 100 tokens on 0 to 8,000 0.64 to 0.87,
+# batches of 8, 32 and 63 portions of 2 to 64 tokens 0.63 to 0.99, but 63 of 2 to 17 tokens on 500 of 24 heads of 128
+# 1.04 to 1.06: a rule on a sequence's own lengths does not see the others).
 WHOLE_HEADS = (64, 128)
 # Their keys are walked by two groups of waves in turn where a sequence makes at most this many workgroups, by head size,
-# and has this many positions (us, one group -> two: heads of 64, 16 x 32 workgroups 37.5 -> 31, 8 x 32 19.4 -> 15.7, 4 x 32 x 6
-# runs 62 -> 61, 64 x 32 307 -> 309, three prompts of up to 190 tokens 6.6 -> 6.8; heads of 128, 8 x 24 26.8 -> 22.3, 4 x
-# 24 x 2 runs 44.5 -> 39.2, 4 x 32 x 4 runs 94 -> 98, 16 x 32 54.7 -> 57, 64 x 32 536 -> 567).
+# and has this many positions (us, one group -> two: heads of 64, 16 x 32 workgroups 36.6 -> 31.3, 8 x 32 19.6 -> 16.9, 4 x 32 x 6
+# runs 58.3 -> 57.0, 64 x 32 314 -> 320, three prompts of up to 190 tokens 5.85 -> 6.23; heads of 128, 8 x 24 28.3 -> 24.3, 4 x
+# 24 x 2 runs 39.6 -> 34.4, 4 x 32 x 4 runs 88.3 -> 93.1, 16 x 32 53.0 -> 57.8, 64 x 32 547 -> 584).
 SHARED_KEYS_MAX_GROUPS = {64: 512, 128: 256}
 SHARED_KEYS_MIN_CONTEXT = 256
 # Otherwise a sequence takes tiles of 128 queries when they make this many workgroups (tiles x heads; 5/3
@@ -167,7 +169,8 @@ class AttentionPlanner(StepPlanner):
         if PREFILL_SPLIT_UNITS <= 0 or groups > PREFILL_SPLIT_UNITS:
             return 1
         # resident workgroups per compute unit: 4 up to head size 64, 3 with tiles of 128
-        # queries, 2 beyond
+        # queries, 2 beyond (of the general form; the kernel for whole heads has 4 and 2, half of
+        # that where two groups of waves share keys, and takes these numbers as they are)
         resident = 2 if self.d > 64 else (3 if tile == WIDE_TILE else 4)
         return max(1, min(PREFILL_SPLIT_UNITS * resident // groups,
                           (cached + new) // PREFILL_SPLIT_MIN_KEYS, PREFILL_MAX_RUNS))
